@@ -144,32 +144,46 @@ struct Plan {
   // point is shared inside the patch
   bool chains = false;
   std::vector<int> uncovered;         // chains: points (caller numbering) of no element of the phase lists
+  // chain plans: the patch whose bottom GLL row is this patch's top row, point by point (-1: none)
+  std::vector<int> above;
   // chains: per device position and GLL point, whether the chain kernel's update of that point is the first of
   // the step (the earliest colour, in launch order, of the patches that contain the point)
   std::vector<uint8_t> first;
 };
 
-// whether elements elems[k0..k1) form a chain (see Plan::chains)
-bool is_chain(const std::vector<int>& ibool, const std::vector<int>& elems, int k0, int k1) {
-  std::vector<int> pts;
-  for (int k = k0; k < k1; k++) {
-    const int* a = ibool.data() + (size_t)elems[k] * NGLL2;
-    if (k + 1 < k1) {
-      const int* b = ibool.data() + (size_t)elems[k + 1] * NGLL2;
-      for (int j = 0; j < NGLL; j++)
-        if (a[j * NGLL + NGLL - 1] != b[j * NGLL]) return false;
-    }
-    pts.insert(pts.end(), a, a + NGLL2);
-  }
-  std::sort(pts.begin(), pts.end());
-  const size_t distinct = std::unique(pts.begin(), pts.end()) - pts.begin();
-  return distinct == (size_t)(NGLL * (4 * (k1 - k0) + 1));
-}
-
 int desc_counts(int ne, int nown, int nhalo) { return ne | (nown << 8) | (nhalo << 20); }
 
-Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np, int mode,
-                int max_elems = Mesh::PATCH_ELEMS) {
+// First-touch flags of a chain plan, in the launch order of the colours (phase 1's, then phase 2's): a lane updates
+// points i = 0..3 of its row, and i = 4 in the patch's last element.  Points that no force launch writes (those of
+// fluid elements only) are listed as uncovered: they join the special points, which the predictor clears.
+void mark_first_touch(Plan& P, const std::vector<int>& ibool, int nspec, int nglob) {
+  P.first.assign((size_t)nspec * NGLL2, 0);
+  std::vector<int> earliest((size_t)nglob, 1 << 30);
+  const int npatch = (int)P.desc.size() / 4;
+  std::vector<int> launch(npatch, 0);
+  for (int ph = 0, base = 0; ph < 2; base += P.ncolour[ph], ph++)
+    for (int c = 0; c < P.ncolour[ph]; c++)
+      for (int q = P.colour_start[ph][c]; q < P.colour_start[ph][c] + P.colour_count[ph][c]; q++) launch[q] = base + c;
+  for (int pass = 0; pass < 2; pass++)
+    for (int q = 0; q < npatch; q++) {
+      const int pos0 = P.desc[4 * q], ne = P.desc[4 * q + 3] & 0xf;
+      for (int k = 0; k < ne; k++)
+        for (int j = 0; j < NGLL; j++)
+          for (int i = 0; i < (k == ne - 1 ? NGLL : NGLL - 1); i++) {
+            const size_t l = (size_t)(pos0 + k) * NGLL2 + j * NGLL + i;
+            const int g = ibool[(size_t)P.order[pos0 + k] * NGLL2 + j * NGLL + i];
+            if (pass == 0)
+              earliest[g] = std::min(earliest[g], launch[q]);
+            else
+              P.first[l] = earliest[g] == launch[q];
+          }
+    }
+  for (int g = 0; g < nglob; g++)
+    if (earliest[g] == (1 << 30)) P.uncovered.push_back(g);
+}
+
+Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np, int mode) {
+  const int max_elems = Mesh::PATCH_ELEMS;
   Plan P;
   std::vector<int>& order = P.order;
   order.reserve(nspec);
@@ -190,7 +204,6 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
   if (mode == 0) {
     P.slot.assign((size_t)nspec * NGLL2, 0);
     P.newid.assign((size_t)nglob, -1);
-    P.chains = true;
   }
   int next_id = 0;
   for (int ph = 0; ph < 2; ph++) {
@@ -217,7 +230,6 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
     // coloured patches; ownership and numbering in phase-list order
     const std::vector<int> pstart = make_patches(ibool, elems, nglob, max_elems);
     const int np_ph = (int)pstart.size() - 1;
-    for (int q = 0; q < np_ph && P.chains; q++) P.chains = is_chain(ibool, elems, pstart[q], pstart[q + 1]);
     std::vector<std::vector<int>> pnodes(np_ph), phalo(np_ph);
     std::vector<int> own0(np_ph), nown(np_ph);
     for (int q = 0; q < np_ph; q++) {
@@ -281,35 +293,6 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
       P.colour_count[ph][c] = (int)P.desc.size() / 4 - P.colour_start[ph][c];
     }
   }
-  if (mode == 0 && P.chains) {
-    // launch order of the colours: phase 1's, then phase 2's; a lane updates points i = 0..3 of its row, and
-    // i = 4 in the patch's last element
-    P.first.assign((size_t)nspec * NGLL2, 0);
-    std::vector<int> earliest((size_t)nglob, 1 << 30);
-    const int npatch = (int)P.desc.size() / 4;
-    std::vector<int> launch(npatch, 0);
-    for (int ph = 0, base = 0; ph < 2; base += P.ncolour[ph], ph++)
-      for (int c = 0; c < P.ncolour[ph]; c++)
-        for (int q = P.colour_start[ph][c]; q < P.colour_start[ph][c] + P.colour_count[ph][c]; q++) launch[q] = base + c;
-    for (int pass = 0; pass < 2; pass++)
-      for (int q = 0; q < npatch; q++) {
-        const int pos0 = P.desc[4 * q], ne = P.desc[4 * q + 3] & 0xf;
-        for (int k = 0; k < ne; k++)
-          for (int j = 0; j < NGLL; j++)
-            for (int i = 0; i < (k == ne - 1 ? NGLL : NGLL - 1); i++) {
-              const size_t l = (size_t)(pos0 + k) * NGLL2 + j * NGLL + i;
-              const int g = ibool[(size_t)order[pos0 + k] * NGLL2 + j * NGLL + i];
-              if (pass == 0)
-                earliest[g] = std::min(earliest[g], launch[q]);
-              else
-                P.first[l] = earliest[g] == launch[q];
-            }
-      }
-    // points that no force launch writes (those of fluid elements only) join the special points, which the
-    // predictor clears
-    for (int g = 0; g < nglob; g++)
-      if (earliest[g] == (1 << 30)) P.uncovered.push_back(g);
-  }
   for (int e = 0; e < nspec; e++)
     if (!placed[e]) order.push_back(e);  // elements outside the elastic phase lists keep their relative order
   if (mode == 0) {
@@ -320,6 +303,141 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
   return P;
 }
 
+// The plan of a mesh whose patches are all chains (mode 0 with patches of up to max_elems elements), for the chain
+// kernels: false, and P unusable, when some patch is not one.  The colours are build_plan's; elements and points are
+// numbered for towers, the stacks of chains whose top GLL row is the next one's bottom row: tower by tower, first the
+// points inside the rows (x = 1 .. 4 ne - 1, row by row upwards, so that a row is consecutive and the next row of the
+// tower follows it), then the left and the right column upwards (consecutive too, where a neighbour has not numbered
+// them).  No slots, halos or owned ranges: those serve the general patch kernel.
+bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
+                      int max_elems, Plan& P) {
+  P = Plan();
+  std::vector<char> placed(nspec, 0);
+  std::vector<int> elems[2];
+  struct Chain { int ph, k0, ne; };
+  std::vector<Chain> ch;
+  std::vector<int> mark((size_t)nglob, -1);
+  for (int ph = 0; ph < 2; ph++) {
+    for (int k = 0; k < np; k++) {
+      const int v = phase_lists[(size_t)ph * np + k];
+      if (v < 1) break;
+      if (v > nspec) fail("phase_ispec_inner_elastic: element %d outside 1..%d", v, nspec);
+      if (placed[v - 1]) fail("phase_ispec_inner_elastic: element %d listed twice", v);
+      placed[v - 1] = 1;
+      elems[ph].push_back(v - 1);
+    }
+    P.phase_count[ph] = (int)elems[ph].size();
+    const std::vector<int> ps = make_patches(ibool, elems[ph], nglob, max_elems);
+    for (size_t q = 0; q + 1 < ps.size(); q++) ch.push_back({ph, ps[q], ps[q + 1] - ps[q]});
+  }
+  auto row_point = [&](const Chain& c, int j, int x) {  // column x of GLL row j
+    const int k = x == 4 * c.ne ? c.ne - 1 : x / 4;
+    return ibool[(size_t)elems[c.ph][c.k0 + k] * NGLL2 + j * NGLL + (x - 4 * k)];
+  };
+  const int nch = (int)ch.size();
+  std::fill(mark.begin(), mark.end(), -1);
+  for (int q = 0; q < nch; q++) {  // the chain property: shared edges, every other point once
+    const Chain& c = ch[q];
+    for (int k = 0; k < c.ne; k++) {
+      const int* a = ibool.data() + (size_t)elems[c.ph][c.k0 + k] * NGLL2;
+      if (k > 0) {
+        const int* l = ibool.data() + (size_t)elems[c.ph][c.k0 + k - 1] * NGLL2;
+        for (int j = 0; j < NGLL; j++)
+          if (l[j * NGLL + NGLL - 1] != a[j * NGLL]) return false;
+      }
+      for (int j = 0; j < NGLL; j++)
+        for (int i = k > 0 ? 1 : 0; i < NGLL; i++) {
+          int& m = mark[a[j * NGLL + i]];
+          if (m == q) return false;
+          m = q;
+        }
+    }
+  }
+  // towers: the chain on top of each chain
+  std::vector<int> above(nch, -1), below(nch, -1);
+  std::fill(mark.begin(), mark.end(), -1);
+  for (int q = 0; q < nch; q++) mark[row_point(ch[q], 0, 1)] = q;
+  for (int q = 0; q < nch; q++) {
+    const int t = mark[row_point(ch[q], NGLL - 1, 1)];
+    if (t < 0 || t == q || below[t] >= 0 || ch[t].ne != ch[q].ne || ch[t].ph != ch[q].ph) continue;
+    bool same = true;
+    for (int x = 0; x <= 4 * ch[q].ne && same; x++) same = row_point(ch[q], NGLL - 1, x) == row_point(ch[t], 0, x);
+    if (!same) continue;
+    above[q] = t;
+    below[t] = q;
+  }
+  P.newid.assign((size_t)nglob, -1);
+  int next_id = 0;
+  auto number = [&](int g) {
+    if (P.newid[g] < 0) P.newid[g] = next_id++;
+  };
+  for (int q = 0; q < nch; q++) {
+    if (below[q] >= 0) continue;  // a closed ring of chains has no bottom: its points are numbered below
+    for (int t = q; t >= 0; t = above[t])
+      for (int j = 0; j < NGLL; j++)
+        for (int x = 1; x < 4 * ch[t].ne; x++) number(row_point(ch[t], j, x));
+    for (int side = 0; side < 2; side++)
+      for (int t = q; t >= 0; t = above[t])
+        for (int j = 0; j < NGLL; j++) number(row_point(ch[t], j, side ? 4 * ch[t].ne : 0));
+  }
+  for (int q = 0; q < nch; q++)
+    for (int j = 0; j < NGLL; j++)
+      for (int x = 0; x <= 4 * ch[q].ne; x++) number(row_point(ch[q], j, x));
+  // colours, in phase-list order
+  std::vector<uint32_t> used((size_t)nglob, 0u);
+  std::vector<int> patch_of(nch, -1), pos(nch, -1);
+  for (int ph = 0, q0 = 0; ph < 2; ph++) {
+    int q1 = q0;
+    while (q1 < nch && ch[q1].ph == ph) q1++;
+    std::fill(used.begin(), used.end(), 0u);
+    std::vector<int> col(q1 - q0, 0);
+    int ncol = 0;
+    for (int q = q0; q < q1; q++) {
+      uint32_t forbidden = 0;
+      for (int k = 0; k < ch[q].ne; k++)
+        for (int p = 0; p < NGLL2; p++) forbidden |= used[ibool[(size_t)elems[ph][ch[q].k0 + k] * NGLL2 + p]];
+      if (forbidden == 0xffffffffu) fail("patch colouring needs more than %d colours", Mesh::MAX_COLOURS);
+      int c = 0;
+      while (forbidden & (1u << c)) c++;
+      col[q - q0] = c;
+      ncol = std::max(ncol, c + 1);
+      for (int k = 0; k < ch[q].ne; k++)
+        for (int p = 0; p < NGLL2; p++) used[ibool[(size_t)elems[ph][ch[q].k0 + k] * NGLL2 + p]] |= 1u << c;
+    }
+    P.ncolour[ph] = ncol;
+    // positions tower by tower, upwards (a tower's element data is consecutive); descriptors colour by colour
+    auto place = [&](int q) {
+      if (pos[q] >= 0) return;
+      pos[q] = (int)P.order.size();
+      for (int k = 0; k < ch[q].ne; k++) P.order.push_back(elems[ph][ch[q].k0 + k]);
+    };
+    for (int q = q0; q < q1; q++)
+      if (below[q] < 0)
+        for (int t = q; t >= 0; t = above[t]) place(t);
+    for (int q = q0; q < q1; q++) place(q);
+    for (int c = 0; c < ncol; c++) {
+      P.colour_start[ph][c] = (int)P.desc.size() / 4;
+      for (int q = q0; q < q1; q++) {
+        if (col[q - q0] != c) continue;
+        patch_of[q] = (int)P.desc.size() / 4;
+        P.desc.insert(P.desc.end(), {pos[q], 0, 0, desc_counts(ch[q].ne, 0, 0)});
+      }
+      P.colour_count[ph][c] = (int)P.desc.size() / 4 - P.colour_start[ph][c];
+    }
+    q0 = q1;
+  }
+  P.above.assign(nch, -1);
+  for (int q = 0; q < nch; q++)
+    if (above[q] >= 0) P.above[patch_of[q]] = patch_of[above[q]];
+  P.chains = true;
+  mark_first_touch(P, ibool, nspec, nglob);
+  for (int e = 0; e < nspec; e++)
+    if (!placed[e]) P.order.push_back(e);
+  for (int g = 0; g < nglob; g++)
+    if (P.newid[g] < 0) P.newid[g] = next_id++;  // points of no elastic element
+  return true;
+}
+
 }  // namespace
 
 // Patches of up to CHAIN_ELEMS elements over the given phase lists (1-based, zero-padded rows of np), coloured so
@@ -328,8 +446,8 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
 bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
                    std::vector<int>& order, std::vector<int>& desc, int ncolour[2],
                    int colour_start[2][Mesh::MAX_COLOURS], int colour_count[2][Mesh::MAX_COLOURS]) {
-  Plan P = build_plan(ibool, nspec, nglob, phase_lists, np, 0, Mesh::CHAIN_ELEMS);
-  if (!P.chains) return false;
+  Plan P;
+  if (!build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P)) return false;
   order = std::move(P.order);
   desc = std::move(P.desc);
   for (int ph = 0; ph < 2; ph++) {
@@ -343,13 +461,14 @@ bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const in
 }
 
 // Row records of chain point ids: per patch (desc: {first position, -, -, ne}) and GLL row j, {base, id of column
-// 0, first-touch mask low, high} such that column x > 0 of the row is point base + x.  ids: per element point (device
-// order) the point id; flagged: the same with the FIRST_TOUCH flags.  False when some row is not numbered
-// consecutively (or a shared column is not shared): the per-point ids are kept then.
+// 0, first-touch mask low, high} such that column 0 < x < 4 ne of the row is point base + x, and the id of column 4 ne
+// (ends).  ids: per element point (device order) the point id; flagged: the same with the FIRST_TOUCH flags.  False when
+// some row is not numbered consecutively (or a shared column is not shared): the per-point ids are kept then.
 bool chain_row_records(const std::vector<int>& desc, const std::vector<int>& ids, const std::vector<int>& flagged,
-                       std::vector<int4>& rows) {
+                       std::vector<int4>& rows, std::vector<int>& ends) {
   const int npatch = (int)desc.size() / 4;
   rows.assign((size_t)npatch * NGLL, make_int4(0, 0, 0, 0));
+  ends.assign((size_t)npatch * NGLL, 0);
   for (int q = 0; q < npatch; q++) {
     const int e0 = desc[4 * q], ne = desc[4 * q + 3] & 0xf;
     if (ne < 1 || 4 * ne + 1 > 64 || (size_t)(e0 + ne) * NGLL2 > ids.size()) return false;
@@ -362,7 +481,7 @@ bool chain_row_records(const std::vector<int>& desc, const std::vector<int>& ids
       const int base = ids[at(1)] - 1;
       unsigned long long mask = 0ull;
       for (int x = 0; x <= 4 * ne; x++) {
-        if (x > 0 && ids[at(x)] != base + x) return false;
+        if (x > 0 && x < 4 * ne && ids[at(x)] != base + x) return false;
         if (flagged[at(x)] & Mesh::FIRST_TOUCH) mask |= 1ull << x;
       }
       // the other element point of each shared column holds the same point (the chain property)
@@ -371,6 +490,7 @@ bool chain_row_records(const std::vector<int>& desc, const std::vector<int>& ids
           return false;
       rows[(size_t)q * NGLL + j] =
           make_int4(base, ids[at(0)], (int)(unsigned)(mask & 0xffffffffull), (int)(unsigned)(mask >> 32));
+      ends[(size_t)q * NGLL + j] = ids[at(4 * ne)];
     }
   }
   return true;
@@ -410,11 +530,16 @@ void upload_chain_ids(Mesh* mp) {
   launch_col_pack(mp);
   // the ids of each chain row as {base, id at x = 0, first-touch mask}, verified point by point
   device_free(mp->d_col_rows);
-  mp->d_col_rows = nullptr;
+  device_free(mp->d_col_ends);
   if (mp->d_col_ids && !getenv("SF2D_COL_IDS")) {
     std::vector<int4> rows;
-    if (chain_row_records(mp->h_patch_desc, mp->h_chain_ids, ids, rows) && !rows.empty())
+    std::vector<int> ends;
+    if (chain_row_records(mp->h_patch_desc, mp->h_chain_ids, ids, rows, ends) && !rows.empty()) {
       mp->d_col_rows = device_copy(rows.data(), rows.size());
+      mp->d_col_ends = device_copy(ends.data(), ends.size());
+      mp->h_col_rows = std::move(rows);
+      mp->h_col_ends = std::move(ends);
+    }
   }
   device_free(mp->d_special);
   mp->nspecial = (int)list.size();
@@ -438,15 +563,11 @@ void sort_elements_by_colour(Mesh* mp, const int* phase_lists, int np) {
     mp->chain_elems = n;
   }
   if (const char* env = getenv("SF2D_SHOTS_PER_WAVE")) mp->shots_per_wave = std::max(1, atoi(env));
-  Plan P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly,
-                      try_chain ? mp->chain_elems : Mesh::PATCH_ELEMS);
-  if (try_chain && !P.chains) {
-    if (mp->attenuation) {  // the memory variables ride in the chain kernel only: atomic assembly otherwise
-      mp->assembly = 2;
-      P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, 2);
-    } else {
-      P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly);
-    }
+  Plan P;
+  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P) &&
+                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))) {
+    if (try_chain && mp->attenuation) mp->assembly = 2;  // the memory variables ride in the chain kernel only
+    P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly);
   }
   std::vector<int>& order = P.order;
   for (int ph = 0; ph < 2; ph++) {
@@ -463,12 +584,14 @@ void sort_elements_by_colour(Mesh* mp, const int* phase_lists, int np) {
   if (mp->assembly == 0) {
     mp->npatch = (int)P.desc.size() / 4;
     mp->h_patch_desc = P.desc;
-
+    mp->h_above = P.above;
     mp->d_patch_desc = reinterpret_cast<int4*>(device_copy(P.desc.data(), P.desc.size()));
-    mp->d_halo_nodes = device_copy(P.halo.data(), P.halo.size());
-    mp->d_elem_slot = device_copy(P.slot.data(), P.slot.size());
+    mp->chain = P.chains;
+    if (!mp->chain) {
+      mp->d_halo_nodes = device_copy(P.halo.data(), P.halo.size());
+      mp->d_elem_slot = device_copy(P.slot.data(), P.slot.size());
+    }
     mp->point_id = std::move(P.newid);
-    mp->chain = P.chains && try_chain;
   }
 
   // the solid's Newmark updates visit ids 0 .. nglob_el-1: up to the largest point id of an elastic element (in
@@ -1029,6 +1152,7 @@ void prepare_cleanup_device_(long* Mesh_pointer, int* ACOUSTIC_SIMULATION, int* 
   (void)hipStreamSynchronize(mp->stream);
   acoustic_release(mp);
   pml_release(mp);
+  tower_release(mp);
   device_free(mp->d_ibool); device_free(mp->d_xix); device_free(mp->d_xiz); device_free(mp->d_gammax);
   device_free(mp->d_gammaz); device_free(mp->d_kappav); device_free(mp->d_muv); device_free(mp->d_att_idx); device_free(mp->d_att_table); device_free(mp->d_att_e); device_free(mp->d_att_old); device_free(mp->d_ispec_is_elastic);
   device_free(mp->d_displ); device_free(mp->d_veloc); device_free(mp->d_accel);
@@ -1062,6 +1186,7 @@ void prepare_cleanup_device_(long* Mesh_pointer, int* ACOUSTIC_SIMULATION, int* 
   device_free(mp->d_col_ids);
   device_free(mp->d_col_mod);
   device_free(mp->d_col_rows);
+  device_free(mp->d_col_ends);
   device_free(mp->d_special);
   if (mp->grad) sf2d_grad_release(Mesh_pointer);
   if (mp->batch) sf2d_batch_release(Mesh_pointer);
@@ -1611,8 +1736,10 @@ extern "C" int sf2d_mesh_affine_elements(long* Mesh_pointer) {
 extern "C" int sf2d_plan_chains(int nspec, int nglob, const int* ibool_1based, int np, const int* phase_lists,
                                 int* first_writes) {
   std::vector<int> ib = to_zero_based(ibool_1based, (size_t)nspec * NGLL2, 1, nglob, "ibool");
-  Plan P = build_plan(ib, nspec, nglob, phase_lists, np, 0, Mesh::CHAIN_ELEMS);  // as the device plan is chosen
-  if (!P.chains) P = build_plan(ib, nspec, nglob, phase_lists, np, 0);
+  Plan P;  // as the device plan is chosen
+  if (!build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P) &&
+      !build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))
+    P = Plan();
   if (first_writes) {
     *first_writes = 0;
     for (uint8_t f : P.first) *first_writes += f;
@@ -1625,9 +1752,10 @@ extern "C" int sf2d_plan_chains(int nspec, int nglob, const int* ibool_1based, i
 extern "C" int sf2d_plan_row_records(int nspec, int nglob, const int* ibool_1based, int np, const int* phase_lists,
                                      int* nrecords) {
   std::vector<int> ib = to_zero_based(ibool_1based, (size_t)nspec * NGLL2, 1, nglob, "ibool");
-  Plan P = build_plan(ib, nspec, nglob, phase_lists, np, 0, Mesh::CHAIN_ELEMS);  // as the device plan is chosen
-  if (!P.chains) P = build_plan(ib, nspec, nglob, phase_lists, np, 0);
-  if (!P.chains) return -1;
+  Plan P;  // as the device plan is chosen
+  if (!build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P) &&
+      !build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))
+    return -1;
   std::vector<int> ids((size_t)nspec * NGLL2);
   for (int pos = 0; pos < nspec; pos++)
     for (int p = 0; p < NGLL2; p++) ids[(size_t)pos * NGLL2 + p] = P.newid[ib[(size_t)P.order[pos] * NGLL2 + p]];
@@ -1635,7 +1763,8 @@ extern "C" int sf2d_plan_row_records(int nspec, int nglob, const int* ibool_1bas
   for (size_t l = 0; l < flagged.size() && l < P.first.size(); l++)
     if (P.first[l]) flagged[l] |= Mesh::FIRST_TOUCH;
   std::vector<int4> rows;
-  const bool ok = chain_row_records(P.desc, ids, flagged, rows);
+  std::vector<int> ends;
+  const bool ok = chain_row_records(P.desc, ids, flagged, rows, ends);
   if (nrecords) *nrecords = ok ? (int)rows.size() : 0;
   if (!ok) return 0;
   // the records reproduce every writer's id and flag
@@ -1646,7 +1775,7 @@ extern "C" int sf2d_plan_row_records(int nspec, int nglob, const int* ibool_1bas
         for (int i = 0; i < NGLL; i++) {
           const int x = 4 * k + i;
           const int4 r = rows[(size_t)q * NGLL + j];
-          const int id = x == 0 ? r.y : r.x + x;
+          const int id = x == 0 ? r.y : x == 4 * ne ? ends[(size_t)q * NGLL + j] : r.x + x;
           const size_t l = (size_t)(e0 + k) * NGLL2 + j * NGLL + i;
           if (id != ids[l]) return 0;
           const bool writer = i < NGLL - 1 || k == ne - 1;

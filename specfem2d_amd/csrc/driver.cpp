@@ -1236,6 +1236,7 @@ void prepare_device(Sim& s) {
     if (s.simulation_type == 3) transfer_b_fields_to_device_(&size, zeros.data(), zeros.data(), zeros.data(), &s.mesh);
   }
   if (s.nshot > 0) sf2d_batch_prepare(&s.mesh, s.nshot, s.src_shot.data());
+  else if (nspec_el > 0) sf2d_tower_prepare(&s.mesh, s.rmassx.data(), s.rmassz.data());
 }
 
 // Relaxation times of n standard linear solids fitting 1/Q over [fmin, fmax] Hz by linear least squares, as
@@ -1757,6 +1758,10 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   auto mark = [&](int step, int k) {
     if (timed && k < nev) hc(hipEventRecord(ev[(size_t)step * nev + k], stream));
   };
+  // the solid's fused step where the handle has one and nothing between its phases is asked for
+  const int st = s->p.seismotype;
+  const bool fused = any_el && !phases && !s->save_forward && !s->grad_save && st != 2 && st != 3 &&
+                     sf2d_tower_ready(&s->mesh);
   for (int it = it_begin; it <= it_end; it++) {
     const int step = it - it_begin;
     mark(step, 2);
@@ -1765,9 +1770,11 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     if (any_ac)
       update_displacement_ac_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,
                                    &b_deltatover2, &one, &zero);
-    if (any_el)
+    if (any_el && !(fused && it > it_begin)) {
       update_displacement_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,
                                 &b_deltatover2);
+      if (fused) sf2d_tower_begin(&s->mesh);
+    }
     mark(step, 3);
     // the fluid first, coupled to the predicted solid displacement (compute_gpu_acoustic.f90:34-220)
     if (any_ac && !any_el) mark(step, 0);
@@ -1791,6 +1798,21 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
       mark(step, 1);
       mark(step, 4);
       mark(step, 5);
+    }
+    if (fused) {
+      // receivers in fluid elements (the solid's are recorded by the fused step)
+      if (any_ac && s->nrec > 0 && it < it_end)
+        compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
+                                  &acoustic_sim, &trick, &zero, &it, &it_end);
+      if (pml) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
+      if (any_ac && nfluid_solid > 0) compute_coupling_el_ac_cuda_(&s->mesh, &one, &nfluid_solid, &one);
+      mark(step, 0);
+      sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, deltat, deltatsqover2, deltatover2);
+      mark(step, 1);
+      if (it == it_end && s->nrec > 0)
+        compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
+                                  &acoustic_sim, &trick, &zero, &it, &it_end);
+      continue;
     }
     // then the solid, coupled to the new fluid pressure (compute_gpu_elastic.f90:34-215)
     for (int iphase = 1; iphase <= 2 && any_el; iphase++) {

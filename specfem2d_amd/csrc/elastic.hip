@@ -13,6 +13,7 @@
 //   * workgroups are remapped so that each XCD walks a contiguous range: neighbouring patches share an L2.
 // Coloured-element (plain read-modify-write per colour) and FP32-atomic variants remain selectable.
 // All kernels run on the handle's stream.  Every launch bounds its indices against the array sizes it was given.
+#include "sf2d_device.h"
 #include "sf2d_mesh.h"
 
 namespace sf2d {
@@ -21,7 +22,6 @@ namespace {
 
 constexpr int FORCE_THREADS = 256;
 constexpr int FORCE_EPB = 10;  // elements per block: 250 of 256 lanes active
-constexpr int NXCD = 8;        // gfx950: 8 accelerator complex dies, workgroups dispatched round-robin
 
 static_assert(Mesh::PATCH_ELEMS == FORCE_EPB, "one workgroup holds one patch");
 static_assert(FORCE_EPB * NGLL2 <= FORCE_THREADS && FORCE_THREADS <= 256, "patch points indexed by 8-bit slots");
@@ -29,8 +29,6 @@ static_assert(Mesh::PATCH_SHARE == 4, "force cells are summed as two float4 per 
 static_assert(Mesh::PATCH_ELEMS <= 15 && Mesh::CHAIN_ELEMS <= 15, "the element count of a patch descriptor has 4 bits");
 static_assert(Mesh::CHAIN_ELEMS * NGLL <= 64 && (4 * Mesh::CHAIN_ELEMS + 1) * NGLL <= 256,
               "a chain patch fills one wave by rows and has 8-bit point slots");
-
-__device__ __forceinline__ void atomic_add_f32(float* p, float v) { unsafeAtomicAdd(p, v); }
 
 // ---------------------------------------------------------------------------
 // Newmark predictor  (src/gpu/kernels/UpdateDispVeloc_kernel.cu:37-66; update_displacement_Newmark.F90:408-454)
@@ -156,54 +154,6 @@ __global__ __launch_bounds__(256) void k_zero_points(float2* __restrict__ a, con
 // {A_kappa, B_kappa, A_mu, B_mu} x 3 solids from a small table through a per-point index; the state (memory
 // variables e1, e11, e13 per solid, previous dux_dxl, duz_dzl, dux_dzl + duz_dxl) is three float4 planes of
 // [3][ne] in device element order (att_load)
-// One point's viscoelastic update (3 standard linear solids): the memory variables ev (e1, e11, e13 per solid)
-// advance by the recursive convolution of compute_attenuation_viscoelastic.f90:93-121 with the coefficient set
-// cf[k] = {A_kappa, B_kappa, A_mu, B_mu}, the previous strains ov (dux_dxl, duz_dzl, dux_dzl + duz_dxl) become
-// this step's, and the stress takes the unrelaxed-moduli correction.
-__device__ __forceinline__ void attenuate_point(const float4 (&cf)[3], float (&ev)[9], float (&ov)[3], float kap,
-                                                float mu, float dux_dxl, float dux_dzl, float duz_dxl, float duz_dzl,
-                                                float& sxx, float& sxz, float& szz) {
-  const float th = dux_dxl + duz_dzl;
-  const float oxx = ov[0], ozz = ov[1], oxz = ov[2];
-  const float th_old = oxx + ozz;
-  float e1s = 0.f, e11s = 0.f, e13s = 0.f;
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const float a1 = cf[k].x, b1 = cf[k].y, a2 = cf[k].z, b2 = cf[k].w;
-    const float e1 = a1 * a1 * ev[3 * k] + b1 * (th + a1 * th_old);
-    const float e11 = a2 * a2 * ev[3 * k + 1] + b2 * (dux_dxl - 0.5f * th + a2 * (oxx - 0.5f * th_old));
-    const float e13 = a2 * a2 * ev[3 * k + 2] + b2 * (dux_dzl + duz_dxl + a2 * oxz);
-    ev[3 * k] = e1;
-    ev[3 * k + 1] = e11;
-    ev[3 * k + 2] = e13;
-    e1s += e1;
-    e11s += e11;
-    e13s += e13;
-  }
-  ov[0] = dux_dxl;
-  ov[1] = duz_dzl;
-  ov[2] = dux_dzl + duz_dxl;
-  sxx += kap * e1s + 2.f * mu * e11s;
-  sxz += mu * e13s;
-  szz += kap * e1s - 2.f * mu * e11s;
-}
-
-// A point's attenuation state as three float4 planes of [3][ne] (ne = element points): the 9 memory variables then
-// the 3 previous strains, {e1, e11, e13} of solid 1, 2, 3 and {dux_dxl, duz_dzl, dux_dzl + duz_dxl}
-__device__ __forceinline__ void att_load(const float* st, long ne, size_t l, float (&ev)[9], float (&ov)[3]) {
-  const float4* s4 = reinterpret_cast<const float4*>(st);
-  const float4 a = s4[l], b = s4[(size_t)ne + l], c = s4[2 * (size_t)ne + l];
-  ev[0] = a.x; ev[1] = a.y; ev[2] = a.z; ev[3] = a.w;
-  ev[4] = b.x; ev[5] = b.y; ev[6] = b.z; ev[7] = b.w;
-  ev[8] = c.x; ov[0] = c.y; ov[1] = c.z; ov[2] = c.w;
-}
-__device__ __forceinline__ void att_store(float* st, long ne, size_t l, const float (&ev)[9], const float (&ov)[3]) {
-  float4* s4 = reinterpret_cast<float4*>(st);
-  s4[l] = make_float4(ev[0], ev[1], ev[2], ev[3]);
-  s4[(size_t)ne + l] = make_float4(ev[4], ev[5], ev[6], ev[7]);
-  s4[2 * (size_t)ne + l] = make_float4(ev[8], ov[0], ov[1], ov[2]);
-}
-
 // RECT: every element an axis-aligned rectangle (xi_z = gamma_x = 0, xi_x and gamma_z constant over the element):
 // one float2 {xi_x, gamma_z} per element (geom_rect, device element order) instead of four per-point arrays
 template <bool ATOMIC, bool ATT, bool RECT>
@@ -355,13 +305,6 @@ struct PatchRegs {
   int g;        // point id loaded by this lane (lanes < nown + nhalo)
   float2 u, a;
 };
-
-// load through a 32-bit byte offset from a uniform base (global_load with saddr + voffset); every array indexed
-// this way is smaller than 4 GiB (checked when the handle is prepared)
-template <typename T>
-__device__ __forceinline__ T ld_off(const T* base, unsigned byte_off) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
-}
 
 // counts word of a patch descriptor: ne (bits 0-3), affine flag (bit 7), nown (bits 8-19), nhalo (bits 20-31)
 __device__ __forceinline__ int patch_ne(int c) { return c & 0xf; }
@@ -761,8 +704,8 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_chain(
 // shared column (4, j) of element k moves to lane 5 (k + 1) by a one-lane shuffle.  Every sum has the row-lane
 // kernel's terms in its order, and the same (element, point) pairs write accel, so the first-touch flags carry over.
 // rows: when not null, the point ids and first-touch flags come from one int4 per GLL row of the patch
-// (Mesh::d_col_rows: id = base + x for column x > 0 of the chain, the id of x = 0, the flags as a 64-bit mask)
-// instead of col_ids
+// (Mesh::d_col_rows: id = base + x for the columns 0 < x < 4 ne of the chain, the id of x = 0, the flags as a 64-bit
+// mask; ends: the id of x = 4 ne) instead of col_ids
 // ATT (one wavefield): viscoelastic attenuation, the memory variables and previous strains as three float4 planes
 // of [3][ne] in lane order (att_e; see att_load) and a coefficient-set index per point in lane order (att_idx)
 struct ColAtt {
@@ -793,7 +736,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
     int first_patch, int npatch, int nshot, int group, long shot_stride, const int4* __restrict__ desc,
     const int* __restrict__ col_ids, const float4* __restrict__ geom, const float4* __restrict__ geom_elem,
     const float2* __restrict__ col_mod, const float2* __restrict__ displ, float2* __restrict__ accel,
-    const Basis basis, const int4* __restrict__ rows, const ColAtt att) {
+    const Basis basis, const int4* __restrict__ rows, const int* __restrict__ ends, const ColAtt att) {
   __shared__ float2 s_t[Mesh::CHAIN_ELEMS + 1][NGLL][NGLL + 1];
   __shared__ float2 s_v[Mesh::CHAIN_ELEMS + 1][NGLL][NGLL + 1];
   __shared__ float s_hp[NGLL2], s_hpw[NGLL2];
@@ -824,10 +767,11 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
   if (rows) {
     const int x = 4 * min(k, ne - 1) + i;  // column of the chain (lanes past it: the last element's)
     const int4* rp = rows + (size_t)(first_patch + item / ngroup) * NGLL;
+    const int* re = ends + (size_t)(first_patch + item / ngroup) * NGLL;
 #pragma unroll
     for (int j = 0; j < NGLL; j++) {
       const int4 r = rp[j];  // the same word for every lane
-      g[j] = x == 0 ? r.y : r.x + x;
+      g[j] = x == 0 ? r.y : x == 4 * ne ? re[j] : r.x + x;
       const unsigned bits = x < 32 ? ((unsigned)r.z >> x) : ((unsigned)r.w >> (x - 32));
       first[j] = FIRST && (bits & 1u);
       mod[j] = ld_off(col_mod, 8u * (c0 + (unsigned)(j * row)));
@@ -1203,48 +1147,24 @@ __global__ __launch_bounds__(256) void k_permute(const T* __restrict__ src, T* _
 }
 
 // ---------------------------------------------------------------------------
-// Stacey absorbing traction (src/gpu/kernels/compute_stacey_elastic_kernel.cu:37-150,
-// src/specfem2D/compute_stacey_elastic.f90:34-1001)
-__global__ __launch_bounds__(64) void k_stacey(int nabs, const int* __restrict__ abs_ispec,
-                                               const int* __restrict__ abs_ij, const float* __restrict__ normal,
-                                               const float* __restrict__ jacw, const int* __restrict__ edge_abs,
-                                               const int* __restrict__ ib, const int* __restrict__ ibool,
-                                               const int* __restrict__ is_elastic, const float* __restrict__ rho_vp,
-                                               const float* __restrict__ rho_vs, const float2* __restrict__ veloc,
+// Stacey absorbing traction (stacey_traction)
+__global__ __launch_bounds__(64) void k_stacey(const StaceyFaces F, const int* __restrict__ edge_abs,
+                                               const int* __restrict__ ib, const float2* __restrict__ veloc,
                                                float* __restrict__ accel, int write_store, float* store_bottom,
                                                float* store_right, float* store_top, float* store_left,
                                                long shot_stride, int ps) {
   veloc += blockIdx.y * shot_stride;
   accel += 2 * blockIdx.y * shot_stride;
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int f = idx / NGLL;
-  const int k = idx - f * NGLL;
-  if (f >= nabs) return;
-  const int i = abs_ij[(f * NGLL + k) * 2];
-  const int j = abs_ij[(f * NGLL + k) * 2 + 1];
-  if (i < 0 || j < 0) return;  // duplicated corner point, handled by the neighbouring edge
-  const int ispec = abs_ispec[f];
-  if (!is_elastic[ispec]) return;
-  const size_t l = (size_t)ispec * NGLL2 + j * NGLL + i;
-  const long g = (long)ibool[l] * ps;
-  const float2 v = veloc[g];
-  const float nx = normal[(f * NGLL + k) * 2];
-  const float nz = normal[(f * NGLL + k) * 2 + 1];
-  const float vn = nx * v.x + nz * v.y;
-  const float rvp = rho_vp[l], rvs = rho_vs[l];
-  const float tx = rvp * vn * nx + rvs * (v.x - vn * nx);
-  const float tz = rvp * vn * nz + rvs * (v.y - vn * nz);
-  const float w = jacw[f * NGLL + k];
-  const float fx = tx * w, fz = tz * w;
-  atomic_add_f32(&accel[2 * (size_t)g], -fx);
-  atomic_add_f32(&accel[2 * (size_t)g + 1], -fz);
-  if (write_store) {
+  const float2 t = stacey_traction(F, idx, veloc, accel, ps);
+  if (write_store && idx < F.nabs * NGLL && F.ij[2 * idx] >= 0 && F.is_elastic[F.ispec[idx / NGLL]]) {
+    const int f = idx / NGLL, k = idx - f * NGLL;
     const int side = edge_abs[f];
     float* st = side == 1 ? store_bottom : side == 2 ? store_right : side == 3 ? store_top : store_left;
     if (st) {
       const int o = (ib[f] * NGLL + k) * 2;
-      st[o] = fx;
-      st[o + 1] = fz;
+      st[o] = t.x;
+      st[o + 1] = t.y;
     }
   }
 }
@@ -1276,23 +1196,15 @@ __global__ __launch_bounds__(64) void k_stacey_backward(int nabs, const int* __r
 }
 
 // ---------------------------------------------------------------------------
-// collocated force sources (src/gpu/kernels/compute_add_sources_kernel.cu:37-70)
-__global__ __launch_bounds__(64) void k_sources(int nsrc, int it, const int* __restrict__ ispec_src,
-                                                const int* __restrict__ is_elastic, const int* __restrict__ ibool,
-                                                const float* __restrict__ sourcearrays, const float* __restrict__ stf,
-                                                float* __restrict__ accel, const int* __restrict__ src_shot,
-                                                long shot_stride, int ps, const int* __restrict__ step) {
+// collocated force sources (source_force)
+__global__ __launch_bounds__(64) void k_sources(const SourceSet S, int it, float* __restrict__ accel,
+                                                const int* __restrict__ src_shot, long shot_stride, int ps,
+                                                const int* __restrict__ step) {
   const int s = blockIdx.x;
-  const int p = threadIdx.x;
-  if (s >= nsrc || p >= NGLL2) return;
+  if (s >= S.nsrc) return;
   if (step) it = *step - 1;  // graph replays: the 1-based step from device memory
   if (src_shot) accel += 2 * (long)src_shot[s] * shot_stride;  // each source drives its own shot's field
-  const int ispec = ispec_src[s];
-  if (!is_elastic[ispec]) return;
-  const long g = (long)ibool[(size_t)ispec * NGLL2 + p] * ps;
-  const float f = stf[(size_t)it * nsrc + s];
-  atomic_add_f32(&accel[2 * (size_t)g], sourcearrays[(s * NGLL2 + p) * 2] * f);
-  atomic_add_f32(&accel[2 * (size_t)g + 1], sourcearrays[(s * NGLL2 + p) * 2 + 1] * f);
+  source_force(S, s, threadIdx.x, it, accel, ps);
 }
 
 // adjoint sources at the receivers (src/gpu/kernels/add_sources_el_SIM_TYPE_2_OR_3_kernel.cu:37-74)
@@ -1316,39 +1228,12 @@ __global__ __launch_bounds__(64) void k_adjoint_sources(int nadj, int it, int ns
 }
 
 // ---------------------------------------------------------------------------
-// seismograms: Lagrange interpolation at the receivers, FP64 accumulation, rotation
-// (src/gpu/kernels/compute_elastic_seismogram_kernel.cu:69-192; compute_interpolated_dva.f90)
-__global__ __launch_bounds__(64) void k_seismograms(int nrec, int nlength, int cur, const int* __restrict__ ispec_rec,
-                                                    const int* __restrict__ ibool, const float* __restrict__ xir,
-                                                    const float* __restrict__ gammar, const float* __restrict__ cosrot,
-                                                    const float* __restrict__ sinrot, const float2* __restrict__ field,
+// seismograms (record_receiver)
+__global__ __launch_bounds__(64) void k_seismograms(const ReceiverSet R, int cur, const float2* __restrict__ field,
                                                     float* __restrict__ dst, long shot_stride, long dst_stride,
                                                     int ps, const int* __restrict__ step) {
   if (step) cur = *step - 1;  // graph replays: the 1-based step from device memory
-  field += blockIdx.y * shot_stride;
-  dst += blockIdx.y * dst_stride;
-  const int r = blockIdx.x;
-  const int p = threadIdx.x;
-  if (r >= nrec) return;
-  double vx = 0.0, vz = 0.0;
-  if (p < NGLL2) {
-    const int i = p % NGLL, j = p / NGLL;
-    const long g = (long)ibool[(size_t)ispec_rec[r] * NGLL2 + p] * ps;
-    const double h = (double)(xir[i * nrec + r] * gammar[j * nrec + r]);
-    const float2 u = field[g];
-    vx = (double)u.x * h;
-    vz = (double)u.y * h;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    vx += __shfl_xor(vx, off, 64);
-    vz += __shfl_xor(vz, off, 64);
-  }
-  if (p == 0) {
-    const double c = cosrot[r], s = sinrot[r];
-    dst[(size_t)r * nlength + cur] = (float)(c * vx + s * vz);
-    dst[((size_t)nrec + r) * nlength + cur] = (float)(-s * vx + c * vz);
-  }
+  record_receiver(R, blockIdx.x, threadIdx.x, cur, field + blockIdx.y * shot_stride, dst + blockIdx.y * dst_stride, ps);
 }
 
 // ---------------------------------------------------------------------------
@@ -1583,7 +1468,7 @@ void launch_elastic_forces_patch(const Mesh* mp, int first_patch, int npatch, co
                              : ckerns[first_touch ? 1 : 0][group > 1 ? 1 : 0][mp->rect ? 1 : 0],
                          dim3(grid), dim3(CHAIN_LANES), 0, mp->stream, first_patch, npatch, nshot, group, shot_stride,
                          (const int4*)mp->d_patch_desc, mp->d_col_ids, mp->d_geom, mp->d_geom_elem, mp->d_col_mod,
-                         (const float2*)displ, (float2*)accel, mp->basis, (const int4*)mp->d_col_rows, ca);
+                         (const float2*)displ, (float2*)accel, mp->basis, (const int4*)mp->d_col_rows, mp->d_col_ends, ca);
       check_hip(hipGetLastError(), "k_elastic_forces_col launch");
       return;
     }
@@ -1706,10 +1591,8 @@ void launch_stacey(const Mesh* mp, const float* veloc, float* accel, int write_s
   if (mp->num_abs <= 0) return;
   if (nshot > 1 && write_store) fail("the Stacey boundary store holds one wavefield");
   hipLaunchKernelGGL(k_stacey, shot_grid((long)mp->num_abs * NGLL, 64, 1 << 20, nshot), dim3(64), 0, mp->stream,
-                     mp->num_abs, mp->d_abs_ispec, mp->d_abs_ij, mp->d_abs_normal, mp->d_abs_jacw, mp->d_edge_abs,
-                     mp->d_ib, mp->d_ibool, mp->d_ispec_is_elastic, mp->d_rho_vp, mp->d_rho_vs, (const float2*)veloc,
-                     accel, write_store, mp->d_b_absorb[1], mp->d_b_absorb[2], mp->d_b_absorb[3], mp->d_b_absorb[4],
-                     shot_stride, ps);
+                     stacey_faces(mp), mp->d_edge_abs, mp->d_ib, (const float2*)veloc, accel, write_store,
+                     mp->d_b_absorb[1], mp->d_b_absorb[2], mp->d_b_absorb[3], mp->d_b_absorb[4], shot_stride, ps);
   check_hip(hipGetLastError(), "k_stacey launch");
 }
 
@@ -1725,9 +1608,8 @@ void launch_stacey_backward(const Mesh* mp, float* b_accel) {
 void launch_sources(const Mesh* mp, float* accel, int it, const int* src_shot, long shot_stride, int ps,
                     const int* step) {
   if (mp->nsources_local <= 0) return;
-  hipLaunchKernelGGL(k_sources, dim3(mp->nsources_local), dim3(64), 0, mp->stream, mp->nsources_local, it,
-                     mp->d_ispec_selected_source, mp->d_ispec_is_elastic, mp->d_ibool, mp->d_sourcearrays, mp->d_stf,
-                     accel, src_shot, shot_stride, ps, step);
+  hipLaunchKernelGGL(k_sources, dim3(mp->nsources_local), dim3(64), 0, mp->stream, source_set(mp), it, accel, src_shot,
+                     shot_stride, ps, step);
   check_hip(hipGetLastError(), "k_sources launch");
 }
 
@@ -1742,10 +1624,8 @@ void launch_adjoint_sources(const Mesh* mp, float* accel, int it) {
 void launch_seismograms(const Mesh* mp, const float* field, float* dst, int seismo_current, int nshot,
                         long shot_stride, long dst_stride, int ps, const int* step) {
   if (mp->nrec_local <= 0) return;
-  hipLaunchKernelGGL(k_seismograms, dim3(mp->nrec_local, nshot), dim3(64), 0, mp->stream, mp->nrec_local,
-                     mp->nlength_seismogram, seismo_current, mp->d_ispec_selected_rec, mp->d_ibool, mp->d_xir,
-                     mp->d_gammar, mp->d_cosrot, mp->d_sinrot, (const float2*)field, dst, shot_stride, dst_stride,
-                     ps, step);
+  hipLaunchKernelGGL(k_seismograms, dim3(mp->nrec_local, nshot), dim3(64), 0, mp->stream, receiver_set(mp),
+                     seismo_current, (const float2*)field, dst, shot_stride, dst_stride, ps, step);
   check_hip(hipGetLastError(), "k_seismograms launch");
 }
 

@@ -16,8 +16,8 @@
 // element's phase.  Per layer element point they stream the point id, the geometry, the moduli (fluid: J/rho), the
 // damping weight w_i w_j rho J (fluid: w_i w_j J/kappa), a 4-byte index into a table of the distinct coefficient
 // sets (the profiles depend on the distance into the layer only, so a few thousand sets serve a layer of millions
-// of points), the previous-step field of the point (written per element point by a pass before the Newmark
-// predictor) and the memory variables (12 planes for a solid point, 6 for a fluid one), all stored
+// of points), the previous-step field of the point (solid: a field of its own; fluid: written per element point by a
+// pass before the Newmark predictor) and the memory variables (12 planes for a solid point, 6 for a fluid one), all stored
 // [plane][layer element point] so that consecutive lanes touch consecutive words.
 #include <algorithm>
 #include <array>
@@ -86,7 +86,7 @@ template <bool VISCO>
 __global__ __launch_bounds__(256) void k_pml_elastic_forces(
     int first, int n, long nq, const int* __restrict__ ids, const float4* __restrict__ geom,
     const float2* __restrict__ moduli, const float* __restrict__ dampw, const unsigned int* __restrict__ cidx,
-    const float4* __restrict__ table, const float2* __restrict__ old, float* __restrict__ rm,
+    const float4* __restrict__ table, const float2* __restrict__ oldp, float* __restrict__ rm,
     const float2* __restrict__ displ, const float2* __restrict__ veloc, float2* __restrict__ accel, const Basis basis,
     const unsigned int* __restrict__ zidx, const float4* __restrict__ ztable, float* __restrict__ zrm) {
   __shared__ float s_hp[NGLL2], s_hpw[NGLL2], s_w[NGLL];
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void k_pml_elastic_forces(
     g = ids[q];
     u = displ[g];
     a_old = accel[g];  // no other element of this colour has the point: read with the fields, in one round trip
-    o = old[q];
+    o = oldp[g];
     v = veloc[g];
     gm = geom[q];
     md = moduli[q];
@@ -360,29 +360,28 @@ __global__ __launch_bounds__(256) void k_pml_acoustic_forces(
   }
 }
 
-// previous-step field of each layer element point, before the Newmark predictor (update_displacement_Newmark.F90:
+// previous-step field of the layer's points, before the Newmark predictor (update_displacement_Newmark.F90:
 // 373-380, 428-433): u_old = u + dt^2/4 a, with a the corrected acceleration (the deferred corrector's mass
 // scaling applied here when it is pending); zero on the layer's outer boundary, which the zero condition clears
-// before the field is used
-__global__ __launch_bounds__(256) void k_pml_old_elastic(long nq, const int* __restrict__ ids,
-                                                         const unsigned int* __restrict__ cidx,
+// before the field is used.  pts: the solid layer's points, those of the outer boundary with ON_EDGE
+__global__ __launch_bounds__(256) void k_pml_old_elastic(int n, const unsigned int* __restrict__ pts,
                                                          const float2* __restrict__ d, const float2* __restrict__ a,
                                                          const float* __restrict__ rmx, const float* __restrict__ rmz,
                                                          int pending, float dt2o4, float2* __restrict__ old) {
-  for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < nq; q += (long)gridDim.x * blockDim.x) {
-    float2 out = make_float2(0.f, 0.f);
-    if (!(cidx[q] & ON_EDGE)) {
-      const int g = ids[q];
-      float2 acc = a[g];
-      if (pending) {
-        acc.x *= rmx[g];
-        acc.y *= rmz[g];
-      }
-      const float2 u = d[g];
-      out = make_float2(u.x + dt2o4 * acc.x, u.y + dt2o4 * acc.y);
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int g = (int)(pts[k] & ~ON_EDGE);
+  float2 out = make_float2(0.f, 0.f);
+  if (!(pts[k] & ON_EDGE)) {
+    float2 acc = a[g];
+    if (pending) {
+      acc.x *= rmx[g];
+      acc.y *= rmz[g];
     }
-    old[q] = out;
+    const float2 u = d[g];
+    out = make_float2(u.x + dt2o4 * acc.x, u.y + dt2o4 * acc.y);
   }
+  old[g] = out;
 }
 
 __global__ __launch_bounds__(256) void k_pml_old_acoustic(long nq, const int* __restrict__ ids,
@@ -625,7 +624,9 @@ struct PmlLayer {  // the solid's or the fluid's layer elements, packed in (phas
   float2* d_mod = nullptr;  // solid {kappa, mu}; fluid {J/rho, 0}
   float* d_dampw = nullptr;
   unsigned int* d_cidx = nullptr;
-  float* d_old = nullptr;   // previous-step field per element point (float2 solid, float fluid)
+  float* d_old = nullptr;   // previous-step field: solid [nglob] float2, fluid per element point
+  int npts = 0;             // solid: the layer's points, ON_EDGE on the outer boundary
+  unsigned int* d_pts = nullptr;
   float* d_rm = nullptr;    // memory variables: solid [3][nelem * 25] float4, fluid [3][nelem * 25] float2
   unsigned int* d_zidx = nullptr;  // solid, viscoelastic layer: Zener set per element point (NO_ZENER: none)
   float* d_zrm = nullptr;          // its memory variables: [3][nelem * 25] float4, then [3][nelem * 25] float2
@@ -654,7 +655,7 @@ namespace {
 void release_layer(PmlLayer& L) {
   device_free(L.d_ids); device_free(L.d_geom); device_free(L.d_mod); device_free(L.d_dampw);
   device_free(L.d_cidx); device_free(L.d_old); device_free(L.d_rm); device_free(L.d_bnd);
-  device_free(L.d_zidx); device_free(L.d_zrm);
+  device_free(L.d_zidx); device_free(L.d_zrm); device_free(L.d_pts);
 }
 
 // greedy colouring of a layer element list (device point ids), then the packed order per phase
@@ -814,7 +815,20 @@ void pml_setup(Mesh* mp, const std::vector<int>& region, const std::vector<int>&
     L.d_mod = device_alloc<float2>((size_t)nq);
     L.d_dampw = device_alloc<float>((size_t)nq);
     L.d_cidx = device_copy(cq.data(), cq.size());
-    L.d_old = device_zeros<float>((size_t)nq * (side ? 1 : 2));
+    L.d_old = device_zeros<float>(side ? (size_t)nq : (size_t)2 * mp->nglob);
+    if (side == 0) {
+      std::vector<unsigned int> pts;
+      pts.reserve((size_t)nq);
+      for (int k = 0; k < L.nelem; k++)
+        for (int p = 0; p < NGLL2; p++) {
+          const int g = ibool_dev[(size_t)pos[k] * NGLL2 + p];
+          pts.push_back((unsigned int)g | (on_edge[g] ? ON_EDGE : 0u));
+        }
+      std::sort(pts.begin(), pts.end(), [](unsigned int a, unsigned int b) { return (a & ~ON_EDGE) < (b & ~ON_EDGE); });
+      pts.erase(std::unique(pts.begin(), pts.end()), pts.end());
+      L.npts = (int)pts.size();
+      L.d_pts = device_copy(pts.data(), pts.size());
+    }
     L.d_rm = device_zeros<float>((size_t)nq * (side ? AC_PLANES : EL_PLANES));
     hipLaunchKernelGGL(k_pml_pack, dim3(grid_for(nq)), dim3(256), 0, mp->stream, nq, side, d_pos, d_rho, mp->d_ibool,
                        mp->d_xix, mp->d_xiz, mp->d_gammax, mp->d_gammaz, mp->d_kappav, mp->d_muv, mp->basis, L.d_ids,
@@ -845,6 +859,16 @@ bool pml_element(const Mesh* mp, int ispec) {
   return mp->pml_state && !mp->pml_state->region.empty() && mp->pml_state->region[ispec] != 0;
 }
 
+std::vector<int> pml_solid_elements(const Mesh* mp) {
+  std::vector<int> out;
+  if (mp->pml_state)
+    for (int e = 0; e < mp->nspec; e++)
+      if (pml_element(mp, e) && (mp->h_is_acoustic.empty() || !mp->h_is_acoustic[e])) out.push_back(e);
+  return out;
+}
+
+float2* pml_old_field(const Mesh* mp) { return mp->pml_state ? (float2*)mp->pml_state->el.d_old : nullptr; }
+
 void pml_release(Mesh* mp) {
   PmlState* S = mp->pml_state;
   if (!S) return;
@@ -862,7 +886,8 @@ void pml_reset(Mesh* mp) {
   for (PmlLayer* L : {&S->el, &S->ac}) {
     if (L->nelem == 0) continue;
     const bool fluid = L == &S->ac;
-    check_hip(hipMemsetAsync(L->d_old, 0, (size_t)L->nq() * (fluid ? 1 : 2) * sizeof(float), mp->stream), "memset");
+    check_hip(hipMemsetAsync(L->d_old, 0, (fluid ? (size_t)L->nq() : (size_t)2 * mp->nglob) * sizeof(float), mp->stream),
+              "memset");
     check_hip(hipMemsetAsync(L->d_rm, 0, (size_t)L->nq() * (fluid ? AC_PLANES : EL_PLANES) * sizeof(float),
                              mp->stream), "memset");
     if (L->d_zrm)
@@ -874,7 +899,7 @@ void pml_elastic_before_predictor(Mesh* mp, float deltatsqover2) {
   PmlState* S = mp->pml_state;
   if (!S || S->el.nelem == 0) return;
   PmlLayer& L = S->el;
-  hipLaunchKernelGGL(k_pml_old_elastic, dim3(grid_for(L.nq())), dim3(256), 0, mp->stream, L.nq(), L.d_ids, L.d_cidx,
+  hipLaunchKernelGGL(k_pml_old_elastic, dim3((L.npts + 255) / 256), dim3(256), 0, mp->stream, L.npts, L.d_pts,
                      (const float2*)mp->d_displ, (const float2*)mp->d_accel, mp->d_rmassx, mp->d_rmassz,
                      mp->pending_corrector[0], 0.5f * deltatsqover2, (float2*)L.d_old);
   check_hip(hipGetLastError(), "k_pml_old_elastic launch");

@@ -29,6 +29,7 @@ struct Basis {
 
 struct AcousticState;  // fluid elements (acoustic.hip)
 struct PmlState;       // CPML layer (pml.hip)
+struct TowerState;     // the solid's fused time step (tower.hip)
 
 struct Mesh {
   int myrank = 0;
@@ -119,11 +120,15 @@ struct Mesh {
   // wave's load of GLL row j reads consecutive words (SF2D_ROW_CHAIN keeps the row-lane kernel)
   int* d_col_ids = nullptr;
   float2* d_col_mod = nullptr;
-  // the column-lane kernel's point ids as rows: when GLL row j of every chain numbers its points x = 1 .. 4 ne
+  // the column-lane kernel's point ids as rows: when GLL row j of every chain numbers its points x = 1 .. 4 ne - 1
   // consecutively (id = base_j + x; the numbering of the plan makes it so), a patch needs per row only base_j, the
-  // id of its point x = 0 and a 64-bit mask of the first-touch flags: int4 {base_j, id(0, j), mask low, mask high}
-  // per (patch, row), 80 B per chain instead of 1200 B of ids (SF2D_COL_IDS keeps the per-point ids)
+  // ids of its points x = 0 and x = 4 ne and a 64-bit mask of the first-touch flags: int4 {base_j, id(0, j), mask low,
+  // mask high} and an int per (patch, row), 100 B per chain instead of 1200 B of ids (SF2D_COL_IDS keeps the ids)
   int4* d_col_rows = nullptr;
+  int* d_col_ends = nullptr;
+  std::vector<int4> h_col_rows;      // host copies of d_col_rows and d_col_ends
+  std::vector<int> h_col_ends;
+  std::vector<int> h_above;          // chain plans: the patch on top of each patch (-1: none), see build_chain_plan
   std::vector<int> h_patch_desc;
   std::vector<uint8_t> h_first;
   // First-touch assembly (forward wavefield of SIMULATION_TYPE=1 and shot batches; SF2D_NO_FIRST_TOUCH turns it
@@ -190,6 +195,7 @@ struct Mesh {
 
   // CPML layer (prepare_pml_device_ / prepare_cpml_device_)
   PmlState* pml_state = nullptr;
+  TowerState* tower = nullptr;
 
   // scratch
   unsigned int* d_scratch_u32 = nullptr;  // reductions
@@ -266,10 +272,16 @@ void pml_elastic_forces(Mesh* mp, int ph);
 void pml_acoustic_before_predictor(Mesh* mp, const float* pot, const float* pdd, float deltatsqover2);
 void pml_acoustic_forces(Mesh* mp, int ph, const float* pot, const float* pd, float* pdd);
 void pml_acoustic_boundary(Mesh* mp, float* pot, float* pd, float* pdd);
+// solid elements of the layer (caller order, 0-based); its previous-step displacement [nglob] (null without a layer)
+std::vector<int> pml_solid_elements(const Mesh* mp);
+float2* pml_old_field(const Mesh* mp);
+// the solid's fused time step (tower.hip)
+void tower_release(Mesh* mp);
+bool tower_masses_fit(const Mesh* mp, const float* rmassx, const float* rmassz);
 // chain-kernel point ids with first-touch flags and the special points, uploaded again when the special points change
 void upload_chain_ids(Mesh* mp);
 bool chain_row_records(const std::vector<int>& desc, const std::vector<int>& ids, const std::vector<int>& flagged,
-                       std::vector<int4>& rows);
+                       std::vector<int4>& rows, std::vector<int>& ends);
 bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
                    std::vector<int>& order, std::vector<int>& desc, int ncolour[2],
                    int colour_start[2][Mesh::MAX_COLOURS], int colour_count[2][Mesh::MAX_COLOURS]);

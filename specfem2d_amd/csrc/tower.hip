@@ -1,0 +1,647 @@
+// A whole time step of the solid in two launches: towers of chains, then the points between them.
+//
+// A tower is a stack of chains (rows of up to 12 elements) in which each chain's top GLL row is the next one's bottom
+// row.  One wave walks up a tower, lane 5 k + i holding column i of element k, and carries the displacement and the
+// force of the shared GLL row in registers from one chain to the next.  A GLL point inside a tower gets all of its
+// force there, so the wave applies the Newmark corrector of this step and the predictor of the next one to it at once
+// and in place: nobody else reads or writes the point.  Per step such a point costs its displacement and velocity read
+// and written, its inverse mass, and the element data once: no acceleration array, no second pass, no colours.
+//
+// The other points -- the tower's outline and every point that something else also acts on or looks at (absorbing
+// edges, sources, fluid-solid edges, CPML elements, receivers, points whose two inverse masses differ) -- are the
+// interface.  For these the wave stores its force into a slot of its own (partial), the boundary kernels add theirs
+// into accel as they always do, and the interface kernel sums the slots of each point in a fixed order, adds and clears
+// accel and makes the same Newmark update.
+//
+// State between two such steps: (d_n, v'_n) predicted, accel zero at the interface points with a boundary term and
+// stale elsewhere.  A run starts from the ordinary predictor; its last step leaves displacement, velocity and
+// acceleration as the callers know them.
+//
+// What bounds it: HBM.  2000 x 1000 elements (32 M points), one step: see the launch rule at tower_chains below.
+#include <algorithm>
+#include <cstdlib>
+#include <vector>
+
+#include "sf2d_device.h"
+#include "sf2d_mesh.h"
+#include "specfem2d_gpu_ext.h"
+
+namespace sf2d {
+
+struct TowerState {
+  int ntower = 0, nrow = 0;
+  int4* d_desc = nullptr;     // [ntower][2] {first element position, chains, elements per chain, first row record},
+                              // {base, id of x = 0, id of x = 4 ne of the bottom GLL row, -}
+  int4* d_row = nullptr;      // [nrow] {mask low, mask high, first partial slot, -} per GLL row, bottom to top; mask
+                              // bit x: point x of the row is an interface point
+  int npartial = 0;
+  float2* d_partial = nullptr;
+  int nif = 0, nif2 = 0;      // interface points; the first nif2 have at most two slots
+  int* d_if_id = nullptr;     // [nif]
+  int2* d_if_s = nullptr;     // [nif] slots 0 and 1 (-1: none)
+  int2* d_if_s2 = nullptr;    // [nif - nif2] slots 2 and 3
+  uint8_t* d_if_flag = nullptr;
+  std::vector<char> is_if;    // [nglob]
+};
+
+namespace {
+
+constexpr int HAS_ACC = 1, PML_POINT = 2, PML_EDGE = 4;  // interface point flags
+
+struct Newmark {
+  float dto2, dt, dt2o2;
+};
+
+
+constexpr int TROW = 64;  // float2 per GLL row in LDS, in lane order: writes and reads without bank conflicts
+
+// attenuation state and coefficient sets in the chain kernel's lane order (att_load); SETS: 0 no attenuation, 1 one
+// coefficient set for every point, 2 a set index per point
+struct TowerAtt {
+  const unsigned int* idx;
+  const float4* table;
+  float* state;
+  long ne;
+};
+
+// The wavefields of a step, shot s at s * stride points: (d, v) = (d_n, v'_n) in, (d_out, v_out) = (d_{n+1}, v'_{n+1})
+// out, which may be the same arrays.  last: the step ends a run instead, accel = a_n and v_out = v_n.  r_out (may be
+// null): the force r_n of every point.  accel holds the boundary terms at interface points.
+struct TowerFields {
+  const float2 *d, *v;
+  float2 *d_out, *v_out, *r_out, *accel;
+  long stride;
+  int nshot, last;
+};
+
+// the point at byte offset o: corrector of this step and predictor of the next (k_corrector's and k_predictor's
+// operations, contracted the same way, so that a run in pieces gives the bits of the run in one) from the force r
+__device__ __forceinline__ void newmark_point(const Newmark& c, const TowerFields& F, long shot, unsigned o, float2 r,
+                                              float wx, float wz, float2 d, float2 v) {
+  auto put = [&](float2* base, float2 value) {
+    *reinterpret_cast<float2*>(reinterpret_cast<char*>(base + shot) + o) = value;
+  };
+  if (F.r_out) put(F.r_out, r);
+  const float2 a = make_float2(r.x * wx, r.y * wz);
+  v.x = fmaf(c.dto2, a.x, v.x);
+  v.y = fmaf(c.dto2, a.y, v.y);
+  if (F.last) {
+    put(F.accel, a);
+  } else {
+    d.x = fmaf(c.dt2o2, a.x, fmaf(c.dt, v.x, d.x));
+    d.y = fmaf(c.dt2o2, a.y, fmaf(c.dt, v.y, d.y));
+    v.x = fmaf(c.dto2, a.x, v.x);
+    v.y = fmaf(c.dto2, a.y, v.y);
+    put(F.d_out, d);
+  }
+  put(F.v_out, v);
+}
+
+// What else the launch does, in workgroups after the towers': Stacey faces, sources, receivers of the step
+struct TowerEdges {
+  StaceyFaces faces;
+  SourceSet sources;
+  ReceiverSet receivers;
+  int it;                  // 0-based time sample
+  int nface_wg, nsource, nreceiver;
+  const int* src_shot;     // shot of each source (null: one shot)
+  float* seismo;           // [shot][2][receiver][time]
+  long seismo_stride;
+  int wgs(int nshot) const { return nface_wg * nshot + nsource + nreceiver * nshot; }
+};
+
+__device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFields& F, int wg) {
+  const int faces = E.nface_wg * F.nshot;
+  if (wg < faces) {
+    const int shot = wg / E.nface_wg;
+    stacey_traction(E.faces, (wg - shot * E.nface_wg) * 64 + threadIdx.x, F.v + shot * F.stride,
+                    (float*)(F.accel + shot * F.stride), 1);
+    return;
+  }
+  wg -= faces;
+  if (wg < E.nsource) {
+    const long shot = E.src_shot ? E.src_shot[wg] : 0;
+    source_force(E.sources, wg, threadIdx.x, E.it, (float*)(F.accel + shot * F.stride), 1);
+    return;
+  }
+  wg -= E.nsource;
+  if (wg >= E.nreceiver * F.nshot) return;
+  const int shot = wg / E.nreceiver, r = wg - shot * E.nreceiver;
+  if (E.faces.is_elastic[E.receivers.ispec[r]])  // receivers in fluid elements are recorded by the fluid
+    record_receiver(E.receivers, r, threadIdx.x, E.it, F.d + shot * F.stride, E.seismo + shot * E.seismo_stride, 1);
+}
+
+// The operands of a lane's column of one chain that the next iteration starts from, loaded one chain ahead: the
+// displacement of GLL rows 1 .. 4, the moduli of rows 0 .. 4, the element's geometry record
+struct ChainRegs {
+  float2 d[NGLL - 1], mod[NGLL];
+  float4 ge;
+};
+
+// GEO: 0 every element a rectangle {xi_x, gamma_z}, 1 every element affine (one record), 2 geometry per point
+template <int GEO, int SETS>
+__global__ __launch_bounds__(64) void k_tower(
+    int ntower, const int4* __restrict__ desc, const int4* __restrict__ rows, const float4* __restrict__ geom,
+    const float4* __restrict__ geom_elem, const float2* __restrict__ mod, const TowerFields F,
+    const float* __restrict__ rm, float2* __restrict__ partial, int npartial, const Newmark nm, const Basis basis,
+    const TowerAtt att, int tower_wgs, const TowerEdges edges) {
+  constexpr bool RECT = GEO == 0;
+  __shared__ float2 s_t[NGLL * TROW + 1];
+  if ((int)blockIdx.x >= tower_wgs) {
+    tower_edges(edges, F, blockIdx.x - tower_wgs);
+    return;
+  }
+  // the shots of a tower are neighbours on one XCD: its element data comes from HBM once
+  const int item = (blockIdx.x % NXCD) * (tower_wgs / NXCD) + blockIdx.x / NXCD;
+  const int tower = F.nshot == 1 ? item : item / F.nshot;
+  if (tower >= ntower) return;  // uniform over the wave
+  const int shot = item - tower * F.nshot;
+  const long at = shot * F.stride;
+  const float2* const __restrict__ d = F.d + at;
+  const float2* const __restrict__ v = F.v + at;
+  partial += (size_t)shot * npartial;
+  const int4 td = desc[2 * tower], tb = desc[2 * tower + 1];
+  const int nch = td.y, ne = td.z;
+  const int4* const row = rows + td.w;
+  const int lane = threadIdx.x;
+  const int k = min(lane / NGLL, Mesh::CHAIN_ELEMS);
+  const int i = lane % NGLL;
+  const int kk = min(k, ne - 1);
+  const int x = 4 * kk + i;
+  const int xe = 4 * ne;
+  const bool active = lane / NGLL < ne;
+  const bool writer = active && (i < NGLL - 1 || k == ne - 1);
+  const unsigned below_lo = x < 32 ? (1u << x) - 1u : ~0u, below_hi = x < 32 ? 0u : (1u << (x - 32)) - 1u;
+  float hpi[NGLL], hwi[NGLL];  // this lane's row of the derivative matrix and column of the weighted one
+#pragma unroll
+  for (int m = 0; m < NGLL; m++) {
+    hpi[m] = basis.hp[i * NGLL + m];
+    hwi[m] = basis.hpw[m * NGLL + i];
+  }
+  const float wi = basis.w[i];
+  // byte offsets: point of this lane in the current bottom row and its step from row to row (fields of 8 bytes), and
+  // word of row 0 of the chain in the element arrays
+  unsigned off = 8u * (unsigned)(x == 0 ? tb.y : x == xe ? tb.z : tb.x + x);
+  const unsigned up = 8u * (x == 0 || x == xe ? 1u : (unsigned)(xe - 1));
+  unsigned word = (unsigned)td.x * NGLL2 + (unsigned)min(lane, NGLL * ne - 1);
+  unsigned elem = (unsigned)(td.x + kk);
+  const unsigned mrow = (unsigned)(NGLL * ne);
+
+  auto load_chain = [&](unsigned o, unsigned w, unsigned e, ChainRegs& q) {
+#pragma unroll
+    for (int j = 0; j < NGLL - 1; j++) q.d[j] = ld_off(d, o + (unsigned)(j + 1) * up);
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) q.mod[j] = ld_off(mod, 8u * (w + (unsigned)j * mrow));
+    if (GEO < 2) q.ge = ld_off(geom_elem, 16u * e);
+  };
+  // the update of one row's point, or its share of an interface point
+  auto finish = [&](const int4 r, unsigned o, float2 f, float2 u, float2 vp, float m) {
+    if (!writer) return;
+    const unsigned bits = x < 32 ? (unsigned)r.x >> x : (unsigned)r.y >> (x - 32);
+    if (bits & 1u) {
+      partial[r.z + __popc((unsigned)r.x & below_lo) + __popc((unsigned)r.y & below_hi)] = f;
+    } else {
+      newmark_point(nm, F, at, o, f, m, m, u, vp);
+    }
+  };
+
+  float2 u0 = ld_off(d, off);
+  float2 carry = make_float2(0.f, 0.f);
+  ChainRegs nx;
+  load_chain(off, word, elem, nx);
+  float4 cf[3];
+  if (SETS == 1) {
+#pragma unroll
+    for (int s = 0; s < 3; s++) cf[s] = att.table[s];
+  }
+  const float2* const el = s_t + NGLL * k;  // this element's five points of GLL row 0
+
+  for (int c = 0; c < nch; c++) {
+    const ChainRegs q = nx;
+    // this chain's velocity and inverse mass (rows 0 .. 3), needed at its end
+    float2 vp[NGLL - 1];
+    float ms[NGLL - 1];
+#pragma unroll
+    for (int j = 0; j < NGLL - 1; j++) {
+      vp[j] = ld_off(v, off + (unsigned)j * up);
+      ms[j] = ld_off(rm, (off + (unsigned)j * up) / 2u);
+    }
+    float4 st[3];  // attenuation state of the next row
+    if (SETS > 0) {
+#pragma unroll
+      for (int s = 0; s < 3; s++) st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + word];
+    }
+    const unsigned noff = off + 4u * up, nword = word + (unsigned)NGLL * mrow, nelem = elem + (unsigned)ne;
+    if (c + 1 < nch) load_chain(noff, nword, nelem, nx);
+    float2 u[NGLL];
+    u[0] = u0;
+#pragma unroll
+    for (int j = 1; j < NGLL; j++) u[j] = q.d[j - 1];
+
+    // xi derivatives: the element's rows through LDS
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) s_t[j * TROW + lane] = u[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float2 t1[NGLL], t2[NGLL];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      const float2 e0 = el[j * TROW], e1 = el[j * TROW + 1], e2 = el[j * TROW + 2], e3 = el[j * TROW + 3],
+                   e4 = el[j * TROW + 4];
+      const float dux_dxi = e0.x * hpi[0] + e1.x * hpi[1] + e2.x * hpi[2] + e3.x * hpi[3] + e4.x * hpi[4];
+      const float duz_dxi = e0.y * hpi[0] + e1.y * hpi[1] + e2.y * hpi[2] + e3.y * hpi[3] + e4.y * hpi[4];
+      float dux_dga = 0.f, duz_dga = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        const float h = basis.hp[j * NGLL + m];
+        dux_dga += u[m].x * h;
+        duz_dga += u[m].y * h;
+      }
+      const float kap = q.mod[j].x, mu = q.mod[j].y;
+      const float lambdal = kap - mu, lp2m = kap + mu;
+      float4 gp = q.ge;
+      if (GEO == 2) gp = ld_off(geom, 16u * (elem * NGLL2 + (unsigned)(j * NGLL + i)));
+      const float xixl = gp.x, xizl = RECT ? 0.f : gp.y, gaxl = RECT ? 0.f : gp.z, gazl = gp.w;
+      const float dux_dxl = RECT ? dux_dxi * xixl : dux_dxi * xixl + dux_dga * gaxl;
+      const float dux_dzl = RECT ? dux_dga * gazl : dux_dxi * xizl + dux_dga * gazl;
+      const float duz_dxl = RECT ? duz_dxi * xixl : duz_dxi * xixl + duz_dga * gaxl;
+      const float duz_dzl = RECT ? duz_dga * gazl : duz_dxi * xizl + duz_dga * gazl;
+      float sxx = lp2m * dux_dxl + lambdal * duz_dzl;
+      float szz = lp2m * duz_dzl + lambdal * dux_dxl;
+      float sxz = mu * (duz_dxl + dux_dzl);
+      if (SETS > 0) {
+        const unsigned la = word + (unsigned)j * mrow;
+        float ev[9] = {st[0].x, st[0].y, st[0].z, st[0].w, st[1].x, st[1].y, st[1].z, st[1].w, st[2].x};
+        float ov[3] = {st[2].y, st[2].z, st[2].w};
+        if (j + 1 < NGLL) {
+#pragma unroll
+          for (int s = 0; s < 3; s++)
+            st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + la + mrow];
+        }
+        if (SETS == 2) {
+          const float4* coef = att.table + 3 * (size_t)att.idx[la];
+#pragma unroll
+          for (int s = 0; s < 3; s++) cf[s] = coef[s];
+        }
+        attenuate_point(cf, ev, ov, kap, mu, dux_dxl, dux_dzl, duz_dxl, duz_dzl, sxx, sxz, szz);
+        if (active) att_store(att.state, att.ne, la, ev, ov);
+      }
+      if (RECT) {  // xi_z = gamma_x = 0: J xi_x = 1 / gamma_z, J gamma_z = 1 / xi_x
+        const float cx = 1.f / gazl, cz = 1.f / xixl;
+        t1[j] = make_float2(cx * sxx, cx * sxz);
+        t2[j] = make_float2(cz * sxz, cz * szz);
+      } else {
+        const float jac = 1.f / (xixl * gazl - gaxl * xizl);
+        t1[j] = make_float2(jac * (sxx * xixl + sxz * xizl), jac * (sxz * xixl + szz * xizl));
+        t2[j] = make_float2(jac * (sxx * gaxl + sxz * gazl), jac * (sxz * gaxl + szz * gazl));
+      }
+    }
+    // xi flux contraction: the element's rows through LDS
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) s_t[j * TROW + lane] = t1[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float2 f[NGLL];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      const float2 e0 = el[j * TROW], e1 = el[j * TROW + 1], e2 = el[j * TROW + 2], e3 = el[j * TROW + 3],
+                   e4 = el[j * TROW + 4];
+      const float sx = e0.x * hwi[0] + e1.x * hwi[1] + e2.x * hwi[2] + e3.x * hwi[3] + e4.x * hwi[4];
+      const float sz = e0.y * hwi[0] + e1.y * hwi[1] + e2.y * hwi[2] + e3.y * hwi[3] + e4.y * hwi[4];
+      float gx = 0.f, gz = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        const float h = basis.hpw[m * NGLL + j];
+        gx += t2[m].x * h;
+        gz += t2[m].y * h;
+      }
+      const float wj = basis.w[j];
+      f[j] = make_float2(-(wj * sx + wi * gx), -(wj * sz + wi * gz));
+    }
+    __builtin_amdgcn_wave_barrier();
+    // the shared column's force moves from element k - 1 (lane 5 k - 1) to element k (lane 5 k)
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      const float fx = __shfl_up(f[j].x, 1, 64);
+      const float fz = __shfl_up(f[j].y, 1, 64);
+      if (i == 0 && k > 0) {
+        f[j].x += fx;
+        f[j].y += fz;
+      }
+    }
+    f[0].x += carry.x;
+    f[0].y += carry.y;
+#pragma unroll
+    for (int j = 0; j < NGLL - 1; j++) finish(row[4 * c + j], off + (unsigned)j * up, f[j], u[j], vp[j], ms[j]);
+    carry = f[NGLL - 1];
+    u0 = u[NGLL - 1];
+    off = noff;
+    word = nword;
+    elem = nelem;
+  }
+  // the tower's top row
+  finish(row[4 * nch], off, carry, u0, ld_off(v, off), ld_off(rm, off / 2u));
+}
+
+// Interface points: the tower slots of each point summed in order, the boundary terms of accel added and cleared, and
+// the Newmark update; old (CPML layer points): u + dt^2 / 4 a of this step, the layer's previous-step field, zero on
+// the layer's outer boundary.
+__global__ __launch_bounds__(256) void k_interface(int n, int n2, const int* __restrict__ ids,
+                                                   const int2* __restrict__ s01, const int2* __restrict__ s23,
+                                                   const uint8_t* __restrict__ flag, const float2* __restrict__ partial,
+                                                   int npartial, const TowerFields F, const float* __restrict__ rmx,
+                                                   const float* __restrict__ rmz, const Newmark nm,
+                                                   float2* __restrict__ old, float dt2o4) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const long at = blockIdx.y * F.stride;
+  partial += (size_t)blockIdx.y * npartial;
+  const int g = ids[q];
+  const int fl = flag[q];
+  const int2 s = s01[q];
+  const float2 dd = F.d[at + g], vv = F.v[at + g];
+  const float wx = rmx[g], wz = rmz[g];
+  float2 r = make_float2(0.f, 0.f);
+  if (s.x >= 0) r = partial[s.x];
+  if (s.y >= 0) {
+    const float2 p = partial[s.y];
+    r.x += p.x;
+    r.y += p.y;
+  }
+  if (q >= n2) {
+    const int2 t = s23[q - n2];
+    const float2 p = partial[t.x];
+    r.x += p.x;
+    r.y += p.y;
+    if (t.y >= 0) {
+      const float2 p2 = partial[t.y];
+      r.x += p2.x;
+      r.y += p2.y;
+    }
+  }
+  if (fl & HAS_ACC) {
+    const float2 a = F.accel[at + g];
+    r.x += a.x;
+    r.y += a.y;
+    if (!F.last) F.accel[at + g] = make_float2(0.f, 0.f);
+  }
+  if ((fl & PML_POINT) && old) {
+    const float ax = r.x * wx, az = r.y * wz;
+    old[g] = (fl & PML_EDGE) ? make_float2(0.f, 0.f) : make_float2(fmaf(dt2o4, ax, dd.x), fmaf(dt2o4, az, dd.y));
+  }
+  newmark_point(nm, F, at, 8u * (unsigned)g, r, wx, wz, dd, vv);
+}
+
+// accel = 0 at the interface points with a boundary term (the start of a run of tower steps)
+__global__ __launch_bounds__(256) void k_interface_clear(int n, const int* __restrict__ ids,
+                                                         const uint8_t* __restrict__ flag, float2* __restrict__ accel) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n && (flag[q] & HAS_ACC)) accel[ids[q]] = make_float2(0.f, 0.f);
+}
+
+// Chains per tower: about one wave per slot of the card (4096 at four waves per SIMD) and at most 16.  A tall tower has
+// few interface rows (1 in 4 x chains), a short one more waves in flight.  Measured, ms of 300 steps of 600 x 300 elements
+// (15,000 chains) at 1, 2, 4, 8, 16 chains: 15.3, 13.9, 13.6, 14.2, 18.7; 40 steps of 2000 x 1000 (166,667 chains) at 2, 4,
+// 8, 16, 32: 19.9, 17.9, 17.2, 17.1, 17.6.
+int tower_chains(int nchain) {
+  if (const char* env = getenv("SF2D_TOWER_CHAINS")) return std::max(1, atoi(env));
+  return std::max(1, std::min(16, (nchain + 4095) / 4096));
+}
+
+// one step of the fields F at time step it (1-based): towers with the step's Stacey faces, sources and (seismo not null)
+// receivers, the CPML layer, the interface
+void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long seismo_stride, const int* src_shot,
+                  const Newmark& nm, bool forward) {
+  const TowerState* T = mp->tower;
+  const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
+  TowerEdges E{stacey_faces(mp), source_set(mp), receiver_set(mp), it - 1, mp->stacey ? (mp->num_abs * NGLL + 63) / 64 : 0,
+               mp->nsources_local, seismo ? mp->nrec_local : 0, src_shot, seismo, seismo_stride};
+  if ((long)(T->ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", T->ntower, F.nshot);
+  const int wgs = (T->ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
+  const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+  const int sets = !mp->attenuation ? 0 : mp->att_ntable == 1 ? 1 : 2;
+  using K = decltype(&k_tower<0, 0>);
+  const K kern[3][3] = {{k_tower<0, 0>, k_tower<0, 1>, k_tower<0, 2>},
+                        {k_tower<1, 0>, k_tower<1, 1>, k_tower<1, 2>},
+                        {k_tower<2, 0>, k_tower<2, 1>, k_tower<2, 2>}};
+  hipLaunchKernelGGL(kern[geo][sets], dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, T->ntower, T->d_desc,
+                     T->d_row, mp->d_geom, mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, T->d_partial, T->npartial, nm,
+                     mp->basis, att, wgs, E);
+  check_hip(hipGetLastError(), "k_tower launch");
+  if (forward)
+    for (int ph = 0; ph < 2; ph++) pml_elastic_forces(mp, ph);
+  if (T->nif == 0) return;
+  hipLaunchKernelGGL(k_interface, dim3((T->nif + 255) / 256, F.nshot), dim3(256), 0, mp->stream, T->nif, T->nif2,
+                     T->d_if_id, T->d_if_s, T->d_if_s2, T->d_if_flag, T->d_partial, T->npartial, F, mp->d_rmassx,
+                     mp->d_rmassz, nm, F.last ? nullptr : pml_old_field(mp), 0.5f * nm.dt2o2);
+  check_hip(hipGetLastError(), "k_interface launch");
+}
+
+}  // namespace
+
+void tower_release(Mesh* mp) {
+  TowerState* T = mp->tower;
+  if (!T) return;
+  device_free(T->d_desc); device_free(T->d_row); device_free(T->d_partial); device_free(T->d_if_id); device_free(T->d_if_s); device_free(T->d_if_s2);
+  device_free(T->d_if_flag);
+  delete T;
+  mp->tower = nullptr;
+}
+
+// whether every point inside a tower has one inverse mass for both components (rmassx, rmassz: caller's numbering)
+bool tower_masses_fit(const Mesh* mp, const float* rmassx, const float* rmassz) {
+  const TowerState* T = mp->tower;
+  for (int g = 0; g < mp->nglob; g++)
+    if (rmassx[g] != rmassz[g]) {
+      const int id = mp->point_id.empty() ? g : mp->point_id[g];
+      if (id < mp->nglob_el && !T->is_if[id]) return false;
+    }
+  return true;
+}
+
+}  // namespace sf2d
+
+using namespace sf2d;
+
+extern "C" {
+
+int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rmassz) {
+  Mesh* mp = handle(Mesh_pointer);
+  tower_release(mp);
+  if (!mp->chain || !mp->first_touch || !mp->d_col_rows || mp->assembly != 0 || mp->anisotropy || mp->batch ||
+      mp->save_forward || getenv("SF2D_NO_TOWERS"))
+    return 0;
+  const int npatch = mp->npatch;
+  const std::vector<int4>& rows = mp->h_col_rows;
+  const std::vector<int>& ends = mp->h_col_ends;
+  const std::vector<int>& pd = mp->h_patch_desc;
+  if ((int)mp->h_above.size() != npatch || (int)ends.size() != npatch * NGLL) return 0;
+  TowerState* T = new TowerState();
+  mp->tower = T;
+  // stacks of chains whose ids and positions go up in constant steps, cut into towers of about the same height
+  std::vector<char> has_below(npatch, 0);
+  for (int a : mp->h_above)
+    if (a >= 0) has_below[a] = 1;
+  auto regular = [&](int q) {  // the chain's own rows
+    const int4* r = rows.data() + (size_t)q * NGLL;
+    const int* e = ends.data() + (size_t)q * NGLL;
+    const int step = 4 * (pd[4 * q + 3] & 0xf) - 1;
+    for (int j = 1; j < NGLL; j++)
+      if (r[j].x != r[j - 1].x + step || r[j].y != r[j - 1].y + 1 || e[j] != e[j - 1] + 1) return false;
+    return true;
+  };
+  const int want = tower_chains(npatch);
+  struct Tower { int level, first, n; };
+  std::vector<Tower> towers;
+  std::vector<int> stack_chains;
+  for (int q = 0; q < npatch; q++) {
+    if (has_below[q]) continue;
+    int t = q;
+    while (t >= 0) {
+      const int s0 = (int)stack_chains.size();
+      do {
+        stack_chains.push_back(t);
+        if (!regular(t)) {  // such a chain needs its row records
+          tower_release(mp);
+          return 0;
+        }
+        const int a = mp->h_above[t];
+        const bool on = a >= 0 && pd[4 * a] == pd[4 * t] + (pd[4 * t + 3] & 0xf);
+        t = a;
+        if (!on) break;
+      } while (t >= 0);
+      const int len = (int)stack_chains.size() - s0, parts = (len + want - 1) / want;
+      for (int p = 0; p < parts; p++) {
+        const int a = (int)((long)len * p / parts), b = (int)((long)len * (p + 1) / parts);
+        towers.push_back({p, s0 + a, b - a});
+      }
+    }
+  }
+  if ((int)stack_chains.size() != npatch) {  // a closed ring of chains has no bottom
+    tower_release(mp);
+    return 0;
+  }
+  std::stable_sort(towers.begin(), towers.end(), [](const Tower& a, const Tower& b) { return a.level < b.level; });
+
+  // points that something besides the towers acts on or looks at
+  const int ng = mp->nglob;
+  std::vector<uint8_t> flag((size_t)ng, 0), cnt((size_t)ng, 0);
+  constexpr uint8_t LOOKED_AT = 0x80;
+  auto mark_element = [&](int ispec, uint8_t f) {
+    const int* ib = mp->h_chain_ids.data() + (size_t)mp->pos_of_ispec[ispec] * NGLL2;
+    for (int p = 0; p < NGLL2; p++) flag[ib[p]] |= f;
+  };
+  for (int e : mp->h_src_ispec) mark_element(e, HAS_ACC);
+  for (int e : mp->h_rec_ispec) mark_element(e, LOOKED_AT);
+  for (int g : mp->h_stacey_points) flag[g] |= HAS_ACC;
+  for (int g : mp->h_uncovered_points) flag[g] |= HAS_ACC;
+  for (int g : mp->h_coupling_points) flag[mp->point_id.empty() ? g : mp->point_id[g]] |= HAS_ACC;
+  for (int e : pml_solid_elements(mp)) mark_element(e, HAS_ACC | PML_POINT);
+  for (int g : mp->h_pml_points) flag[g] |= HAS_ACC | PML_EDGE;
+  for (int g = 0; g < ng; g++)
+    if (rmassx[g] != rmassz[g]) flag[mp->point_id.empty() ? g : mp->point_id[g]] |= LOOKED_AT;
+
+  const int nt = (int)towers.size();
+  std::vector<int4> desc((size_t)2 * nt);
+  int nrow = 0;
+  for (int t = 0; t < nt; t++) {
+    const int q = stack_chains[towers[t].first], n = towers[t].n;
+    const int4 r = rows[(size_t)q * NGLL];
+    desc[2 * t] = make_int4(pd[4 * q], n, pd[4 * q + 3] & 0xf, nrow);
+    desc[2 * t + 1] = make_int4(r.x, r.y, ends[(size_t)q * NGLL], 0);
+    nrow += 4 * n + 1;
+  }
+  // f(row record, first inner id, inner points, id of x = 0, id of x = 4 ne) over every GLL row of every tower
+  auto each_row = [&](auto f) {
+    for (int t = 0; t < nt; t++) {
+      const int4 a = desc[2 * t], b = desc[2 * t + 1];
+      for (int r = 0; r <= 4 * a.y; r++) f(a.w + r, b.x + 1 + r * (4 * a.z - 1), 4 * a.z - 1, b.y + r, b.z + r);
+    }
+  };
+  // how many towers hold each point
+  each_row([&](int, int g0, int n, int left, int right) {
+    for (int x = 0; x < n; x++) cnt[g0 + x]++;
+    cnt[left]++;
+    cnt[right]++;
+  });
+  T->is_if.assign((size_t)ng, 0);
+  std::vector<int> idx((size_t)ng, -1), order2, order4;
+  for (int g = 0; g < mp->nglob_el; g++) {
+    if (cnt[g] == 1 && !flag[g]) continue;
+    T->is_if[g] = 1;
+    if (cnt[g] > 4) {  // more towers around one point than the interface kernel sums
+      tower_release(mp);
+      return 0;
+    }
+    (cnt[g] <= 2 ? order2 : order4).push_back(g);
+  }
+  T->nif2 = (int)order2.size();
+  order2.insert(order2.end(), order4.begin(), order4.end());
+  T->nif = (int)order2.size();
+  for (int q = 0; q < T->nif; q++) idx[order2[q]] = q;
+  std::vector<int4> row((size_t)nrow);
+  std::vector<int> slots((size_t)4 * T->nif, -1);
+  int np = 0;
+  each_row([&](int r, int g0, int n, int left, int right) {
+    unsigned long long m = 0ull;
+    const int first = np;
+    auto take = [&](int x, int g) {
+      if (!T->is_if[g]) return;
+      m |= 1ull << x;
+      int* sl = slots.data() + (size_t)4 * idx[g];
+      while (*sl >= 0) sl++;
+      *sl = np++;
+    };
+    take(0, left);
+    for (int x = 0; x < n; x++) take(x + 1, g0 + x);
+    take(n + 1, right);
+    row[r] = make_int4((int)(unsigned)(m & 0xffffffffull), (int)(unsigned)(m >> 32), first, 0);
+  });
+  std::vector<int2> s01((size_t)T->nif), s23((size_t)(T->nif - T->nif2));
+  std::vector<uint8_t> fl((size_t)T->nif);
+  for (int q = 0; q < T->nif; q++) {
+    s01[q] = make_int2(slots[4 * (size_t)q], slots[4 * (size_t)q + 1]);
+    if (q >= T->nif2) s23[q - T->nif2] = make_int2(slots[4 * (size_t)q + 2], slots[4 * (size_t)q + 3]);
+    fl[q] = flag[order2[q]] & (HAS_ACC | PML_POINT | PML_EDGE);
+  }
+  T->ntower = nt;
+  T->nrow = nrow;
+  T->npartial = np;
+  T->d_desc = device_copy(desc.data(), desc.size());
+  T->d_row = device_copy(row.data(), row.size());
+  T->d_partial = device_alloc<float2>((size_t)np);
+  T->d_if_id = device_copy(order2.data(), order2.size());
+  T->d_if_s = device_copy(s01.data(), s01.size());
+  T->d_if_s2 = device_copy(s23.data(), s23.size());
+  T->d_if_flag = device_copy(fl.data(), fl.size());
+  return 1;
+}
+
+int sf2d_tower_ready(long* Mesh_pointer) { return handle(Mesh_pointer)->tower != nullptr; }
+
+void sf2d_tower_begin(long* Mesh_pointer) {
+  Mesh* mp = handle(Mesh_pointer);
+  const TowerState* T = mp->tower;
+  if (!T) fail("sf2d_tower_begin: no towers");
+  if (T->nif == 0) return;
+  hipLaunchKernelGGL(k_interface_clear, dim3((T->nif + 255) / 256), dim3(256), 0, mp->stream, T->nif, T->d_if_id,
+                     T->d_if_flag, (float2*)mp->d_accel);
+  check_hip(hipGetLastError(), "k_interface_clear launch");
+}
+
+void sf2d_tower_step(long* Mesh_pointer, int it, int last, float deltat, float deltatsqover2, float deltatover2) {
+  Mesh* mp = handle(Mesh_pointer);
+  if (!mp->tower || !mp->accel_partial || mp->pending_corrector[0])
+    fail("sf2d_tower_step: call after update_displacement_cuda and sf2d_tower_begin");
+  if (it < 1 || it > mp->nstep) fail("sf2d_tower_step: it=%d outside 1..%d", it, mp->nstep);
+  float2 *d = (float2*)mp->d_displ, *v = (float2*)mp->d_veloc;
+  const TowerFields F{d, v, d, v, nullptr, (float2*)mp->d_accel, 0, 1, last};
+  // displacement of the receivers in solid elements; the fluid records its own, and the caller the run's last step
+  const int record = !last && mp->nrec_local > 0 && mp->h_seismotype[0] == 1;
+  if (record && it > mp->nlength_seismogram) fail("sf2d_tower_step: step %d after the seismograms' last", it);
+  launch_tower(mp, F, it, record ? mp->d_seismo[0] : nullptr, 0, nullptr, {deltatover2, deltat, deltatsqover2}, true);
+  if (last) mp->accel_partial = 0;
+}
+
+}  // extern "C"

@@ -1,0 +1,91 @@
+"""The fused time step (towers of chains and the interface between them) against the unfused kernels and the oracle,
+at the shapes where it can go wrong: towers of one chain and of a whole column, chain remainders (a mesh width that is
+not a multiple of 12 elements), a single row of elements, the three geometry forms, one and several attenuation
+coefficient sets, and every kind of interface point (Stacey edges, sources, receivers, CPML, fluid-solid edges)."""
+import numpy as np
+import pytest
+
+from oracle.oracle import OracleSim
+from specfem2d_amd import config
+from specfem2d_amd.config import Source
+from specfem2d_amd.driver import Simulation
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / np.linalg.norm(b))
+
+
+def make(form, nx, nz, nstep=160):
+    if form == "coupled":
+        src = [Source(x=nx * 47.0, z=-nz * 70.0, f0=8.0, factor=1.0e9)]
+        rec = np.array([[nx * 30.0, -nz * 80.0], [nx * 80.0, -60.0], [nx * 55.0, -nz * 45.0]])
+        return config.layered_fluid_solid(nx, nz, max(1, nz // 4), 100.0, nstep, 2.0e-3, sources=src, receivers=rec)
+    cfg = config.small_test_mesh(nx=nx, nz=nz, nstep=nstep, gll=True, seed=3)
+    if form in ("cpml", "visco_cpml"):
+        cfg = cfg.replace(stacey=False, pml=True, nelem_pml=3)
+    if form == "layers":  # rows of two heights: affine elements, not all alike; z sources stay inside
+        cfg = cfg.replace(interfaces=[-nz * 100.0, -nz * 45.0, 0.0], nz_layers=[nz // 2, nz - nz // 2])
+    if form in ("visco", "visco_cpml"):
+        cfg = cfg.replace(attenuation=True, qkappa=60.0, qmu=40.0)
+    if form == "visco_sets":  # two coefficient sets
+        q = np.where(np.repeat(np.arange(nx * nz) % nx < nx // 2, 25), 40.0, 70.0)
+        cfg = cfg.replace(attenuation=True, qkappa=q, qmu=0.7 * q)
+    return cfg
+
+
+def run(cfg, pieces=None):
+    sim = Simulation(cfg)
+    seis = np.concatenate([sim.forward(nstep=n)[0] for n in (pieces or [cfg.nstep])], axis=-1)
+    out = [seis, *sim.fields()]
+    if sim.nspec_acoustic:
+        out += list(sim.acoustic_fields())
+    sim.close()
+    return out
+
+
+# displacement and seismograms: sums of the same 32-bit terms in another order, grown over 160 steps: below 1e-5, the
+# bound of every comparison with the oracle here.  The velocity and, more so, the acceleration M^-1 K d hold short
+# waves whose terms cancel: omega_max / omega, about 1e2 at these element sizes, once and twice.
+BOUNDS = [1e-5, 1e-5, 1e-4, 1e-3, 1e-5, 1e-4, 1e-3]
+
+
+@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "layers", "points", "visco", "visco_sets", "visco_cpml"])
+@pytest.mark.parametrize("nx,nz,chains", [(12, 12, 1), (25, 17, 3), (38, 13, 64), (13, 2, 64)])
+def test_fused_step_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
+    if nz < 12 and form not in ("stacey", "points", "visco", "visco_sets"):
+        pytest.skip("too flat for layers")
+    if form == "points":
+        monkeypatch.setenv("SF2D_NO_AFFINE", "1")
+    cfg = make("stacey" if form == "points" else form, nx, nz)
+    monkeypatch.setenv("SF2D_TOWER_CHAINS", str(chains))
+    fused = run(cfg)
+    monkeypatch.setenv("SF2D_NO_TOWERS", "1")
+    plain = run(cfg)
+    for a, b, tol in zip(fused, plain, BOUNDS):
+        assert np.linalg.norm(b) > 0 and rel(a, b) < tol
+    ref = OracleSim(cfg, "sp").forward()
+    assert rel(fused[0], ref) < 1e-5
+
+
+@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "visco"])
+def test_a_run_in_pieces_gives_the_bits_of_the_run_in_one(form):
+    cfg = make(form, 27, 16)
+    for a, b in zip(run(cfg), run(cfg, [1, 2, 57, cfg.nstep - 60])):
+        assert np.array_equal(a, b)
+
+
+def test_setting_the_same_model_again_keeps_the_run():
+    """New materials on a prepared handle: the fused step reads them (and the two inverse masses) from then on."""
+    cfg = make("stacey", 25, 17)
+    sim = Simulation(cfg)
+    want = sim.forward()[0]
+    sim.set_model(1.1 * cfg.rho, cfg.vp, cfg.vs)
+    sim.reset()
+    other = sim.forward()[0]
+    sim.set_model(cfg.rho, cfg.vp, cfg.vs)
+    sim.reset()
+    again = sim.forward()[0]
+    sim.close()
+    assert rel(again, want) < 1e-6 and rel(other, want) > 1e-2
