@@ -58,18 +58,26 @@ int sf2d_mesh_fluid_chain(long* Mesh_pointer);
 /* 1 when every element is affine and axis-aligned (xi_z = gamma_x = 0 to 2^-22 of the element's largest geometry
    entry): the chain kernel then uses its rectangle form (SF2D_NO_RECT keeps the general form) */
 int sf2d_mesh_rect(long* Mesh_pointer);
-/* The fused time step of the solid (forward runs of chain meshes; no counterpart in the reference): corrector of step
-   n and predictor of step n + 1 inside the force kernel, two launches a step.
-   sf2d_tower_prepare, after all other preparation (rmassx, rmassz as prepare_fields_elastic_device_ got them), returns
-   1 when the handle can run it (SF2D_NO_TOWERS: never).  A run of such steps starts after update_displacement_cuda_ of
-   its first step with sf2d_tower_begin; in each step the CPML zero condition and the fluid-solid coupling are called as
-   usual and sf2d_tower_step(it) takes the place of the forces, Stacey edges, sources, kernel_3_a_cuda_, the displacement
-   seismograms of receivers in solid elements and the next step's update_displacement_cuda_.  The run's last step
-   (last = 1) ends with the step's displacement, velocity and acceleration instead, and its seismograms are the caller's. */
+/* The fused time step (forward runs of chain meshes; no counterpart in the reference): corrector of step n and predictor
+   of step n + 1 inside the force kernel.
+   Solid: sf2d_tower_prepare, after all other preparation (rmassx, rmassz as prepare_fields_elastic_device_ got them),
+   returns 1 when the handle can run it (SF2D_NO_TOWERS: never).  A run of such steps starts after
+   update_displacement_cuda_ (and, with CPML, pml_boundary_elastic_cuda_) of its first step with sf2d_tower_begin;
+   sf2d_tower_step(it) takes the place of the forces, Stacey edges, fluid-solid edges, sources, kernel_3_a_cuda_, the
+   displacement seismograms of receivers in solid elements and, for the next step, update_displacement_cuda_ and
+   pml_boundary_elastic_cuda_.  The
+   run's last step (last = 1) ends with the step's displacement, velocity and acceleration instead, and its seismograms
+   are the caller's.
+   Fluid: sf2d_tower_fluid_ready is 1 when it can run; sf2d_tower_fluid_step likewise, from the predicted potential (first:
+   the run's first step, after acoustic_enforce_free_surf_cuda_) and before the solid's step.  trick: pressure is minus the
+   potential; else minus its second derivative, which the next step records. */
 int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rmassz);
 int sf2d_tower_ready(long* Mesh_pointer);
 void sf2d_tower_begin(long* Mesh_pointer);
 void sf2d_tower_step(long* Mesh_pointer, int it, int last, float deltat, float deltatsqover2, float deltatover2);
+int sf2d_tower_fluid_ready(long* Mesh_pointer);
+void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int trick, float deltat, float deltatsqover2,
+                           float deltatover2);
 /* tuning knobs (specfem2d_amd/autotune.py picks them by timing): elements per chain patch, chosen at set-up
    from SF2D_CHAIN_ELEMS (1..12, default 12), and shots per wave of the batched chain kernel (0 = default 8;
    SF2D_SHOTS_PER_WAVE at set-up) */

@@ -25,14 +25,16 @@
 #include <vector>
 
 #include "sf2d_mesh.h"
+#include "sf2d_tower.h"
 #include "specfem2d_gpu.h"
+#include "specfem2d_gpu_ext.h"
 
 namespace sf2d {
 
 namespace {
 constexpr int AC_EPB = 10;  // fluid elements per 256-thread workgroup (250 active lanes)
 
-__device__ __forceinline__ void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
+__device__ __forceinline__ void atomic_add(float* p, float v) { atomic_add_f32(p, v); }
 
 // One colour of fluid elements: pdd -= K pot over elements first .. first+n-1 of the packed colour order
 // (compute_forces_viscoacoustic.f90:107-330; Kernel_2_acoustic_impl in src/gpu/kernels).  RECT: every element is
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(256) void k_acoustic_forces(int first, int n, const
 // shuffle, and each point of the chain is updated by one lane with a read-modify-write of pdd (no point is shared
 // between the chains of one colour).  Same element operator as k_acoustic_forces.
 constexpr int AC_CHAIN = 12;
-constexpr int AC_NXCD = 8;  // XCD-contiguous blocks of chains, as the solid's kernels
+constexpr int AC_NXCD = NXCD;  // XCD-contiguous blocks of chains, as the solid's kernels
 template <bool RECT>
 __global__ __launch_bounds__(64) void k_acoustic_forces_col(int first_patch, int npatch,
                                                             const int4* __restrict__ desc,
@@ -281,18 +283,29 @@ __global__ __launch_bounds__(256) void k_ac_free_surface(const int* __restrict__
   pdd[g] = 0.f;
 }
 
-// compute_stacey_acoustic.f90:34-160: pdd -= pd w / (rho vp) along the fluid's absorbing edges; with store, each
-// term also goes to its edge slot (the SAVE_FORWARD copy b_absorb_acoustic_*, :46-48, 65-67, 86-88, 107-109)
-__global__ __launch_bounds__(256) void k_ac_stacey(int n, const int* __restrict__ pts, const float* __restrict__ w,
-                                                   const float* __restrict__ rvp, const float* __restrict__ pd,
+// the fluid's absorbing edge points: ids, weights, rho vp
+struct FluidStacey {
+  int n;
+  const int* pts;
+  const float *w, *rvp;
+};
+// compute_stacey_acoustic.f90:34-160: pdd -= pd w / (rho vp) along the fluid's absorbing edges; returns the term
+__device__ __forceinline__ float fluid_stacey(const FluidStacey& S, int k, const float* __restrict__ pd,
+                                              float* __restrict__ pdd) {
+  if (k >= S.n) return 0.f;
+  const int g = S.pts[k];
+  const float t = pd[g] * S.w[k] / S.rvp[k];
+  atomic_add(&pdd[g], -t);
+  return t;
+}
+// with store, each term also goes to its edge slot (the SAVE_FORWARD copy b_absorb_acoustic_*, :46-48, 65-67, 86-88,
+// 107-109)
+__global__ __launch_bounds__(256) void k_ac_stacey(const FluidStacey S, const float* __restrict__ pd,
                                                    float* __restrict__ pdd, const int* __restrict__ slot,
                                                    float* __restrict__ store) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int g = pts[k];
-  const float t = pd[g] * w[k] / rvp[k];
-  atomic_add(&pdd[g], -t);
-  if (store) store[slot[k]] = t;
+  const float t = fluid_stacey(S, k, pd, pdd);
+  if (store && k < S.n) store[slot[k]] = t;
 }
 
 // reconstructed field: b_pdd -= the stored term of step NSTEP - it + 1 (compute_stacey_acoustic.f90:162-240)
@@ -304,46 +317,31 @@ __global__ __launch_bounds__(256) void k_ac_stacey_backward(int n, const int* __
   atomic_add(&bpdd[pts[k]], -store[slot[k]]);
 }
 
-// fluid side of a fluid-solid edge: pdd += w (u . n) (compute_coupling_acoustic_el.f90:34-150); sign -1 gives the
-// adjoint run's term, u = minus the adjoint acceleration (:104-109)
-__global__ __launch_bounds__(256) void k_coupling_ac_el(int n, const int* __restrict__ pts,
-                                                        const float2* __restrict__ nrm, const float* __restrict__ w,
-                                                        const float2* __restrict__ displ, float sign,
-                                                        float* __restrict__ pdd) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int g = pts[k];
-  const float2 u = displ[g], nv = nrm[k];
-  const float dn = (sign * u.x) * nv.x + (sign * u.y) * nv.y;
-  atomic_add(&pdd[g], w[k] * dn);
+__global__ __launch_bounds__(256) void k_coupling_ac_el(const CouplingPoints C, const float2* __restrict__ displ,
+                                                        float sign, float* __restrict__ pdd) {
+  couple_fluid(C, blockIdx.x * blockDim.x + threadIdx.x, displ, sign, pdd);
 }
 
-// solid side: accel += w n p with the fluid pressure p = -pdd (compute_coupling_viscoelastic_ac.f90:34-130); with
-// sign -1 and the adjoint potential in place of pdd, the adjoint run's pressure p = potential (:98-102)
-__global__ __launch_bounds__(256) void k_coupling_el_ac(int n, const int* __restrict__ pts,
-                                                        const float2* __restrict__ nrm, const float* __restrict__ w,
-                                                        const float* __restrict__ pdd, float sign,
+__global__ __launch_bounds__(256) void k_coupling_el_ac(const CouplingPoints C, const float* __restrict__ pdd, float sign,
                                                         float* __restrict__ accel) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int g = pts[k];
-  const float pr = sign * -pdd[g];
-  const float2 nv = nrm[k];
-  const float wk = w[k];
-  atomic_add(&accel[2 * (size_t)g], wk * nv.x * pr);
-  atomic_add(&accel[2 * (size_t)g + 1], wk * nv.y * pr);
+  couple_solid(C, blockIdx.x * blockDim.x + threadIdx.x, pdd, sign, accel);
 }
 
+// sources in fluid elements: their rows in the source time functions, points, Lagrange weights and kappa
+struct FluidSources {
+  int n, nsrc;
+  const int *src, *pts;
+  const float *sa, *kap, *stf;
+};
 // pressure sources in fluid elements: pdd += h stf / kappa (compute_add_sources_acoustic.f90:34-75)
-__global__ __launch_bounds__(64) void k_ac_sources(int nas, int it, int nsrc, const int* __restrict__ src,
-                                                   const int* __restrict__ pts, const float* __restrict__ sa,
-                                                   const float* __restrict__ kap, const float* __restrict__ stf,
-                                                   float* __restrict__ pdd) {
-  const int s = blockIdx.x, p = threadIdx.x;
-  if (s >= nas || p >= NGLL2) return;
+__device__ __forceinline__ void fluid_source(const FluidSources& S, int s, int p, int it, float* __restrict__ pdd) {
+  if (s >= S.n || p >= NGLL2) return;
   const size_t l = (size_t)s * NGLL2 + p;
-  const float f = stf[(size_t)it * nsrc + src[s]];
-  atomic_add(&pdd[pts[l]], sa[l] * f / kap[l]);
+  const float f = S.stf[(size_t)it * S.nsrc + S.src[s]];
+  atomic_add(&pdd[S.pts[l]], S.sa[l] * f / S.kap[l]);
+}
+__global__ __launch_bounds__(64) void k_ac_sources(const FluidSources S, int it, float* __restrict__ pdd) {
+  fluid_source(S, blockIdx.x, threadIdx.x, it, pdd);
 }
 
 // adjoint sources of receivers in fluid elements: pdd += h_i h_j adj(NSTEP - it + 1), without a 1/kappa factor
@@ -408,29 +406,25 @@ __global__ __launch_bounds__(256) void k_ac_kernels(int nrows, const int* __rest
   kappa_kl[l] = __fadd_rn(kappa_kl[l], __fmul_rn(__fmul_rn(__fmul_rn(1.f / m.y, pdd[g]), s_b[le][p]), dt));
 }
 
-// pressure (sign = -1: -potential or -potential_dot_dot) or potential (sign = +1) seismograms of the receivers in
-// fluid elements, interpolated with the receivers' Lagrange weights and accumulated in double
-// (write_seismograms.F90:124-170, compute_pressure.f90:460-490, compute_interpolated_dva.f90); receivers in solid
-// elements (pts = -1) record 0
-// displacement, velocity or acceleration seismograms (seismotypes 1, 2, 3) of the receivers in fluid elements: the
-// gradient over the density of the potential or of its first or second time derivative at each point of the element, interpolated with the receivers' Lagrange weights and rotated
-// (compute_elastic_seismogram_kernel.cu:120-175, compute_vector_field.f90:143-210); one block per receiver, blocks
-// of receivers in solid elements (pts = -1) leave the displacement recorded there untouched
-__global__ __launch_bounds__(64) void k_ac_vector_seismograms(int nrec, int nlength, int cur,
-                                                              const int* __restrict__ pts,
-                                                              const float4* __restrict__ geom,
-                                                              const float* __restrict__ rho, Basis b,
-                                                              const float* __restrict__ xir,
-                                                              const float* __restrict__ gammar,
-                                                              const float* __restrict__ cosrot,
-                                                              const float* __restrict__ sinrot,
-                                                              const float* __restrict__ field,
-                                                              float* __restrict__ dst) {
-  __shared__ float s[NGLL2];
-  const int r = blockIdx.x, p = threadIdx.x;
-  if (r >= nrec || pts[(size_t)r * NGLL2] < 0) return;  // uniform over the block
+// receivers: points (-1 rows: receivers in solid elements), geometry and density of the fluid ones
+struct FluidReceivers {
+  int nrec, nlength;
+  const int* pts;
+  const float4* geom;
+  const float* rho;
+  const float *xir, *gammar, *cosrot, *sinrot;
+};
+// displacement, velocity or acceleration (seismotypes 1, 2, 3) of receiver r in a fluid element: the gradient over the
+// density of the potential or of its first or second time derivative at each point of the element, interpolated with
+// the receiver's Lagrange weights and rotated (compute_elastic_seismogram_kernel.cu:120-175,
+// compute_vector_field.f90:143-210); receivers in solid elements (pts = -1) keep what is recorded there.  One wave per
+// receiver; s: 25 floats of LDS of the wave's own
+__device__ __forceinline__ void fluid_vector_receiver(const FluidReceivers& R, int r, int p, int cur, const Basis& b,
+                                                      const float* __restrict__ field, float* __restrict__ dst,
+                                                      float* __restrict__ s) {
+  if (r >= R.nrec || R.pts[(size_t)r * NGLL2] < 0) return;  // uniform over the wave
   const size_t l = (size_t)r * NGLL2 + p;
-  if (p < NGLL2) s[p] = field[pts[l]];
+  if (p < NGLL2) s[p] = field[R.pts[l]];
   __syncthreads();
   double vx = 0.0, vz = 0.0;
   if (p < NGLL2) {
@@ -441,10 +435,10 @@ __global__ __launch_bounds__(64) void k_ac_vector_seismograms(int nrec, int nlen
       t1 += s[j * NGLL + k] * b.hp[i * NGLL + k];
       t2 += s[k * NGLL + i] * b.hp[j * NGLL + k];
     }
-    const float4 g = geom[l];
-    const float fx = (t1 * g.x + t2 * g.z) / rho[l];
-    const float fz = (t1 * g.y + t2 * g.w) / rho[l];
-    const double h = (double)(xir[i * nrec + r] * gammar[j * nrec + r]);
+    const float4 g = R.geom[l];
+    const float fx = (t1 * g.x + t2 * g.z) / R.rho[l];
+    const float fz = (t1 * g.y + t2 * g.w) / R.rho[l];
+    const double h = (double)(R.xir[i * R.nrec + r] * R.gammar[j * R.nrec + r]);
     vx = (double)fx * h;
     vz = (double)fz * h;
   }
@@ -454,32 +448,292 @@ __global__ __launch_bounds__(64) void k_ac_vector_seismograms(int nrec, int nlen
     vz += __shfl_xor(vz, off, 64);
   }
   if (p == 0) {
-    const double c = cosrot[r], sn = sinrot[r];
-    dst[(size_t)r * nlength + cur] = (float)(c * vx + sn * vz);
-    dst[((size_t)nrec + r) * nlength + cur] = (float)(-sn * vx + c * vz);
+    const double c = R.cosrot[r], sn = R.sinrot[r];
+    dst[(size_t)r * R.nlength + cur] = (float)(c * vx + sn * vz);
+    dst[((size_t)R.nrec + r) * R.nlength + cur] = (float)(-sn * vx + c * vz);
   }
 }
 
-__global__ __launch_bounds__(64) void k_ac_seismograms(int nrec, int nlength, int cur, const int* __restrict__ pts,
-                                                       const float* __restrict__ xir, const float* __restrict__ gammar,
-                                                       const float* __restrict__ field, float sign,
-                                                       float* __restrict__ dst) {
-  const int r = blockIdx.x, p = threadIdx.x;
-  if (r >= nrec) return;
+// pressure (sign = -1: -potential or -potential_dot_dot) or potential (sign = +1) of receiver r in a fluid element,
+// interpolated with the receiver's Lagrange weights and accumulated in double (write_seismograms.F90:124-170,
+// compute_pressure.f90:460-490, compute_interpolated_dva.f90); receivers in solid elements (pts = -1) record 0
+__device__ __forceinline__ void fluid_scalar_receiver(const FluidReceivers& R, int r, int p, int cur,
+                                                      const float* __restrict__ field, float sign,
+                                                      float* __restrict__ dst) {
+  if (r >= R.nrec) return;
   double v = 0.0;
   if (p < NGLL2) {
-    const int g = pts[(size_t)r * NGLL2 + p];
+    const int g = R.pts[(size_t)r * NGLL2 + p];
     if (g >= 0) {
       const int i = p % NGLL, j = p / NGLL;
-      const double h = (double)(xir[i * nrec + r] * gammar[j * nrec + r]);
+      const double h = (double)(R.xir[i * R.nrec + r] * R.gammar[j * R.nrec + r]);
       v = (double)(sign * field[g]) * h;
     }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   if (p == 0) {
-    dst[(size_t)r * nlength + cur] = (float)v;
-    dst[((size_t)nrec + r) * nlength + cur] = 0.f;
+    dst[(size_t)r * R.nlength + cur] = (float)v;
+    dst[((size_t)R.nrec + r) * R.nlength + cur] = 0.f;
+  }
+}
+
+__global__ __launch_bounds__(64) void k_ac_vector_seismograms(const FluidReceivers R, int cur, Basis b,
+                                                              const float* __restrict__ field,
+                                                              float* __restrict__ dst) {
+  __shared__ float s[NGLL2];
+  fluid_vector_receiver(R, blockIdx.x, threadIdx.x, cur, b, field, dst, s);
+}
+
+__global__ __launch_bounds__(64) void k_ac_seismograms(const FluidReceivers R, int cur, const float* __restrict__ field,
+                                                       float sign, float* __restrict__ dst) {
+  fluid_scalar_receiver(R, blockIdx.x, threadIdx.x, cur, field, sign, dst);
+}
+
+// The fused step of the fluid (see tower.hip): one wave walks up a tower of chains, lane 5 k + i holding column i of
+// element k, and makes the corrector of this step and the predictor of the next one at every point inside the tower; the
+// forces of interface points go to slots, which k_ac_interface sums.  The free surface and the CPML layer's outer
+// boundary stay zero.  Every point's sum is made in the order and with the roundings of the launch per colour
+// (k_acoustic_forces_col, the CPML layer's kernel, k_ac_corrector, k_ac_predictor): the potential's short waves carry the
+// rounding errors of each step on, and a displacement is its gradient, so that any other order shows in the fifth digit.
+// Small meshes are bound by launches (two a step instead of twelve: 44 x 44 elements, 800 steps, 37.8 -> 14.9 ms), large
+// ones by HBM (with the solid's step and the CPML layer in one launch each, 1000 x 500 fluid-solid elements, 100 steps:
+// 24.1 -> 16.7 ms).
+struct FluidFields {
+  float *pot, *pd, *pdd;
+  float* acc;   // boundary terms at interface points, zero between the steps
+  int last;     // the step ends a run: pdd = a_n, pd = its value of step n
+};
+
+// corrector of this step and predictor of the next one (k_ac_corrector's and k_ac_predictor's operations, contracted the
+// same way) at point g
+__device__ __forceinline__ void fluid_newmark(const Newmark& c, const FluidFields& F, unsigned g, float a, float pot,
+                                              float pd) {
+  pd = fmaf(c.dto2, a, pd);
+  if (F.last) {
+    F.pdd[g] = a;
+  } else {
+    F.pot[g] = fmaf(c.dt2o2, a, fmaf(c.dt, pd, pot));
+    pd = fmaf(c.dto2, a, pd);
+  }
+  F.pd[g] = pd;
+}
+
+struct FluidEdges {
+  FluidStacey faces;
+  FluidSources sources;
+  FluidReceivers receivers;
+  CouplingPoints coupling;
+  const float2* displ;
+  int it;                  // 0-based time sample
+  int nface_wg, nsource, ncoupling_wg, nreceiver;
+  int record, vector;      // the receivers' sample, and whether they record the field's gradient over the density (else
+  float sign;              // sign x field)
+  const float* field;
+  float* seismo;
+};
+
+__device__ __forceinline__ void fluid_edges(const FluidEdges& E, const FluidFields& F, int wg, const Basis& b, float* lds) {
+  const int t = threadIdx.x;
+  if (wg < E.nface_wg) {
+    fluid_stacey(E.faces, wg * 64 + t, F.pd, F.acc);
+    return;
+  }
+  wg -= E.nface_wg;
+  if (wg < E.nsource) {
+    fluid_source(E.sources, wg, t, E.it, F.acc);
+    return;
+  }
+  wg -= E.nsource;
+  if (wg < E.ncoupling_wg) {
+    couple_fluid(E.coupling, wg * 64 + t, E.displ, 1.f, F.acc);
+    return;
+  }
+  wg -= E.ncoupling_wg;
+  if (E.vector)
+    fluid_vector_receiver(E.receivers, wg, t, E.record, b, E.field, E.seismo, lds);
+  else
+    fluid_scalar_receiver(E.receivers, wg, t, E.record, E.field, E.sign, E.seismo);
+}
+
+template <bool RECT>
+__global__ __launch_bounds__(64) void k_ac_tower(int ntower, const int4* __restrict__ desc, const int4* __restrict__ rows,
+                                                 const float* __restrict__ fac, const float4* __restrict__ geom,
+                                                 const float2* __restrict__ rect, const FluidFields F,
+                                                 const float* __restrict__ rm, float* __restrict__ slot, const Newmark nm,
+                                                 const Basis basis, int tower_wgs, const FluidEdges edges) {
+  __shared__ float s_t[NGLL * 64 + 1];
+  if ((int)blockIdx.x >= tower_wgs) {
+    fluid_edges(edges, F, blockIdx.x - tower_wgs, basis, s_t);
+    return;
+  }
+  const int tower = (blockIdx.x % NXCD) * (tower_wgs / NXCD) + blockIdx.x / NXCD;
+  if (tower >= ntower) return;  // uniform over the wave
+  const int4 td = desc[4 * tower], tb = desc[4 * tower + 1], ts = desc[4 * tower + 2], tt = desc[4 * tower + 3];
+  const int nch = td.y, ne = td.z;
+  const int4* const row = rows + td.w;
+  const int lane = threadIdx.x;
+  const int k = min(lane / NGLL, AC_CHAIN);
+  const int i = lane % NGLL;
+  const int kk = min(k, ne - 1);
+  const int x = 4 * kk + i;
+  const int xe = 4 * ne;
+  const bool writer = lane / NGLL < ne && (i < NGLL - 1 || k == ne - 1);
+  const unsigned below_lo = x < 32 ? (1u << x) - 1u : ~0u, below_hi = x < 32 ? 0u : (1u << (x - 32)) - 1u;
+  float hpi[NGLL], hwi[NGLL];
+#pragma unroll
+  for (int m = 0; m < NGLL; m++) {
+    hpi[m] = basis.hp[i * NGLL + m];
+    hwi[m] = basis.hpw[m * NGLL + i];
+  }
+  const float wi = basis.w[i];
+  // point ids: row 0 of the current chain, its row 1 (from there the rows go up by `up`), the tower's topmost row
+  auto point = [&](const int4 r) { return (unsigned)(x == 0 ? r.y : x == xe ? r.z : r.x + x); };
+  unsigned g0 = point(tb), g1 = point(ts);
+  const unsigned gt = point(tt);
+  const unsigned up = x == 0 || x == xe ? 1u : (unsigned)(xe - 1);
+  unsigned word = (unsigned)td.x * NGLL2 + (unsigned)min(lane, NGLL * ne - 1);
+  unsigned elem = (unsigned)(td.x + kk);
+  const unsigned mrow = (unsigned)(NGLL * ne);
+  float nu[NGLL - 1], nf[NGLL];  // the next chain's potential of rows 1 .. 4 and J / rho
+  float2 nr = make_float2(0.f, 0.f);
+  auto load_chain = [&](unsigned o1, bool top, unsigned w, unsigned e) {
+#pragma unroll
+    for (int j = 0; j < NGLL - 2; j++) nu[j] = F.pot[o1 + (unsigned)j * up];
+    nu[NGLL - 2] = F.pot[top ? gt : o1 + (unsigned)(NGLL - 2) * up];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) nf[j] = fac[w + (unsigned)j * mrow];
+    if (RECT) nr = rect[e];
+  };
+  auto finish = [&](const int4 r, unsigned g, float f, float u, float pd, float m) {
+    if (!writer) return;
+    const unsigned bits = x < 32 ? (unsigned)r.x >> x : (unsigned)r.y >> (x - 32);
+    if (bits & 1u)
+      slot[r.z + __popc((unsigned)r.x & below_lo) + __popc((unsigned)r.y & below_hi)] = f;
+    else
+      fluid_newmark(nm, F, g, f * m, u, pd);
+  };
+  auto edge_bit = [&](const int4 r) { return ((xe < 32 ? (unsigned)r.x >> xe : (unsigned)r.y >> (xe - 32)) & 1u) != 0; };
+  float u0 = F.pot[g0], carry = 0.f;
+  load_chain(g1, nch == 1, word, elem);
+  const float* const el = s_t + NGLL * k;
+  for (int c = 0; c < nch; c++) {
+    float u[NGLL], fc[NGLL], pd[NGLL - 1], ms[NGLL - 1];
+    u[0] = u0;
+#pragma unroll
+    for (int j = 1; j < NGLL; j++) u[j] = nu[j - 1];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) fc[j] = nf[j];
+    const float2 gr = nr;
+#pragma unroll
+    for (int j = 0; j < NGLL - 1; j++) {
+      const unsigned g = j == 0 ? g0 : g1 + (unsigned)(j - 1) * up;
+      pd[j] = F.pd[g];
+      ms[j] = rm[g];
+    }
+    const unsigned ng = g1 + 4u * up;
+    const unsigned cword = word, celem = elem;
+    (void)celem;
+    word += (unsigned)NGLL * mrow;
+    elem += (unsigned)ne;
+    if (c + 1 < nch) load_chain(ng, c + 2 == nch, word, elem);
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) s_t[j * 64 + lane] = u[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float t1[NGLL], t2[NGLL];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      float dxi = 0.f, dga = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        dxi += el[j * 64 + m] * hpi[m];
+        dga += u[m] * basis.hp[j * NGLL + m];
+      }
+      if (RECT) {
+        t1[j] = fc[j] * (gr.x * (dxi * gr.x));
+        t2[j] = fc[j] * (gr.y * (dga * gr.y));
+      } else {
+        const float4 gm = geom[cword + (unsigned)j * mrow];
+        const float dxl = dxi * gm.x + dga * gm.z;
+        const float dzl = dxi * gm.y + dga * gm.w;
+        t1[j] = fc[j] * (gm.x * dxl + gm.y * dzl);
+        t2[j] = fc[j] * (gm.z * dxl + gm.w * dzl);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) s_t[j * 64 + lane] = t1[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float f[NGLL];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      float a1 = 0.f, a2 = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        a1 += el[j * 64 + m] * hwi[m];
+        a2 += t2[m] * basis.hpw[m * NGLL + j];
+      }
+      f[j] = basis.w[j] * a1 + wi * a2;
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      const float fl = __shfl_up(f[j], 1, 64);
+      if (i == 0 && k > 0) f[j] += fl;
+      f[j] = -f[j];
+    }
+    // the row below's force, or where the columns are interface points a slot of its own
+    const int4 r0 = row[4 * c];
+    const bool lone = writer && c > 0 && ((x == 0 && (r0.x & 1)) || (x == xe && edge_bit(r0)));
+    if (lone) slot[r0.w + (x == 0 ? 0 : r0.x & 1)] = carry;
+    else f[0] += carry;
+#pragma unroll
+    for (int j = 0; j < NGLL - 1; j++)
+      finish(j == 0 ? r0 : row[4 * c + j], j == 0 ? g0 : g1 + (unsigned)(j - 1) * up, f[j], u[j], pd[j], ms[j]);
+    carry = f[NGLL - 1];
+    u0 = u[NGLL - 1];
+    g0 = g1 + (unsigned)(NGLL - 2) * up;
+    g1 = ng;
+  }
+  finish(row[4 * nch], gt, carry, u0, F.pd[gt], rm[gt]);
+}
+
+// The fluid's interface points; zd, zv at zp: solid points on both the CPML layer's outer boundary and a fluid-solid
+// edge, cleared here because the fluid has read them (pml_boundary_elastic)
+__global__ __launch_bounds__(256) void k_ac_interface(const InterfaceArgs A, const float* __restrict__ slot,
+                                                      const FluidFields F, const float* __restrict__ rm, const Newmark nm,
+                                                      const float2* __restrict__ layer, float* __restrict__ old,
+                                                      float dt2o4, int nz,
+                                                      const int* __restrict__ zp, float2* __restrict__ zd,
+                                                      float2* __restrict__ zv) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nz) {
+    zd[zp[q]] = make_float2(0.f, 0.f);
+    zv[zp[q]] = make_float2(0.f, 0.f);
+  }
+  if (q >= A.n) return;
+  const int g = A.id[q];
+  const int fl = A.flag[q];
+  float r = 0.f;
+  if (fl & IF_ACC) {
+    r = F.acc[g];
+    F.acc[g] = 0.f;
+  }
+  r = sum_towers(A, q, slot, r);
+  each_layer_slot(A, q, [&](int s) { r = (r - layer[s].x) - layer[s].y; });
+  const bool zero = fl & (IF_FREE | IF_PML_EDGE);
+  const float a = zero ? 0.f : r * rm[g];
+  const float pot = F.pot[g];
+  if ((fl & IF_PML) && old) old[g] = (fl & IF_PML_EDGE) ? 0.f : fmaf(dt2o4, a, pot);
+  if (fl & (IF_COUPLED | IF_LOOKED_AT)) F.pdd[g] = a;  // read by the solid, or by receivers in the next step
+  if (zero) {
+    F.pot[g] = 0.f;
+    F.pd[g] = 0.f;
+    if (F.last) F.pdd[g] = 0.f;
+  } else {
+    fluid_newmark(nm, F, (unsigned)g, a, pot, F.pd[g]);
   }
 }
 
@@ -565,6 +819,13 @@ struct AcousticState {
   float4* d_kl_geom = nullptr;
   float2* d_kl_rk = nullptr;
   float *d_rho_kl = nullptr, *d_kappa_kl = nullptr;
+  // the fused step: towers (ntower 0: none), one float per slot, boundary terms [nglob], and (keep) the solid points on
+  // both the CPML layer's outer boundary and a fluid-solid edge
+  TowerPlan plan;
+  float *d_slot = nullptr, *d_acc = nullptr;
+  float2* d_layer = nullptr;  // the CPML layer's two terms per element point
+  int nkeep = 0;
+  int* d_keep = nullptr;
 };
 
 void acoustic_release(Mesh* mp) {
@@ -581,6 +842,8 @@ void acoustic_release(Mesh* mp) {
   device_free(ac->d_bpot); device_free(ac->d_bpd); device_free(ac->d_bpdd);
   device_free(ac->d_kl_ids); device_free(ac->d_kl_geom); device_free(ac->d_kl_rk);
   device_free(ac->d_rho_kl); device_free(ac->d_kappa_kl);
+  ac->plan.release();
+  device_free(ac->d_slot); device_free(ac->d_acc); device_free(ac->d_keep); device_free(ac->d_layer);
   delete ac;
   mp->ac = nullptr;
 }
@@ -634,6 +897,65 @@ std::vector<float> download_rows(const Mesh* mp, const float* d, const std::vect
     std::copy(all.begin() + (size_t)r * NGLL2, all.begin() + (size_t)(r + 1) * NGLL2, out.begin() + q * NGLL2);
   }
   return out;
+}
+
+// the fused step's plan: chains (desc, above, element order, ids in lane order) stacked to towers; none when the point
+// numbering does not allow it (SF2D_NO_TOWERS: none)
+void fluid_towers(Mesh* mp, AcousticState* ac, const IboolView& iv, const std::vector<int>& desc,
+                  const std::vector<int>& above, const std::vector<int>& order, const std::vector<int>& ids) {
+  if (mp->simulation_type != 1 || mp->save_forward || mp->batch || getenv("SF2D_NO_TOWERS")) return;
+  const int n = (int)desc.size() / 4;
+  std::vector<TowerChain> chains(n);
+  std::vector<char> kind(n, CHAIN_STACKED);
+  std::vector<int> rank((size_t)order.size(), 0);  // descriptors lie colour by colour
+  for (int q = 0; q < n; q++) {
+    TowerChain& c = chains[q];
+    c.e0 = desc[4 * q];
+    c.ne = desc[4 * q + 3] & 0xf;
+    const int last = NGLL * c.ne - 1;
+    for (int j = 0; j < NGLL; j++) {
+      const int* r = ids.data() + (size_t)c.e0 * NGLL2 + (size_t)j * NGLL * c.ne;  // (k, i) at 5 k + i
+      c.row[j] = {r[1], r[0], r[last]};
+      for (int x = 1; x < 4 * c.ne; x++) {
+        const int k = x / 4;
+        if (r[NGLL * k + x - 4 * k] != r[1] + x - 1) return;
+      }
+    }
+    rank[c.e0] = q;
+    // a chain all of whose elements belong to the CPML layer has no force of its own; one with a source starts and ends
+    // at interface rows, so that the source's force comes first in the sum
+    bool layer = true, source = false;
+    for (int k = 0; k < c.ne; k++) {
+      layer = layer && pml_element(mp, order[c.e0 + k]);
+      source = source || std::count(mp->h_src_ispec.begin(), mp->h_src_ispec.end(), order[c.e0 + k]) > 0;
+    }
+    if (layer) kind[q] = CHAIN_SKIP;
+    else if (source) kind[q] = CHAIN_ALONE;
+  }
+  std::vector<Tower> towers;
+  if (!chain_towers(above, chains, kind, towers)) return;
+  std::vector<uint8_t> flag((size_t)mp->nglob, 0);
+  auto mark_element = [&](int e, uint8_t f) {
+    if (ac->row_of_ispec[e] < 0) return;
+    for (int p = 0; p < NGLL2; p++) flag[iv.id(e, p)] |= f;
+  };
+  for (int e : mp->h_src_ispec) mark_element(e, IF_ACC);
+  for (int e : mp->h_rec_ispec) mark_element(e, IF_LOOKED_AT);
+  for (size_t k = 0; k < ac->st_e.size(); k++) flag[iv.id(ac->st_e[k], ac->st_ij[k])] |= IF_ACC;
+  for (size_t k = 0; k < ac->free_e.size(); k++) flag[iv.id(ac->free_e[k], ac->free_ij[k])] |= IF_FREE;
+  for (size_t k = 0; k < ac->coup_e.size(); k++) flag[iv.id(ac->coup_e[k], ac->coup_ij[k])] |= IF_ACC | IF_COUPLED;
+  const std::vector<int>& pml = pml_point_ids(mp, true);
+  for (int g : pml) flag[g] |= IF_PML;
+  for (int g : pml_edge_points(mp, true)) flag[g] |= IF_PML_EDGE;
+  if (!build_tower_plan(ac->plan, towers, mp->nglob, flag, pml, rank)) return;
+  ac->d_slot = device_alloc<float>((size_t)ac->plan.nslot);
+  if (!pml.empty()) ac->d_layer = device_alloc<float2>(pml.size());
+  ac->d_acc = device_zeros<float>((size_t)mp->nglob);
+  std::vector<int> keep;
+  for (int g : pml_edge_points(mp, false))
+    if (flag[g] & IF_COUPLED) keep.push_back(g);
+  ac->nkeep = (int)keep.size();
+  if (ac->nkeep) ac->d_keep = device_copy(keep.data(), keep.size());
 }
 
 // resolves the recorded set-up into device arrays (first call of the time loop)
@@ -742,8 +1064,8 @@ AcousticState* ac_ready(Mesh* mp, const char* who) {
       std::vector<int> ibd((size_t)mp->nspec * NGLL2);
       for (int e = 0; e < mp->nspec; e++)
         for (int p = 0; p < NGLL2; p++) ibd[(size_t)e * NGLL2 + p] = iv.id(e, p);
-      std::vector<int> corder, cdesc;
-      if (chain_patches(ibd, mp->nspec, mp->nglob, lists.data(), np, corder, cdesc, ac->cn_colour, ac->cc_start,
+      std::vector<int> corder, cdesc, cabove;
+      if (chain_patches(ibd, mp->nspec, mp->nglob, lists.data(), np, corder, cdesc, cabove, ac->cn_colour, ac->cc_start,
                         ac->cc_count)) {
         // the packed (colour-order) index of each fluid element, for its operands computed above
         std::vector<int> packed((size_t)mp->nspec, -1);
@@ -777,6 +1099,7 @@ AcousticState* ac_ready(Mesh* mp, const char* who) {
           if (rect) ac->d_crect = device_copy(crect.data(), crect.size());
           else ac->d_cgeom = device_copy(cgeom.data(), cgeom.size());
           ac->chain = 1;
+          fluid_towers(mp, ac, iv, cdesc, cabove, corder, cids);
         }
       }
     }
@@ -913,6 +1236,15 @@ AcousticState* ac_ready(Mesh* mp, const char* who) {
   return ac;
 }
 
+FluidReceivers fluid_receivers(const Mesh* mp, const AcousticState* ac) {
+  return {mp->nrec_local, mp->nlength_seismogram, ac->d_rec_pts, ac->d_rec_geom, ac->d_rec_rho,
+          mp->d_xir, mp->d_gammar, mp->d_cosrot, mp->d_sinrot};
+}
+FluidSources fluid_sources(const Mesh* mp, const AcousticState* ac) {
+  return {ac->nas, mp->nsources_local, ac->d_src, ac->d_src_pts, ac->d_src_sa, ac->d_src_kap, mp->d_stf};
+}
+CouplingPoints coupling_points(const AcousticState* ac) { return {ac->ncoup, ac->d_coup, ac->d_coup_n, ac->d_coup_w}; }
+
 // the reconstructed (backward) potential exists only in SIMULATION_TYPE = 3 runs
 void require_backward(const Mesh* mp, const AcousticState* ac, const char* who) {
   if (!ac->d_bpot)
@@ -931,8 +1263,7 @@ void launch_acoustic_pressure_seismograms(Mesh* mp, float* dst, int cur, int use
   if (ac->nrec_fluid != mp->nrec_local)
     fail("compute_seismograms_cuda: pressure or potential of receivers in solid elements is not supported by this "
          "library");
-  hipLaunchKernelGGL(k_ac_seismograms, dim3(mp->nrec_local), dim3(64), 0, mp->stream, mp->nrec_local,
-                     mp->nlength_seismogram, cur, ac->d_rec_pts, mp->d_xir, mp->d_gammar,
+  hipLaunchKernelGGL(k_ac_seismograms, dim3(mp->nrec_local), dim3(64), 0, mp->stream, fluid_receivers(mp, ac), cur,
                      (potential || use_trick) ? ac->d_pot : ac->d_pdd, potential ? 1.f : -1.f, dst);
   check_hip(hipGetLastError(), "k_ac_seismograms launch");
 }
@@ -941,10 +1272,22 @@ void launch_acoustic_vector_seismograms(Mesh* mp, float* dst, int cur, int seism
   AcousticState* ac = ac_ready(mp, "compute_seismograms_cuda");
   if (ac->nrec_fluid == 0) return;
   const float* chi = seismotype == 2 ? ac->d_pd : seismotype == 3 ? ac->d_pdd : ac->d_pot;
-  hipLaunchKernelGGL(k_ac_vector_seismograms, dim3(mp->nrec_local), dim3(64), 0, mp->stream, mp->nrec_local,
-                     mp->nlength_seismogram, cur, ac->d_rec_pts, ac->d_rec_geom, ac->d_rec_rho, mp->basis,
-                     mp->d_xir, mp->d_gammar, mp->d_cosrot, mp->d_sinrot, chi, dst);
+  hipLaunchKernelGGL(k_ac_vector_seismograms, dim3(mp->nrec_local), dim3(64), 0, mp->stream, fluid_receivers(mp, ac),
+                     cur, mp->basis, chi, dst);
   check_hip(hipGetLastError(), "k_ac_vector_seismograms launch");
+}
+
+CouplingPoints acoustic_coupling(Mesh* mp, const float** pdd) {
+  if (!mp->ac) return CouplingPoints{};
+  const AcousticState* ac = ac_ready(mp, "sf2d_tower_step");
+  *pdd = ac->d_pdd;
+  return coupling_points(ac);
+}
+
+std::vector<int> acoustic_elements(const Mesh* mp) {
+  std::vector<int> out;
+  if (mp->ac) out = mp->ac->phase_elems[1];
+  return out;
 }
 
 // number of receivers in fluid elements
@@ -1058,6 +1401,16 @@ void prepare_fields_acoustic_device_(long* Mesh_pointer, realw* rmass_acoustic, 
     for (size_t k = 0; k < ac->coup_e.size(); k++)
       mp->h_coupling_points.push_back(mp->h_ibool[(size_t)ac->coup_e[k] * NGLL2 + ac->coup_ij[k]]);
   }
+  if (nrows == nspec) {
+    // no solid: the points are numbered for the fluid's towers here (else by prepare_fields_elastic_device)
+    std::vector<int> id = fluid_numbering(mp->h_ibool, nglob, ac->phase_elems[1]);
+    if (!id.empty()) {
+      std::vector<int> ib(mp->h_ibool.size());
+      for (size_t l = 0; l < ib.size(); l++) ib[l] = id[mp->h_ibool[l]];
+      check_hip(hipMemcpy(mp->d_ibool, ib.data(), ib.size() * sizeof(int), hipMemcpyHostToDevice), "ibool H2D");
+      mp->point_id = std::move(id);
+    }
+  }
   check_hip(hipDeviceSynchronize(), "prepare_fields_acoustic_device");
 }
 
@@ -1163,8 +1516,8 @@ void compute_stacey_acoustic_cuda_(long* Mesh_pointer, int* iphasef, realw* h_b_
                     h_b_absorb_potential_left};
   const int write_abs = mp->simulation_type == 1 && mp->save_forward && ac->d_absorb;
   if (*compute_wavefield_1 && ac->nst > 0) {
-    hipLaunchKernelGGL(k_ac_stacey, dim3((ac->nst + 255) / 256), dim3(256), 0, mp->stream, ac->nst, ac->d_st,
-                       ac->d_st_w, ac->d_st_rvp, ac->d_pd, ac->d_pdd, ac->d_st_slot,
+    hipLaunchKernelGGL(k_ac_stacey, dim3((ac->nst + 255) / 256), dim3(256), 0, mp->stream,
+                       FluidStacey{ac->nst, ac->d_st, ac->d_st_w, ac->d_st_rvp}, ac->d_pd, ac->d_pdd, ac->d_st_slot,
                        write_abs ? ac->d_absorb : nullptr);
     check_hip(hipGetLastError(), "k_ac_stacey launch");
   }
@@ -1216,8 +1569,7 @@ void compute_add_sources_ac_cuda_(long* Mesh_pointer, int* iphasef, int* itf) { 
   if (ac->nas == 0) return;
   const int it = *itf - 1;
   if (it < 0 || it >= mp->nstep) fail("compute_add_sources_ac_cuda: it %d outside 1..%d", *itf, mp->nstep);
-  hipLaunchKernelGGL(k_ac_sources, dim3(ac->nas), dim3(64), 0, mp->stream, ac->nas, it, mp->nsources_local,
-                     ac->d_src, ac->d_src_pts, ac->d_src_sa, ac->d_src_kap, mp->d_stf, ac->d_pdd);
+  hipLaunchKernelGGL(k_ac_sources, dim3(ac->nas), dim3(64), 0, mp->stream, fluid_sources(mp, ac), it, ac->d_pdd);
   check_hip(hipGetLastError(), "k_ac_sources launch");
 }
 
@@ -1232,8 +1584,7 @@ void compute_add_sources_ac_s3_cuda_(long* Mesh_pointer, int* iphasef, int* itf)
   if (ac->nas == 0) return;
   const int it = *itf - 1;
   if (it < 0 || it >= mp->nstep) fail("compute_add_sources_ac_s3_cuda: it %d outside 1..%d", *itf, mp->nstep);
-  hipLaunchKernelGGL(k_ac_sources, dim3(ac->nas), dim3(64), 0, mp->stream, ac->nas, it, mp->nsources_local,
-                     ac->d_src, ac->d_src_pts, ac->d_src_sa, ac->d_src_kap, mp->d_stf, ac->d_bpdd);
+  hipLaunchKernelGGL(k_ac_sources, dim3(ac->nas), dim3(64), 0, mp->stream, fluid_sources(mp, ac), it, ac->d_bpdd);
   check_hip(hipGetLastError(), "k_ac_sources launch");
 }
 
@@ -1308,8 +1659,8 @@ void compute_coupling_ac_el_cuda_(long* Mesh_pointer, int* iphasef, int* num_cou
     u = mp->d_accel;
     sign = -1.f;
   }
-  hipLaunchKernelGGL(k_coupling_ac_el, dim3((ac->ncoup + 255) / 256), dim3(256), 0, mp->stream, ac->ncoup,
-                     ac->d_coup, ac->d_coup_n, ac->d_coup_w, reinterpret_cast<const float2*>(u), sign, pdd);
+  hipLaunchKernelGGL(k_coupling_ac_el, dim3((ac->ncoup + 255) / 256), dim3(256), 0, mp->stream, coupling_points(ac),
+                     reinterpret_cast<const float2*>(u), sign, pdd);
   check_hip(hipGetLastError(), "k_coupling_ac_el launch");
 }
 
@@ -1337,8 +1688,8 @@ void compute_coupling_el_ac_cuda_(long* Mesh_pointer, int* iphasef, int* num_cou
     p = ac->d_pot;
     sign = -1.f;
   }
-  hipLaunchKernelGGL(k_coupling_el_ac, dim3((ac->ncoup + 255) / 256), dim3(256), 0, mp->stream, ac->ncoup,
-                     ac->d_coup, ac->d_coup_n, ac->d_coup_w, p, sign, acc);
+  hipLaunchKernelGGL(k_coupling_el_ac, dim3((ac->ncoup + 255) / 256), dim3(256), 0, mp->stream, coupling_points(ac),
+                     p, sign, acc);
   check_hip(hipGetLastError(), "k_coupling_el_ac launch");
 }
 
@@ -1449,6 +1800,66 @@ void get_norm_acoustic_from_device_(realw* norm, long* Mesh_pointer, const int* 
   float v;
   std::memcpy(&v, &bits, sizeof(v));
   *norm = v;
+}
+
+// 1 when the fluid has towers for sf2d_tower_fluid_step
+int sf2d_tower_fluid_ready(long* Mesh_pointer) {
+  Mesh* mp = handle(Mesh_pointer);
+  return mp->ac && ac_ready(mp, "sf2d_tower_fluid_ready")->plan.ntower > 0;
+}
+
+// The fluid's step `it` (1-based) on fields whose predictor has run: forces, boundary terms, receivers, corrector and the
+// next step's predictor (last: none, the fields are left as kernel_3_acoustic_cuda leaves them, and the caller records
+// this step's seismograms).  trick: pressure seismograms are minus the potential, else minus its second derivative, which
+// is recorded one step late.
+void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int trick, float deltat, float deltatsqover2,
+                           float deltatover2) {
+  Mesh* mp = handle(Mesh_pointer);
+  AcousticState* ac = ac_ready(mp, "sf2d_tower_fluid_step");
+  const TowerPlan& P = ac->plan;
+  if (P.ntower == 0) fail("sf2d_tower_fluid_step: no towers");
+  if (it < 1 || it > mp->nstep) fail("sf2d_tower_fluid_step: it=%d outside 1..%d", it, mp->nstep);
+  const Newmark nm{deltatover2, deltat, deltatsqover2};
+  const FluidFields F{ac->d_pot, ac->d_pd, ac->d_pdd, ac->d_acc, last};
+  FluidEdges E{};
+  E.faces = {ac->nst, ac->d_st, ac->d_st_w, ac->d_st_rvp};
+  E.sources = fluid_sources(mp, ac);
+  E.receivers = fluid_receivers(mp, ac);
+  E.coupling = coupling_points(ac);
+  E.displ = (const float2*)mp->d_displ;
+  E.it = it - 1;
+  E.nface_wg = (ac->nst + 63) / 64;
+  E.nsource = ac->nas;
+  E.ncoupling_wg = (ac->ncoup + 63) / 64;
+  E.field = ac->d_pot;
+  E.record = it - 1;
+  if (mp->nrec_local > 0) {
+    const int st = mp->h_seismotype[0];
+    if (st == 2) fail("sf2d_tower_fluid_step: velocity seismograms");
+    const bool late = st == 3 || (st == 4 && !trick);
+    E.vector = st == 1 || st == 3;
+    E.sign = st == 6 ? 1.f : -1.f;
+    if (late) {
+      E.field = ac->d_pdd;
+      E.record--;
+    }
+    E.seismo = mp->d_seismo[0];
+    E.nreceiver = (late ? first : last) || ac->nrec_fluid == 0 ? 0 : mp->nrec_local;
+    if (E.record >= mp->nlength_seismogram) fail("sf2d_tower_fluid_step: step %d after the seismograms' last", it);
+  }
+  const int wgs = (P.ntower + NXCD - 1) / NXCD * NXCD;
+  hipLaunchKernelGGL(ac->rect ? k_ac_tower<true> : k_ac_tower<false>,
+                     dim3(wgs + E.nface_wg + E.nsource + E.ncoupling_wg + E.nreceiver), dim3(64), 0, mp->stream, P.ntower,
+                     P.d_desc, P.d_row, ac->d_cfac, ac->d_cgeom, ac->d_crect, F, ac->d_rm, ac->d_slot, nm, mp->basis, wgs,
+                     E);
+  check_hip(hipGetLastError(), "k_ac_tower launch");
+  pml_acoustic_slots(mp, ac->d_pot, ac->d_pd, ac->d_layer);
+  const int n = std::max(P.n, ac->nkeep);
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_ac_interface, dim3((n + 255) / 256), dim3(256), 0, mp->stream, interface_args(P), ac->d_slot, F,
+                     ac->d_rm, nm, ac->d_layer, last ? nullptr : (float*)pml_old_field(mp, true), 0.5f * deltatsqover2, ac->nkeep,
+                     ac->d_keep, (float2*)mp->d_displ, (float2*)mp->d_veloc);
+  check_hip(hipGetLastError(), "k_ac_interface launch");
 }
 
 }  // extern "C"

@@ -303,45 +303,34 @@ Plan build_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* 
   return P;
 }
 
-// The plan of a mesh whose patches are all chains (mode 0 with patches of up to max_elems elements), for the chain
-// kernels: false, and P unusable, when some patch is not one.  The colours are build_plan's; elements and points are
-// numbered for towers, the stacks of chains whose top GLL row is the next one's bottom row: tower by tower, first the
-// points inside the rows (x = 1 .. 4 ne - 1, row by row upwards, so that a row is consecutive and the next row of the
-// tower follows it), then the left and the right column upwards (consecutive too, where a neighbour has not numbered
-// them).  No slots, halos or owned ranges: those serve the general patch kernel.
-bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
-                      int max_elems, Plan& P) {
-  P = Plan();
-  std::vector<char> placed(nspec, 0);
+// Chains of up to max_elems elements over the elements of two phase lists and, for towers (stacks of chains whose top GLL
+// row is the next one's bottom row), the chain on top of and below each.
+struct ChainSet {
   std::vector<int> elems[2];
   struct Chain { int ph, k0, ne; };
   std::vector<Chain> ch;
-  std::vector<int> mark((size_t)nglob, -1);
-  for (int ph = 0; ph < 2; ph++) {
-    for (int k = 0; k < np; k++) {
-      const int v = phase_lists[(size_t)ph * np + k];
-      if (v < 1) break;
-      if (v > nspec) fail("phase_ispec_inner_elastic: element %d outside 1..%d", v, nspec);
-      if (placed[v - 1]) fail("phase_ispec_inner_elastic: element %d listed twice", v);
-      placed[v - 1] = 1;
-      elems[ph].push_back(v - 1);
-    }
-    P.phase_count[ph] = (int)elems[ph].size();
-    const std::vector<int> ps = make_patches(ibool, elems[ph], nglob, max_elems);
-    for (size_t q = 0; q + 1 < ps.size(); q++) ch.push_back({ph, ps[q], ps[q + 1] - ps[q]});
-  }
-  auto row_point = [&](const Chain& c, int j, int x) {  // column x of GLL row j
+  std::vector<int> above, below;
+  int point(const std::vector<int>& ibool, int q, int j, int x) const {  // column x of GLL row j
+    const Chain& c = ch[q];
     const int k = x == 4 * c.ne ? c.ne - 1 : x / 4;
     return ibool[(size_t)elems[c.ph][c.k0 + k] * NGLL2 + j * NGLL + (x - 4 * k)];
-  };
-  const int nch = (int)ch.size();
-  std::fill(mark.begin(), mark.end(), -1);
+  }
+};
+
+// fills the chains of S.elems; false when some patch is not a chain
+bool find_chains(const std::vector<int>& ibool, int nglob, int max_elems, ChainSet& S) {
+  for (int ph = 0; ph < 2; ph++) {
+    const std::vector<int> ps = make_patches(ibool, S.elems[ph], nglob, max_elems);
+    for (size_t q = 0; q + 1 < ps.size(); q++) S.ch.push_back({ph, ps[q], ps[q + 1] - ps[q]});
+  }
+  const int nch = (int)S.ch.size();
+  std::vector<int> mark((size_t)nglob, -1);
   for (int q = 0; q < nch; q++) {  // the chain property: shared edges, every other point once
-    const Chain& c = ch[q];
+    const ChainSet::Chain& c = S.ch[q];
     for (int k = 0; k < c.ne; k++) {
-      const int* a = ibool.data() + (size_t)elems[c.ph][c.k0 + k] * NGLL2;
+      const int* a = ibool.data() + (size_t)S.elems[c.ph][c.k0 + k] * NGLL2;
       if (k > 0) {
-        const int* l = ibool.data() + (size_t)elems[c.ph][c.k0 + k - 1] * NGLL2;
+        const int* l = ibool.data() + (size_t)S.elems[c.ph][c.k0 + k - 1] * NGLL2;
         for (int j = 0; j < NGLL; j++)
           if (l[j * NGLL + NGLL - 1] != a[j * NGLL]) return false;
       }
@@ -353,36 +342,73 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
         }
     }
   }
-  // towers: the chain on top of each chain
-  std::vector<int> above(nch, -1), below(nch, -1);
+  S.above.assign(nch, -1);
+  S.below.assign(nch, -1);
   std::fill(mark.begin(), mark.end(), -1);
-  for (int q = 0; q < nch; q++) mark[row_point(ch[q], 0, 1)] = q;
+  for (int q = 0; q < nch; q++) mark[S.point(ibool, q, 0, 1)] = q;
   for (int q = 0; q < nch; q++) {
-    const int t = mark[row_point(ch[q], NGLL - 1, 1)];
-    if (t < 0 || t == q || below[t] >= 0 || ch[t].ne != ch[q].ne || ch[t].ph != ch[q].ph) continue;
+    const int t = mark[S.point(ibool, q, NGLL - 1, 1)];
+    if (t < 0 || t == q || S.below[t] >= 0 || S.ch[t].ne != S.ch[q].ne || S.ch[t].ph != S.ch[q].ph) continue;
     bool same = true;
-    for (int x = 0; x <= 4 * ch[q].ne && same; x++) same = row_point(ch[q], NGLL - 1, x) == row_point(ch[t], 0, x);
+    for (int x = 0; x <= 4 * S.ch[q].ne && same; x++)
+      same = S.point(ibool, q, NGLL - 1, x) == S.point(ibool, t, 0, x);
     if (!same) continue;
-    above[q] = t;
-    below[t] = q;
+    S.above[q] = t;
+    S.below[t] = q;
   }
-  P.newid.assign((size_t)nglob, -1);
-  int next_id = 0;
+  return true;
+}
+
+// numbers the points of the chains that have no id yet, tower by tower: first the points inside the rows (x = 1 ..
+// 4 ne - 1, row by row upwards, so that a row is consecutive and the next row of the tower follows it), then the left and
+// the right column upwards (consecutive too, where a neighbour has not numbered them)
+void number_points(const std::vector<int>& ibool, const ChainSet& S, std::vector<int>& newid, int& next_id) {
   auto number = [&](int g) {
-    if (P.newid[g] < 0) P.newid[g] = next_id++;
+    if (newid[g] < 0) newid[g] = next_id++;
   };
+  const int nch = (int)S.ch.size();
   for (int q = 0; q < nch; q++) {
-    if (below[q] >= 0) continue;  // a closed ring of chains has no bottom: its points are numbered below
-    for (int t = q; t >= 0; t = above[t])
+    if (S.below[q] >= 0) continue;  // a closed ring of chains has no bottom: its points are numbered below
+    for (int t = q; t >= 0; t = S.above[t])
       for (int j = 0; j < NGLL; j++)
-        for (int x = 1; x < 4 * ch[t].ne; x++) number(row_point(ch[t], j, x));
+        for (int x = 1; x < 4 * S.ch[t].ne; x++) number(S.point(ibool, t, j, x));
     for (int side = 0; side < 2; side++)
-      for (int t = q; t >= 0; t = above[t])
-        for (int j = 0; j < NGLL; j++) number(row_point(ch[t], j, side ? 4 * ch[t].ne : 0));
+      for (int t = q; t >= 0; t = S.above[t])
+        for (int j = 0; j < NGLL; j++) number(S.point(ibool, t, j, side ? 4 * S.ch[t].ne : 0));
   }
   for (int q = 0; q < nch; q++)
     for (int j = 0; j < NGLL; j++)
-      for (int x = 0; x <= 4 * ch[q].ne; x++) number(row_point(ch[q], j, x));
+      for (int x = 0; x <= 4 * S.ch[q].ne; x++) number(S.point(ibool, q, j, x));
+}
+
+// The plan of a mesh whose patches are all chains (mode 0 with patches of up to max_elems elements), for the chain
+// kernels: false, and P unusable, when some patch is not one.  The colours are build_plan's; elements and points are
+// numbered for towers (number_points), after those points the ones of the elements `fluid` in the same way.  No slots,
+// halos or owned ranges: those serve the general patch kernel.
+bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
+                      int max_elems, Plan& P, const std::vector<int>& fluid = {}) {
+  P = Plan();
+  std::vector<char> placed(nspec, 0);
+  ChainSet S;
+  std::vector<int>* const elems = S.elems;
+  for (int ph = 0; ph < 2; ph++) {
+    for (int k = 0; k < np; k++) {
+      const int v = phase_lists[(size_t)ph * np + k];
+      if (v < 1) break;
+      if (v > nspec) fail("phase_ispec_inner_elastic: element %d outside 1..%d", v, nspec);
+      if (placed[v - 1]) fail("phase_ispec_inner_elastic: element %d listed twice", v);
+      placed[v - 1] = 1;
+      elems[ph].push_back(v - 1);
+    }
+    P.phase_count[ph] = (int)elems[ph].size();
+  }
+  if (!find_chains(ibool, nglob, max_elems, S)) return false;
+  const std::vector<ChainSet::Chain>& ch = S.ch;
+  const std::vector<int>&above = S.above, &below = S.below;
+  const int nch = (int)ch.size();
+  P.newid.assign((size_t)nglob, -1);
+  int next_id = 0;
+  number_points(ibool, S, P.newid, next_id);
   // colours, in phase-list order
   std::vector<uint32_t> used((size_t)nglob, 0u);
   std::vector<int> patch_of(nch, -1), pos(nch, -1);
@@ -433,6 +459,11 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
   mark_first_touch(P, ibool, nspec, nglob);
   for (int e = 0; e < nspec; e++)
     if (!placed[e]) P.order.push_back(e);
+  if (!fluid.empty()) {
+    ChainSet F;
+    F.elems[1] = fluid;
+    if (find_chains(ibool, nglob, Mesh::CHAIN_ELEMS, F)) number_points(ibool, F, P.newid, next_id);
+  }
   for (int g = 0; g < nglob; g++)
     if (P.newid[g] < 0) P.newid[g] = next_id++;  // points of no elastic element
   return true;
@@ -440,16 +471,32 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
 
 }  // namespace
 
+// point numbering of a mesh of fluid elements alone (`elems`) for towers; empty when the patches are not chains
+std::vector<int> fluid_numbering(const std::vector<int>& ibool, int nglob, const std::vector<int>& elems) {
+  ChainSet S;
+  S.elems[1] = elems;
+  std::vector<int> id;
+  if (!find_chains(ibool, nglob, Mesh::CHAIN_ELEMS, S)) return id;
+  id.assign((size_t)nglob, -1);
+  int next_id = 0;
+  number_points(ibool, S, id, next_id);
+  for (int& v : id)
+    if (v < 0) v = next_id++;
+  return id;
+}
+
 // Patches of up to CHAIN_ELEMS elements over the given phase lists (1-based, zero-padded rows of np), coloured so
-// that no two patches of a colour share a point; true when every patch is a chain.  For the fluid's chain kernel:
-// only the element order, the patch descriptors and the colour ranges are used (not the plan's point numbering).
+// that no two patches of a colour share a point; true when every patch is a chain.  For the fluid's chain kernels:
+// only the element order, the patch descriptors, the chain above each and the colour ranges are used (not the plan's
+// point numbering).
 bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
-                   std::vector<int>& order, std::vector<int>& desc, int ncolour[2],
+                   std::vector<int>& order, std::vector<int>& desc, std::vector<int>& above, int ncolour[2],
                    int colour_start[2][Mesh::MAX_COLOURS], int colour_count[2][Mesh::MAX_COLOURS]) {
   Plan P;
   if (!build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P)) return false;
   order = std::move(P.order);
   desc = std::move(P.desc);
+  above = std::move(P.above);
   for (int ph = 0; ph < 2; ph++) {
     ncolour[ph] = P.ncolour[ph];
     for (int c = 0; c < Mesh::MAX_COLOURS; c++) {
@@ -564,8 +611,9 @@ void sort_elements_by_colour(Mesh* mp, const int* phase_lists, int np) {
   }
   if (const char* env = getenv("SF2D_SHOTS_PER_WAVE")) mp->shots_per_wave = std::max(1, atoi(env));
   Plan P;
-  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P) &&
-                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))) {
+  const std::vector<int> fluid = acoustic_elements(mp);
+  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, fluid) &&
+                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P, fluid))) {
     if (try_chain && mp->attenuation) mp->assembly = 2;  // the memory variables ride in the chain kernel only
     P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly);
   }

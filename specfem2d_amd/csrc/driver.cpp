@@ -1758,16 +1758,19 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   auto mark = [&](int step, int k) {
     if (timed && k < nev) hc(hipEventRecord(ev[(size_t)step * nev + k], stream));
   };
-  // the solid's fused step where the handle has one and nothing between its phases is asked for
+  // the fused steps of the solid and the fluid where the handle has them and nothing between a step's phases is asked for;
+  // the fluid's alone only without a solid (the receivers of both are recorded together)
   const int st = s->p.seismotype;
-  const bool fused = any_el && !phases && !s->save_forward && !s->grad_save && st != 2 && st != 3 &&
-                     sf2d_tower_ready(&s->mesh);
+  const bool seen = s->nrec == 0 || st == 1 || st == 4 || st == 6 || (st == 3 && !any_el);
+  const bool whole = !phases && !s->save_forward && !s->grad_save && seen;
+  const bool fused = any_el && whole && sf2d_tower_ready(&s->mesh);
+  const bool fused_ac = any_ac && whole && (fused || !any_el) && sf2d_tower_fluid_ready(&s->mesh);
   for (int it = it_begin; it <= it_end; it++) {
     const int step = it - it_begin;
     mark(step, 2);
     // update_displ_Newmark (update_displacement_Newmark.F90:130-300): fluid, then solid
     // compute_b_wavefield = .true. as update_displ_acoustic_forward passes it (update_displacement_Newmark.F90:150-155)
-    if (any_ac)
+    if (any_ac && !(fused_ac && it > it_begin))
       update_displacement_ac_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,
                                    &b_deltatover2, &one, &zero);
     if (any_el && !(fused && it > it_begin)) {
@@ -1778,7 +1781,10 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     mark(step, 3);
     // the fluid first, coupled to the predicted solid displacement (compute_gpu_acoustic.f90:34-220)
     if (any_ac && !any_el) mark(step, 0);
-    if (any_ac) {
+    if (fused_ac) {
+      if (it == it_begin) acoustic_enforce_free_surf_cuda_(&s->mesh, &one, &zero);
+      sf2d_tower_fluid_step(&s->mesh, it, it == it_begin, it == it_end, trick, deltat, deltatsqover2, deltatover2);
+    } else if (any_ac) {
       acoustic_enforce_free_surf_cuda_(&s->mesh, &one, &zero);
       for (int iphase = 1; iphase <= 2; iphase++) {
         compute_forces_acoustic_cuda_(&s->mesh, &iphase, &zero, &nspec_inner_ac, &zero, &one, &zero);
@@ -1801,14 +1807,16 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     }
     if (fused) {
       // receivers in fluid elements (the solid's are recorded by the fused step)
-      if (any_ac && s->nrec > 0 && it < it_end)
+      if (any_ac && !fused_ac && s->nrec > 0 && it < it_end)
         compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
                                   &acoustic_sim, &trick, &zero, &it, &it_end);
-      if (pml) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
-      if (any_ac && nfluid_solid > 0) compute_coupling_el_ac_cuda_(&s->mesh, &one, &nfluid_solid, &one);
+      // the fused steps clear the layer's outer boundary for the next step
+      if (pml && (it == it_begin || (any_ac && !fused_ac))) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
       mark(step, 0);
       sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, deltat, deltatsqover2, deltatover2);
       mark(step, 1);
+    }
+    if (fused || fused_ac) {
       if (it == it_end && s->nrec > 0)
         compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
                                   &acoustic_sim, &trick, &zero, &it, &it_end);

@@ -16,8 +16,7 @@
 // element's phase.  Per layer element point they stream the point id, the geometry, the moduli (fluid: J/rho), the
 // damping weight w_i w_j rho J (fluid: w_i w_j J/kappa), a 4-byte index into a table of the distinct coefficient
 // sets (the profiles depend on the distance into the layer only, so a few thousand sets serve a layer of millions
-// of points), the previous-step field of the point (solid: a field of its own; fluid: written per element point by a
-// pass before the Newmark predictor) and the memory variables (12 planes for a solid point, 6 for a fluid one), all stored
+// of points), the previous-step field of the point (written before the Newmark predictor) and the memory variables (12 planes for a solid point, 6 for a fluid one), all stored
 // [plane][layer element point] so that consecutive lanes touch consecutive words.
 #include <algorithm>
 #include <array>
@@ -27,6 +26,7 @@
 #include <vector>
 
 #include "sf2d_mesh.h"
+#include "sf2d_tower.h"
 #include "specfem2d_gpu.h"
 #include "specfem2d_gpu_ext.h"
 
@@ -82,7 +82,9 @@ __device__ __forceinline__ float conv(const float c[3], float r, float f, float 
 // VISCO: points with a Zener set take the viscoelastic layer formulation (pml_compute_memory_variables.f90:546-894,
 // compute_forces_viscoelastic.F90:545-556: the bulk and shear parts of the stretched gradients convolved with the
 // standard linear solids, stress with the unrelaxed moduli, kappa = lambda + mu).
-template <bool VISCO>
+// SLOTS: every element of the layer in one launch, each element point's force into its own slot of accel ([nq]), which
+// the fused step's interface sums; else one colour of elements, read-modify-writes of accel.
+template <bool VISCO, bool SLOTS>
 __global__ __launch_bounds__(256) void k_pml_elastic_forces(
     int first, int n, long nq, const int* __restrict__ ids, const float4* __restrict__ geom,
     const float2* __restrict__ moduli, const float* __restrict__ dampw, const unsigned int* __restrict__ cidx,
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(256) void k_pml_elastic_forces(
   if (active) {
     g = ids[q];
     u = displ[g];
-    a_old = accel[g];  // no other element of this colour has the point: read with the fields, in one round trip
+    if (!SLOTS) a_old = accel[g];  // no other element of this colour has the point: read with the fields
     o = oldp[g];
     v = veloc[g];
     gm = geom[q];
@@ -264,17 +266,18 @@ __global__ __launch_bounds__(256) void k_pml_elastic_forces(
     float2 a = a_old;
     a.x = (a.x - (s_w[j] * t1x + s_w[i] * t2x)) - pacc.x;
     a.y = (a.y - (s_w[j] * t1z + s_w[i] * t2z)) - pacc.y;
-    accel[g] = a;
+    accel[SLOTS ? q : (size_t)g] = a;
   }
 }
 
 // Fluid layer elements of one colour: pdd -= the element's CPML term (compute_forces_viscoacoustic.f90 with
 // pml_compute_memory_variables.f90:42-224 and pml_compute_accel_contribution.f90:42-181; Newmark).
+template <bool SLOTS>
 __global__ __launch_bounds__(256) void k_pml_acoustic_forces(
     int first, int n, long nq, const int* __restrict__ ids, const float4* __restrict__ geom,
     const float2* __restrict__ fac, const float* __restrict__ dampw, const unsigned int* __restrict__ cidx,
-    const float4* __restrict__ table, const float* __restrict__ old, float* __restrict__ rm,
-    const float* __restrict__ pot, const float* __restrict__ pd, float* __restrict__ pdd, const Basis basis) {
+    const float4* __restrict__ table, const float* __restrict__ oldp, float* __restrict__ rm,
+    const float* __restrict__ pot, const float* __restrict__ pd, float* __restrict__ pdd, float2* __restrict__ slots, const Basis basis) {
   __shared__ float s_hp[NGLL2], s_hpw[NGLL2], s_w[NGLL];
   __shared__ float s_u[256], s_o[256], s_t1[256], s_t2[256];
   const int tid = threadIdx.x;
@@ -298,8 +301,8 @@ __global__ __launch_bounds__(256) void k_pml_acoustic_forces(
     g = ids[q];
     u = pot[g];
     v = pd[g];
-    pdd_old = pdd[g];  // no other element of this colour has the point
-    o = old[q];
+    if (!SLOTS) pdd_old = pdd[g];  // no other element of this colour has the point
+    o = oldp[g];
     gm = geom[q];
     f = fac[q].x;
     w = dampw[q];
@@ -356,7 +359,9 @@ __global__ __launch_bounds__(256) void k_pml_acoustic_forces(
       a1 += s_t1[base + j * NGLL + k] * s_hpw[k * NGLL + i];
       a2 += s_t2[base + k * NGLL + i] * s_hpw[k * NGLL + j];
     }
-    pdd[g] = (pdd_old - (s_w[j] * a1 + s_w[i] * a2)) - pacc;
+    const float flux = s_w[j] * a1 + s_w[i] * a2;
+    if (SLOTS) slots[q] = make_float2(flux, pacc);
+    else pdd[g] = (pdd_old - flux) - pacc;
   }
 }
 
@@ -384,14 +389,13 @@ __global__ __launch_bounds__(256) void k_pml_old_elastic(int n, const unsigned i
   old[g] = out;
 }
 
-__global__ __launch_bounds__(256) void k_pml_old_acoustic(long nq, const int* __restrict__ ids,
-                                                          const unsigned int* __restrict__ cidx,
+__global__ __launch_bounds__(256) void k_pml_old_acoustic(int n, const unsigned int* __restrict__ pts,
                                                           const float* __restrict__ pot, const float* __restrict__ pdd,
                                                           float dt2o4, float* __restrict__ old) {
-  for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < nq; q += (long)gridDim.x * blockDim.x) {
-    const int g = ids[q];
-    old[q] = (cidx[q] & ON_EDGE) ? 0.f : pot[g] + dt2o4 * pdd[g];
-  }
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int g = (int)(pts[k] & ~ON_EDGE);
+  old[g] = (pts[k] & ON_EDGE) ? 0.f : pot[g] + dt2o4 * pdd[g];
 }
 
 // zero condition on the outer boundary of the layer (pml_boundary_elastic / pml_boundary_acoustic)
@@ -624,9 +628,11 @@ struct PmlLayer {  // the solid's or the fluid's layer elements, packed in (phas
   float2* d_mod = nullptr;  // solid {kappa, mu}; fluid {J/rho, 0}
   float* d_dampw = nullptr;
   unsigned int* d_cidx = nullptr;
-  float* d_old = nullptr;   // previous-step field: solid [nglob] float2, fluid per element point
-  int npts = 0;             // solid: the layer's points, ON_EDGE on the outer boundary
+  float* d_old = nullptr;   // previous-step field: solid [nglob] float2, fluid [nglob] float
+  int npts = 0;             // the layer's points, ON_EDGE on the outer boundary
   unsigned int* d_pts = nullptr;
+  std::vector<int> h_ids;   // point of each element point, packed order
+  std::vector<int> h_bnd;   // outer-boundary points
   float* d_rm = nullptr;    // memory variables: solid [3][nelem * 25] float4, fluid [3][nelem * 25] float2
   unsigned int* d_zidx = nullptr;  // solid, viscoelastic layer: Zener set per element point (NO_ZENER: none)
   float* d_zrm = nullptr;          // its memory variables: [3][nelem * 25] float4, then [3][nelem * 25] float2
@@ -783,6 +789,7 @@ void pml_setup(Mesh* mp, const std::vector<int>& region, const std::vector<int>&
     }
     L.nbnd = (int)bids.size();
     if (L.nbnd) L.d_bnd = device_copy(bids.data(), bids.size());
+    L.h_bnd = bids;
     if (side == 0) mp->h_pml_points = bids;
     if (L.nelem == 0) continue;
     const long nq = L.nq();
@@ -815,17 +822,16 @@ void pml_setup(Mesh* mp, const std::vector<int>& region, const std::vector<int>&
     L.d_mod = device_alloc<float2>((size_t)nq);
     L.d_dampw = device_alloc<float>((size_t)nq);
     L.d_cidx = device_copy(cq.data(), cq.size());
-    L.d_old = device_zeros<float>(side ? (size_t)nq : (size_t)2 * mp->nglob);
-    if (side == 0) {
-      std::vector<unsigned int> pts;
-      pts.reserve((size_t)nq);
+    L.d_old = device_zeros<float>((size_t)mp->nglob * (side ? 1 : 2));
+    {
+      L.h_ids.resize((size_t)nq);
       for (int k = 0; k < L.nelem; k++)
-        for (int p = 0; p < NGLL2; p++) {
-          const int g = ibool_dev[(size_t)pos[k] * NGLL2 + p];
-          pts.push_back((unsigned int)g | (on_edge[g] ? ON_EDGE : 0u));
-        }
-      std::sort(pts.begin(), pts.end(), [](unsigned int a, unsigned int b) { return (a & ~ON_EDGE) < (b & ~ON_EDGE); });
-      pts.erase(std::unique(pts.begin(), pts.end()), pts.end());
+        for (int p = 0; p < NGLL2; p++) L.h_ids[(size_t)k * NGLL2 + p] = ibool_dev[(size_t)pos[k] * NGLL2 + p];
+      std::vector<char> in((size_t)mp->nglob, 0);
+      for (int g : L.h_ids) in[g] = 1;
+      std::vector<unsigned int> pts;
+      for (int g = 0; g < mp->nglob; g++)
+        if (in[g]) pts.push_back((unsigned int)g | (on_edge[g] ? ON_EDGE : 0u));
       L.npts = (int)pts.size();
       L.d_pts = device_copy(pts.data(), pts.size());
     }
@@ -859,15 +865,19 @@ bool pml_element(const Mesh* mp, int ispec) {
   return mp->pml_state && !mp->pml_state->region.empty() && mp->pml_state->region[ispec] != 0;
 }
 
-std::vector<int> pml_solid_elements(const Mesh* mp) {
-  std::vector<int> out;
-  if (mp->pml_state)
-    for (int e = 0; e < mp->nspec; e++)
-      if (pml_element(mp, e) && (mp->h_is_acoustic.empty() || !mp->h_is_acoustic[e])) out.push_back(e);
-  return out;
+const std::vector<int>& pml_point_ids(const Mesh* mp, bool fluid) {
+  static const std::vector<int> none;
+  return !mp->pml_state ? none : fluid ? mp->pml_state->ac.h_ids : mp->pml_state->el.h_ids;
 }
 
-float2* pml_old_field(const Mesh* mp) { return mp->pml_state ? (float2*)mp->pml_state->el.d_old : nullptr; }
+const std::vector<int>& pml_edge_points(const Mesh* mp, bool fluid) {
+  static const std::vector<int> none;
+  return !mp->pml_state ? none : fluid ? mp->pml_state->ac.h_bnd : mp->pml_state->el.h_bnd;
+}
+
+void* pml_old_field(const Mesh* mp, bool fluid) {
+  return !mp->pml_state ? nullptr : fluid ? mp->pml_state->ac.d_old : mp->pml_state->el.d_old;
+}
 
 void pml_release(Mesh* mp) {
   PmlState* S = mp->pml_state;
@@ -886,8 +896,7 @@ void pml_reset(Mesh* mp) {
   for (PmlLayer* L : {&S->el, &S->ac}) {
     if (L->nelem == 0) continue;
     const bool fluid = L == &S->ac;
-    check_hip(hipMemsetAsync(L->d_old, 0, (fluid ? (size_t)L->nq() : (size_t)2 * mp->nglob) * sizeof(float), mp->stream),
-              "memset");
+    check_hip(hipMemsetAsync(L->d_old, 0, (size_t)mp->nglob * (fluid ? 1 : 2) * sizeof(float), mp->stream), "memset");
     check_hip(hipMemsetAsync(L->d_rm, 0, (size_t)L->nq() * (fluid ? AC_PLANES : EL_PLANES) * sizeof(float),
                              mp->stream), "memset");
     if (L->d_zrm)
@@ -905,50 +914,67 @@ void pml_elastic_before_predictor(Mesh* mp, float deltatsqover2) {
   check_hip(hipGetLastError(), "k_pml_old_elastic launch");
 }
 
+namespace {
+
+// elements first .. first + n - 1 of the solid's layer, added to accel (one colour) or into slots
+void launch_pml_elastic(Mesh* mp, int first, int n, float2* accel, bool slots) {
+  PmlState* S = mp->pml_state;
+  PmlLayer& L = S->el;
+  if (n <= 0) return;
+  if (S->visco_needed && !S->visco_ready)
+    fail("CPML with viscoelastic attenuation: call prepare_cpml_attenuation_device before the time loop");
+  using K = decltype(&k_pml_elastic_forces<true, true>);
+  const K kern[2][2] = {{k_pml_elastic_forces<false, false>, k_pml_elastic_forces<false, true>},
+                        {k_pml_elastic_forces<true, false>, k_pml_elastic_forces<true, true>}};
+  hipLaunchKernelGGL(kern[L.d_zidx ? 1 : 0][slots ? 1 : 0], dim3((n + PML_EPB - 1) / PML_EPB), dim3(256), 0, mp->stream,
+                     first, n, L.nq(), L.d_ids, L.d_geom, L.d_mod, L.d_dampw, L.d_cidx, S->d_table,
+                     (const float2*)L.d_old, L.d_rm, (const float2*)mp->d_displ, (const float2*)mp->d_veloc, accel,
+                     mp->basis, L.d_zidx, S->d_ztable, L.d_zrm);
+  check_hip(hipGetLastError(), "k_pml_elastic_forces launch");
+}
+
+// slots (not null): the two terms of each element point instead of pdd
+void launch_pml_acoustic(Mesh* mp, int first, int n, const float* pot, const float* pd, float* pdd, float2* slots) {
+  PmlState* S = mp->pml_state;
+  PmlLayer& L = S->ac;
+  if (n <= 0) return;
+  hipLaunchKernelGGL(slots ? k_pml_acoustic_forces<true> : k_pml_acoustic_forces<false>,
+                     dim3((n + PML_EPB - 1) / PML_EPB), dim3(256), 0, mp->stream, first, n, L.nq(), L.d_ids, L.d_geom,
+                     L.d_mod, L.d_dampw, L.d_cidx, S->d_table, L.d_old, L.d_rm, pot, pd, pdd, slots, mp->basis);
+  check_hip(hipGetLastError(), "k_pml_acoustic_forces launch");
+}
+
+}  // namespace
+
 void pml_elastic_forces(Mesh* mp, int ph) {
   PmlState* S = mp->pml_state;
   if (!S || S->el.nelem == 0) return;
-  PmlLayer& L = S->el;
-  if (S->visco_needed && !S->visco_ready)
-    fail("CPML with viscoelastic attenuation: call prepare_cpml_attenuation_device before the time loop");
-  for (int c = 0; c < L.ncolour[ph]; c++) {
-    const int n = L.colour_count[ph][c];
-    if (n <= 0) continue;
-    if (L.d_zidx)
-      hipLaunchKernelGGL(k_pml_elastic_forces<true>, dim3((n + PML_EPB - 1) / PML_EPB), dim3(256), 0, mp->stream,
-                         L.colour_start[ph][c], n, L.nq(), L.d_ids, L.d_geom, L.d_mod, L.d_dampw, L.d_cidx, S->d_table,
-                         (const float2*)L.d_old, L.d_rm, (const float2*)mp->d_displ, (const float2*)mp->d_veloc,
-                         (float2*)mp->d_accel, mp->basis, L.d_zidx, S->d_ztable, L.d_zrm);
-    else
-      hipLaunchKernelGGL(k_pml_elastic_forces<false>, dim3((n + PML_EPB - 1) / PML_EPB), dim3(256), 0, mp->stream,
-                         L.colour_start[ph][c], n, L.nq(), L.d_ids, L.d_geom, L.d_mod, L.d_dampw, L.d_cidx, S->d_table,
-                         (const float2*)L.d_old, L.d_rm, (const float2*)mp->d_displ, (const float2*)mp->d_veloc,
-                         (float2*)mp->d_accel, mp->basis, nullptr, nullptr, nullptr);
-    check_hip(hipGetLastError(), "k_pml_elastic_forces launch");
-  }
+  for (int c = 0; c < S->el.ncolour[ph]; c++)
+    launch_pml_elastic(mp, S->el.colour_start[ph][c], S->el.colour_count[ph][c], (float2*)mp->d_accel, false);
+}
+
+void pml_elastic_slots(Mesh* mp, float2* slots) {
+  if (mp->pml_state) launch_pml_elastic(mp, 0, mp->pml_state->el.nelem, slots, true);
 }
 
 void pml_acoustic_before_predictor(Mesh* mp, const float* pot, const float* pdd, float deltatsqover2) {
   PmlState* S = mp->pml_state;
   if (!S || S->ac.nelem == 0) return;
   PmlLayer& L = S->ac;
-  hipLaunchKernelGGL(k_pml_old_acoustic, dim3(grid_for(L.nq())), dim3(256), 0, mp->stream, L.nq(), L.d_ids, L.d_cidx,
-                     pot, pdd, 0.5f * deltatsqover2, L.d_old);
+  hipLaunchKernelGGL(k_pml_old_acoustic, dim3((L.npts + 255) / 256), dim3(256), 0, mp->stream, L.npts, L.d_pts, pot, pdd,
+                     0.5f * deltatsqover2, L.d_old);
   check_hip(hipGetLastError(), "k_pml_old_acoustic launch");
 }
 
 void pml_acoustic_forces(Mesh* mp, int ph, const float* pot, const float* pd, float* pdd) {
   PmlState* S = mp->pml_state;
   if (!S || S->ac.nelem == 0) return;
-  PmlLayer& L = S->ac;
-  for (int c = 0; c < L.ncolour[ph]; c++) {
-    const int n = L.colour_count[ph][c];
-    if (n <= 0) continue;
-    hipLaunchKernelGGL(k_pml_acoustic_forces, dim3((n + PML_EPB - 1) / PML_EPB), dim3(256), 0, mp->stream,
-                       L.colour_start[ph][c], n, L.nq(), L.d_ids, L.d_geom, L.d_mod, L.d_dampw, L.d_cidx, S->d_table,
-                       L.d_old, L.d_rm, pot, pd, pdd, mp->basis);
-    check_hip(hipGetLastError(), "k_pml_acoustic_forces launch");
-  }
+  for (int c = 0; c < S->ac.ncolour[ph]; c++)
+    launch_pml_acoustic(mp, S->ac.colour_start[ph][c], S->ac.colour_count[ph][c], pot, pd, pdd, nullptr);
+}
+
+void pml_acoustic_slots(Mesh* mp, const float* pot, const float* pd, float2* slots) {
+  if (mp->pml_state) launch_pml_acoustic(mp, 0, mp->pml_state->ac.nelem, pot, pd, nullptr, slots);
 }
 
 void pml_acoustic_boundary(Mesh* mp, float* pot, float* pd, float* pdd) {

@@ -272,9 +272,6 @@ void pml_elastic_forces(Mesh* mp, int ph);
 void pml_acoustic_before_predictor(Mesh* mp, const float* pot, const float* pdd, float deltatsqover2);
 void pml_acoustic_forces(Mesh* mp, int ph, const float* pot, const float* pd, float* pdd);
 void pml_acoustic_boundary(Mesh* mp, float* pot, float* pd, float* pdd);
-// solid elements of the layer (caller order, 0-based); its previous-step displacement [nglob] (null without a layer)
-std::vector<int> pml_solid_elements(const Mesh* mp);
-float2* pml_old_field(const Mesh* mp);
 // the solid's fused time step (tower.hip)
 void tower_release(Mesh* mp);
 bool tower_masses_fit(const Mesh* mp, const float* rmassx, const float* rmassz);
@@ -283,8 +280,12 @@ void upload_chain_ids(Mesh* mp);
 bool chain_row_records(const std::vector<int>& desc, const std::vector<int>& ids, const std::vector<int>& flagged,
                        std::vector<int4>& rows, std::vector<int>& ends);
 bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
-                   std::vector<int>& order, std::vector<int>& desc, int ncolour[2],
+                   std::vector<int>& order, std::vector<int>& desc, std::vector<int>& above, int ncolour[2],
                    int colour_start[2][Mesh::MAX_COLOURS], int colour_count[2][Mesh::MAX_COLOURS]);
+// point numbering of a mesh of fluid elements alone for towers; empty when its patches are not chains
+std::vector<int> fluid_numbering(const std::vector<int>& ibool, int nglob, const std::vector<int>& elems);
+// the fluid's elements in the order of their phase lists (acoustic.hip); empty without a fluid
+std::vector<int> acoustic_elements(const Mesh* mp);
 // fills the column-lane copies of the chain ids and moduli from d_chain_ids and d_moduli (when both are allocated)
 void launch_col_pack(const Mesh* mp);
 // point arrays in the caller's numbering <-> the device numbering (n2 values per point)

@@ -22,36 +22,19 @@
 #include <cstdlib>
 #include <vector>
 
-#include "sf2d_device.h"
 #include "sf2d_mesh.h"
+#include "sf2d_tower.h"
 #include "specfem2d_gpu_ext.h"
 
 namespace sf2d {
 
 struct TowerState {
-  int ntower = 0, nrow = 0;
-  int4* d_desc = nullptr;     // [ntower][2] {first element position, chains, elements per chain, first row record},
-                              // {base, id of x = 0, id of x = 4 ne of the bottom GLL row, -}
-  int4* d_row = nullptr;      // [nrow] {mask low, mask high, first partial slot, -} per GLL row, bottom to top; mask
-                              // bit x: point x of the row is an interface point
-  int npartial = 0;
-  float2* d_partial = nullptr;
-  int nif = 0, nif2 = 0;      // interface points; the first nif2 have at most two slots
-  int* d_if_id = nullptr;     // [nif]
-  int2* d_if_s = nullptr;     // [nif] slots 0 and 1 (-1: none)
-  int2* d_if_s2 = nullptr;    // [nif - nif2] slots 2 and 3
-  uint8_t* d_if_flag = nullptr;
-  std::vector<char> is_if;    // [nglob]
+  TowerPlan plan;
+  float2* d_layer = nullptr; // forces of the CPML layer's element points
+  float2* d_slot = nullptr;  // [plan.nslot] forces of interface points
 };
 
 namespace {
-
-constexpr int HAS_ACC = 1, PML_POINT = 2, PML_EDGE = 4;  // interface point flags
-
-struct Newmark {
-  float dto2, dt, dt2o2;
-};
-
 
 constexpr int TROW = 64;  // float2 per GLL row in LDS, in lane order: writes and reads without bank conflicts
 
@@ -97,17 +80,20 @@ __device__ __forceinline__ void newmark_point(const Newmark& c, const TowerField
   put(F.v_out, v);
 }
 
-// What else the launch does, in workgroups after the towers': Stacey faces, sources, receivers of the step
+// What else the launch does, in workgroups after the towers': Stacey faces, sources, receivers and fluid-solid edges of
+// the step
 struct TowerEdges {
   StaceyFaces faces;
   SourceSet sources;
   ReceiverSet receivers;
   int it;                  // 0-based time sample
-  int nface_wg, nsource, nreceiver;
+  int nface_wg, nsource, nreceiver, ncoupling_wg;
+  CouplingPoints coupling; // fluid-solid edges (one shot)
+  const float* pdd;        // the fluid's acceleration there
   const int* src_shot;     // shot of each source (null: one shot)
   float* seismo;           // [shot][2][receiver][time]
   long seismo_stride;
-  int wgs(int nshot) const { return nface_wg * nshot + nsource + nreceiver * nshot; }
+  int wgs(int nshot) const { return nface_wg * nshot + nsource + nreceiver * nshot + ncoupling_wg; }
 };
 
 __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFields& F, int wg) {
@@ -125,7 +111,10 @@ __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFiel
     return;
   }
   wg -= E.nsource;
-  if (wg >= E.nreceiver * F.nshot) return;
+  if (wg >= E.nreceiver * F.nshot) {
+    couple_solid(E.coupling, (wg - E.nreceiver * F.nshot) * 64 + threadIdx.x, E.pdd, 1.f, (float*)F.accel);
+    return;
+  }
   const int shot = wg / E.nreceiver, r = wg - shot * E.nreceiver;
   if (E.faces.is_elastic[E.receivers.ispec[r]])  // receivers in fluid elements are recorded by the fluid
     record_receiver(E.receivers, r, threadIdx.x, E.it, F.d + shot * F.stride, E.seismo + shot * E.seismo_stride, 1);
@@ -143,7 +132,7 @@ template <int GEO, int SETS>
 __global__ __launch_bounds__(64) void k_tower(
     int ntower, const int4* __restrict__ desc, const int4* __restrict__ rows, const float4* __restrict__ geom,
     const float4* __restrict__ geom_elem, const float2* __restrict__ mod, const TowerFields F,
-    const float* __restrict__ rm, float2* __restrict__ partial, int npartial, const Newmark nm, const Basis basis,
+    const float* __restrict__ rm, float2* __restrict__ slot, int nslot, const Newmark nm, const Basis basis,
     const TowerAtt att, int tower_wgs, const TowerEdges edges) {
   constexpr bool RECT = GEO == 0;
   __shared__ float2 s_t[NGLL * TROW + 1];
@@ -159,8 +148,8 @@ __global__ __launch_bounds__(64) void k_tower(
   const long at = shot * F.stride;
   const float2* const __restrict__ d = F.d + at;
   const float2* const __restrict__ v = F.v + at;
-  partial += (size_t)shot * npartial;
-  const int4 td = desc[2 * tower], tb = desc[2 * tower + 1];
+  slot += (size_t)shot * nslot;
+  const int4 td = desc[4 * tower], tb = desc[4 * tower + 1], ts = desc[4 * tower + 2], tt = desc[4 * tower + 3];
   const int nch = td.y, ne = td.z;
   const int4* const row = rows + td.w;
   const int lane = threadIdx.x;
@@ -179,17 +168,20 @@ __global__ __launch_bounds__(64) void k_tower(
     hwi[m] = basis.hpw[m * NGLL + i];
   }
   const float wi = basis.w[i];
-  // byte offsets: point of this lane in the current bottom row and its step from row to row (fields of 8 bytes), and
-  // word of row 0 of the chain in the element arrays
-  unsigned off = 8u * (unsigned)(x == 0 ? tb.y : x == xe ? tb.z : tb.x + x);
+  // byte offsets of this lane's points (fields of 8 bytes): in row 0 of the current chain, in its row 1 (from there the
+  // rows go up by `up`), in the tower's topmost row; and its word of row 0 of the chain in the element arrays
+  auto point = [&](const int4 r) { return 8u * (unsigned)(x == 0 ? r.y : x == xe ? r.z : r.x + x); };
+  unsigned off0 = point(tb), off1 = point(ts);
+  const unsigned offt = point(tt);
   const unsigned up = 8u * (x == 0 || x == xe ? 1u : (unsigned)(xe - 1));
   unsigned word = (unsigned)td.x * NGLL2 + (unsigned)min(lane, NGLL * ne - 1);
   unsigned elem = (unsigned)(td.x + kk);
   const unsigned mrow = (unsigned)(NGLL * ne);
 
-  auto load_chain = [&](unsigned o, unsigned w, unsigned e, ChainRegs& q) {
+  auto load_chain = [&](unsigned o1, bool top, unsigned w, unsigned e, ChainRegs& q) {
 #pragma unroll
-    for (int j = 0; j < NGLL - 1; j++) q.d[j] = ld_off(d, o + (unsigned)(j + 1) * up);
+    for (int j = 0; j < NGLL - 2; j++) q.d[j] = ld_off(d, o1 + (unsigned)j * up);
+    q.d[NGLL - 2] = ld_off(d, top ? offt : o1 + (unsigned)(NGLL - 2) * up);
 #pragma unroll
     for (int j = 0; j < NGLL; j++) q.mod[j] = ld_off(mod, 8u * (w + (unsigned)j * mrow));
     if (GEO < 2) q.ge = ld_off(geom_elem, 16u * e);
@@ -199,16 +191,16 @@ __global__ __launch_bounds__(64) void k_tower(
     if (!writer) return;
     const unsigned bits = x < 32 ? (unsigned)r.x >> x : (unsigned)r.y >> (x - 32);
     if (bits & 1u) {
-      partial[r.z + __popc((unsigned)r.x & below_lo) + __popc((unsigned)r.y & below_hi)] = f;
+      slot[r.z + __popc((unsigned)r.x & below_lo) + __popc((unsigned)r.y & below_hi)] = f;
     } else {
       newmark_point(nm, F, at, o, f, m, m, u, vp);
     }
   };
 
-  float2 u0 = ld_off(d, off);
+  float2 u0 = ld_off(d, off0);
   float2 carry = make_float2(0.f, 0.f);
   ChainRegs nx;
-  load_chain(off, word, elem, nx);
+  load_chain(off1, nch == 1, word, elem, nx);
   float4 cf[3];
   if (SETS == 1) {
 #pragma unroll
@@ -223,16 +215,17 @@ __global__ __launch_bounds__(64) void k_tower(
     float ms[NGLL - 1];
 #pragma unroll
     for (int j = 0; j < NGLL - 1; j++) {
-      vp[j] = ld_off(v, off + (unsigned)j * up);
-      ms[j] = ld_off(rm, (off + (unsigned)j * up) / 2u);
+      const unsigned o = j == 0 ? off0 : off1 + (unsigned)(j - 1) * up;
+      vp[j] = ld_off(v, o);
+      ms[j] = ld_off(rm, o / 2u);
     }
     float4 st[3];  // attenuation state of the next row
     if (SETS > 0) {
 #pragma unroll
       for (int s = 0; s < 3; s++) st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + word];
     }
-    const unsigned noff = off + 4u * up, nword = word + (unsigned)NGLL * mrow, nelem = elem + (unsigned)ne;
-    if (c + 1 < nch) load_chain(noff, nword, nelem, nx);
+    const unsigned noff = off1 + 4u * up, nword = word + (unsigned)NGLL * mrow, nelem = elem + (unsigned)ne;
+    if (c + 1 < nch) load_chain(noff, c + 2 == nch, nword, nelem, nx);
     float2 u[NGLL];
     u[0] = u0;
 #pragma unroll
@@ -333,62 +326,49 @@ __global__ __launch_bounds__(64) void k_tower(
     f[0].x += carry.x;
     f[0].y += carry.y;
 #pragma unroll
-    for (int j = 0; j < NGLL - 1; j++) finish(row[4 * c + j], off + (unsigned)j * up, f[j], u[j], vp[j], ms[j]);
+    for (int j = 0; j < NGLL - 1; j++) finish(row[4 * c + j], j == 0 ? off0 : off1 + (unsigned)(j - 1) * up, f[j], u[j], vp[j], ms[j]);
     carry = f[NGLL - 1];
     u0 = u[NGLL - 1];
-    off = noff;
+    off0 = off1 + (unsigned)(NGLL - 2) * up;
+    off1 = noff;
     word = nword;
     elem = nelem;
   }
   // the tower's top row
-  finish(row[4 * nch], off, carry, u0, ld_off(v, off), ld_off(rm, off / 2u));
+  finish(row[4 * nch], offt, carry, u0, ld_off(v, offt), ld_off(rm, offt / 2u));
 }
 
-// Interface points: the tower slots of each point summed in order, the boundary terms of accel added and cleared, and
-// the Newmark update; old (CPML layer points): u + dt^2 / 4 a of this step, the layer's previous-step field, zero on
-// the layer's outer boundary.
-__global__ __launch_bounds__(256) void k_interface(int n, int n2, const int* __restrict__ ids,
-                                                   const int2* __restrict__ s01, const int2* __restrict__ s23,
-                                                   const uint8_t* __restrict__ flag, const float2* __restrict__ partial,
-                                                   int npartial, const TowerFields F, const float* __restrict__ rmx,
+// Interface points: the slots of each point summed in order, the boundary terms of accel added and cleared, and the
+// Newmark update; old (CPML layer points): u + dt^2 / 4 a of this step, the layer's previous-step field, zero on the
+// layer's outer boundary, whose displacement and velocity are zero when the next step starts (pml_boundary_elastic;
+// IF_KEEP: not before the fluid has read them).
+__global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
+                                                   const TowerFields F, const float* __restrict__ rmx,
                                                    const float* __restrict__ rmz, const Newmark nm,
-                                                   float2* __restrict__ old, float dt2o4) {
+                                                   const float2* __restrict__ layer, float2* __restrict__ old,
+                                                   float dt2o4) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
+  if (q >= A.n) return;
   const long at = blockIdx.y * F.stride;
-  partial += (size_t)blockIdx.y * npartial;
-  const int g = ids[q];
-  const int fl = flag[q];
-  const int2 s = s01[q];
+  const int g = A.id[q];
+  const int fl = A.flag[q];
   const float2 dd = F.d[at + g], vv = F.v[at + g];
   const float wx = rmx[g], wz = rmz[g];
-  float2 r = make_float2(0.f, 0.f);
-  if (s.x >= 0) r = partial[s.x];
-  if (s.y >= 0) {
-    const float2 p = partial[s.y];
-    r.x += p.x;
-    r.y += p.y;
-  }
-  if (q >= n2) {
-    const int2 t = s23[q - n2];
-    const float2 p = partial[t.x];
-    r.x += p.x;
-    r.y += p.y;
-    if (t.y >= 0) {
-      const float2 p2 = partial[t.y];
-      r.x += p2.x;
-      r.y += p2.y;
-    }
-  }
-  if (fl & HAS_ACC) {
-    const float2 a = F.accel[at + g];
-    r.x += a.x;
-    r.y += a.y;
+  float2 r = sum_towers(A, q, slot + (size_t)blockIdx.y * nslot, make_float2(0.f, 0.f));
+  each_layer_slot(A, q, [&](int s) { add_slot(r, layer[s]); });
+  if (fl & IF_ACC) {
+    add_slot(r, F.accel[at + g]);
     if (!F.last) F.accel[at + g] = make_float2(0.f, 0.f);
   }
-  if ((fl & PML_POINT) && old) {
+  if ((fl & IF_PML) && old) {
     const float ax = r.x * wx, az = r.y * wz;
-    old[g] = (fl & PML_EDGE) ? make_float2(0.f, 0.f) : make_float2(fmaf(dt2o4, ax, dd.x), fmaf(dt2o4, az, dd.y));
+    old[g] = (fl & IF_PML_EDGE) ? make_float2(0.f, 0.f)
+                                : make_float2(fmaf(dt2o4, ax, dd.x), fmaf(dt2o4, az, dd.y));
+  }
+  if ((fl & (IF_PML_EDGE | IF_KEEP)) == IF_PML_EDGE && !F.last) {
+    F.d_out[at + g] = make_float2(0.f, 0.f);
+    F.v_out[at + g] = make_float2(0.f, 0.f);
+    return;
   }
   newmark_point(nm, F, at, 8u * (unsigned)g, r, wx, wz, dd, vv);
 }
@@ -397,8 +377,50 @@ __global__ __launch_bounds__(256) void k_interface(int n, int n2, const int* __r
 __global__ __launch_bounds__(256) void k_interface_clear(int n, const int* __restrict__ ids,
                                                          const uint8_t* __restrict__ flag, float2* __restrict__ accel) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < n && (flag[q] & HAS_ACC)) accel[ids[q]] = make_float2(0.f, 0.f);
+  if (q < n && (flag[q] & IF_ACC)) accel[ids[q]] = make_float2(0.f, 0.f);
 }
+
+// one step of the fields F at time step it (1-based): towers with the step's Stacey faces, sources, fluid-solid edges
+// (forward) and (seismo not null) receivers, the CPML layer, the interface
+void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long seismo_stride, const int* src_shot,
+                  const Newmark& nm, bool forward) {
+  const TowerPlan& P = mp->tower->plan;
+  float2* const slot = mp->tower->d_slot;
+  const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
+  TowerEdges E{};
+  E.faces = stacey_faces(mp);
+  E.sources = source_set(mp);
+  E.receivers = receiver_set(mp);
+  E.it = it - 1;
+  E.nface_wg = mp->stacey ? (mp->num_abs * NGLL + 63) / 64 : 0;
+  E.nsource = mp->nsources_local;
+  E.nreceiver = seismo ? mp->nrec_local : 0;
+  if (forward) E.coupling = acoustic_coupling(mp, &E.pdd);
+  E.ncoupling_wg = (E.coupling.n + 63) / 64;
+  E.src_shot = src_shot;
+  E.seismo = seismo;
+  E.seismo_stride = seismo_stride;
+  if ((long)(P.ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", P.ntower, F.nshot);
+  const int wgs = (P.ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
+  const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+  const int sets = !mp->attenuation ? 0 : mp->att_ntable == 1 ? 1 : 2;
+  using K = decltype(&k_tower<0, 0>);
+  const K kern[3][3] = {{k_tower<0, 0>, k_tower<0, 1>, k_tower<0, 2>},
+                        {k_tower<1, 0>, k_tower<1, 1>, k_tower<1, 2>},
+                        {k_tower<2, 0>, k_tower<2, 1>, k_tower<2, 2>}};
+  hipLaunchKernelGGL(kern[geo][sets], dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, P.ntower, P.d_desc, P.d_row,
+                     mp->d_geom, mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, slot, P.nslot, nm, mp->basis, att, wgs,
+                     E);
+  check_hip(hipGetLastError(), "k_tower launch");
+  if (forward) pml_elastic_slots(mp, mp->tower->d_layer);
+  if (P.n == 0) return;
+  hipLaunchKernelGGL(k_interface, dim3((P.n + 255) / 256, F.nshot), dim3(256), 0, mp->stream, interface_args(P), slot,
+                     P.nslot, F, mp->d_rmassx, mp->d_rmassz, nm, mp->tower->d_layer,
+                     F.last ? nullptr : (float2*)pml_old_field(mp, false), 0.5f * nm.dt2o2);
+  check_hip(hipGetLastError(), "k_interface launch");
+}
+
+}  // namespace
 
 // Chains per tower: about one wave per slot of the card (4096 at four waves per SIMD) and at most 16.  A tall tower has
 // few interface rows (1 in 4 x chains), a short one more waves in flight.  Measured, ms of 300 steps of 600 x 300 elements
@@ -409,53 +431,194 @@ int tower_chains(int nchain) {
   return std::max(1, std::min(16, (nchain + 4095) / 4096));
 }
 
-// one step of the fields F at time step it (1-based): towers with the step's Stacey faces, sources and (seismo not null)
-// receivers, the CPML layer, the interface
-void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long seismo_stride, const int* src_shot,
-                  const Newmark& nm, bool forward) {
-  const TowerState* T = mp->tower;
-  const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
-  TowerEdges E{stacey_faces(mp), source_set(mp), receiver_set(mp), it - 1, mp->stacey ? (mp->num_abs * NGLL + 63) / 64 : 0,
-               mp->nsources_local, seismo ? mp->nrec_local : 0, src_shot, seismo, seismo_stride};
-  if ((long)(T->ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", T->ntower, F.nshot);
-  const int wgs = (T->ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
-  const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
-  const int sets = !mp->attenuation ? 0 : mp->att_ntable == 1 ? 1 : 2;
-  using K = decltype(&k_tower<0, 0>);
-  const K kern[3][3] = {{k_tower<0, 0>, k_tower<0, 1>, k_tower<0, 2>},
-                        {k_tower<1, 0>, k_tower<1, 1>, k_tower<1, 2>},
-                        {k_tower<2, 0>, k_tower<2, 1>, k_tower<2, 2>}};
-  hipLaunchKernelGGL(kern[geo][sets], dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, T->ntower, T->d_desc,
-                     T->d_row, mp->d_geom, mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, T->d_partial, T->npartial, nm,
-                     mp->basis, att, wgs, E);
-  check_hip(hipGetLastError(), "k_tower launch");
-  if (forward)
-    for (int ph = 0; ph < 2; ph++) pml_elastic_forces(mp, ph);
-  if (T->nif == 0) return;
-  hipLaunchKernelGGL(k_interface, dim3((T->nif + 255) / 256, F.nshot), dim3(256), 0, mp->stream, T->nif, T->nif2,
-                     T->d_if_id, T->d_if_s, T->d_if_s2, T->d_if_flag, T->d_partial, T->npartial, F, mp->d_rmassx,
-                     mp->d_rmassz, nm, F.last ? nullptr : pml_old_field(mp), 0.5f * nm.dt2o2);
-  check_hip(hipGetLastError(), "k_interface launch");
+bool cut_towers(const std::vector<TowerChain>& column, int want, std::vector<Tower>& out) {
+  const int n = (int)column.size();
+  const int ne = n ? column[0].ne : 0;
+  auto follows = [&](const TowerRow& a, const TowerRow& b) {  // b one constant step above a
+    return b.inner == a.inner + 4 * ne - 1 && b.left == a.left + 1 && b.right == a.right + 1;
+  };
+  for (int c = 0; c < n; c++) {
+    const TowerRow* r = column[c].row;
+    if (column[c].ne != ne || !follows(r[1], r[2]) || !follows(r[2], r[3])) return false;
+  }
+  for (int c0 = 0; c0 < n;) {
+    int c1 = c0 + 1;
+    while (c1 < n && column[c1].e0 == column[c1 - 1].e0 + ne && follows(column[c1 - 1].row[3], column[c1 - 1].row[4]) &&
+           follows(column[c1 - 1].row[4], column[c1].row[1]))
+      c1++;
+    const int len = c1 - c0, parts = (len + want - 1) / want;
+    for (int p = 0; p < parts; p++) {
+      const int a = c0 + (int)((long)len * p / parts), b = c0 + (int)((long)len * (p + 1) / parts);
+      out.push_back({column[a].e0, b - a, ne, column[a].row[0], column[a].row[1], column[b - 1].row[NGLL - 1]});
+    }
+    c0 = c1;
+  }
+  return true;
 }
 
-}  // namespace
+bool chain_towers(const std::vector<int>& above, const std::vector<TowerChain>& chains, const std::vector<char>& kind,
+                  std::vector<Tower>& out) {
+  const int n = (int)chains.size();
+  std::vector<char> has_below(n, 0);
+  for (int a : above)
+    if (a >= 0) has_below[a] = 1;
+  const int want = tower_chains(n);
+  std::vector<Tower> towers;
+  std::vector<std::pair<int, int>> order;  // height of the tower in its column, tower
+  std::vector<TowerChain> column;
+  int seen = 0;
+  for (int q = 0; q < n; q++) {
+    if (has_below[q]) continue;
+    int level = 0;
+    for (int t = q; t >= 0;) {
+      column.clear();
+      for (; t >= 0 && kind[t] == CHAIN_STACKED; t = above[t], seen++) column.push_back(chains[t]);
+      if (column.empty()) {
+        if (kind[t] == CHAIN_ALONE) column.push_back(chains[t]);
+        t = above[t];
+        seen++;
+      }
+      if (!cut_towers(column, want, towers)) return false;
+      while (order.size() < towers.size()) order.push_back({level++, (int)order.size()});
+    }
+  }
+  if (seen != n) return false;  // a closed ring of chains has no bottom
+  std::stable_sort(order.begin(), order.end(), [](auto& a, auto& b) { return a.first < b.first; });
+  for (auto& o : order) out.push_back(towers[o.second]);
+  return true;
+}
+
+void TowerPlan::release() {
+  device_free(d_desc); device_free(d_row); device_free(d_id); device_free(d_s01); device_free(d_s23);
+  device_free(d_spml); device_free(d_flag);
+  *this = TowerPlan();
+}
+
+bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob, const std::vector<uint8_t>& flag,
+                      const std::vector<int>& pml_ids, const std::vector<int>& rank) {
+  P.release();
+  const int nt = (int)towers.size();
+  std::vector<int4> desc((size_t)4 * nt);
+  for (int t = 0; t < nt; t++) {
+    const Tower& w = towers[t];
+    desc[4 * t] = make_int4(w.e0, w.nch, w.ne, P.nrow);
+    const TowerRow r[3] = {w.first, w.second, w.top};
+    for (int k = 0; k < 3; k++) desc[4 * t + 1 + k] = make_int4(r[k].inner - 1, r[k].left, r[k].right, 0);
+    P.nrow += 4 * w.nch + 1;
+  }
+  const bool split = !rank.empty();
+  auto junction = [&](const Tower& w, int r) { return split && r % 4 == 0 && r > 0 && r < 4 * w.nch; };
+  // how many towers (or chains of them) and layer elements hold each point
+  std::vector<uint8_t> cnt((size_t)nglob, 0), npml((size_t)(pml_ids.empty() ? 0 : nglob), 0), two((size_t)nglob, 0);
+  for (const Tower& w : towers)
+    for (int r = 0; r <= 4 * w.nch; r++) {
+      const TowerRow q = w.at(r);
+      for (int x = 0; x < 4 * w.ne - 1; x++) cnt[q.inner + x]++;
+      cnt[q.left]++;
+      cnt[q.right]++;
+      if (junction(w, r)) {
+        two[q.left]++;
+        two[q.right]++;
+      }
+    }
+  for (int g : pml_ids) npml[g]++;
+  P.is_if.assign((size_t)nglob, 0);
+  std::vector<int> idx((size_t)nglob, -1), order, order4, orderp;
+  for (int g = 0; g < nglob; g++) {
+    const int np = pml_ids.empty() ? 0 : npml[g];
+    if (np == 0 && cnt[g] <= 1 && !flag[g]) continue;
+    const int n = cnt[g] + two[g];
+    if (n > 4 || np > 4) {
+      P.release();
+      return false;
+    }
+    P.is_if[g] = 1;
+    (np ? orderp : n > 2 ? order4 : order).push_back(g);
+  }
+  P.n2 = (int)order.size();
+  order.insert(order.end(), order4.begin(), order4.end());
+  P.n4 = (int)order.size();
+  order.insert(order.end(), orderp.begin(), orderp.end());
+  P.n = (int)order.size();
+  for (int q = 0; q < P.n; q++) idx[order[q]] = q;
+  struct Share { int rank, slot; };
+  std::vector<Share> share((size_t)4 * P.n, Share{0, -1});
+  std::vector<int4> row((size_t)P.nrow);
+  int ns = 0, nr = 0;
+  auto give = [&](int g, int rk) {  // a slot for point g, kept in the order of the ranks
+    Share* s = &share[(size_t)4 * idx[g]];
+    int k = 0;
+    while (s[k].slot >= 0) k++;
+    for (; k > 0 && s[k - 1].rank > rk; k--) s[k] = s[k - 1];
+    s[k] = {rk, ns++};
+  };
+  for (const Tower& w : towers)
+    for (int r = 0; r <= 4 * w.nch; r++) {
+      const TowerRow t = w.at(r);
+      const int c = std::min(r / 4, w.nch - 1);
+      const int rk = split ? rank[w.e0 + c * w.ne] : 0;
+      unsigned long long m = 0ull;
+      const int first = ns;
+      auto take = [&](int x, int g) {
+        if (!P.is_if[g]) return;
+        m |= 1ull << x;
+        give(g, rk);
+      };
+      take(0, t.left);
+      for (int x = 1; x < 4 * w.ne; x++) take(x, t.inner + x - 1);
+      take(4 * w.ne, t.right);
+      const int second = ns;
+      if (junction(w, r)) {
+        const int below = rank[w.e0 + (c - 1) * w.ne];
+        if (P.is_if[t.left]) give(t.left, below);
+        if (P.is_if[t.right]) give(t.right, below);
+      }
+      row[nr++] = make_int4((int)(unsigned)(m & 0xffffffffull), (int)(unsigned)(m >> 32), first, second);
+    }
+  P.nslot = ns;
+  std::vector<int2> s01((size_t)P.n), s23((size_t)(P.n - P.n2));
+  for (int q = 0; q < P.n; q++) {
+    const Share* s = &share[(size_t)4 * q];
+    s01[q] = make_int2(s[0].slot, s[1].slot);
+    if (q >= P.n2) s23[q - P.n2] = make_int2(s[2].slot, s[3].slot);
+  }
+  std::vector<int4> spml((size_t)(P.n - P.n4), make_int4(-1, -1, -1, -1));
+  for (size_t k = 0; k < pml_ids.size(); k++) {
+    int4& p = spml[idx[pml_ids[k]] - P.n4];
+    int* sl[4] = {&p.x, &p.y, &p.z, &p.w};
+    int m = 0;
+    while (*sl[m] >= 0) m++;
+    *sl[m] = (int)k;
+  }
+  std::vector<uint8_t> fl((size_t)P.n);
+  for (int q = 0; q < P.n; q++) fl[q] = flag[order[q]];
+  P.ntower = nt;
+  P.d_desc = device_copy(desc.data(), desc.size());
+  P.d_row = device_copy(row.data(), row.size());
+  P.d_id = device_copy(order.data(), order.size());
+  P.d_s01 = device_copy(s01.data(), s01.size());
+  P.d_s23 = device_copy(s23.data(), s23.size());
+  P.d_spml = device_copy(spml.data(), spml.size());
+  P.d_flag = device_copy(fl.data(), fl.size());
+  return true;
+}
 
 void tower_release(Mesh* mp) {
   TowerState* T = mp->tower;
   if (!T) return;
-  device_free(T->d_desc); device_free(T->d_row); device_free(T->d_partial); device_free(T->d_if_id); device_free(T->d_if_s); device_free(T->d_if_s2);
-  device_free(T->d_if_flag);
+  T->plan.release();
+  device_free(T->d_slot);
+  device_free(T->d_layer);
   delete T;
   mp->tower = nullptr;
 }
 
 // whether every point inside a tower has one inverse mass for both components (rmassx, rmassz: caller's numbering)
 bool tower_masses_fit(const Mesh* mp, const float* rmassx, const float* rmassz) {
-  const TowerState* T = mp->tower;
   for (int g = 0; g < mp->nglob; g++)
     if (rmassx[g] != rmassz[g]) {
       const int id = mp->point_id.empty() ? g : mp->point_id[g];
-      if (id < mp->nglob_el && !T->is_if[id]) return false;
+      if (id < mp->nglob_el && !mp->tower->plan.is_if[id]) return false;
     }
   return true;
 }
@@ -472,149 +635,60 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
   if (!mp->chain || !mp->first_touch || !mp->d_col_rows || mp->assembly != 0 || mp->anisotropy || mp->batch ||
       mp->save_forward || getenv("SF2D_NO_TOWERS"))
     return 0;
-  const int npatch = mp->npatch;
+  const int npatch = mp->npatch, ng = mp->nglob;
   const std::vector<int4>& rows = mp->h_col_rows;
   const std::vector<int>& ends = mp->h_col_ends;
   const std::vector<int>& pd = mp->h_patch_desc;
   if ((int)mp->h_above.size() != npatch || (int)ends.size() != npatch * NGLL) return 0;
-  TowerState* T = new TowerState();
-  mp->tower = T;
-  // stacks of chains whose ids and positions go up in constant steps, cut into towers of about the same height
-  std::vector<char> has_below(npatch, 0);
-  for (int a : mp->h_above)
-    if (a >= 0) has_below[a] = 1;
-  auto regular = [&](int q) {  // the chain's own rows
-    const int4* r = rows.data() + (size_t)q * NGLL;
-    const int* e = ends.data() + (size_t)q * NGLL;
-    const int step = 4 * (pd[4 * q + 3] & 0xf) - 1;
-    for (int j = 1; j < NGLL; j++)
-      if (r[j].x != r[j - 1].x + step || r[j].y != r[j - 1].y + 1 || e[j] != e[j - 1] + 1) return false;
-    return true;
-  };
-  const int want = tower_chains(npatch);
-  struct Tower { int level, first, n; };
-  std::vector<Tower> towers;
-  std::vector<int> stack_chains;
+  // a chain all of whose elements belong to the CPML layer has no force of its own
+  std::vector<TowerChain> chains(npatch);
+  std::vector<char> kind(npatch, CHAIN_STACKED);
   for (int q = 0; q < npatch; q++) {
-    if (has_below[q]) continue;
-    int t = q;
-    while (t >= 0) {
-      const int s0 = (int)stack_chains.size();
-      do {
-        stack_chains.push_back(t);
-        if (!regular(t)) {  // such a chain needs its row records
-          tower_release(mp);
-          return 0;
-        }
-        const int a = mp->h_above[t];
-        const bool on = a >= 0 && pd[4 * a] == pd[4 * t] + (pd[4 * t + 3] & 0xf);
-        t = a;
-        if (!on) break;
-      } while (t >= 0);
-      const int len = (int)stack_chains.size() - s0, parts = (len + want - 1) / want;
-      for (int p = 0; p < parts; p++) {
-        const int a = (int)((long)len * p / parts), b = (int)((long)len * (p + 1) / parts);
-        towers.push_back({p, s0 + a, b - a});
-      }
+    TowerChain& c = chains[q];
+    c.e0 = pd[4 * q];
+    c.ne = pd[4 * q + 3] & 0xf;
+    for (int j = 0; j < NGLL; j++) {
+      const int4 r = rows[(size_t)q * NGLL + j];
+      c.row[j] = {r.x + 1, r.y, ends[(size_t)q * NGLL + j]};
     }
+    bool layer = true;
+    for (int k = 0; k < c.ne && layer; k++) layer = pml_element(mp, mp->ispec_of_pos[c.e0 + k]);
+    if (layer) kind[q] = CHAIN_SKIP;
   }
-  if ((int)stack_chains.size() != npatch) {  // a closed ring of chains has no bottom
-    tower_release(mp);
-    return 0;
-  }
-  std::stable_sort(towers.begin(), towers.end(), [](const Tower& a, const Tower& b) { return a.level < b.level; });
-
+  std::vector<Tower> towers;
+  if (!chain_towers(mp->h_above, chains, kind, towers)) return 0;
   // points that something besides the towers acts on or looks at
-  const int ng = mp->nglob;
-  std::vector<uint8_t> flag((size_t)ng, 0), cnt((size_t)ng, 0);
-  constexpr uint8_t LOOKED_AT = 0x80;
+  std::vector<uint8_t> flag((size_t)ng, 0);
   auto mark_element = [&](int ispec, uint8_t f) {
     const int* ib = mp->h_chain_ids.data() + (size_t)mp->pos_of_ispec[ispec] * NGLL2;
     for (int p = 0; p < NGLL2; p++) flag[ib[p]] |= f;
   };
-  for (int e : mp->h_src_ispec) mark_element(e, HAS_ACC);
-  for (int e : mp->h_rec_ispec) mark_element(e, LOOKED_AT);
-  for (int g : mp->h_stacey_points) flag[g] |= HAS_ACC;
-  for (int g : mp->h_uncovered_points) flag[g] |= HAS_ACC;
-  for (int g : mp->h_coupling_points) flag[mp->point_id.empty() ? g : mp->point_id[g]] |= HAS_ACC;
-  for (int e : pml_solid_elements(mp)) mark_element(e, HAS_ACC | PML_POINT);
-  for (int g : mp->h_pml_points) flag[g] |= HAS_ACC | PML_EDGE;
+  auto dev = [&](int g) { return mp->point_id.empty() ? g : mp->point_id[g]; };
+  auto solid = [&](int e) { return mp->h_is_acoustic.empty() || !mp->h_is_acoustic[e]; };
+  for (int e : mp->h_src_ispec)
+    if (solid(e)) mark_element(e, IF_ACC);
+  for (int e : mp->h_rec_ispec)
+    if (solid(e)) mark_element(e, IF_LOOKED_AT);
+  for (int g : mp->h_stacey_points) flag[g] |= IF_ACC;
+  for (int g : mp->h_uncovered_points)
+    if (g < mp->nglob_el) flag[g] |= IF_ACC;
+  for (int g : mp->h_coupling_points) flag[dev(g)] |= IF_ACC;
+  const std::vector<int>& pml = pml_point_ids(mp, false);
+  for (int g : pml) flag[g] |= IF_PML;
+  for (int g : mp->h_pml_points) flag[g] |= IF_PML_EDGE;
+  for (int g : mp->h_coupling_points)
+    if (flag[dev(g)] & IF_PML_EDGE) flag[dev(g)] |= IF_KEEP;
   for (int g = 0; g < ng; g++)
-    if (rmassx[g] != rmassz[g]) flag[mp->point_id.empty() ? g : mp->point_id[g]] |= LOOKED_AT;
-
-  const int nt = (int)towers.size();
-  std::vector<int4> desc((size_t)2 * nt);
-  int nrow = 0;
-  for (int t = 0; t < nt; t++) {
-    const int q = stack_chains[towers[t].first], n = towers[t].n;
-    const int4 r = rows[(size_t)q * NGLL];
-    desc[2 * t] = make_int4(pd[4 * q], n, pd[4 * q + 3] & 0xf, nrow);
-    desc[2 * t + 1] = make_int4(r.x, r.y, ends[(size_t)q * NGLL], 0);
-    nrow += 4 * n + 1;
+    if (rmassx[g] != rmassz[g]) flag[dev(g)] |= IF_LOOKED_AT;
+  for (int g = mp->nglob_el; g < ng; g++) flag[g] = 0;  // no solid element has these
+  TowerState* T = new TowerState();
+  if (!build_tower_plan(T->plan, towers, ng, flag, pml)) {
+    delete T;
+    return 0;
   }
-  // f(row record, first inner id, inner points, id of x = 0, id of x = 4 ne) over every GLL row of every tower
-  auto each_row = [&](auto f) {
-    for (int t = 0; t < nt; t++) {
-      const int4 a = desc[2 * t], b = desc[2 * t + 1];
-      for (int r = 0; r <= 4 * a.y; r++) f(a.w + r, b.x + 1 + r * (4 * a.z - 1), 4 * a.z - 1, b.y + r, b.z + r);
-    }
-  };
-  // how many towers hold each point
-  each_row([&](int, int g0, int n, int left, int right) {
-    for (int x = 0; x < n; x++) cnt[g0 + x]++;
-    cnt[left]++;
-    cnt[right]++;
-  });
-  T->is_if.assign((size_t)ng, 0);
-  std::vector<int> idx((size_t)ng, -1), order2, order4;
-  for (int g = 0; g < mp->nglob_el; g++) {
-    if (cnt[g] == 1 && !flag[g]) continue;
-    T->is_if[g] = 1;
-    if (cnt[g] > 4) {  // more towers around one point than the interface kernel sums
-      tower_release(mp);
-      return 0;
-    }
-    (cnt[g] <= 2 ? order2 : order4).push_back(g);
-  }
-  T->nif2 = (int)order2.size();
-  order2.insert(order2.end(), order4.begin(), order4.end());
-  T->nif = (int)order2.size();
-  for (int q = 0; q < T->nif; q++) idx[order2[q]] = q;
-  std::vector<int4> row((size_t)nrow);
-  std::vector<int> slots((size_t)4 * T->nif, -1);
-  int np = 0;
-  each_row([&](int r, int g0, int n, int left, int right) {
-    unsigned long long m = 0ull;
-    const int first = np;
-    auto take = [&](int x, int g) {
-      if (!T->is_if[g]) return;
-      m |= 1ull << x;
-      int* sl = slots.data() + (size_t)4 * idx[g];
-      while (*sl >= 0) sl++;
-      *sl = np++;
-    };
-    take(0, left);
-    for (int x = 0; x < n; x++) take(x + 1, g0 + x);
-    take(n + 1, right);
-    row[r] = make_int4((int)(unsigned)(m & 0xffffffffull), (int)(unsigned)(m >> 32), first, 0);
-  });
-  std::vector<int2> s01((size_t)T->nif), s23((size_t)(T->nif - T->nif2));
-  std::vector<uint8_t> fl((size_t)T->nif);
-  for (int q = 0; q < T->nif; q++) {
-    s01[q] = make_int2(slots[4 * (size_t)q], slots[4 * (size_t)q + 1]);
-    if (q >= T->nif2) s23[q - T->nif2] = make_int2(slots[4 * (size_t)q + 2], slots[4 * (size_t)q + 3]);
-    fl[q] = flag[order2[q]] & (HAS_ACC | PML_POINT | PML_EDGE);
-  }
-  T->ntower = nt;
-  T->nrow = nrow;
-  T->npartial = np;
-  T->d_desc = device_copy(desc.data(), desc.size());
-  T->d_row = device_copy(row.data(), row.size());
-  T->d_partial = device_alloc<float2>((size_t)np);
-  T->d_if_id = device_copy(order2.data(), order2.size());
-  T->d_if_s = device_copy(s01.data(), s01.size());
-  T->d_if_s2 = device_copy(s23.data(), s23.size());
-  T->d_if_flag = device_copy(fl.data(), fl.size());
+  T->d_slot = device_alloc<float2>((size_t)T->plan.nslot);
+  if (!pml.empty()) T->d_layer = device_alloc<float2>(pml.size());
+  mp->tower = T;
   return 1;
 }
 
@@ -622,11 +696,11 @@ int sf2d_tower_ready(long* Mesh_pointer) { return handle(Mesh_pointer)->tower !=
 
 void sf2d_tower_begin(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
-  const TowerState* T = mp->tower;
-  if (!T) fail("sf2d_tower_begin: no towers");
-  if (T->nif == 0) return;
-  hipLaunchKernelGGL(k_interface_clear, dim3((T->nif + 255) / 256), dim3(256), 0, mp->stream, T->nif, T->d_if_id,
-                     T->d_if_flag, (float2*)mp->d_accel);
+  if (!mp->tower) fail("sf2d_tower_begin: no towers");
+  const TowerPlan& P = mp->tower->plan;
+  if (P.n == 0) return;
+  hipLaunchKernelGGL(k_interface_clear, dim3((P.n + 255) / 256), dim3(256), 0, mp->stream, P.n, P.d_id, P.d_flag,
+                     (float2*)mp->d_accel);
   check_hip(hipGetLastError(), "k_interface_clear launch");
 }
 

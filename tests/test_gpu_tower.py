@@ -18,10 +18,17 @@ def rel(a, b):
 
 
 def make(form, nx, nz, nstep=160):
-    if form == "coupled":
+    if form.startswith("coupled"):
         src = [Source(x=nx * 47.0, z=-nz * 70.0, f0=8.0, factor=1.0e9)]
         rec = np.array([[nx * 30.0, -nz * 80.0], [nx * 80.0, -60.0], [nx * 55.0, -nz * 45.0]])
-        return config.layered_fluid_solid(nx, nz, max(1, nz // 4), 100.0, nstep, 2.0e-3, sources=src, receivers=rec)
+        cfg = config.layered_fluid_solid(nx, nz, max(1, nz // 4), 100.0, nstep, 2.0e-3, sources=src, receivers=rec)
+        return cfg.replace(stacey=False, pml=True, nelem_pml=3) if form == "coupled_cpml" else cfg
+    if form.startswith("fluid"):  # pressure: minus the potential, or (the second form) its second derivative
+        cfg = config.pressure_source_acoustic_44x44(nstep).replace(
+            nx=nx, nz=nz, nz_layers=[nz], xmin=0.0, xmax=nx * 100.0, interfaces=[-nz * 100.0, 0.0], dt=2.0e-3, absorbtop=False,
+            sources=[Source(x=nx * 46.0, z=-nz * 42.0, f0=15.0, factor=1.0e4)],
+            receivers=np.array([[nx * 16.0, -nz * 60.0], [nx * 62.0, -nz * 18.0]]))
+        return cfg if form == "fluid" else cfg.replace(stacey=False, pml=True, nelem_pml=3, use_trick=False)
     cfg = config.small_test_mesh(nx=nx, nz=nz, nstep=nstep, gll=True, seed=3)
     if form in ("cpml", "visco_cpml"):
         cfg = cfg.replace(stacey=False, pml=True, nelem_pml=3)
@@ -38,7 +45,9 @@ def make(form, nx, nz, nstep=160):
 def run(cfg, pieces=None):
     sim = Simulation(cfg)
     seis = np.concatenate([sim.forward(nstep=n)[0] for n in (pieces or [cfg.nstep])], axis=-1)
-    out = [seis, *sim.fields()]
+    out = [seis]
+    if sim.nspec_acoustic < cfg.nx * sum(cfg.nz_layers):
+        out += list(sim.fields())
     if sim.nspec_acoustic:
         out += list(sim.acoustic_fields())
     sim.close()
@@ -47,14 +56,17 @@ def run(cfg, pieces=None):
 
 # displacement and seismograms: sums of the same 32-bit terms in another order, grown over 160 steps: below 1e-5, the
 # bound of every comparison with the oracle here.  The velocity and, more so, the acceleration M^-1 K d hold short
-# waves whose terms cancel: omega_max / omega, about 1e2 at these element sizes, once and twice.
+# waves whose terms cancel: omega_max / omega, about 1e2 at these element sizes, once and twice.  The potential and its
+# derivatives behave alike; a pressure that is the second derivative is 3e-6 off 64 bits in the 32-bit oracle itself: ten
+# times that.
 BOUNDS = [1e-5, 1e-5, 1e-4, 1e-3, 1e-5, 1e-4, 1e-3]
 
 
-@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "layers", "points", "visco", "visco_sets", "visco_cpml"])
+@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "layers", "points", "visco", "visco_sets", "visco_cpml",
+                                  "coupled_cpml", "fluid", "fluid_cpml"])
 @pytest.mark.parametrize("nx,nz,chains", [(12, 12, 1), (25, 17, 3), (38, 13, 64), (13, 2, 64)])
 def test_fused_step_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
-    if nz < 12 and form not in ("stacey", "points", "visco", "visco_sets"):
+    if nz < 12 and form not in ("stacey", "points", "visco", "visco_sets", "fluid"):
         pytest.skip("too flat for layers")
     if form == "points":
         monkeypatch.setenv("SF2D_NO_AFFINE", "1")
@@ -63,13 +75,16 @@ def test_fused_step_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
     fused = run(cfg)
     monkeypatch.setenv("SF2D_NO_TOWERS", "1")
     plain = run(cfg)
-    for a, b, tol in zip(fused, plain, BOUNDS):
+    bounds = [3e-5] + BOUNDS[1:] if cfg.seismotype == 4 and not cfg.use_trick else BOUNDS
+    for a, b, tol in zip(fused, plain, bounds):
         assert np.linalg.norm(b) > 0 and rel(a, b) < tol
+        # the fluid's sums keep the order of the launch per colour, but for edge points that two Stacey terms meet in
+        assert not form.startswith("fluid") or nz < 12 or np.array_equal(a, b)
     ref = OracleSim(cfg, "sp").forward()
-    assert rel(fused[0], ref) < 1e-5
+    assert rel(fused[0], ref) < bounds[0]
 
 
-@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "visco"])
+@pytest.mark.parametrize("form", ["stacey", "cpml", "coupled", "visco", "coupled_cpml", "fluid", "fluid_cpml"])
 def test_a_run_in_pieces_gives_the_bits_of_the_run_in_one(form):
     cfg = make(form, 27, 16)
     for a, b in zip(run(cfg), run(cfg, [1, 2, 57, cfg.nstep - 60])):
