@@ -65,7 +65,7 @@ int sf2d_mesh_rect(long* Mesh_pointer);
    update_displacement_cuda_ (and, with CPML, pml_boundary_elastic_cuda_) of its first step with sf2d_tower_begin;
    sf2d_tower_step(it) takes the place of the forces, Stacey edges, fluid-solid edges, sources, kernel_3_a_cuda_, the
    displacement seismograms of receivers in solid elements and, for the next step, update_displacement_cuda_ and
-   pml_boundary_elastic_cuda_.  The
+   pml_boundary_elastic_cuda_.  checkpoint >= 0: the state (d_n, v'_n, r_n) also goes to that gradient checkpoint.  The
    run's last step (last = 1) ends with the step's displacement, velocity and acceleration instead, and its seismograms
    are the caller's.
    Fluid: sf2d_tower_fluid_ready is 1 when it can run; sf2d_tower_fluid_step likewise, from the predicted potential (first:
@@ -74,7 +74,8 @@ int sf2d_mesh_rect(long* Mesh_pointer);
 int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rmassz);
 int sf2d_tower_ready(long* Mesh_pointer);
 void sf2d_tower_begin(long* Mesh_pointer);
-void sf2d_tower_step(long* Mesh_pointer, int it, int last, float deltat, float deltatsqover2, float deltatover2);
+void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float deltat, float deltatsqover2,
+                     float deltatover2);
 int sf2d_tower_fluid_ready(long* Mesh_pointer);
 void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int trick, float deltat, float deltatsqover2,
                            float deltatover2);
@@ -164,8 +165,13 @@ void sf2d_grad_result(long* Mesh_pointer, double* g_kappa, double* g_mu, double*
 /* gradient buffers over the shot batch (sf2d_batch_prepare): the calls above then checkpoint and reverse all
    shots together, residuals are [nstep][nshot][nrec][2] and the results are sums over the shots */
 int sf2d_batch_grad_prepare(long* Mesh_pointer, int chunk);
-/* shot batch: recomputes steps n0+1..n1 directly into segment slots 0..n1-n0-1, starting from checkpoint slot
-   ckpt (the state after step n0) or from rest (ckpt = -1 with n0 = 0); replaces restore + forward + saves */
+/* 1 when the sweep begun by sf2d_grad_begin_reverse runs on towers (below): its steps are then recomputed with
+   sf2d_grad_recompute_segment, and sf2d_grad_load_segment(slot) leaves the handle's own fields in a recomputed state */
+int sf2d_grad_fused(long* Mesh_pointer);
+void sf2d_grad_load_segment(long* Mesh_pointer, int slot, float dto2);
+/* shot batches and fused sweeps: recomputes steps n0+1..n1 directly into segment slots 0..n1-n0-1, starting from
+   checkpoint slot ckpt (the state after step n0) or from rest (ckpt = -1 with n0 = 0); replaces restore + forward +
+   saves */
 void sf2d_grad_recompute_segment(long* Mesh_pointer, int ckpt, int n0, int n1, float dt);
 
 /* ---------------------------------------------------------------------------

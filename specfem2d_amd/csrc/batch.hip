@@ -62,6 +62,9 @@ void batch_step_fields(Mesh* mp, BatchState* B, int it, float deltat, float delt
   B->pending_dto2 = deltatover2;
 }
 
+// whether the batch steps on towers (shot-major fields of a handle that has them)
+bool fused_batch(const Mesh* mp, const BatchState* B) { return mp->tower && B->ps == 1; }
+
 void drop_graph(BatchState* B) {
   if (B->graph_exec) (void)hipGraphExecDestroy(B->graph_exec);
   if (B->graph) (void)hipGraphDestroy(B->graph);
@@ -69,17 +72,30 @@ void drop_graph(BatchState* B) {
   B->graph = nullptr;
 }
 
-// captures one steady-state step (corrector pending with dto2 = deltatover2) reading its index from d_step
+// the fused step `it` (or *step on the device) of the batch fields; r: where the forces go too (null: nowhere)
+void fused_step(Mesh* mp, BatchState* B, int it, int last, float* r, int record, float deltat, float deltatsqover2,
+                float deltatover2, const int* step) {
+  tower_step_shots(mp, {B->d, B->v, B->d, B->v, r, B->a, B->stride, B->nshot, last, B->src_shot,
+                        record && !last && mp->nrec_local > 0 ? B->seismo : nullptr, step},
+                   it, deltat, deltatsqover2, deltatover2);
+}
+
+// captures one steady-state step (fused, or with the corrector pending with dto2 = deltatover2) reading its index from
+// d_step
 void capture_step(Mesh* mp, BatchState* B, float deltat, float deltatsqover2, float deltatover2, int record) {
   drop_graph(B);
   if (!B->d_step) B->d_step = device_zeros<int>(1);
   const int pending = B->pending;
   const float pdto2 = B->pending_dto2;
+  const bool fused = fused_batch(mp, B);
   check_hip(hipStreamBeginCapture(mp->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   B->pending = 1;
   B->pending_dto2 = deltatover2;
-  batch_step_fields(mp, B, 1, deltat, deltatsqover2, deltatover2, B->d_step);
-  if (record && mp->nrec_local > 0)
+  if (fused)
+    fused_step(mp, B, 1, 0, nullptr, record, deltat, deltatsqover2, deltatover2, B->d_step);
+  else
+    batch_step_fields(mp, B, 1, deltat, deltatsqover2, deltatover2, B->d_step);
+  if (!fused && record && mp->nrec_local > 0)
     launch_seismograms(mp, B->d, B->seismo, 0, B->nshot, B->stride, (long)2 * mp->nrec_local * mp->nstep, B->ps,
                        B->d_step);
   launch_next_step(B->d_step, mp->stream);
@@ -91,6 +107,7 @@ void capture_step(Mesh* mp, BatchState* B, float deltat, float deltatsqover2, fl
   B->graph_dt[1] = deltatsqover2;
   B->graph_dt[2] = deltatover2;
   B->graph_record = record;
+  B->graph_fused = fused;
 }
 
 }  // namespace
@@ -122,6 +139,12 @@ void batch_step_into(Mesh* mp, int it, const float* d, const float* v, const flo
   }
   batch_forces(mp, B, it, d_out, v_out, a_out, keep);
 }
+
+void batch_drop_graph(Mesh* mp) {
+  if (mp->batch) drop_graph(mp->batch);
+}
+
+const int* batch_source_shots(const Mesh* mp) { return mp->batch ? mp->batch->src_shot : nullptr; }
 
 void batch_set_pending(Mesh* mp, float dto2) {
   BatchState* B = need_batch(mp);
@@ -221,6 +244,35 @@ void sf2d_batch_run(long* Mesh_pointer, int it_begin, int it_end, float deltat, 
   // device-bound and a replay per step costs more than the launches it replaces
   const bool use_graph = getenv("SF2D_BATCH_GRAPH") != nullptr;
   bool counting = false;  // d_step holds the index of the next replay
+  if (fused_batch(mp, B)) {
+    // the first step's predictor here; the last step ends with the fields of step it_end
+    if (B->pending)
+      launch_newmark_corrector_predictor(B->d, B->v, B->a, mp->d_rmassx, mp->d_rmassz, mp->nglob, B->pending_dto2, deltat,
+                                         deltatsqover2, deltatover2, mp->stream, B->nshot, B->stride, 0, 1);
+    else
+      launch_newmark_predictor(B->d, B->v, B->a, mp->nglob, deltat, deltatsqover2, deltatover2, mp->stream, B->nshot,
+                               B->stride, 0, 1);
+    B->pending = 0;
+    tower_begin_shots(mp, B->a, B->stride, B->nshot);
+    for (int it = it_begin; it <= it_end; it++) {
+      const bool last = it == it_end, save = ckpt_every > 0 && it % ckpt_every == 0 && it < mp->nstep;
+      if (use_graph && it > it_begin && !last && !save) {
+        if (!B->graph_exec || !B->graph_fused || B->graph_record != record || B->graph_dt[0] != deltat ||
+            B->graph_dt[1] != deltatsqover2 || B->graph_dt[2] != deltatover2)
+          capture_step(mp, B, deltat, deltatsqover2, deltatover2, record);
+        if (!counting) launch_set_step(B->d_step, it, mp->stream);
+        counting = true;
+        check_hip(hipGraphLaunch(B->graph_exec, mp->stream), "hipGraphLaunch");
+        continue;
+      }
+      counting = false;
+      fused_step(mp, B, it, last ? 1 : 0, save ? grad_checkpoint_inputs(mp, it / ckpt_every - 1) : nullptr, record, deltat,
+                 deltatsqover2, deltatover2, nullptr);
+    }
+    if (record && mp->nrec_local > 0)
+      launch_seismograms(mp, B->d, B->seismo, it_end - 1, B->nshot, B->stride, (long)2 * mp->nrec_local * mp->nstep, 1);
+    return;
+  }
   for (int it = it_begin; it <= it_end; it++) {
     if (!use_graph || !B->pending || B->pending_dto2 != deltatover2) {
       batch_step_fields(mp, B, it, deltat, deltatsqover2, deltatover2, nullptr);
@@ -229,7 +281,7 @@ void sf2d_batch_run(long* Mesh_pointer, int it_begin, int it_end, float deltat, 
                            B->ps);
       counting = false;
     } else {
-      if (!B->graph_exec || B->graph_record != record || B->graph_dt[0] != deltat ||
+      if (!B->graph_exec || B->graph_fused || B->graph_record != record || B->graph_dt[0] != deltat ||
           B->graph_dt[1] != deltatsqover2 || B->graph_dt[2] != deltatover2)
         capture_step(mp, B, deltat, deltatsqover2, deltatover2, record);
       if (!counting) launch_set_step(B->d_step, it, mp->stream);

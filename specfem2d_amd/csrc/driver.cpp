@@ -1236,7 +1236,7 @@ void prepare_device(Sim& s) {
     if (s.simulation_type == 3) transfer_b_fields_to_device_(&size, zeros.data(), zeros.data(), zeros.data(), &s.mesh);
   }
   if (s.nshot > 0) sf2d_batch_prepare(&s.mesh, s.nshot, s.src_shot.data());
-  else if (nspec_el > 0) sf2d_tower_prepare(&s.mesh, s.rmassx.data(), s.rmassz.data());
+  if (nspec_el > 0) sf2d_tower_prepare(&s.mesh, s.rmassx.data(), s.rmassz.data());
 }
 
 // Relaxation times of n standard linear solids fitting 1/Q over [fmin, fmax] Hz by linear least squares, as
@@ -1762,7 +1762,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   // the fluid's alone only without a solid (the receivers of both are recorded together)
   const int st = s->p.seismotype;
   const bool seen = s->nrec == 0 || st == 1 || st == 4 || st == 6 || (st == 3 && !any_el);
-  const bool whole = !phases && !s->save_forward && !s->grad_save && seen;
+  const bool whole = !phases && !s->save_forward && s->grad_save != 2 && seen;
   const bool fused = any_el && whole && sf2d_tower_ready(&s->mesh);
   const bool fused_ac = any_ac && whole && (fused || !any_el) && sf2d_tower_fluid_ready(&s->mesh);
   for (int it = it_begin; it <= it_end; it++) {
@@ -1813,7 +1813,9 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
       // the fused steps clear the layer's outer boundary for the next step
       if (pml && (it == it_begin || (any_ac && !fused_ac))) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
       mark(step, 0);
-      sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, deltat, deltatsqover2, deltatover2);
+      const bool save = s->grad_save == 1 && it % s->grad_chunk == 0 && it < s->p.nstep;
+      sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, save ? it / s->grad_chunk - 1 : -1, deltat, deltatsqover2,
+                      deltatover2);
       mark(step, 1);
     }
     if (fused || fused_ac) {
@@ -2219,8 +2221,8 @@ int sf2d_sim_gradient_backward(void* sim, double* grad, double* parts) {
   const int nseg = (N + C - 1) / C;
   for (int k = nseg - 1; k >= 0; k--) {
     const int n0 = k * C, n1 = std::min(N, n0 + C);
-    if (s->nshot > 0) {
-      // a batch recomputes the segment straight into its state slots
+    if (s->nshot > 0 || sf2d_grad_fused(&s->mesh)) {
+      // a batch, or a fused sweep, recomputes the segment straight into its state slots
       sf2d_grad_recompute_segment(&s->mesh, k - 1, n0, n1, dt);
     } else {
       if (k == 0)
@@ -2236,6 +2238,10 @@ int sf2d_sim_gradient_backward(void* sim, double* grad, double* parts) {
     }
     for (int n = n1; n > n0; n--) sf2d_grad_reverse_step(&s->mesh, n, n - n0 - 1, n == N ? 1 : 0, dt);
     sf2d_grad_flush(&s->mesh);
+  }
+  if (s->nshot == 0 && sf2d_grad_fused(&s->mesh)) {  // the fields end after the first segment, the last one recomputed
+    s->it_done = std::min(N, C);
+    sf2d_grad_load_segment(&s->mesh, s->it_done - 1, dto2);
   }
   const size_t ne = (size_t)s->nspec * NGLL2, nf = (size_t)s->nabs * NGLL;
   std::vector<double> gk(ne), gm(ne), pm((size_t)2 * s->nglob), fvp(std::max<size_t>(1, nf)), fvs(std::max<size_t>(1, nf));

@@ -24,6 +24,7 @@
 // accumulators loop over the shots, so each accumulator is read and written once per step for the batch.
 #include <algorithm>
 
+#include "sf2d_device.h"
 #include "sf2d_mesh.h"
 #include "specfem2d_gpu_ext.h"
 
@@ -42,16 +43,17 @@ struct GradState {
   float *gk32 = nullptr, *gm32 = nullptr, *pm32 = nullptr, *gvp32 = nullptr, *gvs32 = nullptr;
   double *gk = nullptr, *gm = nullptr, *pm = nullptr, *gvp = nullptr, *gvs = nullptr;
   float* res = nullptr;   // [nstep][nshot][nrec][2] = dt (s - o)
+  // the fused sweep (handles with towers, shot-major fields): boundary terms of the recomputed steps [nfield], zero between
+  // them, and the chains' row records with the points that each owns
+  int fused = 0;
+  float* acc = nullptr;
+  int4* rows = nullptr;
 };
 
 namespace {
 
 constexpr int GT = 256;   // threads per workgroup
 
-template <typename T>
-__device__ __forceinline__ T ld_off(const T* base, unsigned byte_off) {  // 32-bit byte offset from a base
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
-}
 constexpr int GEPB = 10;  // elements per workgroup in k_grad_elastic
 
 // fields of shot s hold point g at float2 g + s ss (shot-major batches and single shots); one thread per point,
@@ -118,24 +120,9 @@ __global__ __launch_bounds__(GT) void k_adj_pointwise(int first, int npts, int n
 
 // residual injection; shot blockIdx.y (residuals [nshot][nrec][2] of this step; D point g of shot s at float2
 // g ps + s ss)
-__global__ __launch_bounds__(64) void k_adj_receivers(int nrec, const float* __restrict__ res, const int* __restrict__ ispec_rec,
-                                                      const int* __restrict__ ibool, const float* __restrict__ xir,
-                                                      const float* __restrict__ gammar, const float* __restrict__ cosrot,
-                                                      const float* __restrict__ sinrot, float* __restrict__ D,
-                                                      int ps, long ss) {
-  const int r = blockIdx.x;
-  const int p = threadIdx.x;
-  if (r >= nrec || p >= NGLL2) return;
-  res += (size_t)blockIdx.y * 2 * nrec;
-  D += (size_t)2 * blockIdx.y * ss;
-  const int i = p % NGLL, j = p / NGLL;
-  const float px = res[2 * r], pz = res[2 * r + 1];
-  const float c = cosrot[r], sn = sinrot[r];
-  const float cx = c * px - sn * pz, cz = sn * px + c * pz;
-  const float hl = xir[i * nrec + r] * gammar[j * nrec + r];
-  const size_t g = (size_t)ibool[(size_t)ispec_rec[r] * NGLL2 + p] * ps;
-  atomicAdd(&D[2 * g], hl * cx);
-  atomicAdd(&D[2 * g + 1], hl * cz);
+__global__ __launch_bounds__(64) void k_adj_receivers(const ReceiverSet R, const float* __restrict__ res,
+                                                      float* __restrict__ D, int ps, long ss) {
+  adjoint_receiver(R, blockIdx.x, threadIdx.x, res + (size_t)blockIdx.y * 2 * R.nrec, D + (size_t)2 * blockIdx.y * ss, ps);
 }
 
 // strain products of the forward displacement d_n and the adjoint force R~ at every element point, summed over
@@ -204,31 +191,10 @@ __global__ __launch_bounds__(GT) void k_grad_elastic(int nelem, int nshot, int p
   gm[l] -= sm;
 }
 
-// Stacey traction's dependence on rho vp and rho vs, per absorbing face point (same order as abs_ij), summed over
-// the shots (point g of shot s at float2 g ps + s ss)
-__global__ __launch_bounds__(64) void k_grad_stacey(int nabs, int nshot, int ps, long ss, const int* __restrict__ abs_ispec,
-                                                    const int* __restrict__ abs_ij,
-                                                    const float* __restrict__ normal, const float* __restrict__ jacw,
-                                                    const int* __restrict__ ibool, const float2* __restrict__ vpn,
-                                                    const float2* __restrict__ rb, float* __restrict__ gvp,
-                                                    float* __restrict__ gvs) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nabs * NGLL) return;
-  const int f = q / NGLL;
-  const int ii = abs_ij[2 * q], jj = abs_ij[2 * q + 1];
-  if (ii < 0 || jj < 0) return;  // corner point owned by the other edge
-  const int g = ibool[(size_t)abs_ispec[f] * NGLL2 + jj * NGLL + ii];
-  const float nx = normal[2 * q], nz = normal[2 * q + 1], w = jacw[q];
-  float sp = 0.f, sv = 0.f;
-  for (int s = 0; s < nshot; s++) {
-    const size_t o = (size_t)g * ps + (size_t)s * ss;
-    const float2 v = vpn[o], b = rb[o];
-    const float vn = nx * v.x + nz * v.y, bn = nx * b.x + nz * b.y;
-    sp += w * vn * bn;
-    sv += w * (v.x * b.x + v.y * b.y - vn * bn);
-  }
-  gvp[q] -= sp;
-  gvs[q] -= sv;
+__global__ __launch_bounds__(64) void k_grad_stacey(const StaceyFaces F, int nshot, int ps, long ss,
+                                                    const float2* __restrict__ vpn, const float2* __restrict__ rb,
+                                                    float* __restrict__ gvp, float* __restrict__ gvs) {
+  stacey_gradient(F, blockIdx.x * blockDim.x + threadIdx.x, nshot, ps, ss, vpn, rb, gvp, gvs);
 }
 
 // Shot-minor batches (nshot = 2^lshift values per point, at most 64): the same two reverse-sweep kernels with the
@@ -320,6 +286,127 @@ __global__ __launch_bounds__(64) void k_grad_elastic_minor(int nelem, int nshot,
   }
 }
 
+// k_grad_elastic over chains, one wave per chain with lane 5 k + i holding column i of element k, for the fused reverse
+// sweep: both fields' columns stay in registers, their rows pass through LDS, and the accumulators gk, gm lie in lane order
+// (point (k, i, j) of the chain at e0 at e0 * 25 + j * 5 ne + 5 k + i) so that a wave reads and writes whole lines.  It
+// also adds each point's mass term, pm -= R~ r W, where the chain owns the point (rows: masks of owned points).  Bound by
+// HBM and L2: of a step's traffic the two accumulators, read and written, are a third.  With the fused steps before and
+// after it: 400 x 200 elements, 300 steps in segments of 50, 79 -> 58 ms; 8 shots of 300 x 150, 200 steps, 94.5 -> 67.2.
+// GEO as in tower.hip: 0 rectangles, 1 affine elements, 2 geometry per point.
+template <int GEO>
+__global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nshot, long ss, const int4* __restrict__ desc,
+                                                   const int4* __restrict__ rows, const int* __restrict__ ends,
+                                                   const float4* __restrict__ geom, const float4* __restrict__ geom_elem,
+                                                   const float2* __restrict__ dn, const float2* __restrict__ rb,
+                                                   const float2* __restrict__ rn, const float* __restrict__ rmx,
+                                                   const float* __restrict__ rmz, float* __restrict__ gk,
+                                                   float* __restrict__ gm, float2* __restrict__ pm, const Basis basis) {
+  __shared__ float4 s_t[NGLL * 64 + 1];
+  const int per = gridDim.x / NXCD;  // XCD-contiguous blocks of chains
+  const int q = (blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
+  if (q >= nchain) return;  // uniform over the wave
+  const int4 pd = desc[q];
+  const int e0 = pd.x, ne = pd.w & 0xf;
+  const int lane = threadIdx.x;
+  const int k = min(lane / NGLL, Mesh::CHAIN_ELEMS);
+  const int i = lane % NGLL;
+  const int kk = min(k, ne - 1);
+  const int x = 4 * kk + i;
+  const bool active = lane / NGLL < ne;
+  const bool writer = active && (i < NGLL - 1 || k == ne - 1);
+  unsigned off[NGLL];
+  bool own[NGLL];
+#pragma unroll
+  for (int j = 0; j < NGLL; j++) {
+    const int4 r = rows[q * NGLL + j];
+    off[j] = 8u * (unsigned)(x == 0 ? r.y : x == 4 * ne ? ends[q * NGLL + j] : r.x + x);
+    const unsigned bits = x < 32 ? (unsigned)r.z >> x : (unsigned)r.w >> (x - 32);
+    own[j] = writer && (bits & 1u);
+  }
+  float hpi[NGLL];
+#pragma unroll
+  for (int m = 0; m < NGLL; m++) hpi[m] = basis.hp[i * NGLL + m];
+  float4 ge = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (GEO < 2) ge = geom_elem[e0 + kk];
+  const float4* const el = s_t + NGLL * k;
+  float sk[NGLL], sm[NGLL];
+  float2 dm[NGLL];
+#pragma unroll
+  for (int j = 0; j < NGLL; j++) {
+    sk[j] = sm[j] = 0.f;
+    dm[j] = make_float2(0.f, 0.f);
+  }
+  float2 d[NGLL], b[NGLL], r[NGLL];
+  auto load = [&](long at) {
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      d[j] = ld_off(dn + at, off[j]);
+      b[j] = ld_off(rb + at, off[j]);
+      r[j] = own[j] ? ld_off(rn + at, off[j]) : make_float2(0.f, 0.f);
+    }
+  };
+  load(0);
+  for (int s = 0; s < nshot; s++) {
+    float4 u[NGLL];
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      u[j] = make_float4(d[j].x, d[j].y, b[j].x, b[j].y);
+      dm[j].x += b[j].x * r[j].x;
+      dm[j].y += b[j].y * r[j].y;
+    }
+    if (s + 1 < nshot) load((s + 1) * ss);  // the next shot's values are in flight while this one is computed
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) s_t[j * 64 + lane] = u[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < NGLL; j++) {
+      float4 xi = make_float4(0.f, 0.f, 0.f, 0.f), ga = xi;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        const float4 e = el[j * 64 + m];
+        const float h = basis.hp[j * NGLL + m];
+        xi.x += e.x * hpi[m];
+        xi.y += e.y * hpi[m];
+        xi.z += e.z * hpi[m];
+        xi.w += e.w * hpi[m];
+        ga.x += u[m].x * h;
+        ga.y += u[m].y * h;
+        ga.z += u[m].z * h;
+        ga.w += u[m].w * h;
+      }
+      float4 gp = ge;
+      if (GEO == 2) gp = ld_off(geom, 16u * ((unsigned)(e0 + kk) * NGLL2 + (unsigned)(j * NGLL + i)));
+      const float X = gp.x, Z = GEO ? gp.y : 0.f, G = GEO ? gp.z : 0.f, H = gp.w;
+      const float ux = xi.x * X + ga.x * G, uxz = xi.x * Z + ga.x * H, uzx = xi.y * X + ga.y * G, uz = xi.y * Z + ga.y * H;
+      const float wx = xi.z * X + ga.z * G, wxz = xi.z * Z + ga.z * H, wzx = xi.w * X + ga.w * G, wz = xi.w * Z + ga.w * H;
+      sk[j] += (ux + uz) * (wx + wz);
+      sm[j] += ux * wx + uz * wz - ux * wz - uz * wx + (uxz + uzx) * (wxz + wzx);
+    }
+  }
+  unsigned l = (unsigned)e0 * NGLL2 + (unsigned)lane;
+#pragma unroll
+  for (int j = 0; j < NGLL; j++) {
+    float4 gp = ge;
+    if (GEO == 2) gp = ld_off(geom, 16u * ((unsigned)(e0 + kk) * NGLL2 + (unsigned)(j * NGLL + i)));
+    const float X = gp.x, Z = GEO ? gp.y : 0.f, G = GEO ? gp.z : 0.f, H = gp.w;
+    const float wj = basis.w[i] * basis.w[j] / (X * H - G * Z);
+    if (active) {
+      gk[l] -= wj * sk[j];
+      gm[l] -= wj * sm[j];
+    }
+    l += (unsigned)(NGLL * ne);
+    if (own[j]) {
+      const unsigned g = off[j] / 8u;
+      float2 p = pm[g];
+      p.x -= dm[j].x * rmx[g];
+      p.y -= dm[j].y * rmz[g];
+      pm[g] = p;
+    }
+  }
+}
+
 __global__ __launch_bounds__(GT) void k_flush64(size_t n, float* __restrict__ a32, double* __restrict__ a64) {
   for (size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x) {
     a64[k] += (double)a32[k];
@@ -402,7 +489,43 @@ int grad_prepare(Mesh* mp, long* Mesh_pointer, int chunk, int nrec, int batch) {
   return G->nckpt;
 }
 
+// whether the sweep runs on towers, and what that needs: with a tower per chain stack, shot-major fields and neither a
+// CPML layer nor attenuation (which gradients refuse)
+void choose_sweep(Mesh* mp, GradState* G) {
+  G->fused = mp->tower && G->ps == 1 && !mp->pml && !mp->attenuation;
+  if (!G->fused || G->rows) return;
+  const int n = mp->npatch;
+  std::vector<int4> rows(mp->h_col_rows);
+  std::vector<char> seen((size_t)mp->nglob, 0);
+  for (int q = 0; q < n; q++) {
+    const int ne = mp->h_patch_desc[4 * q + 3] & 0xf;
+    for (int j = 0; j < NGLL; j++) {
+      int4& r = rows[(size_t)q * NGLL + j];
+      unsigned long long mask = 0ull;
+      for (int x = 0; x <= 4 * ne; x++) {
+        char& s = seen[x == 0 ? r.y : x == 4 * ne ? mp->h_col_ends[(size_t)q * NGLL + j] : r.x + x];
+        if (!s) mask |= 1ull << x;
+        s = 1;
+      }
+      r.z = (int)(unsigned)(mask & 0xffffffffull);
+      r.w = (int)(unsigned)(mask >> 32);
+    }
+  }
+  G->rows = device_copy(rows.data(), rows.size());
+  G->acc = device_zeros<float>(G->nfield);
+}
+
 }  // namespace
+
+float* grad_checkpoint_inputs(Mesh* mp, int slot) {
+  GradState* G = need(mp);
+  if (slot < 0 || slot >= G->nckpt) fail("gradient checkpoint %d outside 0..%d", slot, G->nckpt - 1);
+  float* dst = G->ckpt + (size_t)slot * 3 * G->nfield;
+  copy_d2d(dst, G->fd, G->nfield, mp->stream);
+  copy_d2d(dst + G->nfield, G->fv, G->nfield, mp->stream);
+  return dst + 2 * G->nfield;
+}
+
 }  // namespace sf2d
 
 using namespace sf2d;
@@ -428,8 +551,9 @@ void sf2d_grad_release(long* Mesh_pointer) {
   if (!G) return;
   check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_release");
   for (float** p : {&G->ckpt, &G->seg, &G->D, &G->Vb, &G->Rb, &G->gk32, &G->gm32, &G->pm32, &G->gvp32, &G->gvs32,
-                    &G->res})
+                    &G->res, &G->acc})
     device_free(*p);
+  device_free(G->rows);
   for (double** p : {&G->gk, &G->gm, &G->pm, &G->gvp, &G->gvs}) device_free(*p);
   delete G;
   mp->grad = nullptr;
@@ -446,6 +570,23 @@ void sf2d_grad_save_state(long* Mesh_pointer, int kind, int slot) {
   copy_d2d(dst, G->fd, G->nfield, mp->stream);
   copy_d2d(dst + G->nfield, G->fv, G->nfield, mp->stream);
   copy_d2d(dst + 2 * G->nfield, G->fa, G->nfield, mp->stream);
+}
+
+// 1 when the sweep begun by sf2d_grad_begin_reverse recomputes with sf2d_grad_recompute_segment (always so for batches)
+int sf2d_grad_fused(long* Mesh_pointer) { return need(handle(Mesh_pointer))->fused; }
+
+// leaves the handle's own fields in the state of segment slot (the corrector of that step pending)
+void sf2d_grad_load_segment(long* Mesh_pointer, int slot, float dto2) {
+  Mesh* mp = handle(Mesh_pointer);
+  GradState* G = need(mp);
+  if (G->batch || slot < 0 || slot >= G->chunk) fail("sf2d_grad_load_segment: slot %d", slot);
+  const float* src = G->seg + (size_t)slot * 3 * G->nfield;
+  copy_d2d(G->fd, src, G->nfield, mp->stream);
+  copy_d2d(G->fv, src + G->nfield, G->nfield, mp->stream);
+  copy_d2d(G->fa, src + 2 * G->nfield, G->nfield, mp->stream);
+  mp->pending_corrector[0] = 1;
+  mp->pending_dto2[0] = dto2;
+  mp->accel_partial = 0;
 }
 
 // restores checkpoint slot into the forward fields, with the corrector of that step pending (dto2 = dt/2)
@@ -474,6 +615,7 @@ void sf2d_grad_begin_reverse(long* Mesh_pointer, const float* res) {
     check_hip(hipMemcpyAsync(G->res, res, sizeof(float) * 2 * G->nrec * G->nshot * G->nstep, hipMemcpyHostToDevice,
                              mp->stream),
               "residual H2D");
+  choose_sweep(mp, G);
   for (float* p : {G->D, G->Vb, G->Rb}) check_hip(hipMemsetAsync(p, 0, G->nfield * sizeof(float), mp->stream), "zero");
   check_hip(hipMemsetAsync(G->pm32, 0, G->n2 * sizeof(float), mp->stream), "zero");
   for (float* p : {G->gk32, G->gm32}) check_hip(hipMemsetAsync(p, 0, G->ne * sizeof(float), mp->stream), "zero");
@@ -495,6 +637,22 @@ void sf2d_grad_reverse_step(long* Mesh_pointer, int n, int slot, int first, floa
   const float* vpn = dn + G->nfield;
   const float* rn = dn + 2 * G->nfield;
   const float dto2 = (float)(0.5 * (double)dt), h = (float)(0.5 * (double)dt * (double)dt);
+  const float* res = G->res + (size_t)(n - 1) * 2 * G->nrec * G->nshot;
+  if (G->fused) {
+    if (!mp->tower) fail("sf2d_grad_reverse_step: the materials changed during the sweep");
+    // R~_n is complete: the previous step's update made it (zero at n = NSTEP)
+    using K = decltype(&k_grad_chain<0>);
+    const K kern[3] = {k_grad_chain<0>, k_grad_chain<1>, k_grad_chain<2>};
+    const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+    if (!first)
+      hipLaunchKernelGGL(kern[geo], dim3((mp->npatch + NXCD - 1) / NXCD * NXCD), dim3(64), 0, mp->stream, mp->npatch,
+                         G->nshot, G->stride, mp->d_patch_desc, G->rows, mp->d_col_ends, mp->d_geom, mp->d_geom_elem,
+                         (const float2*)dn, (const float2*)G->Rb, (const float2*)rn, mp->d_rmassx, mp->d_rmassz, G->gk32,
+                         G->gm32, (float2*)G->pm32, mp->basis);
+    check_hip(hipGetLastError(), "k_grad_chain launch");
+    tower_step_adjoint(mp, G->Rb, G->D, G->Vb, G->stride, G->nshot, res, vpn, G->gvp32, G->gvs32, dt, h, dto2);
+    return;
+  }
   int lshift = 0;
   while ((1 << lshift) < G->ps) lshift++;
   if (G->ps > 1)
@@ -506,16 +664,15 @@ void sf2d_grad_reverse_step(long* Mesh_pointer, int n, int slot, int first, floa
                        G->nshot, G->stride, dt, dto2, h, (const float2*)G->D, (float2*)G->Vb, (float2*)G->Rb,
                        mp->d_rmassx, mp->d_rmassz, (const float2*)rn, (float2*)G->pm32);
   if (G->nrec > 0)
-    hipLaunchKernelGGL(k_adj_receivers, dim3(G->nrec, G->nshot), dim3(64), 0, mp->stream, G->nrec,
-                       G->res + (size_t)(n - 1) * 2 * G->nrec * G->nshot, mp->d_ispec_selected_rec, mp->d_ibool,
-                       mp->d_xir, mp->d_gammar, mp->d_cosrot, mp->d_sinrot, G->D, G->ps, G->stride);
+    hipLaunchKernelGGL(k_adj_receivers, dim3(G->nrec, G->nshot), dim3(64), 0, mp->stream, receiver_set(mp),
+                       res, G->D, G->ps, G->stride);
   apply_element_forces(mp, 0, G->Rb, G->D, G->nshot, G->stride, 0, G->ps);
   apply_element_forces(mp, 1, G->Rb, G->D, G->nshot, G->stride, 0, G->ps);
   if (mp->stacey && mp->num_abs > 0) {
     launch_stacey(mp, G->Rb, G->Vb, 0, G->nshot, G->stride, G->ps);
-    hipLaunchKernelGGL(k_grad_stacey, dim3((mp->num_abs * NGLL + 63) / 64), dim3(64), 0, mp->stream, mp->num_abs,
-                       G->nshot, G->ps, G->stride, mp->d_abs_ispec, mp->d_abs_ij, mp->d_abs_normal, mp->d_abs_jacw,
-                       mp->d_ibool, (const float2*)vpn, (const float2*)G->Rb, G->gvp32, G->gvs32);
+    hipLaunchKernelGGL(k_grad_stacey, dim3((mp->num_abs * NGLL + 63) / 64), dim3(64), 0, mp->stream,
+                       stacey_faces(mp), G->nshot, G->ps, G->stride, (const float2*)vpn, (const float2*)G->Rb, G->gvp32,
+                       G->gvs32);
   }
   if (G->ps > 1)
     hipLaunchKernelGGL(k_grad_elastic_minor, dim3((mp->nspec + (64 >> lshift) - 1) / (64 >> lshift)), dim3(64), 0,
@@ -528,18 +685,37 @@ void sf2d_grad_reverse_step(long* Mesh_pointer, int n, int slot, int first, floa
   check_hip(hipGetLastError(), "sf2d_grad_reverse_step launch");
 }
 
-// shot batch: recomputes steps n0+1 .. n1 straight into the segment slots, from checkpoint slot ckpt (the state
-// after step n0) or from rest (ckpt = -1, n0 = 0); no state is copied
+// recomputes steps n0+1 .. n1 straight into the segment slots, from checkpoint slot ckpt (the state after step n0) or
+// from rest (ckpt = -1, n0 = 0); no state is copied.  Shot batches, and the handle's own fields in a fused sweep.
 void sf2d_grad_recompute_segment(long* Mesh_pointer, int ckpt, int n0, int n1, float dt) {
   Mesh* mp = handle(Mesh_pointer);
   GradState* G = need(mp);
-  if (!G->batch) fail("sf2d_grad_recompute_segment: the gradient buffers do not follow a shot batch");
+  if (!G->batch && !G->fused) fail("sf2d_grad_recompute_segment: neither a shot batch nor a fused sweep");
   if (n0 < 0 || n1 <= n0 || n1 > G->nstep || n1 - n0 > G->chunk)
     fail("sf2d_grad_recompute_segment: steps %d..%d (segments of at most %d)", n0 + 1, n1, G->chunk);
   if (ckpt < -1 || ckpt >= G->nckpt || (ckpt == -1) != (n0 == 0))
     fail("sf2d_grad_recompute_segment: checkpoint %d for a segment after step %d", ckpt, n0);
   const float dto2 = (float)(0.5 * (double)dt), h = (float)(0.5 * (double)dt * (double)dt);
   const float* src = ckpt < 0 ? nullptr : G->ckpt + (size_t)ckpt * 3 * G->nfield;
+  if (G->fused) {
+    if (!mp->tower) fail("sf2d_grad_recompute_segment: the materials changed during the sweep");
+    if (!src) {  // the predictor of a state at rest is the state at rest
+      for (int f = 0; f < 2; f++)
+        check_hip(hipMemsetAsync(G->seg + f * G->nfield, 0, G->nfield * sizeof(float), mp->stream), "zero");
+    } else {  // into the accelerations of slot 0 too, where the step's forces overwrite them
+      launch_newmark_corrector_predictor_to(src, src + G->nfield, src + 2 * G->nfield, G->seg, G->seg + G->nfield,
+                                            G->seg + 2 * G->nfield, mp->d_rmassx, mp->d_rmassz, mp->nglob, dto2, dt, h,
+                                            dto2, mp->stream, G->nshot, G->stride, 1, 1);
+    }
+    for (int n = n0 + 1; n <= n1; n++) {
+      float* at = G->seg + (size_t)(n - n0 - 1) * 3 * G->nfield;
+      float* next = n < n1 ? at + 3 * G->nfield : at;
+      tower_step_shots(mp, {at, at + G->nfield, next, next + G->nfield, at + 2 * G->nfield, G->acc, G->stride, G->nshot,
+                            n < n1 ? 0 : 2, G->batch ? batch_source_shots(mp) : nullptr, nullptr, nullptr},
+                       n, dt, h, dto2);
+    }
+    return;
+  }
   for (int n = n0 + 1; n <= n1; n++) {
     float* dst = G->seg + (size_t)(n - n0 - 1) * 3 * G->nfield;
     batch_step_into(mp, n, src, src ? src + G->nfield : nullptr, src ? src + 2 * G->nfield : nullptr, dto2, dst,
@@ -569,10 +745,29 @@ void sf2d_grad_result(long* Mesh_pointer, double* gk, double* gm, double* pm, do
   GradState* G = need(mp);
   check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_result");
   std::vector<double> t(std::max(G->ne, G->n2));
+  std::vector<int> first, count;
+  if (G->fused) {
+    first.assign(mp->nspec, 0);
+    count.assign(mp->nspec, 1);
+    for (int q = 0; q < mp->npatch; q++) {
+      const int e0 = mp->h_patch_desc[4 * q], ne = mp->h_patch_desc[4 * q + 3] & 0xf;
+      for (int k = 0; k < ne; k++) {
+        first[e0 + k] = e0;
+        count[e0 + k] = ne;
+      }
+    }
+  }
   auto elem = [&](const double* dev, double* out) {
     check_hip(hipMemcpy(t.data(), dev, G->ne * sizeof(double), hipMemcpyDeviceToHost), "gradient D2H");
     for (int e = 0; e < mp->nspec; e++) {
       const int pos = mp->pos_of_ispec[e];
+      if (G->fused) {  // lane order of the chain at e0
+        const int e0 = first[pos], ne = count[pos];
+        for (int p = 0; p < NGLL2; p++)
+          out[(size_t)e * NGLL2 + p] =
+              t[(size_t)e0 * NGLL2 + (size_t)(p / NGLL) * NGLL * ne + NGLL * (pos - e0) + p % NGLL];
+        continue;
+      }
       for (int p = 0; p < NGLL2; p++) out[(size_t)e * NGLL2 + p] = t[(size_t)pos * NGLL2 + p];
     }
   };

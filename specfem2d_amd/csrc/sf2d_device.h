@@ -165,4 +165,41 @@ __device__ __forceinline__ void record_receiver(const ReceiverSet& R, int r, int
   }
 }
 
+// point p of receiver r's residual {x, z} (its rotated components) into D, the adjoint of record_receiver
+__device__ __forceinline__ void adjoint_receiver(const ReceiverSet& R, int r, int p, const float* __restrict__ res,
+                                                 float* __restrict__ D, int ps) {
+  if (r >= R.nrec || p >= NGLL2) return;
+  const int i = p % NGLL, j = p / NGLL;
+  const float px = res[2 * r], pz = res[2 * r + 1];
+  const float c = R.cosrot[r], sn = R.sinrot[r];
+  const float cx = c * px - sn * pz, cz = sn * px + c * pz;
+  const float hl = R.xir[i * R.nrec + r] * R.gammar[j * R.nrec + r];
+  const size_t g = (size_t)R.ibool[(size_t)R.ispec[r] * NGLL2 + p] * ps;
+  atomicAdd(&D[2 * g], hl * cx);
+  atomicAdd(&D[2 * g + 1], hl * cz);
+}
+
+// the Stacey traction's dependence on rho vp and rho vs at face point q, summed over the shots (point g of shot s at
+// float2 g ps + s ss): gvp, gvs -= R~ . dB v'
+__device__ __forceinline__ void stacey_gradient(const StaceyFaces& F, int q, int nshot, int ps, long ss,
+                                                const float2* __restrict__ vpn, const float2* __restrict__ rb,
+                                                float* __restrict__ gvp, float* __restrict__ gvs) {
+  if (q >= F.nabs * NGLL) return;
+  const int f = q / NGLL;
+  const int ii = F.ij[2 * q], jj = F.ij[2 * q + 1];
+  if (ii < 0 || jj < 0) return;  // corner point owned by the other edge
+  const int g = F.ibool[(size_t)F.ispec[f] * NGLL2 + jj * NGLL + ii];
+  const float nx = F.normal[2 * q], nz = F.normal[2 * q + 1], w = F.jacw[q];
+  float sp = 0.f, sv = 0.f;
+  for (int s = 0; s < nshot; s++) {
+    const size_t o = (size_t)g * ps + (size_t)s * ss;
+    const float2 v = vpn[o], b = rb[o];
+    const float vn = nx * v.x + nz * v.y, bn = nx * b.x + nz * b.y;
+    sp += w * vn * bn;
+    sv += w * (v.x * b.x + v.y * b.y - vn * bn);
+  }
+  gvp[q] -= sp;
+  gvs[q] -= sv;
+}
+
 }  // namespace sf2d

@@ -228,6 +228,7 @@ struct BatchState {
   hipGraphExec_t graph_exec = nullptr;
   float graph_dt[3] = {0.f, 0.f, 0.f};
   int graph_record = -1;
+  int graph_fused = 0;
 };
 
 // shot batch fields and the re-arming of its deferred corrector (batch.hip)
@@ -274,6 +275,29 @@ void pml_acoustic_forces(Mesh* mp, int ph, const float* pot, const float* pd, fl
 void pml_acoustic_boundary(Mesh* mp, float* pot, float* pd, float* pdd);
 // the solid's fused time step (tower.hip)
 void tower_release(Mesh* mp);
+// a fused step of nshot forward fields, shot s at s * stride points: (d, v) -> (d_out, v_out), which may be the same; r_out
+// (may be null): the forces; last 1: the step ends a run (accel, v_out as kernel_3_a_cuda leaves them), 2: r_out only.
+// accel: boundary terms, zero at the start of a run (tower_begin_shots).  seismo (may be null): [shot][2][nrec][nstep]
+struct ShotStep {
+  const float *d, *v;
+  float *d_out, *v_out, *r_out, *accel;
+  long stride;
+  int nshot, last;
+  const int* src_shot;
+  float* seismo;
+  const int* step;  // (may be null) the 1-based step in device memory, for graph replays
+};
+void tower_begin_shots(Mesh* mp, float* accel, long stride, int nshot);
+void tower_step_shots(Mesh* mp, const ShotStep& S, int it, float deltat, float deltatsqover2, float deltatover2);
+// the reverse step of a gradient (gradient.hip): residuals and Stacey terms of the step, D += -K R~, and the next R~
+void tower_step_adjoint(Mesh* mp, float* Rb, float* D, float* Vb, long stride, int nshot, const float* res,
+                        const float* vpn, float* gvp, float* gvs, float dt, float h, float dto2);
+// copies the solid's displacement and velocity into gradient checkpoint `slot`; returns where its forces go
+float* grad_checkpoint_inputs(Mesh* mp, int slot);
+// source shots of the batch (batch.hip; null without a batch)
+const int* batch_source_shots(const Mesh* mp);
+// drops the batch's captured step, whose launches hold the towers' addresses
+void batch_drop_graph(Mesh* mp);
 bool tower_masses_fit(const Mesh* mp, const float* rmassx, const float* rmassz);
 // chain-kernel point ids with first-touch flags and the special points, uploaded again when the special points change
 void upload_chain_ids(Mesh* mp);

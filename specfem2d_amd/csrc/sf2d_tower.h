@@ -42,12 +42,12 @@ struct TowerChain {
   TowerRow row[NGLL];
 };
 bool cut_towers(const std::vector<TowerChain>& column, int want, std::vector<Tower>& out);
-int tower_chains(int nchain);
+int tower_chains(long nchain);
 // the towers of chains (above: the chain on top of each, -1: none), the lowest of all columns first, so that neighbours
 // run together.  kind: CHAIN_ALONE a tower of its own, CHAIN_SKIP none (the chain has no force of its own)
 enum : char { CHAIN_STACKED, CHAIN_ALONE, CHAIN_SKIP };
 bool chain_towers(const std::vector<int>& above, const std::vector<TowerChain>& chains, const std::vector<char>& kind,
-                  std::vector<Tower>& out);
+                  std::vector<Tower>& out, int nshot = 1);
 
 struct TowerPlan {
   int ntower = 0, nrow = 0;

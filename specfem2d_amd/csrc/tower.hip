@@ -31,7 +31,8 @@ namespace sf2d {
 struct TowerState {
   TowerPlan plan;
   float2* d_layer = nullptr; // forces of the CPML layer's element points
-  float2* d_slot = nullptr;  // [plan.nslot] forces of interface points
+  float2* d_slot = nullptr;  // [slot_shots][plan.nslot] forces of interface points
+  int slot_shots = 0;
 };
 
 namespace {
@@ -47,38 +48,72 @@ struct TowerAtt {
   long ne;
 };
 
+template <typename T>
+__device__ __forceinline__ void st_off(T* base, unsigned byte_off, T value) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte_off) = value;
+}
+
 // The wavefields of a step, shot s at s * stride points: (d, v) = (d_n, v'_n) in, (d_out, v_out) = (d_{n+1}, v'_{n+1})
-// out, which may be the same arrays.  last: the step ends a run instead, accel = a_n and v_out = v_n.  r_out (may be
-// null): the force r_n of every point.  accel holds the boundary terms at interface points.
+// out, which may be the same arrays.  r_out (may be null): the force r_n of every point.  last 1: the step ends a run
+// instead, accel = a_n and v_out = v_n; 2: r_out only.  accel holds the boundary terms at interface points.
 struct TowerFields {
   const float2 *d, *v;
   float2 *d_out, *v_out, *r_out, *accel;
   long stride;
   int nshot, last;
-};
-
-// the point at byte offset o: corrector of this step and predictor of the next (k_corrector's and k_predictor's
-// operations, contracted the same way, so that a run in pieces gives the bits of the run in one) from the force r
-__device__ __forceinline__ void newmark_point(const Newmark& c, const TowerFields& F, long shot, unsigned o, float2 r,
-                                              float wx, float wz, float2 d, float2 v) {
-  auto put = [&](float2* base, float2 value) {
-    *reinterpret_cast<float2*>(reinterpret_cast<char*>(base + shot) + o) = value;
+  struct Row {  // a point's operands besides the field that the force is computed from
+    float2 v;
   };
-  if (F.r_out) put(F.r_out, r);
-  const float2 a = make_float2(r.x * wx, r.y * wz);
-  v.x = fmaf(c.dto2, a.x, v.x);
-  v.y = fmaf(c.dto2, a.y, v.y);
-  if (F.last) {
-    put(F.accel, a);
-  } else {
-    d.x = fmaf(c.dt2o2, a.x, fmaf(c.dt, v.x, d.x));
-    d.y = fmaf(c.dt2o2, a.y, fmaf(c.dt, v.y, d.y));
+  __device__ const float2* field() const { return d; }
+  __device__ Row load(long shot, unsigned o) const { return {ld_off(v + shot, o)}; }
+  // the point at byte offset o: corrector of this step and predictor of the next (k_corrector's and k_predictor's
+  // operations, contracted the same way, so that a run in pieces gives the bits of the run in one) from the force r
+  __device__ void update(const Newmark& c, long shot, unsigned o, float2 r, float wx, float wz, float2 d, Row q) const {
+    if (r_out) st_off(r_out + shot, o, r);
+    if (last == 2) return;
+    float2 v = q.v;
+    const float2 a = make_float2(r.x * wx, r.y * wz);
     v.x = fmaf(c.dto2, a.x, v.x);
     v.y = fmaf(c.dto2, a.y, v.y);
-    put(F.d_out, d);
+    if (last) {
+      st_off(accel + shot, o, a);
+    } else {
+      d.x = fmaf(c.dt2o2, a.x, fmaf(c.dt, v.x, d.x));
+      d.y = fmaf(c.dt2o2, a.y, fmaf(c.dt, v.y, d.y));
+      v.x = fmaf(c.dto2, a.x, v.x);
+      v.y = fmaf(c.dto2, a.y, v.y);
+      st_off(d_out + shot, o, d);
+    }
+    st_off(v_out + shot, o, v);
   }
-  put(F.v_out, v);
-}
+};
+
+// The fields of a reverse step (gradient.hip): R~_n in, from which the force is computed, the cotangents D and V', and
+// R~_{n-1} = W A out in place: D += -K R~; V = V' + dt D; A = dt/2 V' + dt^2/2 D + dt/2 V
+struct AdjointFields {
+  float2 *Rb, *D, *Vb;
+  long stride;
+  int nshot;
+  struct Row {
+    float2 D, Vb;
+  };
+  __device__ const float2* field() const { return Rb; }
+  __device__ Row load(long shot, unsigned o) const { return {ld_off(D + shot, o), ld_off(Vb + shot, o)}; }
+  __device__ void update(const Newmark& c, long shot, unsigned o, float2 r, float wx, float wz, float2, Row q) const {
+    float2 db = q.D, v, a;
+    db.x += r.x;
+    db.y += r.y;
+    v.x = q.Vb.x + c.dt * db.x;
+    v.y = q.Vb.y + c.dt * db.y;
+    a.x = c.dto2 * q.Vb.x + c.dt2o2 * db.x;
+    a.y = c.dto2 * q.Vb.y + c.dt2o2 * db.y;
+    a.x = a.x + c.dto2 * v.x;
+    a.y = a.y + c.dto2 * v.y;
+    st_off(D + shot, o, db);
+    st_off(Vb + shot, o, v);
+    st_off(Rb + shot, o, make_float2(wx * a.x, wz * a.y));
+  }
+};
 
 // What else the launch does, in workgroups after the towers': Stacey faces, sources, receivers and fluid-solid edges of
 // the step
@@ -90,6 +125,7 @@ struct TowerEdges {
   int nface_wg, nsource, nreceiver, ncoupling_wg;
   CouplingPoints coupling; // fluid-solid edges (one shot)
   const float* pdd;        // the fluid's acceleration there
+  const int* step;         // (may be null) the 1-based step in device memory in place of it
   const int* src_shot;     // shot of each source (null: one shot)
   float* seismo;           // [shot][2][receiver][time]
   long seismo_stride;
@@ -98,6 +134,7 @@ struct TowerEdges {
 
 __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFields& F, int wg) {
   const int faces = E.nface_wg * F.nshot;
+  const int it = E.step ? *E.step - 1 : E.it;
   if (wg < faces) {
     const int shot = wg / E.nface_wg;
     stacey_traction(E.faces, (wg - shot * E.nface_wg) * 64 + threadIdx.x, F.v + shot * F.stride,
@@ -107,7 +144,7 @@ __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFiel
   wg -= faces;
   if (wg < E.nsource) {
     const long shot = E.src_shot ? E.src_shot[wg] : 0;
-    source_force(E.sources, wg, threadIdx.x, E.it, (float*)(F.accel + shot * F.stride), 1);
+    source_force(E.sources, wg, threadIdx.x, it, (float*)(F.accel + shot * F.stride), 1);
     return;
   }
   wg -= E.nsource;
@@ -117,7 +154,37 @@ __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFiel
   }
   const int shot = wg / E.nreceiver, r = wg - shot * E.nreceiver;
   if (E.faces.is_elastic[E.receivers.ispec[r]])  // receivers in fluid elements are recorded by the fluid
-    record_receiver(E.receivers, r, threadIdx.x, E.it, F.d + shot * F.stride, E.seismo + shot * E.seismo_stride, 1);
+    record_receiver(E.receivers, r, threadIdx.x, it, F.d + shot * F.stride, E.seismo + shot * E.seismo_stride, 1);
+}
+
+// the boundary part of a reverse step: residuals into D, -B R~ into V', and the Stacey terms of the gradient
+struct AdjointEdges {
+  StaceyFaces faces;
+  ReceiverSet receivers;
+  int nface_wg, nreceiver;
+  const float* res;        // [shot][receiver][2] of the step
+  const float2* vpn;       // v'_n of the forward field
+  float *gvp, *gvs;
+  int wgs(int nshot) const { return nface_wg * (nshot + 1) + nreceiver * nshot; }
+};
+
+__device__ __forceinline__ void tower_edges(const AdjointEdges& E, const AdjointFields& F, int wg) {
+  if (wg < E.nface_wg) {
+    stacey_gradient(E.faces, wg * 64 + threadIdx.x, F.nshot, 1, F.stride, E.vpn, F.Rb, E.gvp, E.gvs);
+    return;
+  }
+  wg -= E.nface_wg;
+  const int faces = E.nface_wg * F.nshot;
+  if (wg < faces) {
+    const int shot = wg / E.nface_wg;
+    stacey_traction(E.faces, (wg - shot * E.nface_wg) * 64 + threadIdx.x, F.Rb + shot * F.stride,
+                    (float*)(F.Vb + shot * F.stride), 1);
+    return;
+  }
+  wg -= faces;
+  const int shot = wg / E.nreceiver, r = wg - shot * E.nreceiver;
+  adjoint_receiver(E.receivers, r, threadIdx.x, E.res + (size_t)shot * 2 * E.receivers.nrec,
+                   (float*)(F.D + shot * F.stride), 1);
 }
 
 // The operands of a lane's column of one chain that the next iteration starts from, loaded one chain ahead: the
@@ -128,12 +195,12 @@ struct ChainRegs {
 };
 
 // GEO: 0 every element a rectangle {xi_x, gamma_z}, 1 every element affine (one record), 2 geometry per point
-template <int GEO, int SETS>
+template <int GEO, int SETS, class Fields, class Edges>
 __global__ __launch_bounds__(64) void k_tower(
     int ntower, const int4* __restrict__ desc, const int4* __restrict__ rows, const float4* __restrict__ geom,
-    const float4* __restrict__ geom_elem, const float2* __restrict__ mod, const TowerFields F,
+    const float4* __restrict__ geom_elem, const float2* __restrict__ mod, const Fields F,
     const float* __restrict__ rm, float2* __restrict__ slot, int nslot, const Newmark nm, const Basis basis,
-    const TowerAtt att, int tower_wgs, const TowerEdges edges) {
+    const TowerAtt att, int tower_wgs, const Edges edges) {
   constexpr bool RECT = GEO == 0;
   __shared__ float2 s_t[NGLL * TROW + 1];
   if ((int)blockIdx.x >= tower_wgs) {
@@ -146,8 +213,7 @@ __global__ __launch_bounds__(64) void k_tower(
   if (tower >= ntower) return;  // uniform over the wave
   const int shot = item - tower * F.nshot;
   const long at = shot * F.stride;
-  const float2* const __restrict__ d = F.d + at;
-  const float2* const __restrict__ v = F.v + at;
+  const float2* const __restrict__ d = F.field() + at;
   slot += (size_t)shot * nslot;
   const int4 td = desc[4 * tower], tb = desc[4 * tower + 1], ts = desc[4 * tower + 2], tt = desc[4 * tower + 3];
   const int nch = td.y, ne = td.z;
@@ -187,13 +253,13 @@ __global__ __launch_bounds__(64) void k_tower(
     if (GEO < 2) q.ge = ld_off(geom_elem, 16u * e);
   };
   // the update of one row's point, or its share of an interface point
-  auto finish = [&](const int4 r, unsigned o, float2 f, float2 u, float2 vp, float m) {
+  auto finish = [&](const int4 r, unsigned o, float2 f, float2 u, const typename Fields::Row& vp, float m) {
     if (!writer) return;
     const unsigned bits = x < 32 ? (unsigned)r.x >> x : (unsigned)r.y >> (x - 32);
     if (bits & 1u) {
       slot[r.z + __popc((unsigned)r.x & below_lo) + __popc((unsigned)r.y & below_hi)] = f;
     } else {
-      newmark_point(nm, F, at, o, f, m, m, u, vp);
+      F.update(nm, at, o, f, m, m, u, vp);
     }
   };
 
@@ -211,12 +277,12 @@ __global__ __launch_bounds__(64) void k_tower(
   for (int c = 0; c < nch; c++) {
     const ChainRegs q = nx;
     // this chain's velocity and inverse mass (rows 0 .. 3), needed at its end
-    float2 vp[NGLL - 1];
+    typename Fields::Row vp[NGLL - 1];
     float ms[NGLL - 1];
 #pragma unroll
     for (int j = 0; j < NGLL - 1; j++) {
       const unsigned o = j == 0 ? off0 : off1 + (unsigned)(j - 1) * up;
-      vp[j] = ld_off(v, o);
+      vp[j] = F.load(at, o);
       ms[j] = ld_off(rm, o / 2u);
     }
     float4 st[3];  // attenuation state of the next row
@@ -335,7 +401,7 @@ __global__ __launch_bounds__(64) void k_tower(
     elem = nelem;
   }
   // the tower's top row
-  finish(row[4 * nch], offt, carry, u0, ld_off(v, offt), ld_off(rm, offt / 2u));
+  finish(row[4 * nch], offt, carry, u0, F.load(at, offt), ld_off(rm, offt / 2u));
 }
 
 // Interface points: the slots of each point summed in order, the boundary terms of accel added and cleared, and the
@@ -358,7 +424,7 @@ __global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const 
   each_layer_slot(A, q, [&](int s) { add_slot(r, layer[s]); });
   if (fl & IF_ACC) {
     add_slot(r, F.accel[at + g]);
-    if (!F.last) F.accel[at + g] = make_float2(0.f, 0.f);
+    if (F.last != 1) F.accel[at + g] = make_float2(0.f, 0.f);
   }
   if ((fl & IF_PML) && old) {
     const float ax = r.x * wx, az = r.y * wz;
@@ -370,23 +436,63 @@ __global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const 
     F.v_out[at + g] = make_float2(0.f, 0.f);
     return;
   }
-  newmark_point(nm, F, at, 8u * (unsigned)g, r, wx, wz, dd, vv);
+  F.update(nm, at, 8u * (unsigned)g, r, wx, wz, dd, {vv});
+}
+
+__global__ __launch_bounds__(256) void k_interface_adjoint(const InterfaceArgs A, const float2* __restrict__ slot,
+                                                           int nslot, const AdjointFields F,
+                                                           const float* __restrict__ rmx, const float* __restrict__ rmz,
+                                                           const Newmark nm) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= A.n) return;
+  const long at = blockIdx.y * F.stride;
+  const int g = A.id[q];
+  const AdjointFields::Row row = F.load(at, 8u * (unsigned)g);
+  const float2 r = sum_towers(A, q, slot + (size_t)blockIdx.y * nslot, make_float2(0.f, 0.f));
+  F.update(nm, at, 8u * (unsigned)g, r, rmx[g], rmz[g], make_float2(0.f, 0.f), row);
 }
 
 // accel = 0 at the interface points with a boundary term (the start of a run of tower steps)
 __global__ __launch_bounds__(256) void k_interface_clear(int n, const int* __restrict__ ids,
-                                                         const uint8_t* __restrict__ flag, float2* __restrict__ accel) {
+                                                         const uint8_t* __restrict__ flag, float2* __restrict__ accel,
+                                                         long stride) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < n && (flag[q] & IF_ACC)) accel[ids[q]] = make_float2(0.f, 0.f);
+  if (q < n && (flag[q] & IF_ACC)) accel[ids[q] + blockIdx.y * stride] = make_float2(0.f, 0.f);
+}
+
+// the slots of nshot fields
+float2* tower_slots(TowerState* T, int nshot) {
+  if (nshot > T->slot_shots) {
+    device_free(T->d_slot);
+    T->d_slot = nullptr;
+    T->slot_shots = 0;
+    T->d_slot = device_alloc<float2>((size_t)T->plan.nslot * nshot);
+    T->slot_shots = nshot;
+  }
+  return T->d_slot;
+}
+
+int tower_geometry(const Mesh* mp) {
+  return mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+}
+
+template <class Fields, class Edges, class Kernel>
+void launch_k_tower(Mesh* mp, Kernel kern, const Fields& F, const Edges& E, float2* slot, const Newmark& nm) {
+  const TowerPlan& P = mp->tower->plan;
+  const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
+  if ((long)(P.ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", P.ntower, F.nshot);
+  const int wgs = (P.ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
+  hipLaunchKernelGGL(kern, dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, P.ntower, P.d_desc, P.d_row, mp->d_geom,
+                     mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, slot, P.nslot, nm, mp->basis, att, wgs, E);
+  check_hip(hipGetLastError(), "k_tower launch");
 }
 
 // one step of the fields F at time step it (1-based): towers with the step's Stacey faces, sources, fluid-solid edges
 // (forward) and (seismo not null) receivers, the CPML layer, the interface
 void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long seismo_stride, const int* src_shot,
-                  const Newmark& nm, bool forward) {
+                  const Newmark& nm, bool forward, const int* step = nullptr) {
   const TowerPlan& P = mp->tower->plan;
-  float2* const slot = mp->tower->d_slot;
-  const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
+  float2* const slot = tower_slots(mp->tower, F.nshot);
   TowerEdges E{};
   E.faces = stacey_faces(mp);
   E.sources = source_set(mp);
@@ -400,18 +506,14 @@ void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long se
   E.src_shot = src_shot;
   E.seismo = seismo;
   E.seismo_stride = seismo_stride;
-  if ((long)(P.ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", P.ntower, F.nshot);
-  const int wgs = (P.ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
-  const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+  E.step = step;
   const int sets = !mp->attenuation ? 0 : mp->att_ntable == 1 ? 1 : 2;
-  using K = decltype(&k_tower<0, 0>);
-  const K kern[3][3] = {{k_tower<0, 0>, k_tower<0, 1>, k_tower<0, 2>},
-                        {k_tower<1, 0>, k_tower<1, 1>, k_tower<1, 2>},
-                        {k_tower<2, 0>, k_tower<2, 1>, k_tower<2, 2>}};
-  hipLaunchKernelGGL(kern[geo][sets], dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, P.ntower, P.d_desc, P.d_row,
-                     mp->d_geom, mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, slot, P.nslot, nm, mp->basis, att, wgs,
-                     E);
-  check_hip(hipGetLastError(), "k_tower launch");
+  using K = decltype(&k_tower<0, 0, TowerFields, TowerEdges>);
+#define SF2D_SETS(g) {k_tower<g, 0, TowerFields, TowerEdges>, k_tower<g, 1, TowerFields, TowerEdges>, \
+                      k_tower<g, 2, TowerFields, TowerEdges>}
+  const K kern[3][3] = {SF2D_SETS(0), SF2D_SETS(1), SF2D_SETS(2)};
+#undef SF2D_SETS
+  launch_k_tower(mp, kern[tower_geometry(mp)][sets], F, E, slot, nm);
   if (forward) pml_elastic_slots(mp, mp->tower->d_layer);
   if (P.n == 0) return;
   hipLaunchKernelGGL(k_interface, dim3((P.n + 255) / 256, F.nshot), dim3(256), 0, mp->stream, interface_args(P), slot,
@@ -420,15 +522,59 @@ void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long se
   check_hip(hipGetLastError(), "k_interface launch");
 }
 
+// accel = 0 at the interface points with a boundary term, before the first of a run of steps
+void clear_interface(Mesh* mp, float2* accel, long stride, int nshot) {
+  const TowerPlan& P = mp->tower->plan;
+  if (P.n == 0) return;
+  hipLaunchKernelGGL(k_interface_clear, dim3((P.n + 255) / 256, nshot), dim3(256), 0, mp->stream, P.n, P.d_id, P.d_flag,
+                     accel, stride);
+  check_hip(hipGetLastError(), "k_interface_clear launch");
+}
+
 }  // namespace
 
-// Chains per tower: about one wave per slot of the card (4096 at four waves per SIMD) and at most 16.  A tall tower has
+// shot batches and gradients: nshot forward fields, shot s at s * stride points
+void tower_begin_shots(Mesh* mp, float* accel, long stride, int nshot) {
+  clear_interface(mp, (float2*)accel, stride, nshot);
+}
+void tower_step_shots(Mesh* mp, const ShotStep& S, int it, float deltat, float deltatsqover2, float deltatover2) {
+  const TowerFields F{(const float2*)S.d, (const float2*)S.v, (float2*)S.d_out, (float2*)S.v_out, (float2*)S.r_out,
+                      (float2*)S.accel, S.stride, S.nshot, S.last};
+  launch_tower(mp, F, it, S.seismo, (long)2 * mp->nrec_local * mp->nstep, S.src_shot,
+               {deltatover2, deltat, deltatsqover2}, false, S.step);
+}
+void tower_step_adjoint(Mesh* mp, float* Rb, float* D, float* Vb, long stride, int nshot, const float* res,
+                        const float* vpn, float* gvp, float* gvs, float dt, float h, float dto2) {
+  const TowerPlan& P = mp->tower->plan;
+  float2* const slot = tower_slots(mp->tower, nshot);
+  const AdjointFields F{(float2*)Rb, (float2*)D, (float2*)Vb, stride, nshot};
+  const Newmark nm{dto2, dt, h};
+  AdjointEdges E{};
+  E.faces = stacey_faces(mp);
+  E.receivers = receiver_set(mp);
+  E.nface_wg = mp->stacey ? (mp->num_abs * NGLL + 63) / 64 : 0;
+  E.nreceiver = mp->nrec_local;
+  E.res = res;
+  E.vpn = (const float2*)vpn;
+  E.gvp = gvp;
+  E.gvs = gvs;
+  using K = decltype(&k_tower<0, 0, AdjointFields, AdjointEdges>);
+  const K kern[3] = {k_tower<0, 0, AdjointFields, AdjointEdges>, k_tower<1, 0, AdjointFields, AdjointEdges>,
+                     k_tower<2, 0, AdjointFields, AdjointEdges>};
+  launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, nm);
+  if (P.n == 0) return;
+  hipLaunchKernelGGL(k_interface_adjoint, dim3((P.n + 255) / 256, nshot), dim3(256), 0, mp->stream, interface_args(P),
+                     slot, P.nslot, F, mp->d_rmassx, mp->d_rmassz, nm);
+  check_hip(hipGetLastError(), "k_interface_adjoint launch");
+}
+
+// Chains per tower (nchain: times the shots): about one wave per slot of the card (4096 at four waves per SIMD) and at most 16.  A tall tower has
 // few interface rows (1 in 4 x chains), a short one more waves in flight.  Measured, ms of 300 steps of 600 x 300 elements
 // (15,000 chains) at 1, 2, 4, 8, 16 chains: 15.3, 13.9, 13.6, 14.2, 18.7; 40 steps of 2000 x 1000 (166,667 chains) at 2, 4,
 // 8, 16, 32: 19.9, 17.9, 17.2, 17.1, 17.6.
-int tower_chains(int nchain) {
+int tower_chains(long nchain) {
   if (const char* env = getenv("SF2D_TOWER_CHAINS")) return std::max(1, atoi(env));
-  return std::max(1, std::min(16, (nchain + 4095) / 4096));
+  return (int)std::max(1L, std::min(16L, (nchain + 4095) / 4096));
 }
 
 bool cut_towers(const std::vector<TowerChain>& column, int want, std::vector<Tower>& out) {
@@ -457,12 +603,12 @@ bool cut_towers(const std::vector<TowerChain>& column, int want, std::vector<Tow
 }
 
 bool chain_towers(const std::vector<int>& above, const std::vector<TowerChain>& chains, const std::vector<char>& kind,
-                  std::vector<Tower>& out) {
+                  std::vector<Tower>& out, int nshot) {
   const int n = (int)chains.size();
   std::vector<char> has_below(n, 0);
   for (int a : above)
     if (a >= 0) has_below[a] = 1;
-  const int want = tower_chains(n);
+  const int want = tower_chains((long)n * nshot);
   std::vector<Tower> towers;
   std::vector<std::pair<int, int>> order;  // height of the tower in its column, tower
   std::vector<TowerChain> column;
@@ -606,6 +752,7 @@ bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob,
 void tower_release(Mesh* mp) {
   TowerState* T = mp->tower;
   if (!T) return;
+  batch_drop_graph(mp);
   T->plan.release();
   device_free(T->d_slot);
   device_free(T->d_layer);
@@ -632,8 +779,7 @@ extern "C" {
 int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rmassz) {
   Mesh* mp = handle(Mesh_pointer);
   tower_release(mp);
-  if (!mp->chain || !mp->first_touch || !mp->d_col_rows || mp->assembly != 0 || mp->anisotropy || mp->batch ||
-      mp->save_forward || getenv("SF2D_NO_TOWERS"))
+  if (!mp->chain || !mp->first_touch || !mp->d_col_rows || mp->assembly != 0 || mp->anisotropy || mp->save_forward || getenv("SF2D_NO_TOWERS"))
     return 0;
   const int npatch = mp->npatch, ng = mp->nglob;
   const std::vector<int4>& rows = mp->h_col_rows;
@@ -656,7 +802,7 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     if (layer) kind[q] = CHAIN_SKIP;
   }
   std::vector<Tower> towers;
-  if (!chain_towers(mp->h_above, chains, kind, towers)) return 0;
+  if (!chain_towers(mp->h_above, chains, kind, towers, mp->batch ? mp->batch->nshot : 1)) return 0;
   // points that something besides the towers acts on or looks at
   std::vector<uint8_t> flag((size_t)ng, 0);
   auto mark_element = [&](int ispec, uint8_t f) {
@@ -686,7 +832,6 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     delete T;
     return 0;
   }
-  T->d_slot = device_alloc<float2>((size_t)T->plan.nslot);
   if (!pml.empty()) T->d_layer = device_alloc<float2>(pml.size());
   mp->tower = T;
   return 1;
@@ -697,20 +842,18 @@ int sf2d_tower_ready(long* Mesh_pointer) { return handle(Mesh_pointer)->tower !=
 void sf2d_tower_begin(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
   if (!mp->tower) fail("sf2d_tower_begin: no towers");
-  const TowerPlan& P = mp->tower->plan;
-  if (P.n == 0) return;
-  hipLaunchKernelGGL(k_interface_clear, dim3((P.n + 255) / 256), dim3(256), 0, mp->stream, P.n, P.d_id, P.d_flag,
-                     (float2*)mp->d_accel);
-  check_hip(hipGetLastError(), "k_interface_clear launch");
+  clear_interface(mp, (float2*)mp->d_accel, 0, 1);
 }
 
-void sf2d_tower_step(long* Mesh_pointer, int it, int last, float deltat, float deltatsqover2, float deltatover2) {
+void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float deltat, float deltatsqover2,
+                     float deltatover2) {
   Mesh* mp = handle(Mesh_pointer);
   if (!mp->tower || !mp->accel_partial || mp->pending_corrector[0])
     fail("sf2d_tower_step: call after update_displacement_cuda and sf2d_tower_begin");
   if (it < 1 || it > mp->nstep) fail("sf2d_tower_step: it=%d outside 1..%d", it, mp->nstep);
   float2 *d = (float2*)mp->d_displ, *v = (float2*)mp->d_veloc;
-  const TowerFields F{d, v, d, v, nullptr, (float2*)mp->d_accel, 0, 1, last};
+  float2* const r = checkpoint >= 0 ? (float2*)grad_checkpoint_inputs(mp, checkpoint) : nullptr;
+  const TowerFields F{d, v, d, v, r, (float2*)mp->d_accel, 0, 1, last ? 1 : 0};
   // displacement of the receivers in solid elements; the fluid records its own, and the caller the run's last step
   const int record = !last && mp->nrec_local > 0 && mp->h_seismotype[0] == 1;
   if (record && it > mp->nlength_seismogram) fail("sf2d_tower_step: step %d after the seismograms' last", it);
