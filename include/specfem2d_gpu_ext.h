@@ -58,6 +58,12 @@ int sf2d_mesh_fluid_chain(long* Mesh_pointer);
 /* 1 when every element is affine and axis-aligned (xi_z = gamma_x = 0 to 2^-22 of the element's largest geometry
    entry): the chain kernel then uses its rectangle form (SF2D_NO_RECT keeps the general form) */
 int sf2d_mesh_rect(long* Mesh_pointer);
+/* the fields of a run from rest: displacement, velocity, acceleration and the potential with its derivatives zero */
+void sf2d_mesh_zero_fields(long* Mesh_pointer);
+/* compute_seismograms_cuda_ in two parts: records sample `current` (1-based) on the device; copies `count` samples from
+   `first` (1-based) on to the host and returns them there, [2][nrec][count], until the next call (null without receivers) */
+void sf2d_seismograms_record(long* Mesh_pointer, int i_sig, int current, int trick);
+const float* sf2d_seismograms_read(long* Mesh_pointer, int i_sig, int first, int count);
 /* The fused time step (forward runs of chain meshes; no counterpart in the reference): corrector of step n and predictor
    of step n + 1 inside the force kernel.
    Solid: sf2d_tower_prepare, after all other preparation (rmassx, rmassz as prepare_fields_elastic_device_ got them),

@@ -1284,6 +1284,12 @@ CouplingPoints acoustic_coupling(Mesh* mp, const float** pdd) {
   return coupling_points(ac);
 }
 
+void acoustic_zero_fields(Mesh* mp) {
+  if (!mp->ac) return;
+  for (float* f : {mp->ac->d_pot, mp->ac->d_pd, mp->ac->d_pdd})
+    check_hip(hipMemsetAsync(f, 0, (size_t)mp->nglob * sizeof(float), mp->stream), "zero fields");
+}
+
 std::vector<int> acoustic_elements(const Mesh* mp) {
   std::vector<int> out;
   if (mp->ac) out = mp->ac->phase_elems[1];

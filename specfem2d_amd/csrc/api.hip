@@ -1526,9 +1526,28 @@ void compute_seismograms_cuda_(long* Mesh_pointer_f, int* i_sigf, double* sisux,
   const int i_sig = *i_sigf - 1;
   const int cur = *seismo_currentf - 1;
   const int nlength = *nlength_seismogramf;
-  if (i_sig < 0 || i_sig >= mp->nsigtype) fail("compute_seismograms_cuda: i_sig %d out of range", i_sig + 1);
   if (nlength != mp->nlength_seismogram) fail("compute_seismograms_cuda: nlength_seismogram mismatch");
-  if (cur < 0 || cur >= nlength) fail("compute_seismograms_cuda: seismo_current %d outside 1..%d", cur + 1, nlength);
+  sf2d_seismograms_record(Mesh_pointer_f, *i_sigf, *seismo_currentf, *USE_TRICK_FOR_BETTER_PRESSURE);
+  if (cur == nlength - 1 || *itf == *it_endf) {
+    const size_t size = (size_t)mp->nrec_local * nlength;
+    float* h = mp->h_seismo[i_sig];
+    check_hip(hipMemcpyAsync(h, mp->d_seismo[i_sig], sizeof(float) * 2 * size, hipMemcpyDeviceToHost, mp->stream),
+              "seismo D2H");
+    check_hip(hipStreamSynchronize(mp->stream), "compute_seismograms_cuda");
+    for (size_t k = 0; k < size; k++) {
+      sisux[k] = (double)h[k];
+      sisuz[k] = (double)h[k + size];
+    }
+  }
+}
+
+void sf2d_seismograms_record(long* Mesh_pointer, int i_sig1, int current, int trick) {
+  Mesh* mp = handle(Mesh_pointer);
+  if (mp->nrec_local == 0) return;
+  const int i_sig = i_sig1 - 1, cur = current - 1;
+  if (i_sig < 0 || i_sig >= mp->nsigtype) fail("compute_seismograms_cuda: i_sig %d out of range", i_sig + 1);
+  if (cur < 0 || cur >= mp->nlength_seismogram)
+    fail("compute_seismograms_cuda: seismo_current %d outside 1..%d", cur + 1, mp->nlength_seismogram);
   const int stype = mp->h_seismotype[i_sig];
   const float* field = nullptr;
   if (stype == 2 || stype == 3) flush_correctors(mp);
@@ -1544,23 +1563,27 @@ void compute_seismograms_cuda_(long* Mesh_pointer_f, int* i_sigf, double* sisux,
   }
   float* d_dst = mp->d_seismo[i_sig];
   if (stype == 4 || stype == 6)
-    launch_acoustic_pressure_seismograms(mp, d_dst, cur, *USE_TRICK_FOR_BETTER_PRESSURE, stype == 6);
+    launch_acoustic_pressure_seismograms(mp, d_dst, cur, trick, stype == 6);
   else {
     // receivers in solid elements interpolate the vector field; those in fluid elements then overwrite theirs with
     // the gradient of the matching scalar field over the density
     if (mp->nspec_elastic > 0) launch_seismograms(mp, field, d_dst, cur);
     if (acoustic_receivers(mp) > 0) launch_acoustic_vector_seismograms(mp, d_dst, cur, stype);
   }
-  if (cur == nlength - 1 || *itf == *it_endf) {
-    const size_t size = (size_t)mp->nrec_local * nlength;
-    float* h = mp->h_seismo[i_sig];
-    check_hip(hipMemcpyAsync(h, d_dst, sizeof(float) * 2 * size, hipMemcpyDeviceToHost, mp->stream), "seismo D2H");
-    check_hip(hipStreamSynchronize(mp->stream), "compute_seismograms_cuda");
-    for (size_t k = 0; k < size; k++) {
-      sisux[k] = (double)h[k];
-      sisuz[k] = (double)h[k + size];
-    }
-  }
+}
+
+const float* sf2d_seismograms_read(long* Mesh_pointer, int i_sig1, int first, int count) {
+  Mesh* mp = handle(Mesh_pointer);
+  const int i_sig = i_sig1 - 1, nlength = mp->nlength_seismogram;
+  if (i_sig < 0 || i_sig >= mp->nsigtype || first < 1 || count < 1 || first - 1 + count > nlength)
+    fail("sf2d_seismograms_read: samples %d..%d outside 1..%d", first, first + count - 1, nlength);
+  if (mp->nrec_local == 0) return nullptr;
+  const size_t row = (size_t)count * sizeof(float);
+  check_hip(hipMemcpy2DAsync(mp->h_seismo[i_sig], row, mp->d_seismo[i_sig] + first - 1, (size_t)nlength * sizeof(float),
+                             row, (size_t)2 * mp->nrec_local, hipMemcpyDeviceToHost, mp->stream),
+            "seismo D2H");
+  check_hip(hipStreamSynchronize(mp->stream), "sf2d_seismograms_read");
+  return mp->h_seismo[i_sig];
 }
 
 void compute_kernels_elastic_cuda_(long* Mesh_pointer, realw* deltat) {  // compute_kernels_cuda.cu:47
@@ -1771,6 +1794,17 @@ extern "C" void sf2d_attenuation_reset(long* Mesh_pointer) {
   if (!mp->attenuation) return;
   const size_t ne = (size_t)mp->nspec * NGLL2;
   check_hip(hipMemsetAsync(mp->d_att_e, 0, 12 * ne * sizeof(float), mp->stream), "attenuation reset");
+}
+
+extern "C" void sf2d_mesh_zero_fields(long* Mesh_pointer) {
+  Mesh* mp = handle(Mesh_pointer);
+  const size_t n = (size_t)2 * mp->nglob * sizeof(float);
+  for (float* f : {mp->d_displ, mp->d_veloc, mp->d_accel})
+    if (f) check_hip(hipMemsetAsync(f, 0, n, mp->stream), "zero fields");
+  if (mp->pending_corrector[1]) flush_correctors(mp);
+  mp->pending_corrector[0] = 0;
+  mp->accel_partial = 0;
+  acoustic_zero_fields(mp);
 }
 
 extern "C" void sf2d_pml_reset(long* Mesh_pointer) { pml_reset(handle(Mesh_pointer)); }

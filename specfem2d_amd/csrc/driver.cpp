@@ -1726,18 +1726,14 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   float b_deltat = 0.f, b_deltatover2 = 0.f, b_deltatsqover2 = 0.f;
   int nspec_outer = 0, nspec_inner = s->nspec, zero = 0, one = 1, att = s->attenuation;
   const int it_begin = s->it_done + 1;
-  int i_sig = 1, nlength = s->p.nstep, it_end = s->it_done + nstep_run;
+  const int it_end = s->it_done + nstep_run;
   const bool any_ac = s->nspec_ac > 0, any_el = s->nspec_ac < s->nspec;
   const bool pml = s->nspec_pml > 0;
-  int elastic_sim = any_el ? 1 : 0, acoustic_sim = any_ac ? 1 : 0, trick = s->p.use_trick ? 1 : 0;
+  const int trick = s->p.use_trick ? 1 : 0;
   int nspec_inner_ac = s->nspec_ac, nfluid_solid = (int)s->coup_ac_ispec.size();
   int aniso = s->aniso_elem.empty() ? 0 : 1;
   nspec_inner = s->nspec - s->nspec_ac;
   if (any_ac && s->grad_save) return 1;  // no fluid gradients
-  if (s->sisux.empty()) {
-    s->sisux.assign((size_t)std::max(1, s->nrec) * nlength, 0.0);
-    s->sisuz.assign(s->sisux.size(), 0.0);
-  }
   const int counts[5] = {0, s->nspec_side[1], s->nspec_side[2], s->nspec_side[3], s->nspec_side[4]};
   std::vector<float> slice[5], slice_ac[5];
   for (int c = 1; c <= 4; c++) slice[c].assign((size_t)2 * NGLL * std::max(1, counts[c]), 0.f);
@@ -1746,8 +1742,15 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   const bool timed = timing != nullptr;
   const bool phases = timed && timing[0] < 0.0;
   hipStream_t stream = (hipStream_t)sf2d_mesh_stream(&s->mesh);
+  // the forces' time is measured in the first 4 steps and then in every 16th, and scaled to all steps: a pair of events
+  // costs a small mesh's step more than half of its kernels' time (80 x 60 elements: 20 us a step with, 11 without)
   const int nev = phases ? 10 : 2;  // per step: forces (2) [+ predictor, boundary, corrector, seismograms]
-  std::vector<hipEvent_t> ev(timed ? (size_t)nev * nstep_run : 0);
+  const int every = phases ? 1 : 16, head = 4;
+  auto measured = [&](int step) { return step < head || step % every == 0; };
+  std::vector<int> at;  // index of each measured step
+  int nmeasured = 0;
+  for (int k = 0; timed && k < nstep_run; k++) at.push_back(measured(k) ? nmeasured++ : -1);
+  std::vector<hipEvent_t> ev((size_t)nev * nmeasured);
   for (auto& e : ev) hc(hipEventCreate(&e));
   hipEvent_t loop_start, loop_end;
   if (timed) {
@@ -1756,7 +1759,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     hc(hipEventRecord(loop_start, stream));
   }
   auto mark = [&](int step, int k) {
-    if (timed && k < nev) hc(hipEventRecord(ev[(size_t)step * nev + k], stream));
+    if (timed && k < nev && at[step] >= 0) hc(hipEventRecord(ev[(size_t)at[step] * nev + k], stream));
   };
   // the fused steps of the solid and the fluid where the handle has them and nothing between a step's phases is asked for;
   // the fluid's alone only without a solid (the receivers of both are recorded together)
@@ -1808,8 +1811,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     if (fused) {
       // receivers in fluid elements (the solid's are recorded by the fused step)
       if (any_ac && !fused_ac && s->nrec > 0 && it < it_end)
-        compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
-                                  &acoustic_sim, &trick, &zero, &it, &it_end);
+        sf2d_seismograms_record(&s->mesh, 1, it, trick);
       // the fused steps clear the layer's outer boundary for the next step
       if (pml && (it == it_begin || (any_ac && !fused_ac))) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
       mark(step, 0);
@@ -1820,8 +1822,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     }
     if (fused || fused_ac) {
       if (it == it_end && s->nrec > 0)
-        compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
-                                  &acoustic_sim, &trick, &zero, &it, &it_end);
+        sf2d_seismograms_record(&s->mesh, 1, it, trick);
       continue;
     }
     // then the solid, coupled to the new fluid pressure (compute_gpu_elastic.f90:34-215)
@@ -1864,11 +1865,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     else if (s->grad_save == 2)
       sf2d_grad_save_state(&s->mesh, 1, it - s->grad_seg_base - 1);
     mark(step, 8);
-    if (s->nrec > 0) {
-      int cur = it;
-      compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &cur, &nlength, &elastic_sim,
-                                &acoustic_sim, &trick, &zero, &it, &it_end);
-    }
+    if (s->nrec > 0) sf2d_seismograms_record(&s->mesh, 1, it, trick);
     mark(step, 9);
   }
   s->it_done = it_end;
@@ -1881,13 +1878,14 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
     hc(hipEventElapsedTime(&ms, loop_start, loop_end));
     double acc[6] = {ms, 0, 0, 0, 0, 0};
     const int pairs[5][2] = {{2, 3}, {0, 1}, {4, 5}, {6, 7}, {8, 9}};  // predictor, forces, boundary, corrector, seismo
-    for (int step = 0; step < nstep_run; step++)
+    for (int k = 0; k < nmeasured; k++)
       for (int q = 0; q < 5; q++) {
         if (pairs[q][1] >= nev) continue;
         float t = 0.f;
-        hc(hipEventElapsedTime(&t, ev[(size_t)step * nev + pairs[q][0]], ev[(size_t)step * nev + pairs[q][1]]));
+        hc(hipEventElapsedTime(&t, ev[(size_t)k * nev + pairs[q][0]], ev[(size_t)k * nev + pairs[q][1]]));
         acc[q + 1] += t;
       }
+    for (int q = 1; q < 6; q++) acc[q] *= (double)nstep_run / nmeasured;
     for (int k = 0; k < 6; k++) timing[k] = acc[k];
     for (auto& e : ev) hc(hipEventDestroy(e));
     hc(hipEventDestroy(loop_start));
@@ -1895,12 +1893,13 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   } else {
     hc(hipStreamSynchronize(stream));
   }
-  if (seis)
-    for (int r = 0; r < s->nrec; r++)
-      for (int k = 0; k < nstep_run; k++) {
-        seis[((size_t)r * 2 + 0) * nstep_run + k] = s->sisux[(size_t)r * nlength + it_begin - 1 + k];
-        seis[((size_t)r * 2 + 1) * nstep_run + k] = s->sisuz[(size_t)r * nlength + it_begin - 1 + k];
-      }
+  if (seis && s->nrec > 0) {
+    const float* rows = sf2d_seismograms_read(&s->mesh, 1, it_begin, nstep_run);
+    for (int c = 0; c < 2; c++)
+      for (int r = 0; r < s->nrec; r++)
+        for (int k = 0; k < nstep_run; k++)
+          seis[((size_t)r * 2 + c) * nstep_run + k] = (double)rows[((size_t)c * s->nrec + r) * nstep_run + k];
+  }
   return 0;
 }
 
@@ -2358,13 +2357,8 @@ void sf2d_sim_reset(void* sim) {
   if (!s || !s->mesh) return;
   sf2d_attenuation_reset(&s->mesh);
   sf2d_pml_reset(&s->mesh);
-  std::vector<float> zeros((size_t)2 * s->nglob, 0.f);
-  int size = 2 * s->nglob, nac = s->nglob;
-  if (s->nspec_ac > 0) transfer_fields_ac_to_device_(&nac, zeros.data(), zeros.data(), zeros.data(), &s->mesh);
-  if (s->nspec_ac < s->nspec) transfer_fields_el_to_device_(&size, zeros.data(), zeros.data(), zeros.data(), &s->mesh);
+  sf2d_mesh_zero_fields(&s->mesh);
   s->it_done = 0;
-  std::fill(s->sisux.begin(), s->sisux.end(), 0.0);
-  std::fill(s->sisuz.begin(), s->sisuz.end(), 0.0);
 }
 
 int sf2d_sim_steps_done(void* sim) { return ((Sim*)sim)->it_done; }

@@ -310,6 +310,7 @@ bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const in
 std::vector<int> fluid_numbering(const std::vector<int>& ibool, int nglob, const std::vector<int>& elems);
 // the fluid's elements in the order of their phase lists (acoustic.hip); empty without a fluid
 std::vector<int> acoustic_elements(const Mesh* mp);
+void acoustic_zero_fields(Mesh* mp);  // the potential and its derivatives (acoustic.hip)
 // fills the column-lane copies of the chain ids and moduli from d_chain_ids and d_moduli (when both are allocated)
 void launch_col_pack(const Mesh* mp);
 // point arrays in the caller's numbering <-> the device numbering (n2 values per point)
