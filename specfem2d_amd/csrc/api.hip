@@ -1591,7 +1591,7 @@ void compute_kernels_elastic_cuda_(long* Mesh_pointer, realw* deltat) {  // comp
   Mesh* mp = handle(Mesh_pointer);
   flush_correctors(mp);
   if (!mp->d_rho_kl || !mp->d_b_displ) fail("compute_kernels_elastic_cuda: adjoint arrays not prepared");
-  launch_kernels(mp);
+  launch_kernels(mp, mp->d_displ, mp->d_accel, mp->d_b_displ);
 }
 
 // ---------------------------------------------------------------------------

@@ -1765,7 +1765,7 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
   // the fluid's alone only without a solid (the receivers of both are recorded together)
   const int st = s->p.seismotype;
   const bool seen = s->nrec == 0 || st == 1 || st == 4 || st == 6 || (st == 3 && !any_el);
-  const bool whole = !phases && !s->save_forward && s->grad_save != 2 && seen;
+  const bool whole = s->simulation_type == 1 && !phases && (!s->save_forward || !any_ac) && s->grad_save != 2 && seen;
   const bool fused = any_el && whole && sf2d_tower_ready(&s->mesh);
   const bool fused_ac = any_ac && whole && (fused || !any_el) && sf2d_tower_fluid_ready(&s->mesh);
   for (int it = it_begin; it <= it_end; it++) {
@@ -1816,7 +1816,8 @@ int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, doub
       if (pml && (it == it_begin || (any_ac && !fused_ac))) pml_boundary_elastic_cuda_(&s->mesh, &one, &zero);
       mark(step, 0);
       const bool save = s->grad_save == 1 && it % s->grad_chunk == 0 && it < s->p.nstep;
-      sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, save ? it / s->grad_chunk - 1 : -1, deltat, deltatsqover2,
+      float* const edges = absorb && s->save_forward && s->nabs > 0 ? absorb + (size_t)step * s->nabs * NGLL * 2 : nullptr;
+      sf2d_tower_step(&s->mesh, it, it == it_end ? 1 : 0, save ? it / s->grad_chunk - 1 : -1, edges, deltat, deltatsqover2,
                       deltatover2);
       mark(step, 1);
     }
@@ -2049,8 +2050,24 @@ int sf2d_sim_adjoint_full(void* sim, const float* adj, const float* absorb, cons
     }
     kernel_3_a_cuda_(&s->mesh, &deltatover2, &b_deltatover2, &w1, &w2);
   };
+  // solid meshes: after the first step, which ends with the reconstructed fields read from the last forward frames, both
+  // fields' fused steps where the handle has them
+  const bool fused = any_el && !any_ac && !att && (s->nrec == 0 || s->p.seismotype == 1) && sf2d_tower_ready(&s->mesh);
   for (int it = 1; it <= nstep; it++) {
     const int it_tmp = nstep - it + 1;
+    if (fused && it > 1) {
+      if (it == 2) {
+        update_displacement_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,
+                                  &b_deltatover2);
+        sf2d_tower_adjoint_begin(&s->mesh);
+      }
+      sf2d_tower_adjoint_step(&s->mesh, it, it == nstep ? 1 : 0, absorb, deltat, deltatsqover2, deltatover2, b_deltat,
+                              b_deltatsqover2, b_deltatover2);
+      if (it == nstep && s->nrec > 0)
+        compute_seismograms_cuda_(&s->mesh, &i_sig, s->sisux.data(), s->sisuz.data(), &it, &nlength, &elastic_sim,
+                                  &acoustic_sim, &trick, &zero, &it, &it_end);
+      continue;
+    }
     // update_displ_Newmark: both fields of each domain (update_displacement_Newmark.F90:126-160, 500-548)
     if (any_ac)
       update_displacement_ac_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,

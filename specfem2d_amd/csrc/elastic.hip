@@ -1208,23 +1208,10 @@ __global__ __launch_bounds__(64) void k_sources(const SourceSet S, int it, float
 }
 
 // adjoint sources at the receivers (src/gpu/kernels/add_sources_el_SIM_TYPE_2_OR_3_kernel.cu:37-74)
-__global__ __launch_bounds__(64) void k_adjoint_sources(int nadj, int it, int nstep, const int* __restrict__ ispec_rec,
-                                                        const int* __restrict__ is_elastic,
-                                                        const int* __restrict__ ibool, const float* __restrict__ xir,
-                                                        const float* __restrict__ gammar,
-                                                        const float* __restrict__ adj, float* __restrict__ accel) {
-  const int r = blockIdx.x;
-  const int p = threadIdx.x;
-  if (r >= nadj || p >= NGLL2) return;
-  const int ispec = ispec_rec[r];
-  if (!is_elastic[ispec]) return;
-  const int i = p % NGLL, j = p / NGLL;
-  const int g = ibool[(size_t)ispec * NGLL2 + p];
-  const float h = xir[i * nadj + r] * gammar[j * nadj + r];
-  const float ax = adj[((size_t)0 * nstep + it) * nadj + r];
-  const float az = adj[((size_t)1 * nstep + it) * nadj + r];
-  atomic_add_f32(&accel[2 * (size_t)g], ax * h);
-  atomic_add_f32(&accel[2 * (size_t)g + 1], az * h);
+__global__ __launch_bounds__(64) void k_adjoint_sources(const ReceiverSet R, const int* __restrict__ is_elastic, int it,
+                                                        int nstep, const float* __restrict__ adj,
+                                                        float* __restrict__ accel) {
+  adjoint_source(R, is_elastic, blockIdx.x, threadIdx.x, it, nstep, adj, accel);
 }
 
 // ---------------------------------------------------------------------------
@@ -1615,9 +1602,8 @@ void launch_sources(const Mesh* mp, float* accel, int it, const int* src_shot, l
 
 void launch_adjoint_sources(const Mesh* mp, float* accel, int it) {
   if (mp->nadj_rec_local <= 0) return;
-  hipLaunchKernelGGL(k_adjoint_sources, dim3(mp->nadj_rec_local), dim3(64), 0, mp->stream, mp->nadj_rec_local, it,
-                     mp->nstep, mp->d_ispec_selected_rec, mp->d_ispec_is_elastic, mp->d_ibool, mp->d_xir,
-                     mp->d_gammar, mp->d_source_adjoint, accel);
+  hipLaunchKernelGGL(k_adjoint_sources, dim3(mp->nadj_rec_local), dim3(64), 0, mp->stream, receiver_set(mp),
+                     mp->d_ispec_is_elastic, it, mp->nstep, mp->d_source_adjoint, accel);
   check_hip(hipGetLastError(), "k_adjoint_sources launch");
 }
 
@@ -1629,12 +1615,12 @@ void launch_seismograms(const Mesh* mp, const float* field, float* dst, int seis
   check_hip(hipGetLastError(), "k_seismograms launch");
 }
 
-void launch_kernels(const Mesh* mp) {
+void launch_kernels(const Mesh* mp, const float* displ, const float* accel, const float* b_displ) {
   if (mp->nspec <= 0) return;
   const int nblocks = (mp->nspec + FORCE_EPB - 1) / FORCE_EPB;
   hipLaunchKernelGGL(k_kernels, dim3(nblocks), dim3(FORCE_THREADS), 0, mp->stream, mp->nspec, mp->d_ibool,
                      mp->d_ispec_is_elastic, mp->d_xix, mp->d_xiz, mp->d_gammax, mp->d_gammaz,
-                     (const float2*)mp->d_displ, (const float2*)mp->d_accel, (const float2*)mp->d_b_displ,
+                     (const float2*)displ, (const float2*)accel, (const float2*)b_displ,
                      mp->d_rho_kl, mp->d_mu_kl, mp->d_kappa_kl, mp->basis);
   check_hip(hipGetLastError(), "k_kernels launch");
 }

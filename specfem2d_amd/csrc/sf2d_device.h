@@ -165,6 +165,37 @@ __device__ __forceinline__ void record_receiver(const ReceiverSet& R, int r, int
   }
 }
 
+// stored Stacey terms ([face point][2]) of the forward run, subtracted from the reconstructed field's force
+// (compute_stacey_viscoelastic.f90, the backward part)
+__device__ __forceinline__ void stored_traction(const StaceyFaces& F, int idx, const float2* __restrict__ store,
+                                                float* __restrict__ accel) {
+  const int f = idx / NGLL;
+  if (f >= F.nabs) return;
+  const int i = F.ij[2 * idx], j = F.ij[2 * idx + 1];
+  if (i < 0 || j < 0) return;
+  const int ispec = F.ispec[f];
+  if (!F.is_elastic[ispec]) return;
+  const size_t g = (size_t)F.ibool[(size_t)ispec * NGLL2 + j * NGLL + i];
+  const float2 t = store[idx];
+  atomic_add_f32(&accel[2 * g], -t.x);
+  atomic_add_f32(&accel[2 * g + 1], -t.y);
+}
+
+// adjoint source of receiver r at time sample it (adj: [2][nstep][nrec]), added to accel at its element's point p
+// (compute_add_sources_viscoelastic_cuda.cu:131)
+__device__ __forceinline__ void adjoint_source(const ReceiverSet& R, const int* __restrict__ is_elastic, int r, int p,
+                                               int it, int nstep, const float* __restrict__ adj,
+                                               float* __restrict__ accel) {
+  if (r >= R.nrec || p >= NGLL2) return;
+  const int ispec = R.ispec[r];
+  if (!is_elastic[ispec]) return;
+  const int i = p % NGLL, j = p / NGLL;
+  const size_t g = (size_t)R.ibool[(size_t)ispec * NGLL2 + p];
+  const float h = R.xir[i * R.nrec + r] * R.gammar[j * R.nrec + r];
+  atomic_add_f32(&accel[2 * g], adj[(size_t)it * R.nrec + r] * h);
+  atomic_add_f32(&accel[2 * g + 1], adj[((size_t)nstep + it) * R.nrec + r] * h);
+}
+
 // point p of receiver r's residual {x, z} (its rotated components) into D, the adjoint of record_receiver
 __device__ __forceinline__ void adjoint_receiver(const ReceiverSet& R, int r, int p, const float* __restrict__ res,
                                                  float* __restrict__ D, int ps) {

@@ -411,7 +411,7 @@ void launch_seismograms(const Mesh* mp, const float* field, float* dst, int seis
                         long shot_stride = 0, long dst_stride = 0, int ps = 1, const int* step = nullptr);
 void launch_set_step(int* step, int value, hipStream_t s);
 void launch_next_step(int* step, hipStream_t s);
-void launch_kernels(const Mesh* mp);
+void launch_kernels(const Mesh* mp, const float* displ, const float* accel, const float* b_displ);
 void launch_max_norm(const Mesh* mp, const float* field, unsigned int* result);
 
 }  // namespace sf2d

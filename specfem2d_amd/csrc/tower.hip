@@ -31,6 +31,12 @@ namespace sf2d {
 struct TowerState {
   TowerPlan plan;
   float2* d_layer = nullptr; // forces of the CPML layer's element points
+  // adjoint runs and SAVE_FORWARD runs: `store_steps` steps of Stacey terms [face point] (those from step store_first on);
+  // the second displacement arrays and the boundary terms of the two fields of an adjoint run [nglob]
+  float2* d_store = nullptr;
+  int store_steps = 0, store_first = -1;
+  float* d_other[2] = {nullptr, nullptr};
+  float2* d_acc[2] = {nullptr, nullptr};
   float2* d_slot = nullptr;  // [slot_shots][plan.nslot] forces of interface points
   int slot_shots = 0;
 };
@@ -64,7 +70,8 @@ struct TowerFields {
   struct Row {  // a point's operands besides the field that the force is computed from
     float2 v;
   };
-  __device__ const float2* field() const { return d; }
+  __device__ long ref(int shot) const { return shot * stride; }
+  __device__ const float2* field(long shot) const { return d + shot; }
   __device__ Row load(long shot, unsigned o) const { return {ld_off(v + shot, o)}; }
   // the point at byte offset o: corrector of this step and predictor of the next (k_corrector's and k_predictor's
   // operations, contracted the same way, so that a run in pieces gives the bits of the run in one) from the force r
@@ -97,7 +104,8 @@ struct AdjointFields {
   struct Row {
     float2 D, Vb;
   };
-  __device__ const float2* field() const { return Rb; }
+  __device__ long ref(int shot) const { return shot * stride; }
+  __device__ const float2* field(long shot) const { return Rb + shot; }
   __device__ Row load(long shot, unsigned o) const { return {ld_off(D + shot, o), ld_off(Vb + shot, o)}; }
   __device__ void update(const Newmark& c, long shot, unsigned o, float2 r, float wx, float wz, float2, Row q) const {
     float2 db = q.D, v, a;
@@ -115,6 +123,39 @@ struct AdjointFields {
   }
 };
 
+// The two fields of an adjoint run (SIMULATION_TYPE 3) as two shots: 0 the adjoint field, 1 the reconstructed one, which
+// steps backwards.  As TowerFields, with the outputs in other arrays than the inputs: the kernels need the step's two
+// displacements and the adjoint acceleration (a0).  last: the step ends the run, a0 and a1 = a_n, (v0_out, v1_out) = v_n.
+struct PairFields {
+  const float2 *d0, *v0, *d1, *v1;
+  float2 *d0_out, *v0_out, *a0, *d1_out, *v1_out, *a1;
+  float2 *acc0, *acc1;       // boundary terms, zero between the steps
+  Newmark nm0, nm1;
+  int nshot, last;
+  struct Row {
+    float2 v;
+  };
+  __device__ int ref(int shot) const { return shot; }
+  __device__ const float2* field(int s) const { return s ? d1 : d0; }
+  __device__ Row load(int s, unsigned o) const { return {ld_off(s ? v1 : v0, o)}; }
+  __device__ void update(const Newmark&, int s, unsigned o, float2 r, float wx, float wz, float2 d, Row q) const {
+    const float dto2 = s ? nm1.dto2 : nm0.dto2, dt = s ? nm1.dt : nm0.dt, dt2o2 = s ? nm1.dt2o2 : nm0.dt2o2;
+    const float2 a = make_float2(r.x * wx, r.y * wz);
+    float2 v = q.v;
+    v.x = fmaf(dto2, a.x, v.x);
+    v.y = fmaf(dto2, a.y, v.y);
+    if (s == 0 || last) st_off(s ? a1 : a0, o, a);
+    if (!last) {
+      d.x = fmaf(dt2o2, a.x, fmaf(dt, v.x, d.x));
+      d.y = fmaf(dt2o2, a.y, fmaf(dt, v.y, d.y));
+      v.x = fmaf(dto2, a.x, v.x);
+      v.y = fmaf(dto2, a.y, v.y);
+      st_off(s ? d1_out : d0_out, o, d);
+    }
+    st_off(s ? v1_out : v0_out, o, v);
+  }
+};
+
 // What else the launch does, in workgroups after the towers': Stacey faces, sources, receivers and fluid-solid edges of
 // the step
 struct TowerEdges {
@@ -129,6 +170,7 @@ struct TowerEdges {
   const int* src_shot;     // shot of each source (null: one shot)
   float* seismo;           // [shot][2][receiver][time]
   long seismo_stride;
+  float2* store;           // SAVE_FORWARD: the Stacey terms of the step, [face point] (one shot; null: not kept)
   int wgs(int nshot) const { return nface_wg * nshot + nsource + nreceiver * nshot + ncoupling_wg; }
 };
 
@@ -137,8 +179,9 @@ __device__ __forceinline__ void tower_edges(const TowerEdges& E, const TowerFiel
   const int it = E.step ? *E.step - 1 : E.it;
   if (wg < faces) {
     const int shot = wg / E.nface_wg;
-    stacey_traction(E.faces, (wg - shot * E.nface_wg) * 64 + threadIdx.x, F.v + shot * F.stride,
-                    (float*)(F.accel + shot * F.stride), 1);
+    const int q = (wg - shot * E.nface_wg) * 64 + threadIdx.x;
+    const float2 f = stacey_traction(E.faces, q, F.v + shot * F.stride, (float*)(F.accel + shot * F.stride), 1);
+    if (E.store && q < E.faces.nabs * NGLL) E.store[q] = f;
     return;
   }
   wg -= faces;
@@ -187,6 +230,44 @@ __device__ __forceinline__ void tower_edges(const AdjointEdges& E, const Adjoint
                    (float*)(F.D + shot * F.stride), 1);
 }
 
+// the boundary part of a step of an adjoint run: Stacey edges, adjoint sources and receivers of the adjoint field, the
+// forward run's stored Stacey terms and its sources for the reconstructed one
+struct PairEdges {
+  StaceyFaces faces;
+  ReceiverSet receivers;
+  SourceSet sources;
+  int it, cur, nstep;      // 0-based samples of the forward run's time and of the seismograms
+  int nface_wg, nsource, nadj, nreceiver;
+  const float* adj;        // [2][nstep][receiver]
+  const float2* store;     // [face point]
+  float* seismo;
+  int wgs(int) const { return 2 * nface_wg + nsource + nadj + nreceiver; }
+};
+
+__device__ __forceinline__ void tower_edges(const PairEdges& E, const PairFields& F, int wg) {
+  const int t = threadIdx.x;
+  if (wg < E.nface_wg) {
+    stacey_traction(E.faces, wg * 64 + t, F.v0, (float*)F.acc0, 1);
+    return;
+  }
+  wg -= E.nface_wg;
+  if (wg < E.nface_wg) {
+    stored_traction(E.faces, wg * 64 + t, E.store, (float*)F.acc1);
+    return;
+  }
+  wg -= E.nface_wg;
+  if (wg < E.nsource) {
+    source_force(E.sources, wg, t, E.it, (float*)F.acc1, 1);
+    return;
+  }
+  wg -= E.nsource;
+  if (wg < E.nadj) {
+    adjoint_source(E.receivers, E.faces.is_elastic, wg, t, E.it, E.nstep, E.adj, (float*)F.acc0);
+    return;
+  }
+  record_receiver(E.receivers, wg - E.nadj, t, E.cur, F.d0, E.seismo, 1);
+}
+
 // The operands of a lane's column of one chain that the next iteration starts from, loaded one chain ahead: the
 // displacement of GLL rows 1 .. 4, the moduli of rows 0 .. 4, the element's geometry record
 struct ChainRegs {
@@ -212,8 +293,8 @@ __global__ __launch_bounds__(64) void k_tower(
   const int tower = F.nshot == 1 ? item : item / F.nshot;
   if (tower >= ntower) return;  // uniform over the wave
   const int shot = item - tower * F.nshot;
-  const long at = shot * F.stride;
-  const float2* const __restrict__ d = F.field() + at;
+  const auto at = F.ref(shot);
+  const float2* const __restrict__ d = F.field(at);
   slot += (size_t)shot * nslot;
   const int4 td = desc[4 * tower], tb = desc[4 * tower + 1], ts = desc[4 * tower + 2], tt = desc[4 * tower + 3];
   const int nch = td.y, ne = td.z;
@@ -452,6 +533,24 @@ __global__ __launch_bounds__(256) void k_interface_adjoint(const InterfaceArgs A
   F.update(nm, at, 8u * (unsigned)g, r, rmx[g], rmz[g], make_float2(0.f, 0.f), row);
 }
 
+__global__ __launch_bounds__(256) void k_interface_pair(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
+                                                        const PairFields F, const float* __restrict__ rmx,
+                                                        const float* __restrict__ rmz) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= A.n) return;
+  const int s = blockIdx.y;
+  const int g = A.id[q];
+  const float2 d = F.field(s)[g];
+  const PairFields::Row row = F.load(s, 8u * (unsigned)g);
+  float2 r = sum_towers(A, q, slot + (size_t)s * nslot, make_float2(0.f, 0.f));
+  if (A.flag[q] & (IF_ACC | IF_LOOKED_AT)) {  // receivers' points take the adjoint sources
+    float2* const acc = s ? F.acc1 : F.acc0;
+    add_slot(r, acc[g]);
+    acc[g] = make_float2(0.f, 0.f);
+  }
+  F.update(F.nm0, s, 8u * (unsigned)g, r, rmx[g], rmz[g], d, row);
+}
+
 // accel = 0 at the interface points with a boundary term (the start of a run of tower steps)
 __global__ __launch_bounds__(256) void k_interface_clear(int n, const int* __restrict__ ids,
                                                          const uint8_t* __restrict__ flag, float2* __restrict__ accel,
@@ -490,7 +589,8 @@ void launch_k_tower(Mesh* mp, Kernel kern, const Fields& F, const Edges& E, floa
 // one step of the fields F at time step it (1-based): towers with the step's Stacey faces, sources, fluid-solid edges
 // (forward) and (seismo not null) receivers, the CPML layer, the interface
 void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long seismo_stride, const int* src_shot,
-                  const Newmark& nm, bool forward, const int* step = nullptr) {
+                  const Newmark& nm, bool forward, const int* step = nullptr,
+                  float2* store = nullptr) {
   const TowerPlan& P = mp->tower->plan;
   float2* const slot = tower_slots(mp->tower, F.nshot);
   TowerEdges E{};
@@ -506,6 +606,7 @@ void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long se
   E.src_shot = src_shot;
   E.seismo = seismo;
   E.seismo_stride = seismo_stride;
+  E.store = store;
   E.step = step;
   const int sets = !mp->attenuation ? 0 : mp->att_ntable == 1 ? 1 : 2;
   using K = decltype(&k_tower<0, 0, TowerFields, TowerEdges>);
@@ -529,6 +630,21 @@ void clear_interface(Mesh* mp, float2* accel, long stride, int nshot) {
   hipLaunchKernelGGL(k_interface_clear, dim3((P.n + 255) / 256, nshot), dim3(256), 0, mp->stream, P.n, P.d_id, P.d_flag,
                      accel, stride);
   check_hip(hipGetLastError(), "k_interface_clear launch");
+}
+
+}  // namespace
+
+namespace {
+
+// Stacey terms are kept on the device for as many steps as fit 64 MB and cross to or from the host together: a copy and a
+// synchronisation per step cost more than a step of a small mesh (80 x 32 elements: 100 of 115 us)
+size_t store_points(const Mesh* mp) { return (size_t)mp->num_abs * NGLL; }
+void prepare_store(Mesh* mp, int nstep) {
+  TowerState* T = mp->tower;
+  const size_t step = store_points(mp) * sizeof(float2);
+  if (step == 0 || T->d_store) return;
+  T->store_steps = (int)std::max<size_t>(1, std::min<size_t>((size_t)nstep, ((size_t)64 << 20) / step));
+  T->d_store = device_alloc<float2>(store_points(mp) * T->store_steps);
 }
 
 }  // namespace
@@ -756,6 +872,11 @@ void tower_release(Mesh* mp) {
   T->plan.release();
   device_free(T->d_slot);
   device_free(T->d_layer);
+  device_free(T->d_store);
+  for (int s = 0; s < 2; s++) {
+    device_free(T->d_other[s]);
+    device_free(T->d_acc[s]);
+  }
   delete T;
   mp->tower = nullptr;
 }
@@ -779,7 +900,8 @@ extern "C" {
 int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rmassz) {
   Mesh* mp = handle(Mesh_pointer);
   tower_release(mp);
-  if (!mp->chain || !mp->first_touch || !mp->d_col_rows || mp->assembly != 0 || mp->anisotropy || mp->save_forward || getenv("SF2D_NO_TOWERS"))
+  if (!mp->chain || (!mp->first_touch && mp->simulation_type == 1) || !mp->d_col_rows || mp->assembly != 0 ||
+      mp->anisotropy || getenv("SF2D_NO_TOWERS"))
     return 0;
   const int npatch = mp->npatch, ng = mp->nglob;
   const std::vector<int4>& rows = mp->h_col_rows;
@@ -845,8 +967,8 @@ void sf2d_tower_begin(long* Mesh_pointer) {
   clear_interface(mp, (float2*)mp->d_accel, 0, 1);
 }
 
-void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float deltat, float deltatsqover2,
-                     float deltatover2) {
+void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float* absorb, float deltat,
+                     float deltatsqover2, float deltatover2) {
   Mesh* mp = handle(Mesh_pointer);
   if (!mp->tower || !mp->accel_partial || mp->pending_corrector[0])
     fail("sf2d_tower_step: call after update_displacement_cuda and sf2d_tower_begin");
@@ -857,8 +979,90 @@ void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float
   // displacement of the receivers in solid elements; the fluid records its own, and the caller the run's last step
   const int record = !last && mp->nrec_local > 0 && mp->h_seismotype[0] == 1;
   if (record && it > mp->nlength_seismogram) fail("sf2d_tower_step: step %d after the seismograms' last", it);
-  launch_tower(mp, F, it, record ? mp->d_seismo[0] : nullptr, 0, nullptr, {deltatover2, deltat, deltatsqover2}, true);
+  TowerState* T = mp->tower;
+  float2* store = nullptr;
+  if (absorb && mp->stacey && mp->num_abs > 0) {
+    prepare_store(mp, mp->nstep);
+    if (T->store_first < 0) T->store_first = it;
+    store = T->d_store + store_points(mp) * (it - T->store_first);
+  }
+  launch_tower(mp, F, it, record ? mp->d_seismo[0] : nullptr, 0, nullptr, {deltatover2, deltat, deltatsqover2}, true,
+               nullptr, store);
+  if (store && (last || it - T->store_first + 1 == T->store_steps)) {
+    const int n = it - T->store_first + 1;
+    check_hip(hipMemcpyAsync(absorb - 2 * store_points(mp) * (n - 1), T->d_store, store_points(mp) * n * sizeof(float2),
+                             hipMemcpyDeviceToHost, mp->stream),
+              "Stacey terms D2H");
+    check_hip(hipStreamSynchronize(mp->stream), "sf2d_tower_step");
+    T->store_first = -1;
+  }
   if (last) mp->accel_partial = 0;
+}
+
+void sf2d_tower_adjoint_begin(long* Mesh_pointer) {
+  Mesh* mp = handle(Mesh_pointer);
+  TowerState* T = mp->tower;
+  if (!T || mp->simulation_type != 3) fail("sf2d_tower_adjoint_begin: no towers, or not SIMULATION_TYPE = 3");
+  for (int s = 0; s < 2; s++) {
+    if (!T->d_other[s]) T->d_other[s] = device_alloc<float>((size_t)2 * mp->nglob);
+    if (!T->d_acc[s]) T->d_acc[s] = device_zeros<float2>((size_t)mp->nglob);
+  }
+  if (mp->stacey) prepare_store(mp, mp->nstep);
+  T->store_first = -1;
+}
+
+void sf2d_tower_adjoint_step(long* Mesh_pointer, int it, int last, const float* absorb, float deltat,
+                             float deltatsqover2, float deltatover2, float b_deltat, float b_deltatsqover2,
+                             float b_deltatover2) {
+  Mesh* mp = handle(Mesh_pointer);
+  TowerState* T = mp->tower;
+  if (!T || !T->d_other[0] || mp->pending_corrector[0] || mp->pending_corrector[1])
+    fail("sf2d_tower_adjoint_step: call after update_displacement_cuda and sf2d_tower_adjoint_begin");
+  if (it < 1 || it > mp->nstep) fail("sf2d_tower_adjoint_step: it=%d outside 1..%d", it, mp->nstep);
+  const TowerPlan& P = T->plan;
+  const int sample = mp->nstep - it;  // 0-based time sample of the forward run
+  const size_t np = store_points(mp);
+  const bool edges = mp->stacey && mp->num_abs > 0;
+  if (edges && (T->store_first < 0 || sample < T->store_first)) {
+    T->store_first = std::max(0, sample + 1 - T->store_steps);
+    check_hip(hipMemcpyAsync(T->d_store, absorb + 2 * np * T->store_first,
+                             np * (sample + 1 - T->store_first) * sizeof(float2), hipMemcpyHostToDevice, mp->stream),
+              "Stacey terms H2D");
+  }
+  float2 *d0 = (float2*)mp->d_displ, *v0 = (float2*)mp->d_veloc, *d1 = (float2*)mp->d_b_displ, *v1 = (float2*)mp->d_b_veloc;
+  const PairFields F{d0, v0, d1, v1, (float2*)T->d_other[0], v0, (float2*)mp->d_accel, (float2*)T->d_other[1], v1,
+                     (float2*)mp->d_b_accel,
+                     T->d_acc[0], T->d_acc[1], {deltatover2, deltat, deltatsqover2},
+                     {b_deltatover2, b_deltat, b_deltatsqover2}, 2, last ? 1 : 0};
+  PairEdges E{};
+  E.faces = stacey_faces(mp);
+  E.receivers = receiver_set(mp);
+  E.sources = source_set(mp);
+  E.it = sample;
+  E.cur = it - 1;
+  E.nstep = mp->nstep;
+  E.nface_wg = edges ? (mp->num_abs * NGLL + 63) / 64 : 0;
+  E.nsource = mp->nsources_local;
+  E.nadj = mp->nadj_rec_local;
+  E.nreceiver = last ? 0 : mp->nrec_local;
+  E.adj = mp->d_source_adjoint;
+  E.store = edges ? T->d_store + np * (sample - T->store_first) : nullptr;
+  E.seismo = mp->d_seismo[0];
+  if (E.nreceiver > 0 && it > mp->nlength_seismogram) fail("sf2d_tower_adjoint_step: step %d after the last sample", it);
+  float2* const slot = tower_slots(T, 2);
+  using K = decltype(&k_tower<0, 0, PairFields, PairEdges>);
+  const K kern[3] = {k_tower<0, 0, PairFields, PairEdges>, k_tower<1, 0, PairFields, PairEdges>,
+                      k_tower<2, 0, PairFields, PairEdges>};
+  launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, F.nm0);
+  if (P.n > 0) {
+    hipLaunchKernelGGL(k_interface_pair, dim3((P.n + 255) / 256, 2), dim3(256), 0, mp->stream, interface_args(P), slot,
+                       P.nslot, F, mp->d_rmassx, mp->d_rmassz);
+    check_hip(hipGetLastError(), "k_interface_pair launch");
+  }
+  launch_kernels(mp, mp->d_displ, mp->d_accel, mp->d_b_displ);
+  if (last) return;
+  std::swap(mp->d_displ, T->d_other[0]);
+  std::swap(mp->d_b_displ, T->d_other[1]);
 }
 
 }  // extern "C"

@@ -136,3 +136,41 @@ def test_fused_reverse_sweep_matches_the_unfused_one(form, nx, nz, chains, shots
     for fused, plain in zip(out[:2], out[2:]):
         for a, b, tol in zip(fused, plain, [1e-5] * 5 + BOUNDS[1:4]):
             assert np.linalg.norm(b) > 0 and rel(a, b) < tol
+
+
+@pytest.mark.parametrize("form", ["stacey", "points"])
+@pytest.mark.parametrize("nx,nz,chains", [(12, 12, 1), (25, 17, 3), (13, 2, 64)])
+def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
+    """A SAVE_FORWARD run (its Stacey terms) and the SIMULATION_TYPE 3 run with its kernels.  The reconstruction runs
+    backwards in time on rounded fields: what a change of 1e-7 in the stored terms and the adjoint traces does to the
+    unfused run is the measure, ten times that the bound."""
+    if form == "points":
+        monkeypatch.setenv("SF2D_NO_AFFINE", "1")
+    cfg = make("stacey", nx, nz)
+    rng = np.random.default_rng(1)
+    monkeypatch.setenv("SF2D_TOWER_CHAINS", str(chains))
+
+    def adjoint(traces, store, last):
+        back = Simulation(cfg, simulation_type=3)
+        out = back.adjoint(traces, store, last)
+        back.close()
+        return [out[0], *out[1].values()] if isinstance(out[1], dict) else [out[0], *out[1]]
+
+    runs = []
+    for towers in (True, False):
+        if not towers:
+            monkeypatch.setenv("SF2D_NO_TOWERS", "1")
+        sim = Simulation(cfg, save_forward=True)
+        parts = [sim.forward(nstep=n, save_stacey=True) for n in (70, cfg.nstep - 70)]
+        seis = np.concatenate([p[0] for p in parts], axis=-1)
+        store = np.concatenate([p[2] for p in parts])
+        last = sim.fields()
+        sim.close()
+        runs.append((seis, store, last, adjoint(seis[..., ::-1], store, last)))
+    (seis, store, last, fused), (seis0, store0, last0, plain) = runs
+    assert rel(seis, seis0) < 1e-5 and rel(store, store0) < 1e-4
+    noise = lambda a: a * (1 + 1e-7 * rng.choice([-1.0, 1.0], np.shape(a)))
+    moved = adjoint(noise(seis0[..., ::-1]), noise(store0).astype(np.float32), [noise(x).astype(np.float32) for x in last0])
+    for a, b, c in zip(fused, plain, moved):
+        assert np.linalg.norm(b) > 0 and rel(a, b) < 10 * max(rel(c, b), 1e-6)
+
