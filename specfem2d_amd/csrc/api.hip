@@ -317,13 +317,49 @@ struct ChainSet {
   }
 };
 
-// fills the chains of S.elems; false when some patch is not a chain
-bool find_chains(const std::vector<int>& ibool, int nglob, int max_elems, ChainSet& S) {
+// Puts elements into rows: each one followed by the element whose points (0, j) are its points (4, j), rows from their
+// left ends.  Returns the patches, rows cut every max_elems elements, as make_patches does.
+std::vector<int> make_rows(const std::vector<int>& ibool, std::vector<int>& elems, int nglob, int max_elems) {
+  const int n = (int)elems.size();
+  auto point = [&](int k, int i, int j) { return ibool[(size_t)elems[k] * NGLL2 + j * NGLL + i]; };
+  std::vector<int> left_edge((size_t)nglob, -1), right(n, -1), order, start;
+  std::vector<char> has_left(n, 0), placed(n, 0);
+  for (int k = 0; k < n; k++) left_edge[point(k, 0, 2)] = k;
+  for (int k = 0; k < n; k++) {
+    const int r = left_edge[point(k, NGLL - 1, 2)];
+    if (r < 0 || r == k || has_left[r]) continue;
+    bool same = true;
+    for (int j = 0; j < NGLL && same; j++) same = point(k, NGLL - 1, j) == point(r, 0, j);
+    if (!same) continue;
+    right[k] = r;
+    has_left[r] = 1;
+  }
+  for (int ring = 0; ring < 2; ring++)  // then rows that close on themselves
+    for (int k = 0; k < n; k++) {
+      if (placed[k] || (!ring && has_left[k])) continue;
+      int len = 0;
+      for (int e = k; e >= 0 && !placed[e]; e = right[e], len++) {
+        if (len % max_elems == 0) start.push_back((int)order.size());
+        placed[e] = 1;
+        order.push_back(elems[e]);
+      }
+    }
+  elems.swap(order);
+  start.push_back(n);
+  return start;
+}
+
+// Fills the chains of S.elems from consecutive elements; false when some patch is not a chain.  With rows, the elements
+// are put into rows first, whatever their order (external meshes, meshes narrower than a patch): false when the chains
+// have fewer than 4 elements on average, where most lanes of a chain's wave would idle.
+bool find_chains(const std::vector<int>& ibool, int nglob, int max_elems, ChainSet& S, bool rows = false) {
   for (int ph = 0; ph < 2; ph++) {
-    const std::vector<int> ps = make_patches(ibool, S.elems[ph], nglob, max_elems);
+    const std::vector<int> ps = rows ? make_rows(ibool, S.elems[ph], nglob, max_elems)
+                                     : make_patches(ibool, S.elems[ph], nglob, max_elems);
     for (size_t q = 0; q + 1 < ps.size(); q++) S.ch.push_back({ph, ps[q], ps[q + 1] - ps[q]});
   }
   const int nch = (int)S.ch.size();
+  if (rows && S.elems[0].size() + S.elems[1].size() < (size_t)4 * nch) return false;
   std::vector<int> mark((size_t)nglob, -1);
   for (int q = 0; q < nch; q++) {  // the chain property: shared edges, every other point once
     const ChainSet::Chain& c = S.ch[q];
@@ -359,6 +395,16 @@ bool find_chains(const std::vector<int>& ibool, int nglob, int max_elems, ChainS
   return true;
 }
 
+// the chains that chain_patches finds over the fluid's elements
+bool find_fluid_chains(const std::vector<int>& ibool, int nglob, const std::vector<int>& elems, ChainSet& S) {
+  for (int rows = 0; rows < 2; rows++) {
+    S = ChainSet();
+    S.elems[1] = elems;
+    if (find_chains(ibool, nglob, Mesh::CHAIN_ELEMS, S, rows)) return true;
+  }
+  return false;
+}
+
 // numbers the points of the chains that have no id yet, tower by tower: first the points inside the rows (x = 1 ..
 // 4 ne - 1, row by row upwards, so that a row is consecutive and the next row of the tower follows it), then the left and
 // the right column upwards (consecutive too, where a neighbour has not numbered them)
@@ -386,7 +432,7 @@ void number_points(const std::vector<int>& ibool, const ChainSet& S, std::vector
 // numbered for towers (number_points), after those points the ones of the elements `fluid` in the same way.  No slots,
 // halos or owned ranges: those serve the general patch kernel.
 bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
-                      int max_elems, Plan& P, const std::vector<int>& fluid = {}) {
+                      int max_elems, Plan& P, bool rows = false, const std::vector<int>& fluid = {}) {
   P = Plan();
   std::vector<char> placed(nspec, 0);
   ChainSet S;
@@ -402,7 +448,7 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
     }
     P.phase_count[ph] = (int)elems[ph].size();
   }
-  if (!find_chains(ibool, nglob, max_elems, S)) return false;
+  if (!find_chains(ibool, nglob, max_elems, S, rows)) return false;
   const std::vector<ChainSet::Chain>& ch = S.ch;
   const std::vector<int>&above = S.above, &below = S.below;
   const int nch = (int)ch.size();
@@ -461,8 +507,7 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
     if (!placed[e]) P.order.push_back(e);
   if (!fluid.empty()) {
     ChainSet F;
-    F.elems[1] = fluid;
-    if (find_chains(ibool, nglob, Mesh::CHAIN_ELEMS, F)) number_points(ibool, F, P.newid, next_id);
+    if (find_fluid_chains(ibool, nglob, fluid, F)) number_points(ibool, F, P.newid, next_id);
   }
   for (int g = 0; g < nglob; g++)
     if (P.newid[g] < 0) P.newid[g] = next_id++;  // points of no elastic element
@@ -474,9 +519,8 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
 // point numbering of a mesh of fluid elements alone (`elems`) for towers; empty when the patches are not chains
 std::vector<int> fluid_numbering(const std::vector<int>& ibool, int nglob, const std::vector<int>& elems) {
   ChainSet S;
-  S.elems[1] = elems;
   std::vector<int> id;
-  if (!find_chains(ibool, nglob, Mesh::CHAIN_ELEMS, S)) return id;
+  if (!find_fluid_chains(ibool, nglob, elems, S)) return id;
   id.assign((size_t)nglob, -1);
   int next_id = 0;
   number_points(ibool, S, id, next_id);
@@ -493,7 +537,9 @@ bool chain_patches(const std::vector<int>& ibool, int nspec, int nglob, const in
                    std::vector<int>& order, std::vector<int>& desc, std::vector<int>& above, int ncolour[2],
                    int colour_start[2][Mesh::MAX_COLOURS], int colour_count[2][Mesh::MAX_COLOURS]) {
   Plan P;
-  if (!build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P)) return false;
+  if (!build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P) &&
+      !build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P, true))
+    return false;
   order = std::move(P.order);
   desc = std::move(P.desc);
   above = std::move(P.above);
@@ -612,8 +658,9 @@ void sort_elements_by_colour(Mesh* mp, const int* phase_lists, int np) {
   if (const char* env = getenv("SF2D_SHOTS_PER_WAVE")) mp->shots_per_wave = std::max(1, atoi(env));
   Plan P;
   const std::vector<int> fluid = acoustic_elements(mp);
-  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, fluid) &&
-                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P, fluid))) {
+  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, false, fluid) &&
+                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P, false, fluid) &&
+                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, true, fluid))) {
     if (try_chain && mp->attenuation) mp->assembly = 2;  // the memory variables ride in the chain kernel only
     P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly);
   }

@@ -174,3 +174,36 @@ def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, monkeyp
     for a, b, c in zip(fused, plain, moved):
         assert np.linalg.norm(b) > 0 and rel(a, b) < 10 * max(rel(c, b), 1e-6)
 
+
+def blocks(nx, nz, h=100.0):
+    """A grid of deformed quadrilaterals whose elements are numbered in blocks 5 wide and 3 high."""
+    o = np.array([(x, z) for bz in range(0, nz, 3) for bx in range(0, nx, 5) for z in range(bz, min(bz + 3, nz))
+                  for x in range(bx, min(bx + 5, nx))])
+    X, Z = np.meshgrid(np.arange(nx + 1) * h, np.arange(nz + 1) * h - nz * h)
+    rng = np.random.default_rng(4)
+    X[1:-1, 1:-1] += 0.15 * h * rng.uniform(-1, 1, (nz - 1, nx - 1))
+    Z[1:-1, 1:-1] += 0.15 * h * rng.uniform(-1, 1, (nz - 1, nx - 1))
+    n0 = o[:, 1] * (nx + 1) + o[:, 0]
+    edges = np.array([(e, c) for e, (x, z) in enumerate(o) for c, on in ((1, z == 0), (2, x == nx - 1), (4, x == 0)) if on],
+                     np.int32)
+    none = np.zeros(0, np.int32)
+    return config.ExternalMesh(knods=np.stack([n0, n0 + 1, n0 + nx + 2, n0 + nx + 1], 1).astype(np.int32),
+                               coorg=np.stack([X, Z], -1).reshape(-1, 2), material=np.ones(len(o), np.int32),
+                               free_elem=none, free_code=none, abs_elem=edges[:, 0], abs_code=edges[:, 1])
+
+
+@pytest.mark.parametrize("nx,nz,rows", [(12, 6, 1), (17, 9, 1), (4, 5, 1), (3, 7, 0)])
+@pytest.mark.parametrize("external", [False, True])
+def test_elements_in_any_order_form_rows(nx, nz, rows, external):
+    """Elements numbered in blocks, and rows narrower than a patch, step on chains where these have four elements on
+    average, and on the general kernel otherwise."""
+    if not external and nx >= 10:
+        pytest.skip("consecutive rows are chains as they are")
+    cfg = make("stacey", nx, nz)
+    if external:
+        cfg = cfg.replace(mesh=blocks(nx, nz))
+    sim = Simulation(cfg)
+    assert sim.chain_kernel() == bool(rows)
+    seis = sim.forward()[0]
+    sim.close()
+    assert rel(seis, OracleSim(cfg, "sp").forward()) < 1e-5
