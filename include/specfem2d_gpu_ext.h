@@ -176,6 +176,13 @@ void sf2d_grad_flush(long* Mesh_pointer);
    parts d chi / d (rho vp), d (rho vs) per absorbing face point [nabs][5] */
 void sf2d_grad_result(long* Mesh_pointer, double* g_kappa, double* g_mu, double* g_mass, double* g_rho_vp,
                       double* g_rho_vs);
+/* the model of the chain rule, rho, vp, vs and the Jacobian [nspec][25] in ispec order: before the first
+   sf2d_grad_model_result after sf2d_grad_prepare (sf2d_grad_has_model: 1 when it is there) and after each change */
+void sf2d_grad_set_model(long* Mesh_pointer, const double* rho, const double* vp, const double* vs, const float* jacobian);
+int sf2d_grad_has_model(long* Mesh_pointer);
+/* d chi / d (rho, vp, vs) [3][nspec][25] (ispec order) and, with parts, d chi / d (kappa, mu, rho through the mass,
+   rho vp, rho vs) [5][nspec][25]; dto2 = dt / 2 */
+void sf2d_grad_model_result(long* Mesh_pointer, float dto2, double* grad, double* parts);
 /* gradient buffers over the shot batch (sf2d_batch_prepare): the calls above then checkpoint and reverse all
    shots together, residuals are [nstep][nshot][nrec][2] and the results are sums over the shots */
 int sf2d_batch_grad_prepare(long* Mesh_pointer, int chunk);

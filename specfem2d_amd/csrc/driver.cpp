@@ -181,6 +181,7 @@ struct Sim {
   // gradient: state saves inside the forward loop (0 none, 1 checkpoints every grad_chunk steps, 2 every step
   // of the segment that starts after step grad_seg_base)
   int grad_save = 0, grad_chunk = 0, grad_seg_base = 0, grad_ready = 0;
+  bool grad_model_stale = false;   // set_model since the handle last got the model for the gradient's chain rule
   std::vector<float> grad_res;     // [nstep][nrec][2] dt (s - o)
   std::vector<double> sisux, sisuz;  // host seismograms (nlength = NSTEP), as the Fortran caller keeps them
   // shot batch: nshot > 0 runs every shot's sources in its own wavefield (src_shot[k] = shot of source k)
@@ -2174,6 +2175,7 @@ int sf2d_sim_set_model(void* sim, const double* rho, const double* vp, const dou
   s->model_rho.assign(rho, rho + ne);
   s->model_vp.assign(vp, vp + ne);
   s->model_vs.assign(vs, vs + ne);
+  s->grad_model_stale = true;
   build_mass(*s);
   if (s->mesh)
     sf2d_mesh_set_materials(&s->mesh, s->kappa.data(), s->mu.data(), s->rho_vp.data(), s->rho_vs.data(),
@@ -2259,47 +2261,10 @@ int sf2d_sim_gradient_backward(void* sim, double* grad, double* parts) {
     s->it_done = std::min(N, C);
     sf2d_grad_load_segment(&s->mesh, s->it_done - 1, dto2);
   }
-  const size_t ne = (size_t)s->nspec * NGLL2, nf = (size_t)s->nabs * NGLL;
-  std::vector<double> gk(ne), gm(ne), pm((size_t)2 * s->nglob), fvp(std::max<size_t>(1, nf)), fvs(std::max<size_t>(1, nf));
-  sf2d_grad_result(&s->mesh, gk.data(), gm.data(), pm.data(), fvp.data(), fvs.data());
-  // mass term: M_c(g) = sum w_i w_j J rho (+ the Stacey term below)
-  std::vector<double> gr(ne, 0.0), gvp(ne, 0.0), gvs(ne, 0.0);
-  for (int e = 0; e < s->nspec; e++)
-    for (int p = 0; p < NGLL2; p++) {
-      const size_t l = (size_t)e * NGLL2 + p;
-      const int g = s->ibool[l] - 1;
-      const double w = (double)s->basis.w[p % NGLL] * (double)s->basis.w[p / NGLL] * (double)s->jacobian[l];
-      gr[l] = w * (pm[2 * (size_t)g] + pm[2 * (size_t)g + 1]);
-    }
-  // Stacey traction and its Newmark mass term T_c = dt/2 w [rho_vp (nx+nz) n_c + rho_vs (1 - (nx+nz) n_c)]
-  for (int f = 0; f < s->nabs; f++) {
-    const int e = s->abs_ispec[f] - 1;
-    for (int k = 0; k < NGLL; k++) {
-      const size_t q = (size_t)f * NGLL + k;
-      const int ii = s->abs_ij[2 * q], jj = s->abs_ij[2 * q + 1];
-      if (ii > NGLL || jj > NGLL) continue;
-      const size_t l = (size_t)e * NGLL2 + (jj - 1) * NGLL + (ii - 1);
-      const int g = s->ibool[l] - 1;
-      const double nx = s->abs_normal[2 * q], nz = s->abs_normal[2 * q + 1], w = s->abs_jacw[q];
-      const double sn = nx + nz, px = pm[2 * (size_t)g], pz = pm[2 * (size_t)g + 1];
-      gvp[l] += fvp[q] + w * (double)dto2 * (px * sn * nx + pz * sn * nz);
-      gvs[l] += fvs[q] + w * (double)dto2 * (px * (1.0 - sn * nx) + pz * (1.0 - sn * nz));
-    }
-  }
-  // chain to (rho, vp, vs): mu = rho vs^2, kappa = rho vp^2 - mu, rho_vp = rho vp, rho_vs = rho vs
-  for (size_t l = 0; l < ne; l++) {
-    const double rho = s->model_rho[l], vp = s->model_vp[l], vs = s->model_vs[l];
-    grad[l] = gk[l] * (vp * vp - vs * vs) + gm[l] * vs * vs + gr[l] + gvp[l] * vp + gvs[l] * vs;
-    grad[ne + l] = gk[l] * 2.0 * rho * vp + gvp[l] * rho;
-    grad[2 * ne + l] = -gk[l] * 2.0 * rho * vs + gm[l] * 2.0 * rho * vs + gvs[l] * rho;
-    if (parts) {
-      parts[l] = gk[l];
-      parts[ne + l] = gm[l];
-      parts[2 * ne + l] = gr[l];
-      parts[3 * ne + l] = gvp[l];
-      parts[4 * ne + l] = gvs[l];
-    }
-  }
+  if (s->grad_model_stale || !sf2d_grad_has_model(&s->mesh))
+    sf2d_grad_set_model(&s->mesh, s->model_rho.data(), s->model_vp.data(), s->model_vs.data(), s->jacobian.data());
+  s->grad_model_stale = false;
+  sf2d_grad_model_result(&s->mesh, dto2, grad, parts);
   return 0;
 }
 
