@@ -48,6 +48,9 @@ struct GradState {
   int fused = 0;
   float* acc = nullptr;
   int4* rows = nullptr;
+  // R~ of the last nrb steps, Rb in a ring of nrb fields; the current step's is in slot rb_at.  npend steps, the first with
+  // the forward state in segment slot pend_slot and R~ in ring slot pend_rb, wait for their strain products
+  int nrb = 1, rb_at = 0, npend = 0, pend_slot = 0, pend_rb = 0;
   // the chain rule to (rho, vp, vs): model [3][ne] and Jacobian [ne] in the caller's element order, where each caller
   // element's accumulators lie, and the result [3 or 8][ne]
   double *model = nullptr, *out = nullptr;
@@ -59,6 +62,7 @@ struct GradState {
 namespace {
 
 constexpr int GT = 256;   // threads per workgroup
+constexpr int RING = 4;   // steps per launch of k_grad_chain
 
 constexpr int GEPB = 10;  // elements per workgroup in k_grad_elastic
 
@@ -295,12 +299,14 @@ __global__ __launch_bounds__(64) void k_grad_elastic_minor(int nelem, int nshot,
 // k_grad_elastic over chains, one wave per chain with lane 5 k + i holding column i of element k, for the fused reverse
 // sweep: both fields' columns stay in registers, their rows pass through LDS, and the accumulators gk, gm lie in lane order
 // (point (k, i, j) of the chain at e0 at e0 * 25 + j * 5 ne + 5 k + i) so that a wave reads and writes whole lines.  It
-// also adds each point's mass term, pm -= R~ r W, where the chain owns the point (rows: masks of owned points).  Bound by
-// HBM and L2: of a step's traffic the two accumulators, read and written, are a third.  With the fused steps before and
-// after it: 400 x 200 elements, 300 steps in segments of 50, 79 -> 58 ms; 8 shots of 300 x 150, 200 steps, 94.5 -> 67.2.
+// also adds each point's mass term, pm -= R~ r W, where the chain owns the point (rows: masks of owned points).
 // GEO as in tower.hip: 0 rectangles, 1 affine elements, 2 geometry per point.
+// One launch takes nstep reverse steps: step t's fields are dn - t * state, rn - t * state and slot (rb0 + t) mod nrb of rb.
+// Bound by HBM and L2, half of it the accumulators, read and written once a launch: 400 x 200
+// elements 27 us for one step, 45 us for four; 8 shots of 300 x 150 46 and 145.
 template <int GEO>
-__global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nshot, long ss, const int4* __restrict__ desc,
+__global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nstep, long state, int rb0, int nrb, long field,
+                                                   int nshot, long ss, const int4* __restrict__ desc,
                                                    const int4* __restrict__ rows, const int* __restrict__ ends,
                                                    const float4* __restrict__ geom, const float4* __restrict__ geom_elem,
                                                    const float2* __restrict__ dn, const float2* __restrict__ rb,
@@ -343,16 +349,24 @@ __global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nshot, long s
     dm[j] = make_float2(0.f, 0.f);
   }
   float2 d[NGLL], b[NGLL], r[NGLL];
-  auto load = [&](long at) {
+  int step = 0, shot = 0;  // of the fields loaded next
+  auto load = [&]() {
+    const int slot = rb0 + step < nrb ? rb0 + step : rb0 + step - nrb;
+    const long at = shot * ss - step * state, bt = shot * ss + slot * field;
 #pragma unroll
     for (int j = 0; j < NGLL; j++) {
       d[j] = ld_off(dn + at, off[j]);
-      b[j] = ld_off(rb + at, off[j]);
+      b[j] = ld_off(rb + bt, off[j]);
       r[j] = own[j] ? ld_off(rn + at, off[j]) : make_float2(0.f, 0.f);
     }
+    if (++shot == nshot) {
+      shot = 0;
+      step++;
+    }
   };
-  load(0);
-  for (int s = 0; s < nshot; s++) {
+  load();
+  const int n = nstep * nshot;
+  for (int s = 0; s < n; s++) {
     float4 u[NGLL];
 #pragma unroll
     for (int j = 0; j < NGLL; j++) {
@@ -360,7 +374,7 @@ __global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nshot, long s
       dm[j].x += b[j].x * r[j].x;
       dm[j].y += b[j].y * r[j].y;
     }
-    if (s + 1 < nshot) load((s + 1) * ss);  // the next shot's values are in flight while this one is computed
+    if (s + 1 < n) load();  // the next shot's or step's values are in flight while this one is computed
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int j = 0; j < NGLL; j++) s_t[j * 64 + lane] = u[j];
@@ -556,11 +570,41 @@ int grad_prepare(Mesh* mp, long* Mesh_pointer, int chunk, int nrec, int batch) {
   return G->nckpt;
 }
 
+// the strain products of the steps that wait for them
+void flush_pending(Mesh* mp, GradState* G) {
+  if (G->npend == 0) return;
+  using K = decltype(&k_grad_chain<0>);
+  const K kern[3] = {k_grad_chain<0>, k_grad_chain<1>, k_grad_chain<2>};
+  const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+  const long field = (long)(G->nfield / 2);
+  const float2* dn = (const float2*)(G->seg + (size_t)G->pend_slot * 3 * G->nfield);
+  hipLaunchKernelGGL(kern[geo], dim3((mp->npatch + NXCD - 1) / NXCD * NXCD), dim3(64), 0, mp->stream, mp->npatch, G->npend,
+                     3 * field, G->pend_rb, G->nrb, field, G->nshot, G->stride, mp->d_patch_desc, G->rows, mp->d_col_ends,
+                     mp->d_geom, mp->d_geom_elem, dn, (const float2*)G->Rb, dn + 2 * field, mp->d_rmassx, mp->d_rmassz,
+                     G->gk32, G->gm32, (float2*)G->pm32, mp->basis);
+  check_hip(hipGetLastError(), "k_grad_chain launch");
+  G->npend = 0;
+}
+
 // whether the sweep runs on towers, and what that needs: with a tower per chain stack, shot-major fields and neither a
 // CPML layer nor attenuation (which gradients refuse)
 void choose_sweep(Mesh* mp, GradState* G) {
+  G->rb_at = G->npend = 0;
   G->fused = mp->tower && G->ps == 1 && !mp->pml && !mp->attenuation;
   if (!G->fused || G->rows) return;
+  // the boundary terms' field has to fit, and a ring of R~ has to leave most of the memory free: steps to take at once
+  size_t free_bytes = 0, total = 0;
+  check_hip(hipMemGetInfo(&free_bytes, &total), "hipMemGetInfo");
+  const size_t bytes = G->nfield * sizeof(float);
+  if (free_bytes < 2 * bytes) {
+    G->fused = 0;
+    return;
+  }
+  if (free_bytes > 8 * RING * bytes) {
+    device_free(G->Rb);
+    G->Rb = device_zeros<float>(RING * G->nfield);
+    G->nrb = RING;
+  }
   const int n = mp->npatch;
   std::vector<int4> rows(mp->h_col_rows);
   std::vector<char> seen((size_t)mp->nglob, 0);
@@ -685,7 +729,8 @@ void sf2d_grad_begin_reverse(long* Mesh_pointer, const float* res) {
                              mp->stream),
               "residual H2D");
   choose_sweep(mp, G);
-  for (float* p : {G->D, G->Vb, G->Rb}) check_hip(hipMemsetAsync(p, 0, G->nfield * sizeof(float), mp->stream), "zero");
+  for (float* p : {G->D, G->Vb}) check_hip(hipMemsetAsync(p, 0, G->nfield * sizeof(float), mp->stream), "zero");
+  check_hip(hipMemsetAsync(G->Rb, 0, G->nrb * G->nfield * sizeof(float), mp->stream), "zero");
   check_hip(hipMemsetAsync(G->pm32, 0, G->n2 * sizeof(float), mp->stream), "zero");
   for (float* p : {G->gk32, G->gm32}) check_hip(hipMemsetAsync(p, 0, G->ne * sizeof(float), mp->stream), "zero");
   for (double* p : {G->gk, G->gm}) check_hip(hipMemsetAsync(p, 0, G->ne * sizeof(double), mp->stream), "zero");
@@ -710,16 +755,17 @@ void sf2d_grad_reverse_step(long* Mesh_pointer, int n, int slot, int first, floa
   if (G->fused) {
     if (!mp->tower) fail("sf2d_grad_reverse_step: the materials changed during the sweep");
     // R~_n is complete: the previous step's update made it (zero at n = NSTEP)
-    using K = decltype(&k_grad_chain<0>);
-    const K kern[3] = {k_grad_chain<0>, k_grad_chain<1>, k_grad_chain<2>};
-    const int geo = mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
-    if (!first)
-      hipLaunchKernelGGL(kern[geo], dim3((mp->npatch + NXCD - 1) / NXCD * NXCD), dim3(64), 0, mp->stream, mp->npatch,
-                         G->nshot, G->stride, mp->d_patch_desc, G->rows, mp->d_col_ends, mp->d_geom, mp->d_geom_elem,
-                         (const float2*)dn, (const float2*)G->Rb, (const float2*)rn, mp->d_rmassx, mp->d_rmassz, G->gk32,
-                         G->gm32, (float2*)G->pm32, mp->basis);
-    check_hip(hipGetLastError(), "k_grad_chain launch");
-    tower_step_adjoint(mp, G->Rb, G->D, G->Vb, G->stride, G->nshot, res, vpn, G->gvp32, G->gvs32, dt, h, dto2);
+    if (!first) {
+      if (G->npend == 0) {
+        G->pend_slot = slot;
+        G->pend_rb = G->rb_at;
+      }
+      if (++G->npend == G->nrb) flush_pending(mp, G);
+    }
+    const int next = (G->rb_at + 1) % G->nrb;
+    tower_step_adjoint(mp, G->Rb + G->rb_at * G->nfield, G->Rb + next * G->nfield, G->D, G->Vb, G->stride, G->nshot, res,
+                       vpn, G->gvp32, G->gvs32, dt, h, dto2);
+    G->rb_at = next;
     return;
   }
   int lshift = 0;
@@ -797,6 +843,7 @@ void sf2d_grad_recompute_segment(long* Mesh_pointer, int ckpt, int n0, int n1, f
 void sf2d_grad_flush(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
   GradState* G = need(mp);
+  flush_pending(mp, G);
   hipLaunchKernelGGL(k_flush64, dim3(grid_for(G->ne)), dim3(GT), 0, mp->stream, G->ne, G->gk32, G->gk);
   hipLaunchKernelGGL(k_flush64, dim3(grid_for(G->ne)), dim3(GT), 0, mp->stream, G->ne, G->gm32, G->gm);
   hipLaunchKernelGGL(k_flush64, dim3(grid_for(G->n2)), dim3(GT), 0, mp->stream, G->n2, G->pm32, G->pm);

@@ -290,7 +290,7 @@ struct ShotStep {
 void tower_begin_shots(Mesh* mp, float* accel, long stride, int nshot);
 void tower_step_shots(Mesh* mp, const ShotStep& S, int it, float deltat, float deltatsqover2, float deltatover2);
 // the reverse step of a gradient (gradient.hip): residuals and Stacey terms of the step, D += -K R~, and the next R~
-void tower_step_adjoint(Mesh* mp, float* Rb, float* D, float* Vb, long stride, int nshot, const float* res,
+void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, float* Vb, long stride, int nshot, const float* res,
                         const float* vpn, float* gvp, float* gvs, float dt, float h, float dto2);
 // copies the solid's displacement and velocity into gradient checkpoint `slot`; returns where its forces go
 float* grad_checkpoint_inputs(Mesh* mp, int slot);

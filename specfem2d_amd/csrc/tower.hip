@@ -96,9 +96,10 @@ struct TowerFields {
 };
 
 // The fields of a reverse step (gradient.hip): R~_n in, from which the force is computed, the cotangents D and V', and
-// R~_{n-1} = W A out in place: D += -K R~; V = V' + dt D; A = dt/2 V' + dt^2/2 D + dt/2 V
+// R~_{n-1} = W A out: D += -K R~; V = V' + dt D; A = dt/2 V' + dt^2/2 D + dt/2 V
 struct AdjointFields {
-  float2 *Rb, *D, *Vb;
+  const float2* Rb;
+  float2 *Rb_out, *D, *Vb;  // Rb_out may be Rb
   long stride;
   int nshot;
   struct Row {
@@ -119,7 +120,7 @@ struct AdjointFields {
     a.y = a.y + c.dto2 * v.y;
     st_off(D + shot, o, db);
     st_off(Vb + shot, o, v);
-    st_off(Rb + shot, o, make_float2(wx * a.x, wz * a.y));
+    st_off(Rb_out + shot, o, make_float2(wx * a.x, wz * a.y));
   }
 };
 
@@ -659,11 +660,11 @@ void tower_step_shots(Mesh* mp, const ShotStep& S, int it, float deltat, float d
   launch_tower(mp, F, it, S.seismo, (long)2 * mp->nrec_local * mp->nstep, S.src_shot,
                {deltatover2, deltat, deltatsqover2}, false, S.step);
 }
-void tower_step_adjoint(Mesh* mp, float* Rb, float* D, float* Vb, long stride, int nshot, const float* res,
+void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, float* Vb, long stride, int nshot, const float* res,
                         const float* vpn, float* gvp, float* gvs, float dt, float h, float dto2) {
   const TowerPlan& P = mp->tower->plan;
   float2* const slot = tower_slots(mp->tower, nshot);
-  const AdjointFields F{(float2*)Rb, (float2*)D, (float2*)Vb, stride, nshot};
+  const AdjointFields F{(const float2*)Rb, (float2*)Rb_out, (float2*)D, (float2*)Vb, stride, nshot};
   const Newmark nm{dto2, dt, h};
   AdjointEdges E{};
   E.faces = stacey_faces(mp);
