@@ -702,7 +702,7 @@ __global__ __launch_bounds__(64) void k_ac_tower(int ntower, const int4* __restr
 
 // The fluid's interface points; zd, zv at zp: solid points on both the CPML layer's outer boundary and a fluid-solid
 // edge, cleared here because the fluid has read them (pml_boundary_elastic)
-__global__ __launch_bounds__(256) void k_ac_interface(const InterfaceArgs A, const float* __restrict__ slot,
+__global__ __launch_bounds__(IF_T) void k_ac_interface(const InterfaceArgs A, const float* __restrict__ slot,
                                                       const FluidFields F, const float* __restrict__ rm, const Newmark nm,
                                                       const float2* __restrict__ layer, float* __restrict__ old,
                                                       float dt2o4, int nz,
@@ -716,16 +716,20 @@ __global__ __launch_bounds__(256) void k_ac_interface(const InterfaceArgs A, con
   if (q >= A.n) return;
   const int g = A.id[q];
   const int fl = A.flag[q];
-  float r = 0.f;
-  if (fl & IF_ACC) {
-    r = F.acc[g];
-    F.acc[g] = 0.f;
-  }
-  r = sum_towers(A, q, slot, r);
-  each_layer_slot(A, q, [&](int s) { r = (r - layer[s].x) - layer[s].y; });
+  const SlotIds s = slot_ids(A, q);
+  const float pot = F.pot[g], pd = F.pd[g], w = rm[g];
+  float acc = 0.f;
+  if (fl & IF_ACC) acc = F.acc[g];
+  const SlotValues<float> x = slot_values(q >= A.n2, s.t, slot);
+  SlotValues<float2> y{};
+  if (q >= A.n4) y = slot_values(true, s.p, layer);
+  if (fl & IF_ACC) F.acc[g] = 0.f;
+  float r = sum_slots(s.t, x, acc);
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (s.p[k] >= 0) r = (r - y.v[k].x) - y.v[k].y;
   const bool zero = fl & (IF_FREE | IF_PML_EDGE);
-  const float a = zero ? 0.f : r * rm[g];
-  const float pot = F.pot[g];
+  const float a = zero ? 0.f : r * w;
   if ((fl & IF_PML) && old) old[g] = (fl & IF_PML_EDGE) ? 0.f : fmaf(dt2o4, a, pot);
   if (fl & (IF_COUPLED | IF_LOOKED_AT)) F.pdd[g] = a;  // read by the solid, or by receivers in the next step
   if (zero) {
@@ -733,7 +737,7 @@ __global__ __launch_bounds__(256) void k_ac_interface(const InterfaceArgs A, con
     F.pd[g] = 0.f;
     if (F.last) F.pdd[g] = 0.f;
   } else {
-    fluid_newmark(nm, F, (unsigned)g, a, pot, F.pd[g]);
+    fluid_newmark(nm, F, (unsigned)g, a, pot, pd);
   }
 }
 
@@ -948,7 +952,7 @@ void fluid_towers(Mesh* mp, AcousticState* ac, const IboolView& iv, const std::v
   for (int g : pml) flag[g] |= IF_PML;
   for (int g : pml_edge_points(mp, true)) flag[g] |= IF_PML_EDGE;
   if (!build_tower_plan(ac->plan, towers, mp->nglob, flag, pml, rank)) return;
-  ac->d_slot = device_alloc<float>((size_t)ac->plan.nslot);
+  ac->d_slot = device_alloc<float>(std::max<size_t>(1, (size_t)ac->plan.nslot));
   if (!pml.empty()) ac->d_layer = device_alloc<float2>(pml.size());
   ac->d_acc = device_zeros<float>((size_t)mp->nglob);
   std::vector<int> keep;
@@ -1862,7 +1866,7 @@ void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int 
   pml_acoustic_slots(mp, ac->d_pot, ac->d_pd, ac->d_layer);
   const int n = std::max(P.n, ac->nkeep);
   if (n == 0) return;
-  hipLaunchKernelGGL(k_ac_interface, dim3((n + 255) / 256), dim3(256), 0, mp->stream, interface_args(P), ac->d_slot, F,
+  hipLaunchKernelGGL(k_ac_interface, dim3((n + IF_T - 1) / IF_T), dim3(IF_T), 0, mp->stream, interface_args(P), ac->d_slot, F,
                      ac->d_rm, nm, ac->d_layer, last ? nullptr : (float*)pml_old_field(mp, true), 0.5f * deltatsqover2, ac->nkeep,
                      ac->d_keep, (float2*)mp->d_displ, (float2*)mp->d_veloc);
   check_hip(hipGetLastError(), "k_ac_interface launch");

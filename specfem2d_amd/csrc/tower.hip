@@ -490,7 +490,7 @@ __global__ __launch_bounds__(64) void k_tower(
 // Newmark update; old (CPML layer points): u + dt^2 / 4 a of this step, the layer's previous-step field, zero on the
 // layer's outer boundary, whose displacement and velocity are zero when the next step starts (pml_boundary_elastic;
 // IF_KEEP: not before the fluid has read them).
-__global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
+__global__ __launch_bounds__(IF_T) void k_interface(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
                                                    const TowerFields F, const float* __restrict__ rmx,
                                                    const float* __restrict__ rmz, const Newmark nm,
                                                    const float2* __restrict__ layer, float2* __restrict__ old,
@@ -500,12 +500,17 @@ __global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const 
   const long at = blockIdx.y * F.stride;
   const int g = A.id[q];
   const int fl = A.flag[q];
+  const SlotIds s = slot_ids(A, q);
   const float2 dd = F.d[at + g], vv = F.v[at + g];
   const float wx = rmx[g], wz = rmz[g];
-  float2 r = sum_towers(A, q, slot + (size_t)blockIdx.y * nslot, make_float2(0.f, 0.f));
-  each_layer_slot(A, q, [&](int s) { add_slot(r, layer[s]); });
+  float2 acc = make_float2(0.f, 0.f);
+  if (fl & IF_ACC) acc = F.accel[at + g];
+  const SlotValues<float2> x = slot_values(q >= A.n2, s.t, slot + (size_t)blockIdx.y * nslot);
+  SlotValues<float2> y{};
+  if (q >= A.n4) y = slot_values(true, s.p, layer);
+  float2 r = sum_slots(s.p, y, sum_slots(s.t, x, make_float2(0.f, 0.f)));
   if (fl & IF_ACC) {
-    add_slot(r, F.accel[at + g]);
+    add_slot(r, acc);
     if (F.last != 1) F.accel[at + g] = make_float2(0.f, 0.f);
   }
   if ((fl & IF_PML) && old) {
@@ -521,7 +526,7 @@ __global__ __launch_bounds__(256) void k_interface(const InterfaceArgs A, const 
   F.update(nm, at, 8u * (unsigned)g, r, wx, wz, dd, {vv});
 }
 
-__global__ __launch_bounds__(256) void k_interface_adjoint(const InterfaceArgs A, const float2* __restrict__ slot,
+__global__ __launch_bounds__(IF_T) void k_interface_adjoint(const InterfaceArgs A, const float2* __restrict__ slot,
                                                            int nslot, const AdjointFields F,
                                                            const float* __restrict__ rmx, const float* __restrict__ rmz,
                                                            const Newmark nm) {
@@ -529,27 +534,36 @@ __global__ __launch_bounds__(256) void k_interface_adjoint(const InterfaceArgs A
   if (q >= A.n) return;
   const long at = blockIdx.y * F.stride;
   const int g = A.id[q];
+  const SlotIds s = slot_ids(A, q);
   const AdjointFields::Row row = F.load(at, 8u * (unsigned)g);
-  const float2 r = sum_towers(A, q, slot + (size_t)blockIdx.y * nslot, make_float2(0.f, 0.f));
-  F.update(nm, at, 8u * (unsigned)g, r, rmx[g], rmz[g], make_float2(0.f, 0.f), row);
+  const float wx = rmx[g], wz = rmz[g];
+  const SlotValues<float2> x = slot_values(q >= A.n2, s.t, slot + (size_t)blockIdx.y * nslot);
+  const float2 r = sum_slots(s.t, x, make_float2(0.f, 0.f));
+  F.update(nm, at, 8u * (unsigned)g, r, wx, wz, make_float2(0.f, 0.f), row);
 }
 
-__global__ __launch_bounds__(256) void k_interface_pair(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
+__global__ __launch_bounds__(IF_T) void k_interface_pair(const InterfaceArgs A, const float2* __restrict__ slot, int nslot,
                                                         const PairFields F, const float* __restrict__ rmx,
                                                         const float* __restrict__ rmz) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= A.n) return;
-  const int s = blockIdx.y;
+  const int f = blockIdx.y;
   const int g = A.id[q];
-  const float2 d = F.field(s)[g];
-  const PairFields::Row row = F.load(s, 8u * (unsigned)g);
-  float2 r = sum_towers(A, q, slot + (size_t)s * nslot, make_float2(0.f, 0.f));
-  if (A.flag[q] & (IF_ACC | IF_LOOKED_AT)) {  // receivers' points take the adjoint sources
-    float2* const acc = s ? F.acc1 : F.acc0;
-    add_slot(r, acc[g]);
+  const int fl = A.flag[q];
+  const SlotIds s = slot_ids(A, q);
+  const float2 d = F.field(f)[g];
+  const PairFields::Row row = F.load(f, 8u * (unsigned)g);
+  const float wx = rmx[g], wz = rmz[g];
+  float2 b = make_float2(0.f, 0.f);
+  float2* const acc = f ? F.acc1 : F.acc0;
+  if (fl & (IF_ACC | IF_LOOKED_AT)) b = acc[g];  // receivers' points take the adjoint sources
+  const SlotValues<float2> x = slot_values(q >= A.n2, s.t, slot + (size_t)f * nslot);
+  float2 r = sum_slots(s.t, x, make_float2(0.f, 0.f));
+  if (fl & (IF_ACC | IF_LOOKED_AT)) {
+    add_slot(r, b);
     acc[g] = make_float2(0.f, 0.f);
   }
-  F.update(F.nm0, s, 8u * (unsigned)g, r, rmx[g], rmz[g], d, row);
+  F.update(F.nm0, f, 8u * (unsigned)g, r, wx, wz, d, row);
 }
 
 // accel = 0 at the interface points with a boundary term (the start of a run of tower steps)
@@ -566,7 +580,7 @@ float2* tower_slots(TowerState* T, int nshot) {
     device_free(T->d_slot);
     T->d_slot = nullptr;
     T->slot_shots = 0;
-    T->d_slot = device_alloc<float2>((size_t)T->plan.nslot * nshot);
+    T->d_slot = device_alloc<float2>(std::max<size_t>(1, (size_t)T->plan.nslot * nshot));
     T->slot_shots = nshot;
   }
   return T->d_slot;
@@ -618,7 +632,7 @@ void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long se
   launch_k_tower(mp, kern[tower_geometry(mp)][sets], F, E, slot, nm);
   if (forward) pml_elastic_slots(mp, mp->tower->d_layer);
   if (P.n == 0) return;
-  hipLaunchKernelGGL(k_interface, dim3((P.n + 255) / 256, F.nshot), dim3(256), 0, mp->stream, interface_args(P), slot,
+  hipLaunchKernelGGL(k_interface, dim3((P.n + IF_T - 1) / IF_T, F.nshot), dim3(IF_T), 0, mp->stream, interface_args(P), slot,
                      P.nslot, F, mp->d_rmassx, mp->d_rmassz, nm, mp->tower->d_layer,
                      F.last ? nullptr : (float2*)pml_old_field(mp, false), 0.5f * nm.dt2o2);
   check_hip(hipGetLastError(), "k_interface launch");
@@ -680,7 +694,7 @@ void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, floa
                      k_tower<2, 0, AdjointFields, AdjointEdges>};
   launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, nm);
   if (P.n == 0) return;
-  hipLaunchKernelGGL(k_interface_adjoint, dim3((P.n + 255) / 256, nshot), dim3(256), 0, mp->stream, interface_args(P),
+  hipLaunchKernelGGL(k_interface_adjoint, dim3((P.n + IF_T - 1) / IF_T, nshot), dim3(IF_T), 0, mp->stream, interface_args(P),
                      slot, P.nslot, F, mp->d_rmassx, mp->d_rmassz, nm);
   check_hip(hipGetLastError(), "k_interface_adjoint launch");
 }
@@ -1056,7 +1070,7 @@ void sf2d_tower_adjoint_step(long* Mesh_pointer, int it, int last, const float* 
                       k_tower<2, 0, PairFields, PairEdges>};
   launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, F.nm0);
   if (P.n > 0) {
-    hipLaunchKernelGGL(k_interface_pair, dim3((P.n + 255) / 256, 2), dim3(256), 0, mp->stream, interface_args(P), slot,
+    hipLaunchKernelGGL(k_interface_pair, dim3((P.n + IF_T - 1) / IF_T, 2), dim3(IF_T), 0, mp->stream, interface_args(P), slot,
                        P.nslot, F, mp->d_rmassx, mp->d_rmassz);
     check_hip(hipGetLastError(), "k_interface_pair launch");
   }
