@@ -71,12 +71,12 @@ struct TowerPlan {
 
 // builds the plan over the points of the towers and the flagged ones; pml_ids: point of each CPML element point.  False
 // when more than four towers (chains) or layer elements meet in a point.
-// With rank (of the chain at each first element position) the slots of a point are in the order of the ranks, and where
-// two chains of a tower meet, the interface points of its left and right column take the two chains' forces in slots of
-// their own (the lower one's are the row's split slots): the interface then sums a point's forces one chain at a time
-// in the order in which a launch per colour adds them.
+// The slots of a point are in the order of rank (of the chain at each first element position), and where two chains of a
+// tower meet, the interface points of its left and right column take the two chains' forces in slots of their own (the
+// lower one's are the row's split slots): the interface then sums a point's forces one chain at a time in the order in
+// which a launch per colour adds them.
 bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob, const std::vector<uint8_t>& flag,
-                      const std::vector<int>& pml_ids, const std::vector<int>& rank = {});
+                      const std::vector<int>& pml_ids, const std::vector<int>& rank);
 
 constexpr int IF_T = 64;  // threads per workgroup of the interface kernels: one wave, so that few points spread over many CUs
 

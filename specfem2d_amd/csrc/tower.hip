@@ -345,6 +345,7 @@ __global__ __launch_bounds__(64) void k_tower(
     }
   };
 
+  auto edge_bit = [&](const int4 r) { return ((xe < 32 ? (unsigned)r.x >> xe : (unsigned)r.y >> (xe - 32)) & 1u) != 0; };
   float2 u0 = ld_off(d, off0);
   float2 carry = make_float2(0.f, 0.f);
   ChainRegs nx;
@@ -387,10 +388,13 @@ __global__ __launch_bounds__(64) void k_tower(
     float2 t1[NGLL], t2[NGLL];
 #pragma unroll
     for (int j = 0; j < NGLL; j++) {
-      const float2 e0 = el[j * TROW], e1 = el[j * TROW + 1], e2 = el[j * TROW + 2], e3 = el[j * TROW + 3],
-                   e4 = el[j * TROW + 4];
-      const float dux_dxi = e0.x * hpi[0] + e1.x * hpi[1] + e2.x * hpi[2] + e3.x * hpi[3] + e4.x * hpi[4];
-      const float duz_dxi = e0.y * hpi[0] + e1.y * hpi[1] + e2.y * hpi[2] + e3.y * hpi[3] + e4.y * hpi[4];
+      float dux_dxi = 0.f, duz_dxi = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        const float2 e = el[j * TROW + m];
+        dux_dxi += e.x * hpi[m];
+        duz_dxi += e.y * hpi[m];
+      }
       float dux_dga = 0.f, duz_dga = 0.f;
 #pragma unroll
       for (int m = 0; m < NGLL; m++) {
@@ -407,9 +411,10 @@ __global__ __launch_bounds__(64) void k_tower(
       const float dux_dzl = RECT ? dux_dga * gazl : dux_dxi * xizl + dux_dga * gazl;
       const float duz_dxl = RECT ? duz_dxi * xixl : duz_dxi * xixl + duz_dga * gaxl;
       const float duz_dzl = RECT ? duz_dga * gazl : duz_dxi * xizl + duz_dga * gazl;
-      float sxx = lp2m * dux_dxl + lambdal * duz_dzl;
-      float szz = lp2m * duz_dzl + lambdal * dux_dxl;
-      float sxz = mu * (duz_dxl + dux_dzl);
+      // contracted as in k_elastic_forces_col, so that both kernels give the same bits
+      float sxx = fmaf(lp2m, dux_dxl, lambdal * duz_dzl);
+      float szz = fmaf(lambdal, dux_dxl, lp2m * duz_dzl);
+      float sxz = mu * (RECT && SETS == 0 ? fmaf(duz_dxi, xixl, dux_dzl) : duz_dxl + dux_dzl);
       if (SETS > 0) {
         const unsigned la = word + (unsigned)j * mrow;
         float ev[9] = {st[0].x, st[0].y, st[0].z, st[0].w, st[1].x, st[1].y, st[1].z, st[1].w, st[2].x};
@@ -433,8 +438,8 @@ __global__ __launch_bounds__(64) void k_tower(
         t2[j] = make_float2(cz * sxz, cz * szz);
       } else {
         const float jac = 1.f / (xixl * gazl - gaxl * xizl);
-        t1[j] = make_float2(jac * (sxx * xixl + sxz * xizl), jac * (sxz * xixl + szz * xizl));
-        t2[j] = make_float2(jac * (sxx * gaxl + sxz * gazl), jac * (sxz * gaxl + szz * gazl));
+        t1[j] = make_float2(jac * fmaf(xixl, sxx, xizl * sxz), jac * fmaf(xixl, sxz, xizl * szz));
+        t2[j] = make_float2(jac * fmaf(gaxl, sxx, gazl * sxz), jac * fmaf(gaxl, sxz, gazl * szz));
       }
     }
     // xi flux contraction: the element's rows through LDS
@@ -446,10 +451,13 @@ __global__ __launch_bounds__(64) void k_tower(
     float2 f[NGLL];
 #pragma unroll
     for (int j = 0; j < NGLL; j++) {
-      const float2 e0 = el[j * TROW], e1 = el[j * TROW + 1], e2 = el[j * TROW + 2], e3 = el[j * TROW + 3],
-                   e4 = el[j * TROW + 4];
-      const float sx = e0.x * hwi[0] + e1.x * hwi[1] + e2.x * hwi[2] + e3.x * hwi[3] + e4.x * hwi[4];
-      const float sz = e0.y * hwi[0] + e1.y * hwi[1] + e2.y * hwi[2] + e3.y * hwi[3] + e4.y * hwi[4];
+      float sx = 0.f, sz = 0.f;
+#pragma unroll
+      for (int m = 0; m < NGLL; m++) {
+        const float2 e = el[j * TROW + m];
+        sx += e.x * hwi[m];
+        sz += e.y * hwi[m];
+      }
       float gx = 0.f, gz = 0.f;
 #pragma unroll
       for (int m = 0; m < NGLL; m++) {
@@ -471,10 +479,17 @@ __global__ __launch_bounds__(64) void k_tower(
         f[j].y += fz;
       }
     }
-    f[0].x += carry.x;
-    f[0].y += carry.y;
+    // the row below's force, or where the columns are interface points a slot of its own
+    const int4 r0 = row[4 * c];
+    const bool lone = writer && c > 0 && ((x == 0 && (r0.x & 1)) || (x == xe && edge_bit(r0)));
+    if (lone) {
+      slot[r0.w + (x == 0 ? 0 : r0.x & 1)] = carry;
+    } else {
+      f[0].x += carry.x;
+      f[0].y += carry.y;
+    }
 #pragma unroll
-    for (int j = 0; j < NGLL - 1; j++) finish(row[4 * c + j], j == 0 ? off0 : off1 + (unsigned)(j - 1) * up, f[j], u[j], vp[j], ms[j]);
+    for (int j = 0; j < NGLL - 1; j++) finish(j == 0 ? r0 : row[4 * c + j], j == 0 ? off0 : off1 + (unsigned)(j - 1) * up, f[j], u[j], vp[j], ms[j]);
     carry = f[NGLL - 1];
     u0 = u[NGLL - 1];
     off0 = off1 + (unsigned)(NGLL - 2) * up;
@@ -508,11 +523,8 @@ __global__ __launch_bounds__(IF_T) void k_interface(const InterfaceArgs A, const
   const SlotValues<float2> x = slot_values(q >= A.n2, s.t, slot + (size_t)blockIdx.y * nslot);
   SlotValues<float2> y{};
   if (q >= A.n4) y = slot_values(true, s.p, layer);
-  float2 r = sum_slots(s.p, y, sum_slots(s.t, x, make_float2(0.f, 0.f)));
-  if (fl & IF_ACC) {
-    add_slot(r, acc);
-    if (F.last != 1) F.accel[at + g] = make_float2(0.f, 0.f);
-  }
+  const float2 r = sum_slots(s.p, y, sum_slots(s.t, x, acc));
+  if ((fl & IF_ACC) && F.last != 1) F.accel[at + g] = make_float2(0.f, 0.f);
   if ((fl & IF_PML) && old) {
     const float ax = r.x * wx, az = r.y * wz;
     old[g] = (fl & IF_PML_EDGE) ? make_float2(0.f, 0.f)
@@ -558,11 +570,8 @@ __global__ __launch_bounds__(IF_T) void k_interface_pair(const InterfaceArgs A, 
   float2* const acc = f ? F.acc1 : F.acc0;
   if (fl & (IF_ACC | IF_LOOKED_AT)) b = acc[g];  // receivers' points take the adjoint sources
   const SlotValues<float2> x = slot_values(q >= A.n2, s.t, slot + (size_t)f * nslot);
-  float2 r = sum_slots(s.t, x, make_float2(0.f, 0.f));
-  if (fl & (IF_ACC | IF_LOOKED_AT)) {
-    add_slot(r, b);
-    acc[g] = make_float2(0.f, 0.f);
-  }
+  const float2 r = sum_slots(s.t, x, b);
+  if (fl & (IF_ACC | IF_LOOKED_AT)) acc[g] = make_float2(0.f, 0.f);
   F.update(F.nm0, f, 8u * (unsigned)g, r, wx, wz, d, row);
 }
 
@@ -783,8 +792,7 @@ bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob,
     for (int k = 0; k < 3; k++) desc[4 * t + 1 + k] = make_int4(r[k].inner - 1, r[k].left, r[k].right, 0);
     P.nrow += 4 * w.nch + 1;
   }
-  const bool split = !rank.empty();
-  auto junction = [&](const Tower& w, int r) { return split && r % 4 == 0 && r > 0 && r < 4 * w.nch; };
+  auto junction = [&](const Tower& w, int r) { return r % 4 == 0 && r > 0 && r < 4 * w.nch; };
   // how many towers (or chains of them) and layer elements hold each point
   std::vector<uint8_t> cnt((size_t)nglob, 0), npml((size_t)(pml_ids.empty() ? 0 : nglob), 0), two((size_t)nglob, 0);
   for (const Tower& w : towers)
@@ -833,7 +841,7 @@ bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob,
     for (int r = 0; r <= 4 * w.nch; r++) {
       const TowerRow t = w.at(r);
       const int c = std::min(r / 4, w.nch - 1);
-      const int rk = split ? rank[w.e0 + c * w.ne] : 0;
+      const int rk = rank[w.e0 + c * w.ne];
       unsigned long long m = 0ull;
       const int first = ns;
       auto take = [&](int x, int g) {
@@ -926,6 +934,11 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
   // a chain all of whose elements belong to the CPML layer has no force of its own
   std::vector<TowerChain> chains(npatch);
   std::vector<char> kind(npatch, CHAIN_STACKED);
+  std::vector<int> rank((size_t)mp->nspec, 0);  // descriptors lie colour by colour
+  std::vector<char> source((size_t)mp->nspec, 0);
+  for (int e : mp->h_src_ispec) source[e] = 1;
+  if (mp->simulation_type == 3)
+    for (int e : mp->h_rec_ispec) source[e] = 1;  // adjoint sources
   for (int q = 0; q < npatch; q++) {
     TowerChain& c = chains[q];
     c.e0 = pd[4 * q];
@@ -934,9 +947,16 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
       const int4 r = rows[(size_t)q * NGLL + j];
       c.row[j] = {r.x + 1, r.y, ends[(size_t)q * NGLL + j]};
     }
-    bool layer = true;
-    for (int k = 0; k < c.ne && layer; k++) layer = pml_element(mp, mp->ispec_of_pos[c.e0 + k]);
+    rank[c.e0] = q;
+    // a chain with a source starts and ends at interface rows, so that the source's force comes first in the sum
+    bool layer = true, alone = false;
+    for (int k = 0; k < c.ne; k++) {
+      const int e = mp->ispec_of_pos[c.e0 + k];
+      layer = layer && pml_element(mp, e);
+      alone = alone || source[e];
+    }
     if (layer) kind[q] = CHAIN_SKIP;
+    else if (alone) kind[q] = CHAIN_ALONE;
   }
   std::vector<Tower> towers;
   if (!chain_towers(mp->h_above, chains, kind, towers, mp->batch ? mp->batch->nshot : 1)) return 0;
@@ -965,7 +985,7 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     if (rmassx[g] != rmassz[g]) flag[dev(g)] |= IF_LOOKED_AT;
   for (int g = mp->nglob_el; g < ng; g++) flag[g] = 0;  // no solid element has these
   TowerState* T = new TowerState();
-  if (!build_tower_plan(T->plan, towers, ng, flag, pml)) {
+  if (!build_tower_plan(T->plan, towers, ng, flag, pml, rank)) {
     delete T;
     return 0;
   }
