@@ -830,6 +830,9 @@ struct AcousticState {
   float2* d_layer = nullptr;  // the CPML layer's two terms per element point
   int nkeep = 0;
   int* d_keep = nullptr;
+  // of a fluid without fluid-solid edges: a stream of its own for the fused steps, and the events that fork and join it
+  hipStream_t apart = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
 };
 
 void acoustic_release(Mesh* mp) {
@@ -847,6 +850,11 @@ void acoustic_release(Mesh* mp) {
   device_free(ac->d_kl_ids); device_free(ac->d_kl_geom); device_free(ac->d_kl_rk);
   device_free(ac->d_rho_kl); device_free(ac->d_kappa_kl);
   ac->plan.release();
+  if (ac->apart) {
+    (void)hipEventDestroy(ac->fork);
+    (void)hipEventDestroy(ac->join);
+    (void)hipStreamDestroy(ac->apart);
+  }
   device_free(ac->d_slot); device_free(ac->d_acc); device_free(ac->d_keep); device_free(ac->d_layer);
   delete ac;
   mp->ac = nullptr;
@@ -1829,6 +1837,24 @@ void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int 
   const TowerPlan& P = ac->plan;
   if (P.ntower == 0) fail("sf2d_tower_fluid_step: no towers");
   if (it < 1 || it > mp->nstep) fail("sf2d_tower_fluid_step: it=%d outside 1..%d", it, mp->nstep);
+  // Without fluid-solid edges the fluid's steps depend on nothing of the solid's: they run beside them, on a stream that
+  // waits for the run's preparation and that the handle's stream waits for at its end.  A step's kernels of 10 to 20 us
+  // leave much of the card idle (an uneven batch of 8
+  // with solids and fluids, 366 steps: 27.0 ms on one stream, 21.4 on two).
+  hipStream_t const own = mp->stream;
+  const bool apart = mp->nspec_elastic > 0 && ac->ncoup == 0;
+  if (apart) {
+    if (!ac->apart) {
+      check_hip(hipStreamCreateWithFlags(&ac->apart, hipStreamNonBlocking), "hipStreamCreate");
+      check_hip(hipEventCreateWithFlags(&ac->fork, hipEventDisableTiming), "hipEventCreate");
+      check_hip(hipEventCreateWithFlags(&ac->join, hipEventDisableTiming), "hipEventCreate");
+    }
+    if (first) {
+      check_hip(hipEventRecord(ac->fork, own), "fork");
+      check_hip(hipStreamWaitEvent(ac->apart, ac->fork, 0), "fork");
+    }
+    mp->stream = ac->apart;
+  }
   const Newmark nm{deltatover2, deltat, deltatsqover2};
   const FluidFields F{ac->d_pot, ac->d_pd, ac->d_pdd, ac->d_acc, last};
   FluidEdges E{};
@@ -1865,11 +1891,17 @@ void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int 
   check_hip(hipGetLastError(), "k_ac_tower launch");
   pml_acoustic_slots(mp, ac->d_pot, ac->d_pd, ac->d_layer);
   const int n = std::max(P.n, ac->nkeep);
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_ac_interface, dim3((n + IF_T - 1) / IF_T), dim3(IF_T), 0, mp->stream, interface_args(P), ac->d_slot, F,
+  if (n > 0)
+    hipLaunchKernelGGL(k_ac_interface, dim3((n + IF_T - 1) / IF_T), dim3(IF_T), 0, mp->stream, interface_args(P), ac->d_slot, F,
                      ac->d_rm, nm, ac->d_layer, last ? nullptr : (float*)pml_old_field(mp, true), 0.5f * deltatsqover2, ac->nkeep,
                      ac->d_keep, (float2*)mp->d_displ, (float2*)mp->d_veloc);
   check_hip(hipGetLastError(), "k_ac_interface launch");
+  if (!apart) return;
+  mp->stream = own;
+  if (last) {
+    check_hip(hipEventRecord(ac->join, ac->apart), "join");
+    check_hip(hipStreamWaitEvent(own, ac->join, 0), "join");
+  }
 }
 
 }  // extern "C"
