@@ -496,9 +496,9 @@ __global__ __launch_bounds__(64) void k_ac_seismograms(const FluidReceivers R, i
 // boundary stay zero.  Every point's sum is made in the order and with the roundings of the launch per colour
 // (k_acoustic_forces_col, the CPML layer's kernel, k_ac_corrector, k_ac_predictor): the potential's short waves carry the
 // rounding errors of each step on, and a displacement is its gradient, so that any other order shows in the fifth digit.
-// Small meshes are bound by launches (two a step instead of twelve: 44 x 44 elements, 800 steps, 37.8 -> 14.9 ms), large
-// ones by HBM (with the solid's step and the CPML layer in one launch each, 1000 x 500 fluid-solid elements, 100 steps:
-// 24.1 -> 16.7 ms).
+// Small meshes are bound by the latency of launches and loads (two launches a step instead of twelve: 44 x 44 elements, 800
+// steps, 37.8 -> 14.9 ms, 7.0 with fewer events), large ones by HBM (with the solid's step and the CPML layer in one launch
+// each, 1000 x 500 fluid-solid elements, 100 steps: 24.1 -> 16.7 ms).
 struct FluidFields {
   float *pot, *pd, *pdd;
   float* acc;   // boundary terms at interface points, zero between the steps
@@ -920,6 +920,8 @@ void fluid_towers(Mesh* mp, AcousticState* ac, const IboolView& iv, const std::v
   std::vector<TowerChain> chains(n);
   std::vector<char> kind(n, CHAIN_STACKED);
   std::vector<int> rank((size_t)order.size(), 0);  // descriptors lie colour by colour
+  std::vector<char> has_source((size_t)mp->nspec, 0);
+  for (int e : mp->h_src_ispec) has_source[e] = 1;
   for (int q = 0; q < n; q++) {
     TowerChain& c = chains[q];
     c.e0 = desc[4 * q];
@@ -939,7 +941,7 @@ void fluid_towers(Mesh* mp, AcousticState* ac, const IboolView& iv, const std::v
     bool layer = true, source = false;
     for (int k = 0; k < c.ne; k++) {
       layer = layer && pml_element(mp, order[c.e0 + k]);
-      source = source || std::count(mp->h_src_ispec.begin(), mp->h_src_ispec.end(), order[c.e0 + k]) > 0;
+      source = source || has_source[order[c.e0 + k]];
     }
     if (layer) kind[q] = CHAIN_SKIP;
     else if (source) kind[q] = CHAIN_ALONE;

@@ -63,7 +63,7 @@ void batch_step_fields(Mesh* mp, BatchState* B, int it, float deltat, float delt
 }
 
 // whether the batch steps on towers (shot-major fields of a handle that has them)
-bool fused_batch(const Mesh* mp, const BatchState* B) { return mp->tower && B->ps == 1; }
+bool fused_batch(const Mesh* mp, const BatchState* B) { return B->ps == 1 && tower_takes(mp, B->nshot); }
 
 void drop_graph(BatchState* B) {
   if (B->graph_exec) (void)hipGraphExecDestroy(B->graph_exec);

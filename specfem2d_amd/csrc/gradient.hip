@@ -590,7 +590,7 @@ void flush_pending(Mesh* mp, GradState* G) {
 // CPML layer nor attenuation (which gradients refuse)
 void choose_sweep(Mesh* mp, GradState* G) {
   G->rb_at = G->npend = 0;
-  G->fused = mp->tower && G->ps == 1 && !mp->pml && !mp->attenuation;
+  G->fused = G->ps == 1 && tower_takes(mp, G->nshot) && !mp->pml && !mp->attenuation;
   if (!G->fused || G->rows) return;
   // the boundary terms' field has to fit, and a ring of R~ has to leave most of the memory free: steps to take at once
   size_t free_bytes = 0, total = 0;

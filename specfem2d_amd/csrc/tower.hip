@@ -9,15 +9,17 @@
 //
 // The other points -- the tower's outline and every point that something else also acts on or looks at (absorbing
 // edges, sources, fluid-solid edges, CPML elements, receivers, points whose two inverse masses differ) -- are the
-// interface.  For these the wave stores its force into a slot of its own (partial), the boundary kernels add theirs
-// into accel as they always do, and the interface kernel sums the slots of each point in a fixed order, adds and clears
-// accel and makes the same Newmark update.
+// interface.  For these the wave stores its force into a slot of its own, further workgroups of the same launch add the
+// boundary terms into accel, and the interface kernel sums the boundary terms and the slots of each point in the order in
+// which a launch per colour adds them, clears accel and makes the same Newmark update.
 //
 // State between two such steps: (d_n, v'_n) predicted, accel zero at the interface points with a boundary term and
 // stale elsewhere.  A run starts from the ordinary predictor; its last step leaves displacement, velocity and
 // acceleration as the callers know them.
 //
-// What bounds it: HBM.  2000 x 1000 elements (32 M points), one step: see the launch rule at tower_chains below.
+// What bounds it: on large meshes HBM.  2000 x 1000 elements (32 M points): k_tower moves 1.74 GB in 371 us (4.7 TB/s, what a
+// copy reaches on this card), k_interface 0.17 GB in 31 us; four colour launches and a corrector-predictor pass took 576 us.
+// On small meshes the latency of launches and dependent loads: 80 x 60 elements 6.0 and 3.2 us.
 #include <algorithm>
 #include <cstdlib>
 #include <vector>
@@ -603,7 +605,6 @@ template <class Fields, class Edges, class Kernel>
 void launch_k_tower(Mesh* mp, Kernel kern, const Fields& F, const Edges& E, float2* slot, const Newmark& nm) {
   const TowerPlan& P = mp->tower->plan;
   const TowerAtt att{mp->d_att_idx, mp->d_att_table, mp->d_att_e, (long)mp->nspec * NGLL2};
-  if ((long)(P.ntower + NXCD) * F.nshot > (1L << 30)) fail("tower launch: %d towers x %d shots", P.ntower, F.nshot);
   const int wgs = (P.ntower * F.nshot + NXCD - 1) / NXCD * NXCD;
   hipLaunchKernelGGL(kern, dim3(wgs + E.wgs(F.nshot)), dim3(64), 0, mp->stream, P.ntower, P.d_desc, P.d_row, mp->d_geom,
                      mp->d_geom_elem, mp->d_col_mod, F, mp->d_rmassx, slot, P.nslot, nm, mp->basis, att, wgs, E);
@@ -673,6 +674,11 @@ void prepare_store(Mesh* mp, int nstep) {
 
 }  // namespace
 
+bool tower_takes(const Mesh* mp, int nshot) {
+  const long per_shot = (mp->tower ? mp->tower->plan.ntower : 0) + (long)mp->num_abs * NGLL / 64 + 1 + mp->nrec_local;
+  return mp->tower && per_shot * nshot + mp->nsources_local < (1L << 25);  // workgroups of 64: below 2^32 threads
+}
+
 // shot batches and gradients: nshot forward fields, shot s at s * stride points
 void tower_begin_shots(Mesh* mp, float* accel, long stride, int nshot) {
   clear_interface(mp, (float2*)accel, stride, nshot);
@@ -708,10 +714,10 @@ void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, floa
   check_hip(hipGetLastError(), "k_interface_adjoint launch");
 }
 
-// Chains per tower (nchain: times the shots): about one wave per slot of the card (4096 at four waves per SIMD) and at most 16.  A tall tower has
-// few interface rows (1 in 4 x chains), a short one more waves in flight.  Measured, ms of 300 steps of 600 x 300 elements
-// (15,000 chains) at 1, 2, 4, 8, 16 chains: 15.3, 13.9, 13.6, 14.2, 18.7; 40 steps of 2000 x 1000 (166,667 chains) at 2, 4,
-// 8, 16, 32: 19.9, 17.9, 17.2, 17.1, 17.6.
+// Chains per tower (nchain: times the shots): about one wave per slot of the card (4096 at four waves per SIMD) and at
+// most 16.  A tall tower has few interface rows (1 in 4 x chains), a short one more waves in flight; a wave takes 2.3 us per
+// chain.  Measured, ms of 300 steps of 600 x 300 elements (15,000 chains) at 1, 2, 4, 8, 16 chains: 12.9, 11.7, 10.7, 12.0,
+// 17.2; 40 steps of 2000 x 1000 (167,000 chains) at 4, 8, 16: 17.1, 16.5, 16.4; 1000 steps of 80 x 60 (420) at 1, 2: 9.9, 11.9.
 int tower_chains(long nchain) {
   if (const char* env = getenv("SF2D_TOWER_CHAINS")) return std::max(1, atoi(env));
   return (int)std::max(1L, std::min(16L, (nchain + 4095) / 4096));

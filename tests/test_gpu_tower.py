@@ -78,8 +78,10 @@ def test_fused_step_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
     bounds = [3e-5] + BOUNDS[1:] if cfg.seismotype == 4 and not cfg.use_trick else BOUNDS
     for a, b, tol in zip(fused, plain, bounds):
         assert np.linalg.norm(b) > 0 and rel(a, b) < tol
-        # the fluid's sums keep the order of the launch per colour, but for edge points that two Stacey terms meet in
-        assert not form.startswith("fluid") or nz < 12 or np.array_equal(a, b)
+        # sums keep the order and the roundings of the launch per colour, but for points where several boundary terms meet
+        # (the flattest mesh, ends of the sea floor) and, in solids, attenuation and CPML
+        if nz >= 12 and form in ("stacey", "points", "layers", "fluid", "fluid_cpml"):
+            assert np.array_equal(a, b)
     ref = OracleSim(cfg, "sp").forward()
     assert rel(fused[0], ref) < bounds[0]
 
