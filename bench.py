@@ -49,6 +49,12 @@ def kernel_min_bytes(nspec: int, nglob: int, n_affine: int, chain: bool, rows: b
     return per_elem * nspec + 16 * n_affine + 400 * (nspec - n_affine) + 24 * nglob
 
 
+def fused_min_bytes(nspec: int, nglob: int, n_affine: int) -> int:
+    """Minimal bytes of the fused step's representation: per element 200 B of moduli, about 9 B of row records and the
+    geometry as above; per unique point displacement and velocity read and written and the inverse mass (36 B)."""
+    return 209 * nspec + 16 * n_affine + 400 * (nspec - n_affine) + 36 * nglob
+
+
 def force_kernel_bytes(nspec: int, nglob: int) -> int:
     """Algorithmic bytes of one element-force launch: per element 25 x (ibool + xix, xiz,
     gammax, gammaz, kappa, mu) = 700 B; per unique point displ read (8 B) and accel
@@ -224,10 +230,10 @@ def batch_forward(nshot: int, nstep: int, shots_per_wave: int = 0):
     return out
 
 
-def read_traffic(name: str):
-    """HBM bytes per force launch (FETCH_SIZE + WRITE_SIZE, calibrated against a plain copy) from the
-    committed rocprofv3 PMC summary of this workload, if present."""
-    path = os.path.join(ROOT, "profiles", f"elastic_forces_{name}_traffic.md")
+def read_traffic(name: str, fused: bool = False):
+    """HBM bytes per force launch, or per fused step (FETCH_SIZE + WRITE_SIZE, calibrated against a plain copy), from
+    the committed rocprofv3 PMC summary of this workload, if present."""
+    path = os.path.join(ROOT, "profiles", f"{'fused_step' if fused else 'elastic_forces'}_{name}_traffic.md")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -278,11 +284,11 @@ def c2_coupled(steps: int = 100, warmup: int = 10):
 def c2_attenuation(steps: int = 50, warmup: int = 5):
     """Forward of the C2 elastic mesh (2000 x 1000 elements of 10 m, the random-field model) with viscoelastic
     attenuation everywhere (Qkappa 60, Qmu 30, 3 standard linear solids): GLL-point updates per second, and the
-    element-force launches' share of the step with the survey's algorithmic bytes for this kernel, the elastic
+    element-force launches' share of the step (all of it where the step is fused) with the survey's algorithmic bytes for this kernel, the elastic
     700 B per element plus 3600 B per element of attenuation, plus 24 B per point.  This build's chain kernel
     reads and writes 2723 B per element (25 points x (moduli 8 B, coefficient-set index 4 B, 9 memory variables and
     3 previous strains read and written 96 B), a 16-byte geometry record and about 7 B of point-id row records per
-    element) plus 24 B per point."""
+    element) plus 24 B per point, 36 B where the Newmark updates are fused in."""
     import torch
     from specfem2d_amd.driver import Simulation
     cfg = make_config("c2_mesh_elastic_2000x1000", warmup + steps).replace(attenuation=True, qkappa=60.0, qmu=30.0)
@@ -290,11 +296,11 @@ def c2_attenuation(steps: int = 50, warmup: int = 5):
     sim.forward(nstep=warmup)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
-    seis, timing = sim.forward(nstep=steps, phase_timing=True)
+    seis, timing = sim.forward(nstep=steps)
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     traffic = (700 + 3600) * sim.nspec + 24 * sim.nglob
-    own = 2723 * sim.nspec + 24 * sim.nglob
+    own = 2723 * sim.nspec + (36 if sim.fused_step() else 24) * sim.nglob
     forces_s = timing["forces_ms"] * 1e-3 / steps
     out = {"workload": "c2_mesh_elastic_2000x1000 + attenuation (Qkappa 60, Qmu 30, N_SLS 3)", "nspec": sim.nspec,
            "nglob": sim.nglob, "steps": steps, "ms_per_step": wall * 1e3 / steps, "value": sim.nglob * steps / wall,
@@ -326,8 +332,10 @@ def c2_elastic(steps: int, warmup: int):
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     nglob, nspec = sim.nglob, sim.nspec
-    # one force launch per colour; the events bracket all launches of a step
-    launches = sim.colours(2)
+    # fused: one step is the tower launch and the interface launch, Newmark updates included, priced by the same formula
+    # (the forces' bytes alone); else one force launch per colour.  The events bracket all launches of a step
+    fused = sim.fused_step()
+    launches = 1 if fused else sim.colours(2)
     patch_mode = os.environ.get("SF2D_ASSEMBLY", "patch") == "patch"
     n_affine = sim.affine_elements() if patch_mode else 0
     chain = patch_mode and sim.chain_kernel()
@@ -336,7 +344,8 @@ def c2_elastic(steps: int, warmup: int):
     achieved = fk_bytes / (fk_ms * 1e-3) / 1e9
     roofline = {
         "bound": "hbm",
-        "kernel": (("k_elastic_forces_chain" if os.environ.get("SF2D_ROW_CHAIN") else "k_elastic_forces_col")
+        "kernel": "k_tower + k_interface (forces and Newmark updates)" if fused else
+                  (("k_elastic_forces_chain" if os.environ.get("SF2D_ROW_CHAIN") else "k_elastic_forces_col")
                    if chain else "k_elastic_forces_patch") if patch_mode
                   else "k_elastic_forces",
         "measured_on": name,
@@ -345,12 +354,13 @@ def c2_elastic(steps: int, warmup: int):
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": achieved / HBM_PEAK_GBS,
-        "traffic": read_traffic(name),
+        "traffic": read_traffic(name, fused),
         "algorithmic_bytes_per_launch": fk_bytes,
         "avg_launch_ms": fk_ms,
         # the bytes this kernel's own representation needs at minimum: affine elements carry one 16-byte
         # geometry record instead of 25 x 16 bytes (what it reads, not the formula above)
-        "kernel_min_bytes_per_launch": kernel_min_bytes(nspec, nglob, n_affine, chain,
+        "kernel_min_bytes_per_launch": fused_min_bytes(nspec, nglob, n_affine) if fused else
+                                       kernel_min_bytes(nspec, nglob, n_affine, chain,
                                                         chain and sim.col_rows()) / launches,
         "chain_row_records": bool(chain and sim.col_rows()),
     }

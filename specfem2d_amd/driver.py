@@ -136,6 +136,8 @@ def load_libraries():
     gpu.sf2d_mesh_fluid_chain.restype = C.c_int
     gpu.sf2d_mesh_chain.argtypes = [C.POINTER(C.c_long)]
     gpu.sf2d_mesh_chain.restype = C.c_int
+    gpu.sf2d_tower_ready.argtypes = [C.POINTER(C.c_long)]
+    gpu.sf2d_tower_ready.restype = C.c_int
     gpu.sf2d_mesh_colours.argtypes = [C.POINTER(C.c_long), C.c_int]
     gpu.sf2d_mesh_colours.restype = C.c_int
     gpu.sf2d_mesh_synchronize.argtypes = [C.POINTER(C.c_long)]
@@ -281,6 +283,12 @@ class Simulation:
         self._need_device()
         mp = C.c_long(self.mesh_pointer)
         return bool(self.gpu.sf2d_mesh_chain(C.byref(mp)))
+
+    def fused_step(self) -> bool:
+        """Whether the solid has towers for the fused time step (its runs use it unless every phase is timed)."""
+        self._need_device()
+        mp = C.c_long(self.mesh_pointer)
+        return bool(self.gpu.sf2d_tower_ready(C.byref(mp)))
 
     def chain_elems(self) -> int:
         """Elements per chain patch of this handle's plan."""
