@@ -924,7 +924,8 @@ void prepare_constants_device_(long* Mesh_pointer, int* h_NGLLX, int* NSPEC_AB, 
   mp->pml = *PML_BOUNDARY_CONDITIONS;
   mp->nstep = *NSTEP;
   if (mp->nspec <= 0 || mp->nglob <= 0) fail("empty mesh (nspec=%d, nglob=%d)", mp->nspec, mp->nglob);
-  // the force kernels address element arrays and fields with 32-bit byte offsets
+  // the force kernels address fields and element arrays of 4 bytes a point with 32-bit byte offsets (wider element arrays
+  // through a base of their own per chain or patch)
   if ((long long)mp->nspec * NGLL2 * 4 >= (1LL << 32) || (long long)mp->nglob * 8 >= (1LL << 32))
     fail("mesh too large for one handle (nspec=%d, nglob=%d): element arrays and fields must stay below 4 GiB",
          mp->nspec, mp->nglob);
@@ -1859,6 +1860,12 @@ extern "C" void sf2d_pml_reset(long* Mesh_pointer) { pml_reset(handle(Mesh_point
 extern "C" int sf2d_mesh_affine_elements(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
   return mp->no_affine ? 0 : mp->n_affine;
+}
+
+// host-only: where the force kernels look for point p of the k-th element of the chain, tower or patch at position `first`
+// in an element array of `bytes` a point: at_element's base and a 32-bit offset
+extern "C" long sf2d_plan_element_byte(int bytes, int first, int k, int p) {
+  return (long)(element_point((unsigned)first) * (size_t)bytes) + (long)((unsigned)bytes * (unsigned)(k * NGLL2 + p));
 }
 
 // whether every patch of the plan for this mesh is a chain of elements (host only)

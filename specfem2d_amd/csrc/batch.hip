@@ -175,8 +175,7 @@ int sf2d_batch_prepare(long* Mesh_pointer, int nshot, const int* src_shot) {
   // the default: with one wave walking a whole patch, the lane-per-shot force kernel has too few waves per SIMD
   // to hide its load latency and runs slower per shot than the patch kernels.
   const bool minor = getenv("SF2D_SHOT_MINOR") && !getenv("SF2D_SHOT_MAJOR") && nshot > 1 && nshot <= 64 &&
-                     (nshot & (nshot - 1)) == 0 && mp->chain && mp->assembly == 0 &&
-                     (size_t)mp->nglob * nshot * 8 < ((size_t)1 << 32);
+                     (nshot & (nshot - 1)) == 0 && mp->chain && mp->assembly == 0 && shot_minor_fits(mp, nshot);
   const long stride = minor ? 1 : ((long)mp->nglob + 63) / 64 * 64;
   const size_t n = minor ? (size_t)2 * mp->nglob * nshot : (size_t)2 * stride * nshot;
   if (n * 3 * sizeof(float) > ((size_t)1 << 38)) fail("sf2d_batch_prepare: %d shots exceed 256 GiB of fields", nshot);

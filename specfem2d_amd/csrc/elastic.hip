@@ -359,8 +359,9 @@ __global__ __launch_bounds__(FORCE_THREADS) void k_elastic_forces_patch(
     const unsigned e = (unsigned)(d.x + min(le, patch_ne(d.w) - 1));
     const unsigned l = e * NGLL2 + p;
     r.slot = ld_off(elem_slot, 2u * l);
-    r.geo = patch_affine(d.w) ? ld_off(geom_elem, 16u * e) : ld_off(geom, 16u * l);
-    r.mod = ld_off(moduli, 8u * l);
+    const unsigned in = l - (unsigned)d.x * NGLL2;  // counted from the patch's first element
+    r.geo = patch_affine(d.w) ? ld_off(geom_elem, 16u * e) : ld_off(at_element(geom, d.x), 16u * in);
+    r.mod = ld_off(at_element(moduli, d.x), 8u * in);
   };
   auto load_halo_id = [&](const int4 d) -> int {
     const int h = min(max(tid - patch_nown(d.w), 0), max(patch_nhalo(d.w) - 1, 0));
@@ -535,6 +536,9 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_chain(
   const bool active = lane / NGLL < ne;
   const int e = d.x + min(k, ne - 1);
   const unsigned l0 = (unsigned)e * NGLL2 + j * NGLL;  // first point of this lane's row
+  const unsigned r0 = l0 - (unsigned)d.x * NGLL2;      // the same from the patch's first element
+  geom = at_element(geom, d.x);
+  moduli = at_element(moduli, d.x);
   int g[NGLL];
   bool first[NGLL];
   float2 u[NGLL], mod[NGLL];
@@ -544,7 +548,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_chain(
     const int id = ld_off(ids, 4u * (l0 + i));
     g[i] = id & ~Mesh::FIRST_TOUCH;
     first[i] = FIRST && (id & Mesh::FIRST_TOUCH);
-    mod[i] = ld_off(moduli, 8u * (l0 + i));
+    mod[i] = ld_off(moduli, 8u * (r0 + i));
   }
   if (RECT || patch_affine(d.w)) {
     const float4 ge = ld_off(geom_elem, 16u * (unsigned)e);
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_chain(
     for (int i = 0; i < NGLL; i++) geo[i] = ge;
   } else {
 #pragma unroll
-    for (int i = 0; i < NGLL; i++) geo[i] = ld_off(geom, 16u * (l0 + i));
+    for (int i = 0; i < NGLL; i++) geo[i] = ld_off(geom, 16u * (r0 + i));
   }
   const bool last = k == ne - 1;
   float2 un[NGLL];  // the displacement of the group's next shot, loaded while the current one is computed
@@ -760,6 +764,9 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
   const int e = d.x + min(k, ne - 1);
   const int row = NGLL * ne;                                   // words per GLL row of the patch in lane order
   const unsigned c0 = (unsigned)d.x * NGLL2 + (unsigned)min(lane, row - 1);  // this lane's word of row 0
+  const unsigned r0 = (unsigned)min(lane, row - 1);            // the same from the patch's first element
+  geom = at_element(geom, d.x);
+  col_mod = at_element(col_mod, d.x);
   int g[NGLL];
   bool first[NGLL];
   float2 u[NGLL], mod[NGLL];
@@ -774,7 +781,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
       g[j] = x == 0 ? r.y : x == 4 * ne ? re[j] : r.x + x;
       const unsigned bits = x < 32 ? ((unsigned)r.z >> x) : ((unsigned)r.w >> (x - 32));
       first[j] = FIRST && (bits & 1u);
-      mod[j] = ld_off(col_mod, 8u * (c0 + (unsigned)(j * row)));
+      mod[j] = ld_off(col_mod, 8u * (r0 + (unsigned)(j * row)));
     }
   } else {
 #pragma unroll
@@ -782,7 +789,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
       const int id = ld_off(col_ids, 4u * (c0 + (unsigned)(j * row)));
       g[j] = id & ~Mesh::FIRST_TOUCH;
       first[j] = FIRST && (id & Mesh::FIRST_TOUCH);
-      mod[j] = ld_off(col_mod, 8u * (c0 + (unsigned)(j * row)));
+      mod[j] = ld_off(col_mod, 8u * (r0 + (unsigned)(j * row)));
     }
   }
   if (RECT || patch_affine(d.w)) {
@@ -791,7 +798,7 @@ __global__ __launch_bounds__(CHAIN_LANES) void k_elastic_forces_col(
     for (int j = 0; j < NGLL; j++) geo[j] = ge;
   } else {
 #pragma unroll
-    for (int j = 0; j < NGLL; j++) geo[j] = ld_off(geom, 16u * ((unsigned)e * NGLL2 + j * NGLL + i));
+    for (int j = 0; j < NGLL; j++) geo[j] = ld_off(geom, 16u * ((unsigned)(e - d.x) * NGLL2 + j * NGLL + i));
   }
   const bool last = k == ne - 1;
   const bool writer = active && (i < NGLL - 1 || last);  // the shared column is written by the next element's lane
@@ -959,7 +966,7 @@ __device__ __forceinline__ void walk_body(
   const int itc = min(item, nitem - 1);
   const int shot = (itc % ngroup) * (1 << lshift) + (lane & ((1 << lshift) - 1));
   const bool live = item < nitem && shot < nshot;
-  // 32-bit element offsets (the launcher checks that points x shots x 8 B stays below 4 GiB)
+  // 32-bit offsets (shot_minor_fits: points x shots x 8 B and element points x 16 B stay below 4 GiB)
   const unsigned sh = (unsigned)min(shot, nshot - 1);
   const unsigned ps = (unsigned)nshot;
   const int4 d = desc[first_patch + itc / ngroup];
@@ -1478,8 +1485,9 @@ void launch_elastic_forces_walk(const Mesh* mp, int first_patch, int npatch, con
                                 int nshot, int first_touch) {
   if (npatch <= 0) return;
   if (!mp->chain) fail("shot-minor batches need chain patches");
-  if ((size_t)mp->nglob * nshot * sizeof(float2) >= ((size_t)1 << 32))
-    fail("shot-minor batch fields of %d points x %d shots exceed the 4 GiB of 32-bit offsets", mp->nglob, nshot);
+  if (!shot_minor_fits(mp, nshot))
+    fail("shot-minor batch of %d points x %d shots, %d elements exceeds the 4 GiB of 32-bit offsets", mp->nglob, nshot,
+         mp->nspec);
   if (first_touch && !mp->first_touch) fail("first-touch assembly is not set up for this handle");
   if (first_patch < 0 || first_patch + npatch > mp->npatch)
     fail("patch range [%d, %d) outside the %d patches", first_patch, first_patch + npatch, mp->npatch);

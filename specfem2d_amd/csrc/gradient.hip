@@ -340,6 +340,7 @@ __global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nstep, long s
   for (int m = 0; m < NGLL; m++) hpi[m] = basis.hp[i * NGLL + m];
   float4 ge = make_float4(0.f, 0.f, 0.f, 0.f);
   if (GEO < 2) ge = geom_elem[e0 + kk];
+  geom = at_element(geom, e0);
   const float4* const el = s_t + NGLL * k;
   float sk[NGLL], sm[NGLL];
   float2 dm[NGLL];
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nstep, long s
         ga.w += u[m].w * h;
       }
       float4 gp = ge;
-      if (GEO == 2) gp = ld_off(geom, 16u * ((unsigned)(e0 + kk) * NGLL2 + (unsigned)(j * NGLL + i)));
+      if (GEO == 2) gp = ld_off(geom, 16u * (unsigned)(kk * NGLL2 + j * NGLL + i));
       const float X = gp.x, Z = GEO ? gp.y : 0.f, G = GEO ? gp.z : 0.f, H = gp.w;
       const float ux = xi.x * X + ga.x * G, uxz = xi.x * Z + ga.x * H, uzx = xi.y * X + ga.y * G, uz = xi.y * Z + ga.y * H;
       const float wx = xi.z * X + ga.z * G, wxz = xi.z * Z + ga.z * H, wzx = xi.w * X + ga.w * G, wz = xi.w * Z + ga.w * H;
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(64) void k_grad_chain(int nchain, int nstep, long s
 #pragma unroll
   for (int j = 0; j < NGLL; j++) {
     float4 gp = ge;
-    if (GEO == 2) gp = ld_off(geom, 16u * ((unsigned)(e0 + kk) * NGLL2 + (unsigned)(j * NGLL + i)));
+    if (GEO == 2) gp = ld_off(geom, 16u * (unsigned)(kk * NGLL2 + j * NGLL + i));
     const float X = gp.x, Z = GEO ? gp.y : 0.f, G = GEO ? gp.z : 0.f, H = gp.w;
     const float wj = basis.w[i] * basis.w[j] / (X * H - G * Z);
     if (active) {

@@ -27,6 +27,13 @@ struct Basis {
   float w[NGLL];     // GLL weights
 };
 
+// the first point of the element at position e in an element array [nspec][25]
+__host__ __device__ inline size_t element_point(unsigned e) { return (size_t)e * NGLL2; }
+template <typename T>
+__host__ __device__ inline T* at_element(T* array, unsigned e) {
+  return array + element_point(e);
+}
+
 struct AcousticState;  // fluid elements (acoustic.hip)
 struct PmlState;       // CPML layer (pml.hip)
 struct TowerState;     // the solid's fused time step (tower.hip)
@@ -231,6 +238,11 @@ struct BatchState {
   int graph_fused = 0;
 };
 
+// whether the lane-per-shot kernels' 32-bit offsets reach everything: fields of nshot values a point, geometry per point
+inline bool shot_minor_fits(const Mesh* mp, int nshot) {
+  const size_t reach = (size_t)1 << 32;
+  return (size_t)mp->nglob * nshot * sizeof(float2) < reach && element_point(mp->nspec) * sizeof(float4) < reach;
+}
 // shot batch fields and the re-arming of its deferred corrector (batch.hip)
 void batch_fields(Mesh* mp, float** d, float** v, float** a, int* nshot, long* stride, int* ps);
 void batch_set_pending(Mesh* mp, float dto2);

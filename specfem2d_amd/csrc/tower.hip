@@ -324,8 +324,14 @@ __global__ __launch_bounds__(64) void k_tower(
   unsigned off0 = point(tb), off1 = point(ts);
   const unsigned offt = point(tt);
   const unsigned up = 8u * (x == 0 || x == xe ? 1u : (unsigned)(xe - 1));
-  unsigned word = (unsigned)td.x * NGLL2 + (unsigned)min(lane, NGLL * ne - 1);
-  unsigned elem = (unsigned)(td.x + kk);
+  // counted from the tower's first element
+  unsigned word = (unsigned)min(lane, NGLL * ne - 1);
+  unsigned elem = (unsigned)kk;
+  mod = at_element(mod, td.x);
+  geom = at_element(geom, td.x);
+  geom_elem += td.x;
+  const unsigned* const att_idx = at_element(att.idx, td.x);
+  float4* const att_state = at_element(reinterpret_cast<float4*>(att.state), td.x);
   const unsigned mrow = (unsigned)(NGLL * ne);
 
   auto load_chain = [&](unsigned o1, bool top, unsigned w, unsigned e, ChainRegs& q) {
@@ -373,7 +379,7 @@ __global__ __launch_bounds__(64) void k_tower(
     float4 st[3];  // attenuation state of the next row
     if (SETS > 0) {
 #pragma unroll
-      for (int s = 0; s < 3; s++) st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + word];
+      for (int s = 0; s < 3; s++) st[s] = att_state[(size_t)s * att.ne + word];
     }
     const unsigned noff = off1 + 4u * up, nword = word + (unsigned)NGLL * mrow, nelem = elem + (unsigned)ne;
     if (c + 1 < nch) load_chain(noff, c + 2 == nch, nword, nelem, nx);
@@ -424,15 +430,15 @@ __global__ __launch_bounds__(64) void k_tower(
         if (j + 1 < NGLL) {
 #pragma unroll
           for (int s = 0; s < 3; s++)
-            st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + la + mrow];
+            st[s] = att_state[(size_t)s * att.ne + la + mrow];
         }
         if (SETS == 2) {
-          const float4* coef = att.table + 3 * (size_t)att.idx[la];
+          const float4* coef = att.table + 3 * (size_t)att_idx[la];
 #pragma unroll
           for (int s = 0; s < 3; s++) cf[s] = coef[s];
         }
         attenuate_point(cf, ev, ov, kap, mu, dux_dxl, dux_dzl, duz_dxl, duz_dzl, sxx, sxz, szz);
-        if (active) att_store(att.state, att.ne, la, ev, ov);
+        if (active) att_store(reinterpret_cast<float*>(att_state), att.ne, la, ev, ov);
       }
       if (RECT) {  // xi_z = gamma_x = 0: J xi_x = 1 / gamma_z, J gamma_z = 1 / xi_x
         const float cx = 1.f / gazl, cz = 1.f / xixl;
@@ -719,7 +725,7 @@ void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, floa
 // chain.  Measured, ms of 300 steps of 600 x 300 elements (15,000 chains) at 1, 2, 4, 8, 16 chains: 12.9, 11.7, 10.7, 12.0,
 // 17.2; 40 steps of 2000 x 1000 (167,000 chains) at 4, 8, 16: 17.1, 16.5, 16.4; 1000 steps of 80 x 60 (420) at 1, 2: 9.9, 11.9.
 int tower_chains(long nchain) {
-  if (const char* env = getenv("SF2D_TOWER_CHAINS")) return std::max(1, atoi(env));
+  if (const char* env = getenv("SF2D_TOWER_CHAINS")) return std::max(1, std::min(4096, atoi(env)));
   return (int)std::max(1L, std::min(16L, (nchain + 4095) / 4096));
 }
 

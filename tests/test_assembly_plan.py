@@ -150,3 +150,17 @@ def test_chain_row_records(nx, expect):
     if expect == 1:
         chains_per_row = -(-nx // 12) if nx >= 12 else 1  # rows narrower than 12 elements: one chain of 10
         assert n == 5 * chains_per_row * cfg.nz
+
+
+def test_element_arrays_beyond_4_gib():
+    """Element arrays of 8 and 16 bytes a point (moduli, geometry per point) pass 4 GiB at 21.5 and 10.7 million elements,
+    which a handle takes (it refuses 4 GiB of an array of 4 bytes a point, 42.9 million): their last points lie where they
+    should."""
+    gpu, _ = driver.load_libraries()
+    f = gpu.sf2d_plan_element_byte
+    f.restype = C.c_long
+    for bytes_, first in ((4, 42949660), (8, 21474836), (8, 21474837), (8, 42949660), (16, 10737418), (16, 10737419),
+                          (16, 42949660)):
+        for k in (0, 1, 11, 16 * 12 - 1):  # a chain, and a tower of 16
+            for p in (0, 24):
+                assert f(bytes_, first, k, p) == bytes_ * ((first + k) * 25 + p)

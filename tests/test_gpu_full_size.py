@@ -10,7 +10,9 @@
   pairing) against the same gradient;
 * the batched 600 x 300-element, 1500-step FWI workload: the gradient of a batch of 4 shots equals the sum of the
   4 single-shot gradients, and central finite differences of the batched misfit along 2 smooth directions agree
-  with it.
+  with it;
+* 4800 x 2300 elements with geometry per point, whose array is longer than 4 GiB: the fused step against the kernel
+  that takes one element at a time.
 
 Every measured error is printed (run pytest with -s to see them).
 """
@@ -220,3 +222,33 @@ def test_c4_batched_misfit_finite_differences(c4):
         worst = max(worst, min(errs))
     b.set_model(base["rho"], base["vp"], base["vs"])
     assert worst < 1e-3
+
+
+# ---------------------------------------------------------------------------------------------------------------
+# element arrays beyond 4 GiB
+def test_geometry_per_point_beyond_4_gib(monkeypatch):
+    """11.04 million elements in two layers of different heights: the last 300,000 hold their geometry beyond 4 GiB (10.74
+    million elements of 400 bytes), where 32-bit offsets would find the lower layer's.  One source among them, one among
+    the first.  60 steps of the same sums in another order, below the bound of every comparison with the oracle."""
+    from specfem2d_amd.config import SimulationConfig
+    from specfem2d_amd.driver import Simulation
+    nx, nz, h = 4800, 2300, 10.0
+    src = [Source(x=x, z=z, f0=40.0, factor=1.0e10, anglesource=30.0)
+           for x, z in ((nx * h - 83.0, -47.0), (92.0, -nz * h + 64.0))]
+    rec = np.array([[s.x + dx, s.z + dz] for s in src for dx, dz in ((12.0, -9.0), (-18.0, -15.0), (0.0, 0.0))])
+    cfg = SimulationConfig(name="large", nx=nx, nz=nz, xmin=0.0, xmax=nx * h, interfaces=[-nz * h, -nz * h / 3, 0.0],
+                           nz_layers=[nz // 2, nz - nz // 2], nstep=60, dt=2.0e-4, rho=2500.0, vp=3000.0, vs=1732.0,
+                           material_mode=0, stacey=True, absorbtop=False, sources=src, receivers=rec)
+    out = []
+    for fused, env in ((True, ("SF2D_NO_AFFINE", "1")), (False, ("SF2D_ASSEMBLY", "colour"))):
+        with monkeypatch.context() as m:
+            m.setenv(*env)
+            sim = Simulation(cfg)
+            assert sim.fused_step() == fused
+            out.append(sim.forward()[0])
+            sim.close()
+        print(f"4800x2300 elements, fused {fused}: ran", flush=True)
+    for k in (slice(0, 3), slice(3, 6)):
+        e = _rel(out[0][k], out[1][k])
+        print(f"4800x2300 elements, geometry per point, fused vs colour assembly: rel-L2 {e:.2e}", flush=True)
+        assert np.abs(out[1][k]).max() > 0 and e < 1e-5
