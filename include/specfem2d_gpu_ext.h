@@ -184,7 +184,7 @@ void sf2d_grad_result(long* Mesh_pointer, double* g_kappa, double* g_mu, double*
 void sf2d_grad_set_model(long* Mesh_pointer, const double* rho, const double* vp, const double* vs, const float* jacobian);
 int sf2d_grad_has_model(long* Mesh_pointer);
 /* d chi / d (rho, vp, vs) [3][nspec][25] (ispec order) and, with parts, d chi / d (kappa, mu, rho through the mass,
-   rho vp, rho vs) [5][nspec][25]; dto2 = dt / 2 */
+   rho vp, rho vs) [5][nspec][25]; dto2 = dt / 2.  Overwrites the segment's state slots. */
 void sf2d_grad_model_result(long* Mesh_pointer, float dto2, double* grad, double* parts);
 /* gradient buffers over the shot batch (sf2d_batch_prepare): the calls above then checkpoint and reverse all
    shots together, residuals are [nstep][nshot][nrec][2] and the results are sums over the shots */

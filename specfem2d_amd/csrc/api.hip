@@ -44,6 +44,15 @@ void check_hip(hipError_t err, const char* what) {
   if (err != hipSuccess) fail("%s: %s", what, hipGetErrorString(err));
 }
 
+size_t spare_memory() {
+  size_t free_bytes = 0, total = 0;
+  check_hip(hipMemGetInfo(&free_bytes, &total), "hipMemGetInfo");
+  const size_t keep = (size_t)64 << 20;
+  size_t spare = free_bytes > keep ? free_bytes - keep : 0;
+  if (const char* env = getenv("SF2D_SPARE_MEMORY")) spare = std::min<size_t>(spare, strtoull(env, nullptr, 10));
+  return spare;
+}
+
 // the z inverse mass for the Newmark kernels: null when it equals the x one at every point (one array read)
 const float* rmass_z(const Mesh* mp) { return mp->same_mass ? nullptr : mp->d_rmassz; }
 

@@ -51,12 +51,12 @@ struct GradState {
   // R~ of the last nrb steps, Rb in a ring of nrb fields; the current step's is in slot rb_at.  npend steps, the first with
   // the forward state in segment slot pend_slot and R~ in ring slot pend_rb, wait for their strain products
   int nrb = 1, rb_at = 0, npend = 0, pend_slot = 0, pend_rb = 0;
-  // the chain rule to (rho, vp, vs): model [3][ne] and Jacobian [ne] in the caller's element order, where each caller
-  // element's accumulators lie, and the result [3 or 8][ne]
-  double *model = nullptr, *out = nullptr;
+  // the chain rule to (rho, vp, vs): model [3][ne] and Jacobian [ne] in the caller's element order, on the device or, where
+  // that has little memory left, on the host
+  double* model = nullptr;
   float* jac = nullptr;
-  int4* where = nullptr;
-  int nout = 0;
+  std::vector<double> h_model;
+  std::vector<float> h_jac;
 };
 
 namespace {
@@ -436,11 +436,13 @@ __global__ __launch_bounds__(GT) void k_flush64(size_t n, float* __restrict__ a3
 }
 
 // The chain rule from the accumulators to (rho, vp, vs) in 64 bits, one thread per element point in the caller's order:
-// mu = rho vs^2, kappa = rho vp^2 - mu, and the mass term M_c(g) = sum w_i w_j J rho.  where[e]: {element position, first
-// accumulator word, words from one j to the next, -}.  out: [3][ne] gradient, then (parts) [5][ne] d chi / d (kappa, mu, rho
-// through the mass, rho vp, rho vs).  Bound by its reads and writes, 100 bytes a point; on the host the same loops, with
-// their arrays, took half of a gradient (400 x 200 elements: 30 of 59 ms).
-__global__ __launch_bounds__(GT) void k_grad_model(long ne, const int4* __restrict__ where, const int* __restrict__ ibool,
+// mu = rho vs^2, kappa = rho vp^2 - mu, and the mass term M_c(g) = sum w_i w_j J rho.  For the ne element points of a range
+// of elements, of which where, jac, model (components mstride apart) and out hold the range alone.  where[e]: {element
+// position, first accumulator word, words from one j to the next, -}.  out: [3][ne] gradient, then (parts) [5][ne]
+// d chi / d (kappa, mu, rho through the mass, rho vp, rho vs).  Bound by its reads and writes, 100 bytes a point; on the host
+// the same loops, with their arrays, took half of a gradient (400 x 200 elements: 30 of 59 ms).
+__global__ __launch_bounds__(GT) void k_grad_model(long ne, long mstride, const int4* __restrict__ where,
+                                                   const int* __restrict__ ibool,
                                                    const double* __restrict__ gk, const double* __restrict__ gm,
                                                    const double* __restrict__ pm, const double* __restrict__ model,
                                                    const float* __restrict__ jac, double* __restrict__ out, int parts,
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(GT) void k_grad_model(long ne, const int4* __restri
   const double a = gk[at], b = gm[at];
   const double w = (double)basis.w[i] * (double)basis.w[j] * (double)jac[l];
   const double r = w * (pm[2 * g] + pm[2 * g + 1]);
-  const double rho = model[l], vp = model[ne + l], vs = model[2 * ne + l];
+  const double rho = model[l], vp = model[mstride + l], vs = model[2 * mstride + l];
   out[l] = a * (vp * vp - vs * vs) + b * vs * vs + r;
   out[ne + l] = a * 2.0 * rho * vp;
   out[2 * ne + l] = -a * 2.0 * rho * vs + b * 2.0 * rho * vs;
@@ -468,8 +470,9 @@ __global__ __launch_bounds__(GT) void k_grad_model(long ne, const int4* __restri
 }
 
 // the Stacey traction's part and its Newmark mass term T_c = dt/2 w [rho_vp (nx+nz) n_c + rho_vs (1 - (nx+nz) n_c)], one
-// thread per face point; ispec_of_pos: the caller's element at each position
-__global__ __launch_bounds__(64) void k_grad_model_stacey(const StaceyFaces F, long ne, const int* __restrict__ ispec_of_pos,
+// thread per face point, of the faces in elements e0 .. e0 + ne / 25 - 1; ispec_of_pos: the caller's element at each position
+__global__ __launch_bounds__(64) void k_grad_model_stacey(const StaceyFaces F, int e0, long ne, long mstride,
+                                                          const int* __restrict__ ispec_of_pos,
                                                           const double* __restrict__ gvp, const double* __restrict__ gvs,
                                                           const double* __restrict__ pm,
                                                           const double* __restrict__ model, double dto2,
@@ -480,12 +483,13 @@ __global__ __launch_bounds__(64) void k_grad_model_stacey(const StaceyFaces F, l
   if (ii < 0 || jj < 0) return;
   const int pos = F.ispec[q / NGLL], p = jj * NGLL + ii;
   const size_t g = (size_t)F.ibool[(size_t)pos * NGLL2 + p];
-  const size_t l = (size_t)ispec_of_pos[pos] * NGLL2 + p;
+  const long l = (long)(ispec_of_pos[pos] - e0) * NGLL2 + p;
+  if (l < 0 || l >= ne) return;
   const double nx = F.normal[2 * q], nz = F.normal[2 * q + 1], w = F.jacw[q];
   const double sn = nx + nz, px = pm[2 * g], pz = pm[2 * g + 1];
   const double a = gvp[q] + w * dto2 * (px * sn * nx + pz * sn * nz);
   const double b = gvs[q] + w * dto2 * (px * (1.0 - sn * nx) + pz * (1.0 - sn * nz));
-  const double rho = model[l], vp = model[ne + l], vs = model[2 * ne + l];
+  const double rho = model[l], vp = model[mstride + l], vs = model[2 * mstride + l];
   // corner elements have two faces, hence atomics; two terms added to a third in either order differ in the last bit
   unsafeAtomicAdd(&out[l], a * vp + b * vs);
   unsafeAtomicAdd(&out[ne + l], a * rho);
@@ -594,8 +598,7 @@ void choose_sweep(Mesh* mp, GradState* G) {
   G->fused = G->ps == 1 && tower_takes(mp, G->nshot) && !mp->pml && !mp->attenuation;
   if (!G->fused || G->rows) return;
   // the boundary terms' field has to fit, and a ring of R~ has to leave most of the memory free: steps to take at once
-  size_t free_bytes = 0, total = 0;
-  check_hip(hipMemGetInfo(&free_bytes, &total), "hipMemGetInfo");
+  const size_t free_bytes = spare_memory();
   const size_t bytes = G->nfield * sizeof(float);
   if (free_bytes < 2 * bytes) {
     G->fused = 0;
@@ -667,8 +670,7 @@ void sf2d_grad_release(long* Mesh_pointer) {
     device_free(*p);
   device_free(G->rows);
   device_free(G->jac);
-  device_free(G->where);
-  for (double** p : {&G->gk, &G->gm, &G->pm, &G->gvp, &G->gvs, &G->model, &G->out}) device_free(*p);
+  for (double** p : {&G->gk, &G->gm, &G->pm, &G->gvp, &G->gvs, &G->model}) device_free(*p);
   delete G;
   mp->grad = nullptr;
   mp->grad_batch = 0;
@@ -903,36 +905,42 @@ void sf2d_grad_result(long* Mesh_pointer, double* gk, double* gm, double* pm, do
 }
 
 // the model of the chain rule, after sf2d_grad_prepare and whenever the model changes: rho, vp, vs and the Jacobian
-// [nspec][25] in ispec order
+// [nspec][25] in ispec order.  It stays on the device where it takes an eighth of the spare memory at most: checkpoints are
+// made to fill the card, and a gradient must not fail at its end.
 void sf2d_grad_set_model(long* Mesh_pointer, const double* rho, const double* vp, const double* vs, const float* jacobian) {
   Mesh* mp = handle(Mesh_pointer);
   GradState* G = need(mp);
+  const double* m[3] = {rho, vp, vs};
+  if (!G->model && spare_memory() / 8 < G->ne * (3 * sizeof(double) + sizeof(float))) {
+    G->h_model.resize(3 * G->ne);
+    for (int k = 0; k < 3; k++) std::copy(m[k], m[k] + G->ne, G->h_model.begin() + k * G->ne);
+    G->h_jac.assign(jacobian, jacobian + G->ne);
+    return;
+  }
   if (!G->model) {
     G->model = device_alloc<double>(3 * G->ne);
     G->jac = device_alloc<float>(G->ne);
   }
-  const double* m[3] = {rho, vp, vs};
   for (int k = 0; k < 3; k++)
     check_hip(hipMemcpyAsync(G->model + k * G->ne, m[k], G->ne * sizeof(double), hipMemcpyHostToDevice, mp->stream),
               "model H2D");
   check_hip(hipMemcpyAsync(G->jac, jacobian, G->ne * sizeof(float), hipMemcpyHostToDevice, mp->stream), "model H2D");
   check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_set_model");
 }
-int sf2d_grad_has_model(long* Mesh_pointer) { return need(handle(Mesh_pointer))->model != nullptr; }
+int sf2d_grad_has_model(long* Mesh_pointer) {
+  const GradState* G = need(handle(Mesh_pointer));
+  return G->model != nullptr || !G->h_model.empty();
+}
 
 // d chi / d (rho, vp, vs) [3][nspec][25] in ispec order and (parts not null) d chi / d (kappa, mu, rho through the mass,
-// rho vp, rho vs) [5][nspec][25]
+// rho vp, rho vs) [5][nspec][25].  Formed in the segment's state slots, which the sweep no longer needs, as many elements at
+// a time as they hold (all of them where a segment has at least seven steps).
 void sf2d_grad_model_result(long* Mesh_pointer, float dto2, double* grad, double* parts) {
   Mesh* mp = handle(Mesh_pointer);
   GradState* G = need(mp);
-  if (!G->model) fail("sf2d_grad_model_result: call sf2d_grad_set_model first");
+  const bool resident = G->model != nullptr;
+  if (!resident && G->h_model.empty()) fail("sf2d_grad_model_result: call sf2d_grad_set_model first");
   const int nout = parts ? 8 : 3;
-  if (nout > G->nout) {
-    check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_model_result");
-    device_free(G->out);
-    G->out = device_alloc<double>(nout * G->ne);
-    G->nout = nout;
-  }
   // where the accumulators lie: element position by position, or in the lane order of the chain at e0
   std::vector<int4> where((size_t)mp->nspec);
   for (int e = 0; e < mp->nspec; e++) {
@@ -944,24 +952,55 @@ void sf2d_grad_model_result(long* Mesh_pointer, float dto2, double* grad, double
       const int e0 = mp->h_patch_desc[4 * q], n = mp->h_patch_desc[4 * q + 3] & 0xf;
       for (int k = 0; k < n; k++) where[mp->ispec_of_pos[e0 + k]] = make_int4(e0 + k, e0 * NGLL2 + NGLL * k, NGLL * n, 0);
     }
-  if (!G->where) G->where = device_alloc<int4>(where.size());
-  check_hip(hipMemcpyAsync(G->where, where.data(), where.size() * sizeof(int4), hipMemcpyHostToDevice, mp->stream), "H2D");
-  hipLaunchKernelGGL(k_grad_model, dim3((unsigned)((G->ne + GT - 1) / GT)), dim3(GT), 0, mp->stream, (long)G->ne, G->where,
-                     mp->d_ibool, G->gk, G->gm, G->pm, G->model, G->jac, G->out, parts ? 1 : 0, mp->basis);
-  check_hip(hipGetLastError(), "k_grad_model launch");
-  if (G->nf) {
-    int* order = device_copy(mp->ispec_of_pos.data(), mp->ispec_of_pos.size());
-    hipLaunchKernelGGL(k_grad_model_stacey, dim3((unsigned)((G->nf + 63) / 64)), dim3(64), 0, mp->stream, stacey_faces(mp),
-                       (long)G->ne, order, G->gvp, G->gvs, G->pm, G->model, (double)dto2, G->out, parts ? 1 : 0);
-    check_hip(hipGetLastError(), "k_grad_model_stacey launch");
-    check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_model_result");
-    device_free(order);
+  // the scratch memory: ispec_of_pos, then of the elements in hand where, (model, Jacobian) and the result
+  const size_t per = sizeof(int4) + NGLL2 * (nout * sizeof(double) + (resident ? 0 : 3 * sizeof(double) + sizeof(float)));
+  const size_t order_bytes = G->nf ? ((size_t)mp->nspec * sizeof(int) + 15) / 16 * 16 : 0;
+  size_t room = 3 * G->nfield * G->chunk * sizeof(float);
+  char* base = reinterpret_cast<char*>(G->seg);
+  char* own = nullptr;
+  const size_t few = order_bytes + per * std::min(mp->nspec, 64);
+  if (room < few) base = own = device_alloc<char>(room = few);  // meshes of a few elements, segments of one step
+  const int most = (int)std::min<size_t>(mp->nspec, (room - order_bytes) / per);
+  auto put = [&](void* dst, const void* src, size_t bytes) {
+    check_hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, mp->stream), "gradient H2D");
+  };
+  int* const order = reinterpret_cast<int*>(base);
+  if (G->nf) put(order, mp->ispec_of_pos.data(), (size_t)mp->nspec * sizeof(int));
+  for (int e0 = 0; e0 < mp->nspec; e0 += most) {
+    const int n = std::min(most, mp->nspec - e0);
+    const size_t np = (size_t)n * NGLL2, l0 = element_point(e0);
+    int4* const at = reinterpret_cast<int4*>(base + order_bytes);
+    double* const out = reinterpret_cast<double*>(at + n);
+    put(at, where.data() + e0, n * sizeof(int4));
+    const double* model = G->model + l0;
+    const float* jac = G->jac + l0;
+    if (!resident) {
+      double* const m = out + nout * np;
+      for (int k = 0; k < 3; k++) put(m + k * np, G->h_model.data() + k * G->ne + l0, np * sizeof(double));
+      put(m + 3 * np, G->h_jac.data() + l0, np * sizeof(float));
+      model = m;
+      jac = reinterpret_cast<const float*>(m + 3 * np);
+    }
+    const long mstride = (long)(resident ? G->ne : np);
+    hipLaunchKernelGGL(k_grad_model, dim3((unsigned)((np + GT - 1) / GT)), dim3(GT), 0, mp->stream, (long)np, mstride, at,
+                       mp->d_ibool, G->gk, G->gm, G->pm, model, jac, out, parts ? 1 : 0, mp->basis);
+    check_hip(hipGetLastError(), "k_grad_model launch");
+    if (G->nf) {
+      hipLaunchKernelGGL(k_grad_model_stacey, dim3((unsigned)((G->nf + 63) / 64)), dim3(64), 0, mp->stream, stacey_faces(mp),
+                         e0, (long)np, mstride, order, G->gvp, G->gvs, G->pm, model, (double)dto2, out, parts ? 1 : 0);
+      check_hip(hipGetLastError(), "k_grad_model_stacey launch");
+    }
+    auto get = [&](double* dst, int c0, int nc) {  // components c0 .. c0 + nc - 1 of the range
+      for (int c = 0; c < nc; c += n == mp->nspec ? nc : 1)
+        check_hip(hipMemcpyAsync(dst + c * G->ne + l0, out + (c0 + c) * np, (n == mp->nspec ? nc : 1) * np * sizeof(double),
+                                 hipMemcpyDeviceToHost, mp->stream),
+                  "gradient D2H");
+    };
+    get(grad, 0, 3);
+    if (parts) get(parts, 3, 5);
   }
-  check_hip(hipMemcpyAsync(grad, G->out, 3 * G->ne * sizeof(double), hipMemcpyDeviceToHost, mp->stream), "gradient D2H");
-  if (parts)
-    check_hip(hipMemcpyAsync(parts, G->out + 3 * G->ne, 5 * G->ne * sizeof(double), hipMemcpyDeviceToHost, mp->stream),
-              "gradient D2H");
   check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_model_result");
+  device_free(own);
 }
 
 // replaces the materials of a prepared handle: kappa, mu, rho vp, rho vs [nspec][25] in ispec order and the

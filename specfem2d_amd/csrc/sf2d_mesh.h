@@ -342,6 +342,10 @@ unsigned int* noalloc_scratch();
 [[noreturn]] void fail(const char* fmt, ...);
 void check_hip(hipError_t err, const char* what);
 
+// Device memory that something with another way to go may take: what is free, less 64 MB for the granularity of the
+// allocations.  SF2D_SPARE_MEMORY (bytes) says that there is less.
+size_t spare_memory();
+
 inline Mesh* handle(long* p) {
   Mesh* mp = reinterpret_cast<Mesh*>(*p);
   if (!mp) fail("invalid Mesh_pointer (not prepared)");
