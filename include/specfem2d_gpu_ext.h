@@ -70,14 +70,15 @@ const float* sf2d_seismograms_read(long* Mesh_pointer, int i_sig, int first, int
 /* The fused time step (forward runs of chain meshes; no counterpart in the reference): corrector of step n and predictor
    of step n + 1 inside the force kernel.
    Solid: sf2d_tower_prepare, after all other preparation (rmassx, rmassz as prepare_fields_elastic_device_ got them),
-   returns 1 when the handle can run it (SF2D_NO_TOWERS: never).  A run of such steps starts after
-   update_displacement_cuda_ (and, with CPML, pml_boundary_elastic_cuda_) of its first step with sf2d_tower_begin;
-   sf2d_tower_step(it) takes the place of the forces, Stacey edges, fluid-solid edges, sources, kernel_3_a_cuda_, the
-   displacement seismograms of receivers in solid elements and, for the next step, update_displacement_cuda_ and
-   pml_boundary_elastic_cuda_.  checkpoint >= 0: the state (d_n, v'_n, r_n) also goes to that gradient checkpoint.  absorb
-   (SAVE_FORWARD; may be null): where the step's Stacey terms [face][5][2] go, consecutive steps one after the other; they
-   are there when the run's last step has returned.  The run's last step (last = 1) ends with the step's displacement, velocity and acceleration instead, and its seismograms
-   are the caller's.
+   returns 1 when the handle can run it (SF2D_NO_TOWERS: never; nor where the spare device memory, SF2D_SPARE_MEMORY bytes
+   at most, does not hold its arrays).  A run of such steps starts after update_displacement_cuda_ (and, with CPML,
+   pml_boundary_elastic_cuda_) of its first step with sf2d_tower_begin; sf2d_tower_step(it) takes the place of the forces,
+   Stacey edges, fluid-solid edges, sources, kernel_3_a_cuda_, the displacement seismograms of receivers in solid elements
+   and, for the next step, update_displacement_cuda_ and pml_boundary_elastic_cuda_.  checkpoint >= 0: the state (d_n, v'_n,
+   r_n) also goes to that gradient checkpoint.  absorb (SAVE_FORWARD; may be null): where the step's Stacey terms
+   [face][5][2] go, consecutive steps one after the other; they are there when the run's last step has returned.  The run's
+   last step (last = 1) ends with the step's displacement, velocity and acceleration instead, and its seismograms are the
+   caller's.
    Fluid: sf2d_tower_fluid_ready is 1 when it can run; sf2d_tower_fluid_step likewise, from the predicted potential (first:
    the run's first step, after acoustic_enforce_free_surf_cuda_) and before the solid's step.  trick: pressure is minus the
    potential; else minus its second derivative, which the next step records. */
@@ -86,11 +87,12 @@ int sf2d_tower_ready(long* Mesh_pointer);
 void sf2d_tower_begin(long* Mesh_pointer);
 void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float* absorb, float deltat,
                      float deltatsqover2, float deltatover2);
-/* SIMULATION_TYPE 3 of solid meshes: sf2d_tower_adjoint_begin after update_displacement_cuda_ of the first fused step,
-   then sf2d_tower_adjoint_step takes the place of the forces, Stacey edges (absorb: the forward run's terms of all steps,
+/* SIMULATION_TYPE 3 of solid meshes: sf2d_tower_adjoint_begin before the run (0: the second field arrays do not fit the
+   spare memory, and the run takes the entry points one by one), then after update_displacement_cuda_ of the first fused
+   step sf2d_tower_adjoint_step takes the place of the forces, Stacey edges (absorb: the forward run's terms of all steps,
    [NSTEP][face][5][2]), adjoint sources, sources, kernel_3_a_cuda_, displacement seismograms, compute_kernels_elastic_cuda_
    and the next step's update_displacement_cuda_, for the adjoint and the reconstructed field; last as above. */
-void sf2d_tower_adjoint_begin(long* Mesh_pointer);
+int sf2d_tower_adjoint_begin(long* Mesh_pointer);
 void sf2d_tower_adjoint_step(long* Mesh_pointer, int it, int last, const float* absorb, float deltat, float deltatsqover2,
                              float deltatover2, float b_deltat, float b_deltatsqover2, float b_deltatover2);
 int sf2d_tower_fluid_ready(long* Mesh_pointer);

@@ -961,7 +961,9 @@ void fluid_towers(Mesh* mp, AcousticState* ac, const IboolView& iv, const std::v
   const std::vector<int>& pml = pml_point_ids(mp, true);
   for (int g : pml) flag[g] |= IF_PML;
   for (int g : pml_edge_points(mp, true)) flag[g] |= IF_PML_EDGE;
-  if (!build_tower_plan(ac->plan, towers, mp->nglob, flag, pml, rank)) return;
+  if (!build_tower_plan(ac->plan, towers, mp->nglob, flag, pml, rank, sizeof(float),
+                        mp->nglob * sizeof(float) + pml.size() * sizeof(float2)))
+    return;
   ac->d_slot = device_alloc<float>(std::max<size_t>(1, (size_t)ac->plan.nslot));
   if (!pml.empty()) ac->d_layer = device_alloc<float2>(pml.size());
   ac->d_acc = device_zeros<float>((size_t)mp->nglob);

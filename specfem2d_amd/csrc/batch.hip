@@ -63,7 +63,7 @@ void batch_step_fields(Mesh* mp, BatchState* B, int it, float deltat, float delt
 }
 
 // whether the batch steps on towers (shot-major fields of a handle that has them)
-bool fused_batch(const Mesh* mp, const BatchState* B) { return B->ps == 1 && tower_takes(mp, B->nshot); }
+bool fused_batch(Mesh* mp, const BatchState* B) { return B->ps == 1 && tower_takes(mp, B->nshot); }
 
 void drop_graph(BatchState* B) {
   if (B->graph_exec) (void)hipGraphExecDestroy(B->graph_exec);
@@ -180,6 +180,7 @@ int sf2d_batch_prepare(long* Mesh_pointer, int nshot, const int* src_shot) {
   const size_t n = minor ? (size_t)2 * mp->nglob * nshot : (size_t)2 * stride * nshot;
   if (n * 3 * sizeof(float) > ((size_t)1 << 38)) fail("sf2d_batch_prepare: %d shots exceed 256 GiB of fields", nshot);
   if (mp->batch) sf2d_batch_release(Mesh_pointer);
+  if (n * 3 * sizeof(float) > spare_memory()) tower_release(mp);  // the fields before a faster step
   BatchState* B = new BatchState();
   B->nshot = nshot;
   B->stride = stride;

@@ -2053,15 +2053,14 @@ int sf2d_sim_adjoint_full(void* sim, const float* adj, const float* absorb, cons
   };
   // solid meshes: after the first step, which ends with the reconstructed fields read from the last forward frames, both
   // fields' fused steps where the handle has them
-  const bool fused = any_el && !any_ac && !att && (s->nrec == 0 || s->p.seismotype == 1) && sf2d_tower_ready(&s->mesh);
+  const bool fused = any_el && !any_ac && !att && (s->nrec == 0 || s->p.seismotype == 1) && sf2d_tower_ready(&s->mesh) &&
+                     sf2d_tower_adjoint_begin(&s->mesh);
   for (int it = 1; it <= nstep; it++) {
     const int it_tmp = nstep - it + 1;
     if (fused && it > 1) {
-      if (it == 2) {
+      if (it == 2)
         update_displacement_cuda_(&s->mesh, &deltat, &deltatsqover2, &deltatover2, &b_deltat, &b_deltatsqover2,
                                   &b_deltatover2);
-        sf2d_tower_adjoint_begin(&s->mesh);
-      }
       sf2d_tower_adjoint_step(&s->mesh, it, it == nstep ? 1 : 0, absorb, deltat, deltatsqover2, deltatover2, b_deltat,
                               b_deltatsqover2, b_deltatover2);
       if (it == nstep && s->nrec > 0)

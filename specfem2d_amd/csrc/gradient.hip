@@ -554,6 +554,8 @@ int grad_prepare(Mesh* mp, long* Mesh_pointer, int chunk, int nrec, int batch) {
   const size_t states = (size_t)std::max(1, G->nckpt) + G->chunk;
   if (states * 3 * G->nfield * sizeof(float) > ((size_t)240 << 30))
     fail("gradient: %zu states of %d shots exceed 240 GiB; use a longer chunk or fewer shots", states, G->nshot);
+  // the states before a faster step
+  if ((states + 1) * 3 * G->nfield * sizeof(float) + (3 * G->ne + 2 * G->n2) * sizeof(double) > spare_memory()) tower_release(mp);
   G->ckpt = device_alloc<float>(3 * G->nfield * std::max(1, G->nckpt));  // written before they are read
   G->seg = device_alloc<float>(3 * G->nfield * G->chunk);
   G->D = device_zeros<float>(G->nfield);

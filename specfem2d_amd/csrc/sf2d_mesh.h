@@ -299,8 +299,8 @@ struct ShotStep {
   float* seismo;
   const int* step;  // (may be null) the 1-based step in device memory, for graph replays
 };
-// whether the handle has towers, and nshot fields' towers, edges and receivers fit one launch
-bool tower_takes(const Mesh* mp, int nshot);
+// whether the handle has towers, nshot fields' towers, edges and receivers fit one launch and their slots the memory
+bool tower_takes(Mesh* mp, int nshot);
 void tower_begin_shots(Mesh* mp, float* accel, long stride, int nshot);
 void tower_step_shots(Mesh* mp, const ShotStep& S, int it, float deltat, float deltatsqover2, float deltatover2);
 // the reverse step of a gradient (gradient.hip): residuals and Stacey terms of the step, D += -K R~, and the next R~

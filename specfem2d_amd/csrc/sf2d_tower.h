@@ -75,8 +75,9 @@ struct TowerPlan {
 // tower meet, the interface points of its left and right column take the two chains' forces in slots of their own (the
 // lower one's are the row's split slots): the interface then sums a point's forces one chain at a time in the order in
 // which a launch per colour adds them.
+// False too when the spare memory does not hold the plan, slot_bytes for each slot and more_bytes.
 bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob, const std::vector<uint8_t>& flag,
-                      const std::vector<int>& pml_ids, const std::vector<int>& rank);
+                      const std::vector<int>& pml_ids, const std::vector<int>& rank, size_t slot_bytes, size_t more_bytes);
 
 constexpr int IF_T = 64;  // threads per workgroup of the interface kernels: one wave, so that few points spread over many CUs
 

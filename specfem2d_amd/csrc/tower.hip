@@ -591,15 +591,20 @@ __global__ __launch_bounds__(256) void k_interface_clear(int n, const int* __res
   if (q < n && (flag[q] & IF_ACC)) accel[ids[q] + blockIdx.y * stride] = make_float2(0.f, 0.f);
 }
 
-// the slots of nshot fields
-float2* tower_slots(TowerState* T, int nshot) {
-  if (nshot > T->slot_shots) {
-    device_free(T->d_slot);
-    T->d_slot = nullptr;
-    T->slot_shots = 0;
-    T->d_slot = device_alloc<float2>(std::max<size_t>(1, (size_t)T->plan.nslot * nshot));
-    T->slot_shots = nshot;
-  }
+// the slots of nshot fields; false (what is there stays) when the spare memory does not hold them
+bool reserve_slots(Mesh* mp, int nshot) {
+  TowerState* T = mp->tower;
+  if (nshot <= T->slot_shots) return true;
+  const size_t n = std::max<size_t>(1, (size_t)T->plan.nslot * nshot);
+  if (n * sizeof(float2) > spare_memory()) return false;
+  batch_drop_graph(mp);  // its launches hold the address
+  device_free(T->d_slot);
+  T->d_slot = device_alloc<float2>(n);
+  T->slot_shots = nshot;
+  return true;
+}
+float2* tower_slots(const TowerState* T, int nshot) {
+  if (nshot > T->slot_shots) fail("fused step of %d fields: slots for %d", nshot, T->slot_shots);
   return T->d_slot;
 }
 
@@ -668,21 +673,25 @@ void clear_interface(Mesh* mp, float2* accel, long stride, int nshot) {
 namespace {
 
 // Stacey terms are kept on the device for as many steps as fit 64 MB and cross to or from the host together: a copy and a
-// synchronisation per step cost more than a step of a small mesh (80 x 32 elements: 100 of 115 us)
+// synchronisation per step cost more than a step of a small mesh (80 x 32 elements: 100 of 115 us).  Less where the spare
+// memory is less than twice that; SF2D_STACEY_STEPS sets the steps.
 size_t store_points(const Mesh* mp) { return (size_t)mp->num_abs * NGLL; }
 void prepare_store(Mesh* mp, int nstep) {
   TowerState* T = mp->tower;
   const size_t step = store_points(mp) * sizeof(float2);
   if (step == 0 || T->d_store) return;
-  T->store_steps = (int)std::max<size_t>(1, std::min<size_t>((size_t)nstep, ((size_t)64 << 20) / step));
+  size_t steps = std::min((size_t)64 << 20, spare_memory() / 2) / step;
+  if (const char* env = getenv("SF2D_STACEY_STEPS")) steps = strtoull(env, nullptr, 10);
+  T->store_steps = (int)std::max<size_t>(1, std::min<size_t>((size_t)nstep, steps));
   T->d_store = device_alloc<float2>(store_points(mp) * T->store_steps);
 }
 
 }  // namespace
 
-bool tower_takes(const Mesh* mp, int nshot) {
+bool tower_takes(Mesh* mp, int nshot) {
   const long per_shot = (mp->tower ? mp->tower->plan.ntower : 0) + (long)mp->num_abs * NGLL / 64 + 1 + mp->nrec_local;
-  return mp->tower && per_shot * nshot + mp->nsources_local < (1L << 25);  // workgroups of 64: below 2^32 threads
+  return mp->tower && per_shot * nshot + mp->nsources_local < (1L << 25) &&  // workgroups of 64: below 2^32 threads
+         reserve_slots(mp, nshot);
 }
 
 // shot batches and gradients: nshot forward fields, shot s at s * stride points
@@ -793,7 +802,7 @@ void TowerPlan::release() {
 }
 
 bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob, const std::vector<uint8_t>& flag,
-                      const std::vector<int>& pml_ids, const std::vector<int>& rank) {
+                      const std::vector<int>& pml_ids, const std::vector<int>& rank, size_t slot_bytes, size_t more_bytes) {
   P.release();
   const int nt = (int)towers.size();
   std::vector<int4> desc((size_t)4 * nt);
@@ -873,6 +882,12 @@ bool build_tower_plan(TowerPlan& P, const std::vector<Tower>& towers, int nglob,
       row[nr++] = make_int4((int)(unsigned)(m & 0xffffffffull), (int)(unsigned)(m >> 32), first, second);
     }
   P.nslot = ns;
+  const size_t point_bytes = sizeof(int) + 2 * sizeof(int2) + sizeof(uint8_t);
+  if (desc.size() * sizeof(int4) + row.size() * sizeof(int4) + (size_t)P.n * point_bytes +
+          (size_t)(P.n - P.n4) * sizeof(int4) + (size_t)ns * slot_bytes + more_bytes > spare_memory()) {
+    P.release();
+    return false;
+  }
   std::vector<int2> s01((size_t)P.n), s23((size_t)(P.n - P.n2));
   for (int q = 0; q < P.n; q++) {
     const Share* s = &share[(size_t)4 * q];
@@ -997,13 +1012,15 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     if (rmassx[g] != rmassz[g]) flag[dev(g)] |= IF_LOOKED_AT;
   for (int g = mp->nglob_el; g < ng; g++) flag[g] = 0;  // no solid element has these
   TowerState* T = new TowerState();
-  if (!build_tower_plan(T->plan, towers, ng, flag, pml, rank)) {
+  const int nshot = mp->batch && mp->batch->ps == 1 ? mp->batch->nshot : 1;
+  if (!build_tower_plan(T->plan, towers, ng, flag, pml, rank, nshot * sizeof(float2), pml.size() * sizeof(float2))) {
     delete T;
     return 0;
   }
   if (!pml.empty()) T->d_layer = device_alloc<float2>(pml.size());
   mp->tower = T;
-  return 1;
+  if (!reserve_slots(mp, nshot)) tower_release(mp);
+  return mp->tower != nullptr;
 }
 
 int sf2d_tower_ready(long* Mesh_pointer) { return handle(Mesh_pointer)->tower != nullptr; }
@@ -1046,16 +1063,20 @@ void sf2d_tower_step(long* Mesh_pointer, int it, int last, int checkpoint, float
   if (last) mp->accel_partial = 0;
 }
 
-void sf2d_tower_adjoint_begin(long* Mesh_pointer) {
+int sf2d_tower_adjoint_begin(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
   TowerState* T = mp->tower;
   if (!T || mp->simulation_type != 3) fail("sf2d_tower_adjoint_begin: no towers, or not SIMULATION_TYPE = 3");
+  const size_t field = (size_t)mp->nglob * sizeof(float2), slots = (size_t)T->plan.nslot * 2 * sizeof(float2);
+  if (!T->d_acc[1] && 4 * field + slots > spare_memory()) return 0;
+  if (!reserve_slots(mp, 2)) return 0;
   for (int s = 0; s < 2; s++) {
     if (!T->d_other[s]) T->d_other[s] = device_alloc<float>((size_t)2 * mp->nglob);
     if (!T->d_acc[s]) T->d_acc[s] = device_zeros<float2>((size_t)mp->nglob);
   }
   if (mp->stacey) prepare_store(mp, mp->nstep);
   T->store_first = -1;
+  return 1;
 }
 
 void sf2d_tower_adjoint_step(long* Mesh_pointer, int it, int last, const float* absorb, float deltat,

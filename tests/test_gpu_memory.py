@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import test_gpu_tower as towers
 from specfem2d_amd import config
 from specfem2d_amd.config import Source
 from specfem2d_amd.driver import ShotBatch, Simulation
@@ -79,3 +80,74 @@ def test_gradient_formed_in_pieces(nx, nz, spare, monkeypatch):
     got, _, _ = gradient(nx, nz, 1, 1, None if spare is None else lambda sim: spare, monkeypatch)
     for a, b in zip(got, want):
         assert np.linalg.norm(b) > 0 and rel(a, b) < 1e-5
+
+
+def fluid_ready(sim):
+    return sim.gpu.sf2d_tower_fluid_ready(C.byref(C.c_long(sim.mesh_pointer)))
+
+
+@pytest.mark.parametrize("form", ["stacey", "coupled_cpml", "fluid_cpml"])
+def test_no_towers_on_a_full_card(form, monkeypatch):
+    """A handle made with nothing to spare steps phase by phase, as with SF2D_NO_TOWERS: the same bits where no atomics meet."""
+    cfg = towers.make(form, 25, 17)
+    out = []
+    for env in (("SF2D_SPARE_MEMORY", "0"), ("SF2D_NO_TOWERS", "1")):
+        with monkeypatch.context() as m:
+            m.setenv(*env)
+            sim = Simulation(cfg)
+            seis = sim.forward()[0]
+            assert not fluid_ready(sim) and (form == "fluid_cpml" or not sim.fused_step())
+            sim.close()
+        out.append(seis)
+    assert np.linalg.norm(out[1]) > 0 and rel(*out) < (1e-5 if form == "coupled_cpml" else 1e-12)
+
+
+def test_states_before_towers(monkeypatch):
+    """A gradient whose states need what the towers hold gives these up."""
+    sim, obs = make(25, 17, 1)
+    assert sim.fused_step()
+    chi, seis = sim.gradient_forward(obs, chunk=40)
+    want = sim.gradient_backward()
+    sim.close()
+    sim, obs = make(25, 17, 1)
+    monkeypatch.setenv("SF2D_SPARE_MEMORY", "0")
+    chi0, seis0 = sim.gradient_forward(obs, chunk=40)
+    assert not sim.fused_step()
+    got = sim.gradient_backward()
+    sim.close()
+    assert abs(chi0 - chi) < 1e-5 * chi and rel(seis0, seis) < 1e-5
+    for k in want:
+        assert rel(got[k], want[k]) < 1e-5
+
+
+def test_adjoint_run_on_a_full_card(monkeypatch):
+    """No room for the second field arrays: the run takes the entry points one by one, as with SF2D_NO_TOWERS."""
+    cfg = towers.make("stacey", 25, 17)
+    sim = Simulation(cfg, save_forward=True)
+    seis, _, store = sim.forward(save_stacey=True)
+    last = sim.fields()
+    sim.close()
+
+    def adjoint(env=None):
+        with monkeypatch.context() as m:
+            back = Simulation(cfg, simulation_type=3)
+            assert back.fused_step()
+            if env:
+                m.setenv(*env)
+            before = free_bytes()
+            adj, kernels = back.adjoint(seis[..., ::-1], store, last)
+            taken = before - free_bytes()
+            back.close()
+        return [adj, *(kernels.values() if isinstance(kernels, dict) else kernels)], taken
+
+    fused, _ = adjoint()
+    plain, taken = adjoint(("SF2D_SPARE_MEMORY", "0"))
+    assert taken <= 0
+    with monkeypatch.context() as m:
+        m.setenv("SF2D_NO_TOWERS", "1")
+        back = Simulation(cfg, simulation_type=3)
+        adj, kernels = back.adjoint(seis[..., ::-1], store, last)
+        back.close()
+    ref = [adj, *(kernels.values() if isinstance(kernels, dict) else kernels)]
+    for a, b, c in zip(plain, ref, fused):
+        assert np.linalg.norm(b) > 0 and rel(a, b) <= max(1e-6, 10 * rel(c, b))
