@@ -37,9 +37,9 @@ int sf2d_plan_validate(int nspec, int nglob, const int* ibool_1based, int np, co
 /* host only: the byte at which the force kernels look for GLL point p (0..24) of the k-th element of a chain, tower or patch
    whose first element lies at position `first`, in an element array of `bytes` bytes a point */
 long sf2d_plan_element_byte(int bytes, int first, int k, int p);
-/* 1 when every patch of the coloured-patch plan for this mesh is a chain (element k's right edge is element
-   k+1's left edge, no other point shared inside the patch): such meshes use the row-lane force kernel.
-   Host only, same arguments as sf2d_plan_validate; first_writes (if not NULL) receives the number of element
+/* 1 when the elements of this mesh, consecutive ones or put into rows along shared edges, form chains (element k's right
+   edge is element k+1's left edge, no other point shared inside the chain): such meshes use the chain kernels and towers.
+   Host only, same arguments as sf2d_plan_validate, chosen as a handle chooses; first_writes (if not NULL) receives the number of element
    points whose update is the first of its point in a step (first-touch assembly: nglob when every point has
    exactly one, 0 when the plan cannot use it). */
 int sf2d_plan_chains(int nspec, int nglob, const int* ibool_1based, int np, const int* phase_lists,

@@ -523,6 +523,15 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
   return true;
 }
 
+// the chain plan that a handle of the mesh takes: chains of up to max_elems consecutive elements, of up to PATCH_ELEMS, or of
+// elements put into rows; false (P unusable) when the elements form none of them
+bool choose_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np, int max_elems,
+                       Plan& P, const std::vector<int>& fluid = {}) {
+  return build_chain_plan(ibool, nspec, nglob, phase_lists, np, max_elems, P, false, fluid) ||
+         build_chain_plan(ibool, nspec, nglob, phase_lists, np, Mesh::PATCH_ELEMS, P, false, fluid) ||
+         build_chain_plan(ibool, nspec, nglob, phase_lists, np, max_elems, P, true, fluid);
+}
+
 }  // namespace
 
 // point numbering of a mesh of fluid elements alone (`elems`) for towers; empty when the patches are not chains
@@ -667,9 +676,7 @@ void sort_elements_by_colour(Mesh* mp, const int* phase_lists, int np) {
   if (const char* env = getenv("SF2D_SHOTS_PER_WAVE")) mp->shots_per_wave = std::max(1, atoi(env));
   Plan P;
   const std::vector<int> fluid = acoustic_elements(mp);
-  if (!try_chain || (!build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, false, fluid) &&
-                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, Mesh::PATCH_ELEMS, P, false, fluid) &&
-                     !build_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, true, fluid))) {
+  if (!try_chain || !choose_chain_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->chain_elems, P, fluid)) {
     if (try_chain && mp->attenuation) mp->assembly = 2;  // the memory variables ride in the chain kernel only
     P = build_plan(mp->h_ibool, nspec, mp->nglob, phase_lists, np, mp->assembly);
   }
@@ -1877,14 +1884,12 @@ extern "C" long sf2d_plan_element_byte(int bytes, int first, int k, int p) {
   return (long)(element_point((unsigned)first) * (size_t)bytes) + (long)((unsigned)bytes * (unsigned)(k * NGLL2 + p));
 }
 
-// whether every patch of the plan for this mesh is a chain of elements (host only)
+// whether the elements of this mesh form a chain plan (host only; chains of up to CHAIN_ELEMS elements)
 extern "C" int sf2d_plan_chains(int nspec, int nglob, const int* ibool_1based, int np, const int* phase_lists,
                                 int* first_writes) {
   std::vector<int> ib = to_zero_based(ibool_1based, (size_t)nspec * NGLL2, 1, nglob, "ibool");
-  Plan P;  // as the device plan is chosen
-  if (!build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P) &&
-      !build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))
-    P = Plan();
+  Plan P;
+  if (!choose_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P)) P = Plan();
   if (first_writes) {
     *first_writes = 0;
     for (uint8_t f : P.first) *first_writes += f;
@@ -1897,10 +1902,8 @@ extern "C" int sf2d_plan_chains(int nspec, int nglob, const int* ibool_1based, i
 extern "C" int sf2d_plan_row_records(int nspec, int nglob, const int* ibool_1based, int np, const int* phase_lists,
                                      int* nrecords) {
   std::vector<int> ib = to_zero_based(ibool_1based, (size_t)nspec * NGLL2, 1, nglob, "ibool");
-  Plan P;  // as the device plan is chosen
-  if (!build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P) &&
-      !build_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::PATCH_ELEMS, P))
-    return -1;
+  Plan P;
+  if (!choose_chain_plan(ib, nspec, nglob, phase_lists, np, Mesh::CHAIN_ELEMS, P)) return -1;
   std::vector<int> ids((size_t)nspec * NGLL2);
   for (int pos = 0; pos < nspec; pos++)
     for (int p = 0; p < NGLL2; p++) ids[(size_t)pos * NGLL2 + p] = P.newid[ib[(size_t)P.order[pos] * NGLL2 + p]];

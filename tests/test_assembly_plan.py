@@ -100,12 +100,11 @@ def chains(ibool, nglob, lists, first=None):
     return rc
 
 
-@pytest.mark.parametrize("nx,expect", [(80, 1), (12, 1), (13, 1), (10, 1), (8, 0), (1, 0)])
+@pytest.mark.parametrize("nx,expect", [(80, 1), (12, 1), (13, 1), (10, 1), (8, 1), (4, 1), (3, 0), (1, 0)])
 def test_chain_patches_on_structured_meshes(nx, expect):
-    """Rows of at least ten elements split into strips that are chains (the row-lane force kernel applies);
-    narrower meshes make patches that wrap into the next row (a 2-D block) and fall back to the general
-    patch kernel.  The chain property itself is re-derived here from ibool: along a strip of consecutive
-    elements of one row, element k's points (4, j) are element k+1's points (0, j)."""
+    """Rows of elements split into strips that are chains, whether they are listed row by row or in any order; meshes
+    narrower than four elements fall back to the general patch kernel.  The chain property itself is re-derived here from
+    ibool: along a strip of consecutive elements of one row, element k's points (4, j) are element k+1's points (0, j)."""
     cfg = config.small_test_mesh(nx=nx, nz=4, nstep=2)
     o = OracleSim(cfg, "sp")
     ib = o.ibool()
@@ -118,11 +117,13 @@ def test_chain_patches_on_structured_meshes(nx, expect):
         left, right = e[:, 1:].reshape(-1), e[:, :-1].reshape(-1)
         b = ib.reshape(-1, 5, 5)
         np.testing.assert_array_equal(b[right][:, :, 4], b[left][:, :, 0])
-    # a shuffled element list breaks the strips
+    # a shuffled element list is put into rows again
     rng = np.random.default_rng(3)
     lists = inner_only(o.nspec)
     lists[1] = rng.permutation(lists[1])
-    assert chains(ib, o.nglob, lists) == 0
+    first = []
+    assert chains(ib, o.nglob, lists, first) == expect
+    assert first[0] == (o.nglob if expect else 0)
 
 
 def row_records(ibool, nglob, lists):
@@ -137,19 +138,22 @@ def row_records(ibool, nglob, lists):
     return rc, n.value
 
 
-@pytest.mark.parametrize("nx,expect", [(80, 1), (12, 1), (13, 1), (10, 1), (8, -1)])
-def test_chain_row_records(nx, expect):
+@pytest.mark.parametrize("nx,expect", [(80, 1), (12, 1), (13, 1), (10, 1), (8, 1), (4, 1), (3, -1)])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_chain_row_records(nx, expect, shuffled):
     """The column-lane kernel's point ids as one record per chain row: in the plan's numbering every GLL row of a
     chain is numbered consecutively (column x > 0 at base + x), so {base, id of column 0, first-touch mask} per row
     reproduces the id and first-touch flag of every writing lane (checked point by point on the host); meshes whose
     patches are not chains have no records."""
     cfg = config.small_test_mesh(nx=nx, nz=4, nstep=2)
     o = OracleSim(cfg, "sp")
-    rc, n = row_records(o.ibool(), o.nglob, inner_only(o.nspec))
+    lists = inner_only(o.nspec)
+    if shuffled:
+        lists[1] = np.random.default_rng(3).permutation(lists[1])
+    rc, n = row_records(o.ibool(), o.nglob, lists)
     assert rc == expect
     if expect == 1:
-        chains_per_row = -(-nx // 12) if nx >= 12 else 1  # rows narrower than 12 elements: one chain of 10
-        assert n == 5 * chains_per_row * cfg.nz
+        assert n == 5 * -(-nx // 12) * cfg.nz
 
 
 def test_element_arrays_beyond_4_gib():
