@@ -437,9 +437,9 @@ void number_points(const std::vector<int>& ibool, const ChainSet& S, std::vector
 }
 
 // The plan of a mesh whose patches are all chains (mode 0 with patches of up to max_elems elements), for the chain
-// kernels: false, and P unusable, when some patch is not one.  The colours are build_plan's; elements and points are
-// numbered for towers (number_points), after those points the ones of the elements `fluid` in the same way.  No slots,
-// halos or owned ranges: those serve the general patch kernel.
+// kernels: false, and P unusable, when some patch is not one or more than MAX_COLOURS of them meet.  The colours are
+// build_plan's; elements and points are numbered for towers (number_points), after those points the ones of the elements
+// `fluid` in the same way.  No slots, halos or owned ranges: those serve the general patch kernel.
 bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const int* phase_lists, int np,
                       int max_elems, Plan& P, bool rows = false, const std::vector<int>& fluid = {}) {
   P = Plan();
@@ -477,7 +477,7 @@ bool build_chain_plan(const std::vector<int>& ibool, int nspec, int nglob, const
       uint32_t forbidden = 0;
       for (int k = 0; k < ch[q].ne; k++)
         for (int p = 0; p < NGLL2; p++) forbidden |= used[ibool[(size_t)elems[ph][ch[q].k0 + k] * NGLL2 + p]];
-      if (forbidden == 0xffffffffu) fail("patch colouring needs more than %d colours", Mesh::MAX_COLOURS);
+      if (forbidden == 0xffffffffu) return false;
       int c = 0;
       while (forbidden & (1u << c)) c++;
       col[q - q0] = c;

@@ -7,12 +7,17 @@ permutation in which every patch owns one contiguous id range (ranges disjoint) 
 points owned by other patches as its halo.  On structured meshes a 10-element strip owns its upper four
 GLL rows (160 points) and reads 45 halo points (the row below and the column to its left)."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 from oracle.oracle import OracleSim
 from specfem2d_amd import config, driver
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def validate(ibool, nglob, lists, mode):
@@ -154,6 +159,36 @@ def test_chain_row_records(nx, expect, shuffled):
     assert rc == expect
     if expect == 1:
         assert n == 5 * -(-nx // 12) * cfg.nz
+
+
+ROWS = """
+import sys
+import numpy as np
+from tests.test_assembly_plan import chains, inner_only, validate
+rows, long = {rows}, 12
+# rows of twelve elements without neighbours above or below, but every two rows share one point of their top edges
+g = np.arange(rows * 5 * (4 * long + 1), dtype=np.int64).reshape(rows, 5, 4 * long + 1)
+for a in range(rows):
+    for b in range(a):
+        g[a, 4, b + 1] = g[b, 4, a + 1]
+ib = np.zeros((rows, long, 5, 5), np.int64)
+for k in range(long):
+    ib[:, k] = g[:, :, 4 * k:4 * k + 5]
+_, ib = np.unique(ib, return_inverse=True)
+ib = ib.reshape(rows, long, 25) + 1
+ib = np.ascontiguousarray(ib.transpose(1, 0, 2)).reshape(rows * long, 25).astype(np.int32)  # column by column
+lists = inner_only(rows * long)
+assert validate(ib, ib.max(), lists, 0)[0] == 0, "the general patches"
+print("chains", chains(ib, int(ib.max()), lists), flush=True)
+"""
+
+
+@pytest.mark.parametrize("rows,expect", [(32, 1), (33, 0), (46, 0)])
+def test_rows_that_need_too_many_colours_are_no_chains(rows, expect):
+    """Rows can meet in more points than patches do: where 32 colours do not keep them apart, the mesh keeps the general
+    patches (in a process of its own, which an error ends)."""
+    out = subprocess.run([sys.executable, "-c", ROWS.format(rows=rows)], capture_output=True, text=True, cwd=ROOT)
+    assert out.returncode == 0 and f"chains {expect}" in out.stdout, out.stdout + out.stderr
 
 
 def test_element_arrays_beyond_4_gib():
