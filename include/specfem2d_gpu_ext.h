@@ -100,7 +100,7 @@ void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int 
                            float deltatover2);
 /* tuning knobs (specfem2d_amd/autotune.py picks them by timing): elements per chain patch, chosen at set-up
    from SF2D_CHAIN_ELEMS (1..12, default 12), and shots per wave of the batched chain kernel (0 = default 8;
-   SF2D_SHOTS_PER_WAVE at set-up) */
+   SF2D_SHOTS_PER_WAVE at set-up; the fused step does not read it) */
 int sf2d_mesh_chain_elems(long* Mesh_pointer);
 void sf2d_mesh_set_shots_per_wave(long* Mesh_pointer, int shots);
 /* Elements per chain patch (1..12; 0 = the default 12) of the handle's element plan: call between

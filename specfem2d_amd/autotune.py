@@ -1,12 +1,13 @@
-"""Autotuner for the force kernel's launch shape: elements per chain patch and shots per wave.
+"""Autotuner for the launch shape of a time step: elements per chain patch and shots per wave.
 
-The patch plan of a mesh (``sf2d_mesh_set_chain_elems``, elements per chain patch, 1..12) fixes how many element rows
-one wave of the chain kernel holds and how many waves a colour launch has; the shots per wave of a batched
-launch (``sf2d_mesh_set_shots_per_wave``) trade element-data reuse against waves in flight.  Which pair is
+The patch plan of a mesh (``sf2d_mesh_set_chain_elems``, elements per chain patch, 1..12) fixes how many elements one
+wave of the fused step or of the chain kernel holds and how many waves there are; the shots per wave of a batch that
+steps phase by phase (``sf2d_mesh_set_shots_per_wave``) trade element-data reuse against waves in flight.  Which is
 fastest depends on the mesh size, the number of shots and the device, so it is measured: every candidate runs
 a short forward (``steps`` time steps from rest) on the workload's own mesh, model and shots, and the fastest
-device time wins.  The colour schedule itself is the plan's greedy colouring (four colours on the structured
-meshes), in launch order.
+device time wins.  The fused step takes one shot per wave and does not read the second knob: a chain length is timed once
+there, for all its candidates, and the choice leaves the knob at 0, its default.  The height of the towers is the
+library's own rule and is not tuned.
 
 ``tune(cfg, shots)`` returns the choice and the table; ``settings(choice)`` gives it as the ``chain_elems`` and
 ``shots_per_wave`` arguments of the handle it is for (``Simulation`` / ``ShotBatch``): per handle, nothing
@@ -36,27 +37,33 @@ def tune(cfg: SimulationConfig, shots: Optional[Sequence[list]] = None, steps: i
          chain_elems: Iterable[int] = CHAIN_ELEMS, shots_per_wave: Iterable[int] = SHOTS_PER_WAVE) -> Dict:
     """Time a ``steps``-step forward for every (elements per chain patch, shots per wave) candidate on this
     workload (a ShotBatch of ``shots`` when given, else a single simulation) and return
-    ``{"chain_elems", "shots_per_wave", "ms_per_step", "table"}``; ``table`` lists every candidate."""
+    ``{"chain_elems", "shots_per_wave", "ms_per_step", "table"}``; ``table`` lists every candidate.  A batch on the fused
+    step does not read the shots per wave: one time for all, and 0 as the choice."""
     small = cfg.replace(nstep=steps)
     batch = shots is not None
     groups: List[int] = sorted({min(g, len(shots)) for g in shots_per_wave}) if batch else [0]
-    table = []
+    table, unread = [], {}
     for n in chain_elems:
         sim = ShotBatch(small, shots, chain_elems=n) if batch else Simulation(small, chain_elems=n)
         try:
             if not sim.chain_kernel():
                 continue  # the mesh's patches are not chains: nothing to tune
+            read = batch and (sim.shot_minor() or not sim.fused_step())
+            unread[sim.chain_elems()] = not read
             for g in groups:
-                if batch:
-                    sim.set_shots_per_wave(g)
-                _forward_ms(sim, steps, batch)  # warm-up
-                ms = _forward_ms(sim, steps, batch)
+                if read or g == groups[0]:
+                    if read:
+                        sim.set_shots_per_wave(g)
+                    _forward_ms(sim, steps, batch)  # warm-up
+                    ms = _forward_ms(sim, steps, batch)
                 table.append({"chain_elems": sim.chain_elems(), "shots_per_wave": g, "ms_per_step": ms / steps})
         finally:
             sim.close()
     if not table:
         return {"chain_elems": None, "shots_per_wave": None, "ms_per_step": None, "table": []}
     best = min(table, key=lambda r: r["ms_per_step"])
+    if unread[best["chain_elems"]]:
+        best = dict(best, shots_per_wave=0)
     return dict(best, table=table)
 
 

@@ -223,6 +223,21 @@ def test_autotuner_picks_a_candidate_and_keeps_the_results(case, monkeypatch):
     assert _rel(out[0], out[1]) < 2e-6
 
 
+@pytest.mark.parametrize("fused", [True, False])
+def test_autotuner_times_only_what_is_read(case, fused, monkeypatch):
+    """The fused step does not read the shots per wave: one time per chain length, and the knob at its default."""
+    from specfem2d_amd import autotune
+    cfg, shots = case
+    if not fused:
+        monkeypatch.setenv("SF2D_NO_TOWERS", "1")
+    timed = []
+    forward = autotune._forward_ms
+    monkeypatch.setattr(autotune, "_forward_ms", lambda *a: timed.append(1) or forward(*a))
+    choice = autotune.tune(cfg, shots, steps=10, chain_elems=(4, 12), shots_per_wave=(1, 4))
+    assert len(timed) == (4 if fused else 8) and len(choice["table"]) == 4
+    assert (choice["shots_per_wave"] == 0) if fused else (choice["shots_per_wave"] in (1, 4))
+
+
 def test_graph_replayed_steps_match_launched_steps(case, observed, monkeypatch):
     """With SF2D_BATCH_GRAPH, every batch step after the first of a run is one replay of a captured HIP graph
     (the step index read from device memory); it gives the same seismograms as launching every kernel, and so
