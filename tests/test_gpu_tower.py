@@ -2,13 +2,15 @@
 at the shapes where it can go wrong: towers of one chain and of a whole column, chain remainders (a mesh width that is
 not a multiple of 12 elements), a single row of elements, the three geometry forms, one and several attenuation
 coefficient sets, and every kind of interface point (Stacey edges, sources, receivers, CPML, fluid-solid edges)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle.oracle import OracleSim
 from specfem2d_amd import config
 from specfem2d_amd.config import Source
-from specfem2d_amd.driver import ShotBatch, Simulation
+from specfem2d_amd.driver import ShotBatch, Simulation, UnevenBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -42,8 +44,18 @@ def make(form, nx, nz, nstep=160):
     return cfg
 
 
-def run(cfg, pieces=None):
+def check_route(sim, fused):
+    """The solid and the fluid of a handle, where it has them, step on towers or do not."""
+    mp = C.byref(C.c_long(sim.mesh_pointer))
+    if sim.nspec_acoustic < sim.nspec:
+        assert sim.fused_step() == fused
+    if sim.nspec_acoustic:
+        assert bool(sim.gpu.sf2d_tower_fluid_ready(mp)) == fused
+
+
+def run(cfg, pieces=None, fused=True):
     sim = Simulation(cfg)
+    check_route(sim, fused)
     seis = np.concatenate([sim.forward(nstep=n)[0] for n in (pieces or [cfg.nstep])], axis=-1)
     out = [seis]
     if sim.nspec_acoustic < cfg.nx * sum(cfg.nz_layers):
@@ -74,7 +86,7 @@ def test_fused_step_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
     monkeypatch.setenv("SF2D_TOWER_CHAINS", str(chains))
     fused = run(cfg)
     monkeypatch.setenv("SF2D_NO_TOWERS", "1")
-    plain = run(cfg)
+    plain = run(cfg, fused=False)
     bounds = [3e-5] + BOUNDS[1:] if cfg.seismotype == 4 and not cfg.use_trick else BOUNDS
     for a, b, tol in zip(fused, plain, bounds):
         assert np.linalg.norm(b) > 0 and rel(a, b) < tol
@@ -129,9 +141,11 @@ def test_fused_reverse_sweep_matches_the_unfused_one(form, nx, nz, chains, shots
             monkeypatch.setenv("SF2D_NO_TOWERS", "1")
         sim = Simulation(cfg) if shots == 1 else ShotBatch(cfg, more)
         obs = np.zeros((cfg.nrec, 2, cfg.nstep) if shots == 1 else (shots, cfg.nrec, 2, cfg.nstep))
+        check_route(sim, towers)
         for chunk in (64, 160):
             chi, seis = sim.gradient_forward(obs, chunk=chunk)
             out.append([np.array([chi]), seis, *sim.gradient_backward().values()])
+            assert sim.gpu.sf2d_grad_fused(C.byref(C.c_long(sim.mesh_pointer))) == towers
         if shots == 1:  # both sweeps leave the fields after the first segment
             out[-1] += list(sim.fields())
         sim.close()
@@ -140,20 +154,25 @@ def test_fused_reverse_sweep_matches_the_unfused_one(form, nx, nz, chains, shots
             assert np.linalg.norm(b) > 0 and rel(a, b) < tol
 
 
-@pytest.mark.parametrize("form", ["stacey", "points"])
-@pytest.mark.parametrize("nx,nz,chains", [(12, 12, 1), (25, 17, 3), (13, 2, 64)])
-def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, monkeypatch):
-    """A SAVE_FORWARD run (its Stacey terms) and the SIMULATION_TYPE 3 run with its kernels.  The reconstruction runs
-    backwards in time on rounded fields: what a change of 1e-7 in the stored terms and the adjoint traces does to the
-    unfused run is the measure, ten times that the bound."""
+@pytest.mark.parametrize("form,nx,nz,chains,block", [
+    *[(f, *s, 0) for f in ("stacey", "points") for s in ((12, 12, 1), (25, 17, 3), (13, 2, 64))], ("layers", 25, 17, 3, 0),
+    ("stacey", 25, 17, 3, 7), ("layers", 12, 12, 1, 1), ("stacey", 12, 12, 1, 159)])
+def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, block, monkeypatch):
+    """A SAVE_FORWARD run (its Stacey terms) and the SIMULATION_TYPE 3 run with its kernels, the terms in one block of all
+    160 steps and in blocks that do and do not divide them.  The reconstruction runs backwards in time on rounded fields:
+    what a change of 1e-7 in the stored terms and the adjoint traces does to the unfused run is the measure, ten times that
+    the bound."""
     if form == "points":
         monkeypatch.setenv("SF2D_NO_AFFINE", "1")
-    cfg = make("stacey", nx, nz)
+    if block:
+        monkeypatch.setenv("SF2D_STACEY_STEPS", str(block))
+    cfg = make("stacey" if form == "points" else form, nx, nz)
     rng = np.random.default_rng(1)
     monkeypatch.setenv("SF2D_TOWER_CHAINS", str(chains))
 
-    def adjoint(traces, store, last):
+    def adjoint(traces, store, last, fused):
         back = Simulation(cfg, simulation_type=3)
+        check_route(back, fused)
         out = back.adjoint(traces, store, last)
         back.close()
         return [out[0], *out[1].values()] if isinstance(out[1], dict) else [out[0], *out[1]]
@@ -163,18 +182,38 @@ def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, monkeyp
         if not towers:
             monkeypatch.setenv("SF2D_NO_TOWERS", "1")
         sim = Simulation(cfg, save_forward=True)
+        check_route(sim, towers)
         parts = [sim.forward(nstep=n, save_stacey=True) for n in (70, cfg.nstep - 70)]
         seis = np.concatenate([p[0] for p in parts], axis=-1)
         store = np.concatenate([p[2] for p in parts])
         last = sim.fields()
         sim.close()
-        runs.append((seis, store, last, adjoint(seis[..., ::-1], store, last)))
+        runs.append((seis, store, last, adjoint(seis[..., ::-1], store, last, towers)))
     (seis, store, last, fused), (seis0, store0, last0, plain) = runs
     assert rel(seis, seis0) < 1e-5 and rel(store, store0) < 1e-4
     noise = lambda a: a * (1 + 1e-7 * rng.choice([-1.0, 1.0], np.shape(a)))
-    moved = adjoint(noise(seis0[..., ::-1]), noise(store0).astype(np.float32), [noise(x).astype(np.float32) for x in last0])
+    moved = adjoint(noise(seis0[..., ::-1]), noise(store0).astype(np.float32), [noise(x).astype(np.float32) for x in last0],
+                    False)
     for a, b, c in zip(fused, plain, moved):
         assert np.linalg.norm(b) > 0 and rel(a, b) < 10 * max(rel(c, b), 1e-6)
+
+
+def test_a_union_in_pieces_and_after_a_reset():
+    """A union of a solid and two fluids, of which the fluids step on a stream of their own: forked from the handle's and
+    joined again in each piece of a run.  A missing wait would leave whole samples out; the order of atomics is 5e-6."""
+    cfgs = [make("visco_cpml", 25, 17).replace(dt=2.0e-3), make("fluid", 19, 14), make("fluid_cpml", 26, 12)]
+    cfgs = [c.replace(seismotype=1, use_trick=True) for c in cfgs]
+    u = UnevenBatch(cfgs)
+    check_route(u, True)
+    runs = []
+    for pieces in ([160], [1, 2, 57, 100], [1] * 20 + [140], [160]):
+        u.reset()
+        seis = np.concatenate([Simulation.forward(u, nstep=n)[0] for n in pieces], axis=-1)
+        runs.append([seis, *u.fields(), *u.acoustic_fields()])
+    u.close()
+    for other in runs[1:]:
+        for a, b, tol in zip(other, runs[0], BOUNDS):
+            assert np.linalg.norm(b) > 0 and rel(a, b) < min(tol, 5e-6)
 
 
 def blocks(nx, nz, h=100.0):
@@ -206,6 +245,7 @@ def test_elements_in_any_order_form_rows(nx, nz, rows, external):
         cfg = cfg.replace(mesh=blocks(nx, nz))
     sim = Simulation(cfg)
     assert sim.chain_kernel() == bool(rows)
+    check_route(sim, bool(rows))
     seis = sim.forward()[0]
     sim.close()
     assert rel(seis, OracleSim(cfg, "sp").forward()) < 1e-5
