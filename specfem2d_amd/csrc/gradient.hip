@@ -632,6 +632,22 @@ void choose_sweep(Mesh* mp, GradState* G) {
   G->acc = device_zeros<float>(G->nfield);
 }
 
+// where each caller element's accumulators lie: {element position, first word, words from one j to the next, -}, element
+// position by position or, in a fused sweep, in the lane order of the chain at e0
+std::vector<int4> accumulator_places(const Mesh* mp, const GradState* G) {
+  std::vector<int4> where((size_t)mp->nspec);
+  for (int e = 0; e < mp->nspec; e++) {
+    const int pos = mp->pos_of_ispec[e];
+    where[e] = make_int4(pos, pos * NGLL2, NGLL, 0);
+  }
+  if (G->fused)
+    for (int q = 0; q < mp->npatch; q++) {
+      const int e0 = mp->h_patch_desc[4 * q], n = mp->h_patch_desc[4 * q + 3] & 0xf;
+      for (int k = 0; k < n; k++) where[mp->ispec_of_pos[e0 + k]] = make_int4(e0 + k, e0 * NGLL2 + NGLL * k, NGLL * n, 0);
+    }
+  return where;
+}
+
 }  // namespace
 
 float* grad_checkpoint_inputs(Mesh* mp, int slot) {
@@ -866,31 +882,12 @@ void sf2d_grad_result(long* Mesh_pointer, double* gk, double* gm, double* pm, do
   GradState* G = need(mp);
   check_hip(hipStreamSynchronize(mp->stream), "sf2d_grad_result");
   std::vector<double> t(std::max(G->ne, G->n2));
-  std::vector<int> first, count;
-  if (G->fused) {
-    first.assign(mp->nspec, 0);
-    count.assign(mp->nspec, 1);
-    for (int q = 0; q < mp->npatch; q++) {
-      const int e0 = mp->h_patch_desc[4 * q], ne = mp->h_patch_desc[4 * q + 3] & 0xf;
-      for (int k = 0; k < ne; k++) {
-        first[e0 + k] = e0;
-        count[e0 + k] = ne;
-      }
-    }
-  }
+  const std::vector<int4> where = accumulator_places(mp, G);
   auto elem = [&](const double* dev, double* out) {
     check_hip(hipMemcpy(t.data(), dev, G->ne * sizeof(double), hipMemcpyDeviceToHost), "gradient D2H");
-    for (int e = 0; e < mp->nspec; e++) {
-      const int pos = mp->pos_of_ispec[e];
-      if (G->fused) {  // lane order of the chain at e0
-        const int e0 = first[pos], ne = count[pos];
-        for (int p = 0; p < NGLL2; p++)
-          out[(size_t)e * NGLL2 + p] =
-              t[(size_t)e0 * NGLL2 + (size_t)(p / NGLL) * NGLL * ne + NGLL * (pos - e0) + p % NGLL];
-        continue;
-      }
-      for (int p = 0; p < NGLL2; p++) out[(size_t)e * NGLL2 + p] = t[(size_t)pos * NGLL2 + p];
-    }
+    for (int e = 0; e < mp->nspec; e++)
+      for (int p = 0; p < NGLL2; p++)
+        out[(size_t)e * NGLL2 + p] = t[(size_t)where[e].y + (size_t)(p / NGLL) * where[e].z + p % NGLL];
   };
   elem(G->gk, gk);
   elem(G->gm, gm);
@@ -943,17 +940,7 @@ void sf2d_grad_model_result(long* Mesh_pointer, float dto2, double* grad, double
   const bool resident = G->model != nullptr;
   if (!resident && G->h_model.empty()) fail("sf2d_grad_model_result: call sf2d_grad_set_model first");
   const int nout = parts ? 8 : 3;
-  // where the accumulators lie: element position by position, or in the lane order of the chain at e0
-  std::vector<int4> where((size_t)mp->nspec);
-  for (int e = 0; e < mp->nspec; e++) {
-    const int pos = mp->pos_of_ispec[e];
-    where[e] = make_int4(pos, pos * NGLL2, NGLL, 0);
-  }
-  if (G->fused)
-    for (int q = 0; q < mp->npatch; q++) {
-      const int e0 = mp->h_patch_desc[4 * q], n = mp->h_patch_desc[4 * q + 3] & 0xf;
-      for (int k = 0; k < n; k++) where[mp->ispec_of_pos[e0 + k]] = make_int4(e0 + k, e0 * NGLL2 + NGLL * k, NGLL * n, 0);
-    }
+  const std::vector<int4> where = accumulator_places(mp, G);
   // the scratch memory: ispec_of_pos, then of the elements in hand where, (model, Jacobian) and the result
   const size_t per = sizeof(int4) + NGLL2 * (nout * sizeof(double) + (resident ? 0 : 3 * sizeof(double) + sizeof(float)));
   const size_t order_bytes = G->nf ? ((size_t)mp->nspec * sizeof(int) + 15) / 16 * 16 : 0;

@@ -144,3 +144,32 @@ def test_reference_adjoint_kernels_match_the_gradient(case, gpu_grad):
         err = _rel(ker[name], ours)
         print(f"SIMULATION_TYPE=3 K_{name} vs exact gradient: rel L2 {err:.2e}")
         assert err < 1e-3, (name, err)
+
+
+@pytest.mark.parametrize("towers", [True, False])
+def test_accumulators_are_the_parts_of_the_gradient(towers, monkeypatch):
+    """sf2d_grad_result, the accumulators themselves (in a fused sweep they lie in the lane order of the chains): kappa and mu
+    are the gradient's parts, and the derivative with respect to the mass gives the mass part, w_i w_j J times its two
+    components."""
+    import ctypes as C
+
+    from specfem2d_amd.driver import Simulation
+    if not towers:
+        monkeypatch.setenv("SF2D_NO_TOWERS", "1")
+    cfg = config.small_test_mesh(nx=25, nz=17, nstep=160, gll=True, seed=3)
+    sim = Simulation(cfg)
+    sim.gradient_forward(np.zeros((cfg.nrec, 2, cfg.nstep)), chunk=50)
+    _, parts = sim.gradient_backward(parts=True)
+    mp = C.byref(C.c_long(sim.mesh_pointer))
+    assert sim.gpu.sf2d_grad_fused(mp) == towers
+    out = [np.zeros((sim.nspec, 25)), np.zeros((sim.nspec, 25)), np.zeros((sim.nglob, 2)),
+           *(np.zeros((max(1, sim.nabs), 5)) for _ in range(2))]
+    sim.gpu.sf2d_grad_result(mp, *(a.ctypes.data_as(C.c_void_p) for a in out))
+    w = np.array([0.1, 49 / 90, 32 / 45, 49 / 90, 0.1])
+    mass = (w[:, None] * w[None, :]).reshape(1, 25) * out[2].sum(1)[sim.ibool().reshape(-1, 25) - 1]
+    sim.close()
+    assert np.abs(out[0]).max() > 0 and np.array_equal(out[0], parts["kappa"])
+    assert np.array_equal(out[1], parts["mu"])
+    used = np.abs(mass) > 1e-6 * np.abs(mass).max()
+    jac = parts["rho_mass"][used] / mass[used]
+    assert np.ptp(jac) < 1e-6 * jac.mean()  # equal rectangles, weights and Jacobians in 32 bits
