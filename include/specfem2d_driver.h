@@ -132,7 +132,9 @@ void sf2d_sim_get_stacey(void* sim, int* ispec, int* ij, float* normal, float* j
    the traction of a solid face, the potential term of a fluid face in component 0).  If timing is not NULL, HIP
    events on the library stream give {loop ms, predictor ms, forces ms, boundary+sources ms, corrector ms, seismogram
    ms}: the loop and the element-force launches always (the latter measured in the first 4 steps and every 16th, and
-   scaled to all), the other phases, in every step, only when timing[0] < 0 on entry.  Returns 0 on success. */
+   scaled to all: an estimate; of fused steps the solid's launches, boundary terms and Newmark updates among them, or the
+   fluid's where there is no solid, so that a fluid beside a solid is left out), the other phases, in every step, only when
+   timing[0] < 0 on entry.  Returns 0 on success. */
 int sf2d_sim_forward(void* sim, int nstep_run, double* seis, float* absorb, double* timing);
 /* Adjoint run (SIMULATION_TYPE=3, simulation created with simulation_type 3): adj[nrec][2][NSTEP]
    adjoint source traces (x then z), absorb[NSTEP][nabs][5][2] and the last frame from a save_forward

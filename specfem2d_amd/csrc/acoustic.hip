@@ -632,8 +632,7 @@ __global__ __launch_bounds__(64) void k_ac_tower(int ntower, const int4* __restr
       ms[j] = rm[g];
     }
     const unsigned ng = g1 + 4u * up;
-    const unsigned cword = word, celem = elem;
-    (void)celem;
+    const unsigned cword = word;
     word += (unsigned)NGLL * mrow;
     elem += (unsigned)ne;
     if (c + 1 < nch) load_chain(ng, c + 2 == nch, word, elem);
@@ -1843,8 +1842,9 @@ void sf2d_tower_fluid_step(long* Mesh_pointer, int it, int first, int last, int 
   if (it < 1 || it > mp->nstep) fail("sf2d_tower_fluid_step: it=%d outside 1..%d", it, mp->nstep);
   // Without fluid-solid edges the fluid's steps depend on nothing of the solid's: they run beside them, on a stream that
   // waits for the run's preparation and that the handle's stream waits for at its end.  A step's kernels of 10 to 20 us
-  // leave much of the card idle (an uneven batch of 8
-  // with solids and fluids, 366 steps: 27.0 ms on one stream, 21.4 on two).
+  // leave much of the card idle (an uneven batch of 8 with solids and fluids, 366 steps: 27.0 ms on one stream; on two 21.4
+  // where the runtime gives these a hardware queue each, and up to 25.5 where they share one, which it decides by how many
+  // streams the process has made before).
   hipStream_t const own = mp->stream;
   const bool apart = mp->nspec_elastic > 0 && ac->ncoup == 0;
   if (apart) {
