@@ -41,6 +41,7 @@ struct TowerState {
   float2* d_acc[2] = {nullptr, nullptr};
   float2* d_slot = nullptr;  // [slot_shots][plan.nslot] forces of interface points
   int slot_shots = 0;
+  int geo = 0;               // k_tower's GEO
 };
 
 namespace {
@@ -278,14 +279,16 @@ struct ChainRegs {
   float4 ge;
 };
 
-// GEO: 0 every element a rectangle {xi_x, gamma_z}, 1 every element affine (one record), 2 geometry per point
+// GEO: 0 every element a rectangle {xi_x, gamma_z}, 1 every element affine (one record), 2 geometry per point; 3 and 4 are 1
+// and 2 with offsets that count from the tower's first element, for element arrays that pass 4 GiB (tower_geometry: a base
+// of the tower's own costs scalar registers that the kernel has too few of already, 1 to 2.5 percent of a small mesh's step)
 template <int GEO, int SETS, class Fields, class Edges>
 __global__ __launch_bounds__(64) void k_tower(
     int ntower, const int4* __restrict__ desc, const int4* __restrict__ rows, const float4* __restrict__ geom,
     const float4* __restrict__ geom_elem, const float2* __restrict__ mod, const Fields F,
     const float* __restrict__ rm, float2* __restrict__ slot, int nslot, const Newmark nm, const Basis basis,
     const TowerAtt att, int tower_wgs, const Edges edges) {
-  constexpr bool RECT = GEO == 0;
+  constexpr bool RECT = GEO == 0, WIDE = GEO >= 3, PER_POINT = GEO == 2 || GEO == 4;
   __shared__ float2 s_t[NGLL * TROW + 1];
   if ((int)blockIdx.x >= tower_wgs) {
     tower_edges(edges, F, blockIdx.x - tower_wgs);
@@ -324,14 +327,15 @@ __global__ __launch_bounds__(64) void k_tower(
   unsigned off0 = point(tb), off1 = point(ts);
   const unsigned offt = point(tt);
   const unsigned up = 8u * (x == 0 || x == xe ? 1u : (unsigned)(xe - 1));
-  // counted from the tower's first element
-  unsigned word = (unsigned)min(lane, NGLL * ne - 1);
-  unsigned elem = (unsigned)kk;
-  mod = at_element(mod, td.x);
-  geom = at_element(geom, td.x);
-  geom_elem += td.x;
-  const unsigned* const att_idx = at_element(att.idx, td.x);
-  float4* const att_state = at_element(reinterpret_cast<float4*>(att.state), td.x);
+  const unsigned first = WIDE ? 0u : (unsigned)td.x;
+  const unsigned att0 = WIDE ? (unsigned)td.x * NGLL2 : 0u;  // indices, not bytes: within 32 bits
+  unsigned word = first * NGLL2 + (unsigned)min(lane, NGLL * ne - 1);
+  unsigned elem = first + (unsigned)kk;
+  if (WIDE) {
+    mod = at_element(mod, td.x);
+    geom = at_element(geom, td.x);
+    geom_elem += td.x;
+  }
   const unsigned mrow = (unsigned)(NGLL * ne);
 
   auto load_chain = [&](unsigned o1, bool top, unsigned w, unsigned e, ChainRegs& q) {
@@ -340,7 +344,7 @@ __global__ __launch_bounds__(64) void k_tower(
     q.d[NGLL - 2] = ld_off(d, top ? offt : o1 + (unsigned)(NGLL - 2) * up);
 #pragma unroll
     for (int j = 0; j < NGLL; j++) q.mod[j] = ld_off(mod, 8u * (w + (unsigned)j * mrow));
-    if (GEO < 2) q.ge = ld_off(geom_elem, 16u * e);
+    if (!PER_POINT) q.ge = ld_off(geom_elem, 16u * e);
   };
   // the update of one row's point, or its share of an interface point
   auto finish = [&](const int4 r, unsigned o, float2 f, float2 u, const typename Fields::Row& vp, float m) {
@@ -379,7 +383,7 @@ __global__ __launch_bounds__(64) void k_tower(
     float4 st[3];  // attenuation state of the next row
     if (SETS > 0) {
 #pragma unroll
-      for (int s = 0; s < 3; s++) st[s] = att_state[(size_t)s * att.ne + word];
+      for (int s = 0; s < 3; s++) st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + (att0 + word)];
     }
     const unsigned noff = off1 + 4u * up, nword = word + (unsigned)NGLL * mrow, nelem = elem + (unsigned)ne;
     if (c + 1 < nch) load_chain(noff, c + 2 == nch, nword, nelem, nx);
@@ -413,7 +417,7 @@ __global__ __launch_bounds__(64) void k_tower(
       const float kap = q.mod[j].x, mu = q.mod[j].y;
       const float lambdal = kap - mu, lp2m = kap + mu;
       float4 gp = q.ge;
-      if (GEO == 2) gp = ld_off(geom, 16u * (elem * NGLL2 + (unsigned)(j * NGLL + i)));
+      if (PER_POINT) gp = ld_off(geom, 16u * (elem * NGLL2 + (unsigned)(j * NGLL + i)));
       const float xixl = gp.x, xizl = RECT ? 0.f : gp.y, gaxl = RECT ? 0.f : gp.z, gazl = gp.w;
       const float dux_dxl = RECT ? dux_dxi * xixl : dux_dxi * xixl + dux_dga * gaxl;
       const float dux_dzl = RECT ? dux_dga * gazl : dux_dxi * xizl + dux_dga * gazl;
@@ -424,21 +428,21 @@ __global__ __launch_bounds__(64) void k_tower(
       float szz = fmaf(lambdal, dux_dxl, lp2m * duz_dzl);
       float sxz = mu * (RECT && SETS == 0 ? fmaf(duz_dxi, xixl, dux_dzl) : duz_dxl + dux_dzl);
       if (SETS > 0) {
-        const unsigned la = word + (unsigned)j * mrow;
+        const unsigned la = att0 + word + (unsigned)j * mrow;
         float ev[9] = {st[0].x, st[0].y, st[0].z, st[0].w, st[1].x, st[1].y, st[1].z, st[1].w, st[2].x};
         float ov[3] = {st[2].y, st[2].z, st[2].w};
         if (j + 1 < NGLL) {
 #pragma unroll
           for (int s = 0; s < 3; s++)
-            st[s] = att_state[(size_t)s * att.ne + la + mrow];
+            st[s] = reinterpret_cast<const float4*>(att.state)[(size_t)s * att.ne + la + mrow];
         }
         if (SETS == 2) {
-          const float4* coef = att.table + 3 * (size_t)att_idx[la];
+          const float4* coef = att.table + 3 * (size_t)att.idx[la];
 #pragma unroll
           for (int s = 0; s < 3; s++) cf[s] = coef[s];
         }
         attenuate_point(cf, ev, ov, kap, mu, dux_dxl, dux_dzl, duz_dxl, duz_dzl, sxx, sxz, szz);
-        if (active) att_store(reinterpret_cast<float*>(att_state), att.ne, la, ev, ov);
+        if (active) att_store(att.state, att.ne, la, ev, ov);
       }
       if (RECT) {  // xi_z = gamma_x = 0: J xi_x = 1 / gamma_z, J gamma_z = 1 / xi_x
         const float cx = 1.f / gazl, cz = 1.f / xixl;
@@ -608,8 +612,14 @@ float2* tower_slots(const TowerState* T, int nshot) {
   return T->d_slot;
 }
 
+// The kernel's GEO: offsets from the start of the element arrays where these stay below 4 GiB, 21.4 million elements of
+// moduli and 10.7 of geometry per point (SF2D_WIDE_OFFSETS: from the tower on any mesh)
 int tower_geometry(const Mesh* mp) {
-  return mp->rect ? 0 : (!mp->no_affine && mp->n_affine == mp->nspec) ? 1 : 2;
+  const bool affine = !mp->no_affine && mp->n_affine == mp->nspec;
+  const size_t bytes = element_point(mp->nspec) * (affine ? sizeof(float2) : sizeof(float4));
+  const bool wide = bytes >= ((size_t)1 << 32) || getenv("SF2D_WIDE_OFFSETS");
+  if (affine) return wide ? 3 : mp->rect ? 0 : 1;
+  return wide ? 4 : 2;
 }
 
 template <class Fields, class Edges, class Kernel>
@@ -648,9 +658,9 @@ void launch_tower(Mesh* mp, const TowerFields& F, int it, float* seismo, long se
   using K = decltype(&k_tower<0, 0, TowerFields, TowerEdges>);
 #define SF2D_SETS(g) {k_tower<g, 0, TowerFields, TowerEdges>, k_tower<g, 1, TowerFields, TowerEdges>, \
                       k_tower<g, 2, TowerFields, TowerEdges>}
-  const K kern[3][3] = {SF2D_SETS(0), SF2D_SETS(1), SF2D_SETS(2)};
+  const K kern[5][3] = {SF2D_SETS(0), SF2D_SETS(1), SF2D_SETS(2), SF2D_SETS(3), SF2D_SETS(4)};
 #undef SF2D_SETS
-  launch_k_tower(mp, kern[tower_geometry(mp)][sets], F, E, slot, nm);
+  launch_k_tower(mp, kern[mp->tower->geo][sets], F, E, slot, nm);
   if (forward) pml_elastic_slots(mp, mp->tower->d_layer);
   if (P.n == 0) return;
   hipLaunchKernelGGL(k_interface, dim3((P.n + IF_T - 1) / IF_T, F.nshot), dim3(IF_T), 0, mp->stream, interface_args(P), slot,
@@ -720,9 +730,10 @@ void tower_step_adjoint(Mesh* mp, const float* Rb, float* Rb_out, float* D, floa
   E.gvp = gvp;
   E.gvs = gvs;
   using K = decltype(&k_tower<0, 0, AdjointFields, AdjointEdges>);
-  const K kern[3] = {k_tower<0, 0, AdjointFields, AdjointEdges>, k_tower<1, 0, AdjointFields, AdjointEdges>,
-                     k_tower<2, 0, AdjointFields, AdjointEdges>};
-  launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, nm);
+  const K kern[5] = {k_tower<0, 0, AdjointFields, AdjointEdges>, k_tower<1, 0, AdjointFields, AdjointEdges>,
+                     k_tower<2, 0, AdjointFields, AdjointEdges>, k_tower<3, 0, AdjointFields, AdjointEdges>,
+                     k_tower<4, 0, AdjointFields, AdjointEdges>};
+  launch_k_tower(mp, kern[mp->tower->geo], F, E, slot, nm);
   if (P.n == 0) return;
   hipLaunchKernelGGL(k_interface_adjoint, dim3((P.n + IF_T - 1) / IF_T, nshot), dim3(IF_T), 0, mp->stream, interface_args(P),
                      slot, P.nslot, F, mp->d_rmassx, mp->d_rmassz, nm);
@@ -1018,6 +1029,7 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     return 0;
   }
   if (!pml.empty()) T->d_layer = device_alloc<float2>(pml.size());
+  T->geo = tower_geometry(mp);
   mp->tower = T;
   if (!reserve_slots(mp, nshot)) tower_release(mp);
   return mp->tower != nullptr;
@@ -1119,9 +1131,10 @@ void sf2d_tower_adjoint_step(long* Mesh_pointer, int it, int last, const float* 
   if (E.nreceiver > 0 && it > mp->nlength_seismogram) fail("sf2d_tower_adjoint_step: step %d after the last sample", it);
   float2* const slot = tower_slots(T, 2);
   using K = decltype(&k_tower<0, 0, PairFields, PairEdges>);
-  const K kern[3] = {k_tower<0, 0, PairFields, PairEdges>, k_tower<1, 0, PairFields, PairEdges>,
-                      k_tower<2, 0, PairFields, PairEdges>};
-  launch_k_tower(mp, kern[tower_geometry(mp)], F, E, slot, F.nm0);
+  const K kern[5] = {k_tower<0, 0, PairFields, PairEdges>, k_tower<1, 0, PairFields, PairEdges>,
+                     k_tower<2, 0, PairFields, PairEdges>, k_tower<3, 0, PairFields, PairEdges>,
+                     k_tower<4, 0, PairFields, PairEdges>};
+  launch_k_tower(mp, kern[mp->tower->geo], F, E, slot, F.nm0);
   if (P.n > 0) {
     hipLaunchKernelGGL(k_interface_pair, dim3((P.n + IF_T - 1) / IF_T, 2), dim3(IF_T), 0, mp->stream, interface_args(P), slot,
                        P.nslot, F, mp->d_rmassx, mp->d_rmassz);

@@ -198,6 +198,39 @@ def test_fused_adjoint_run_matches_the_unfused_one(form, nx, nz, chains, block, 
         assert np.linalg.norm(b) > 0 and rel(a, b) < 10 * max(rel(c, b), 1e-6)
 
 
+@pytest.mark.parametrize("form", ["stacey", "layers", "points", "visco", "visco_sets", "cpml"])
+def test_offsets_that_count_from_the_tower(form, monkeypatch):
+    """The kernels for element arrays beyond 4 GiB, on a small mesh: the bits of the others (affine kernels on both sides) in a
+    run; atomics meet in gradients and adjoint runs, whose bounds are those of a run repeated."""
+    monkeypatch.setenv("SF2D_NO_RECT", "1")
+    monkeypatch.setenv("SF2D_TOWER_CHAINS", "3")
+    if form == "points":
+        monkeypatch.setenv("SF2D_NO_AFFINE", "1")
+    cfg = make("stacey" if form == "points" else form, 25, 17)
+    out = []
+    for wide in (False, True):
+        if wide:
+            monkeypatch.setenv("SF2D_WIDE_OFFSETS", "1")
+        exact, close = run(cfg), []
+        if form in ("stacey", "layers", "points"):
+            sim = Simulation(cfg)
+            sim.gradient_forward(np.zeros((cfg.nrec, 2, cfg.nstep)), chunk=40)
+            close += sim.gradient_backward().values()
+            sim.close()
+            sim = Simulation(cfg, save_forward=True)
+            seis, _, store = sim.forward(save_stacey=True)
+            back = Simulation(cfg, simulation_type=3)
+            adj, kernels = back.adjoint(seis[..., ::-1], store, sim.fields())
+            close += [adj, *kernels.values()]
+            back.close()
+            sim.close()
+        out.append((exact, close))
+    for a, b in zip(out[1][0], out[0][0]):
+        assert np.linalg.norm(b) > 0 and np.array_equal(a, b)
+    for a, b in zip(out[1][1], out[0][1]):
+        assert np.linalg.norm(b) > 0 and rel(a, b) < 1e-5
+
+
 def test_a_union_in_pieces_and_after_a_reset():
     """A union of a solid and two fluids, of which the fluids step on a stream of their own: forked from the handle's and
     joined again in each piece of a run.  A missing wait would leave whole samples out; the order of atomics is 5e-6."""
