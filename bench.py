@@ -342,6 +342,7 @@ def c2_elastic(steps: int, warmup: int):
     fk_ms = timing["forces_ms"] / steps / launches
     fk_bytes = force_kernel_bytes(nspec, nglob) / launches
     achieved = fk_bytes / (fk_ms * 1e-3) / 1e9
+    traffic = read_traffic(name, fused)
     roofline = {
         "bound": "hbm",
         "kernel": "k_tower + k_interface (forces and Newmark updates)" if fused else
@@ -354,7 +355,10 @@ def c2_elastic(steps: int, warmup: int):
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": achieved / HBM_PEAK_GBS,
-        "traffic": read_traffic(name, fused),
+        # the bytes that rocprofv3 counted (profiles/), and the share of the peak at which they moved: of a fused step, whose
+        # formula above prices the forces of the phase-by-phase step, the one that tells how busy the memory is
+        "traffic": traffic,
+        "traffic_frac": traffic / (fk_ms * 1e-3) / 1e9 / HBM_PEAK_GBS if traffic else None,
         "algorithmic_bytes_per_launch": fk_bytes,
         "avg_launch_ms": fk_ms,
         # the bytes this kernel's own representation needs at minimum: affine elements carry one 16-byte
