@@ -1023,7 +1023,7 @@ int sf2d_tower_prepare(long* Mesh_pointer, const float* rmassx, const float* rma
     if (rmassx[g] != rmassz[g]) flag[dev(g)] |= IF_LOOKED_AT;
   for (int g = mp->nglob_el; g < ng; g++) flag[g] = 0;  // no solid element has these
   TowerState* T = new TowerState();
-  const int nshot = mp->batch && mp->batch->ps == 1 ? mp->batch->nshot : 1;
+  const int nshot = mp->simulation_type == 3 ? 2 : mp->batch && mp->batch->ps == 1 ? mp->batch->nshot : 1;
   if (!build_tower_plan(T->plan, towers, ng, flag, pml, rank, nshot * sizeof(float2), pml.size() * sizeof(float2))) {
     delete T;
     return 0;
@@ -1079,9 +1079,7 @@ int sf2d_tower_adjoint_begin(long* Mesh_pointer) {
   Mesh* mp = handle(Mesh_pointer);
   TowerState* T = mp->tower;
   if (!T || mp->simulation_type != 3) fail("sf2d_tower_adjoint_begin: no towers, or not SIMULATION_TYPE = 3");
-  const size_t field = (size_t)mp->nglob * sizeof(float2), slots = (size_t)T->plan.nslot * 2 * sizeof(float2);
-  if (!T->d_acc[1] && 4 * field + slots > spare_memory()) return 0;
-  if (!reserve_slots(mp, 2)) return 0;
+  if (!T->d_acc[1] && 4 * (size_t)mp->nglob * sizeof(float2) > spare_memory()) return 0;
   for (int s = 0; s < 2; s++) {
     if (!T->d_other[s]) T->d_other[s] = device_alloc<float>((size_t)2 * mp->nglob);
     if (!T->d_acc[s]) T->d_acc[s] = device_zeros<float2>((size_t)mp->nglob);
