@@ -11,9 +11,9 @@ __device__ __forceinline__ void atomic_add_f32(float* p, float v) { unsafeAtomic
 constexpr int NXCD = 8;  // gfx950: 8 accelerator complex dies, workgroups dispatched round-robin
 
 // Load through a 32-bit byte offset from a uniform base (global_load with saddr + voffset).  Within its reach are a field
-// and an element array of 4 bytes a point, below 4 GiB (checked when the handle is prepared); of the element arrays of 8
-// and 16 bytes a point, which are longer from 21.5 and 10.7 million elements on, what at_element reaches: the elements of
-// one chain, tower or patch.
+// and an element array of 4 bytes a point, below 4 GiB (checked when the handle is prepared).  The element arrays of 8 and
+// 16 bytes a point are longer from 21.5 and 10.7 million elements on: offsets into them count from at_element, the first
+// element of a chain, tower or patch, or the kernel is chosen only where they are short (tower_geometry, shot_minor_fits).
 template <typename T>
 __device__ __forceinline__ T ld_off(const T* base, unsigned byte_off) {
   return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
